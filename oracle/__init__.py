@@ -41,7 +41,7 @@ def build(force: bool = False) -> None:
     if force or not os.path.exists(_LIB_PATH):
         subprocess.run(["make", "-C", _HERE, "-B" if force else "-s", "liborc.so"], check=True,
                        stdout=subprocess.DEVNULL)
-    if os.path.isdir(REFERENCE_DIR) and (force or not os.path.exists(_REF_RPOLY_PATH)):
+    if os.path.exists(os.path.join(REFERENCE_DIR, "src", "rpoly.h")) and (force or not os.path.exists(_REF_RPOLY_PATH)):
         subprocess.run(["make", "-C", _HERE, "-B" if force else "-s", "ref"], check=True,
                        stdout=subprocess.DEVNULL)
 
