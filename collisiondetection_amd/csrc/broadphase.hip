@@ -4,23 +4,20 @@
 // The reference builds a top-down median-split tree of 13-axis swept k-DOPs and traverses it against
 // itself.  Its output does not depend on the tree's shape (interior bounds are exact unions of child
 // bounds, KDOPBroadPhase.cpp:85-98, so a leaf pair is visited iff its two leaf bounds overlap), so this
-// file builds a linear BVH instead:
+// file sorts the leaves along a Morton curve and searches 64-wide levels of boxes over that order:
 //   1. leaf bounds: per face, 13 axes x (3 vertices x history entries), min/max of pos.axis -/+ eta in
-//      FP64 exactly as KDOPBroadPhase.cpp:60-70 (bit-identical), plus an FP32 copy rounded outward;
-//   2. 63-bit Morton codes of the leaf centres, radix-sorted (rocPRIM);
-//   3. Karras' binary radix tree over the sorted codes (index tie-break for equal codes);
-//   4. bottom-up refit of FP32 interior bounds with one atomic arrival counter per node;
-//   5. escape ("rope") links: in the Karras layout the node after the subtree of a node covering
-//      leaves [l, r] is internal node r+1 when that node's range starts at r+1, else leaf r+1;
-//   6. stackless traversal, one lane per leaf i, starting at leaf i's escape link, which visits
-//      exactly the subtrees holding leaves after i: every unordered face pair is found once.  The FP32
-//      test culls; the leaf-leaf decision is the reference's FP64 13-axis test (touching overlaps)
-//      followed by the shared-vertex test (Mesh.cpp:13-20).  Pairs are queued per lane in registers
-//      and written in wavefront-wide flushes (one atomic each);
-//   7. expansion of each face pair into its 6 vertex-face and 9 edge-edge stencils
+//      FP64 exactly as KDOPBroadPhase.cpp:60-70 (bit-identical);
+//   2. 63-bit Morton codes of the leaf centres, radix-sorted (devprims.hip);
+//   3. box records quantised to 16 bits per bound: one per leaf, one per 64 leaves (a cluster), one per
+//      64 clusters, and so on: the width of a wavefront;
+//   4. the pair search: one wavefront per cluster finds the clusters its box meets, 64 box tests at a
+//      time, and tests each as a 64 x 64 tile of leaves.  The quantised test culls; the leaf-leaf
+//      decision is the reference's FP64 13-axis test (touching overlaps) and the shared-vertex test
+//      (Mesh.cpp:13-20), run on full wavefronts from a queue in LDS;
+//   5. expansion of each face pair into its 6 vertex-face and 9 edge-edge stencils
 //      (KDOPBroadPhase.cpp:150-184) with owner-computes deduplication: a stencil is written only by
 //      the smallest face pair that generates it, which is decided from the face -> related faces table
-//      built from the traversal's pairs (rows sorted; one wavefront per face) and the vertex->face
+//      built from the search's pairs (rows sorted; one wavefront per face) and the vertex->face
 //      table, so the unique set comes out with no global sort.
 // Meshes with degenerate faces (a repeated vertex) or duplicate faces break the owner rule's
 // assumptions; for them the raw stencils are emitted and deduplicated by sorting.
@@ -35,7 +32,6 @@ namespace {
 
 constexpr int KAX = 13;
 constexpr int NB = 2 * KAX;   // bounds per node: 13 mins then 13 maxs
-constexpr uint32_t NIL = 0xffffffffu;
 
 struct Axes {
     double a[KAX][3];
@@ -269,83 +265,82 @@ __global__ __launch_bounds__(256) void k_face_instance(const int64_t *__restrict
 }
 
 // ------------------------------------------------------------------------------------------------
-// 3. Karras binary radix tree.  Internal nodes 0..F-2, leaf j is node F-1+j.
+// 3. Leaf, cluster and group records
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ int delta(const uint64_t *__restrict__ k, int64_t F, int64_t i, int64_t j)
-{
-    if (j < 0 || j >= F) return -1;
-    uint64_t a = k[i], b = k[j];
-    if (a == b) return 64 + __clz((uint32_t)(i ^ j));
-    return __clzll(a ^ b);
-}
-
-__global__ __launch_bounds__(256) void k_karras(const uint64_t *__restrict__ keys, int64_t F,
-                                                uint32_t *__restrict__ left, uint32_t *__restrict__ rng_first,
-                                                uint32_t *__restrict__ rng_last, uint32_t *__restrict__ parent)
-{
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= F - 1) return;
-    int d = (delta(keys, F, i, i + 1) - delta(keys, F, i, i - 1)) >= 0 ? 1 : -1;
-    int dmin = delta(keys, F, i, i - d);
-    int64_t lmax = 2;
-    while (delta(keys, F, i, i + lmax * d) > dmin) lmax *= 2;
-    int64_t l = 0;
-    for (int64_t t = lmax / 2; t >= 1; t /= 2)
-        if (delta(keys, F, i, i + (l + t) * d) > dmin) l += t;
-    int64_t j = i + l * d;
-    int dnode = delta(keys, F, i, j);
-    int64_t s = 0;
-    int64_t t = l;
-    do {
-        t = (t + 1) >> 1;
-        if (delta(keys, F, i, i + (s + t) * d) > dnode) s += t;
-    } while (t > 1);
-    int64_t gamma = i + s * d + (d < 0 ? -1 : 0);
-    int64_t lo = i < j ? i : j, hi = i < j ? j : i;
-    uint32_t lc = (lo == gamma) ? (uint32_t)(F - 1 + gamma) : (uint32_t)gamma;
-    uint32_t rc = (hi == gamma + 1) ? (uint32_t)(F - 1 + gamma + 1) : (uint32_t)(gamma + 1);
-    left[i] = lc;
-    rng_first[i] = (uint32_t)lo;
-    rng_last[i] = (uint32_t)hi;
-    parent[lc] = (uint32_t)i;
-    parent[rc] = (uint32_t)i;
-    // The right child is found from the left: it follows the left child's subtree.
-}
-
-// Escape link of every node (internal and leaf) from the ranges.
-__global__ __launch_bounds__(256) void k_escape(const uint32_t *__restrict__ rng_first,
-                                                const uint32_t *__restrict__ rng_last, int64_t F,
-                                                uint32_t *__restrict__ escape)
-{
-    int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (n >= 2 * F - 1) return;
-    int64_t r = n < F - 1 ? (int64_t)rng_last[n] : n - (F - 1);
-    uint32_t e;
-    if (r == F - 1)
-        e = NIL;
-    else if (r + 1 <= F - 2 && (int64_t)rng_first[r + 1] == r + 1)
-        e = (uint32_t)(r + 1);
-    else
-        e = (uint32_t)(F - 1 + r + 1);
-    escape[n] = e;
-}
-
-// Node record used by the traversal: 26 bounds quantised to 16 bits, then the first child (internal)
-// or the sorted leaf index (leaf), then the escape link: 60 bytes, one 64-byte line (112 with FP32
-// bounds; the traversal is bound by fetching node records, so their size is its cost).
+// A record holds a box's 26 bounds quantised to 16 bits, two axes to a 32-bit word: lo[w] has the lower
+// bounds of axes 2w (low half) and 2w + 1, hi[w] the upper ones; the 14th slot is a padding axis that
+// separates nothing (lo 0, hi 65535).  Two boxes are disjoint on some axis exactly when a saturating
+// subtraction a.lo - b.hi or b.lo - a.hi leaves a nonzero half, so a box test is 14 packed
+// subtractions.  64 consecutive sorted leaves form a cluster (level 1), 64 clusters a group (level 2),
+// 64 groups a level-3 record; each record is the union of its children.
 //
 // Quantisation.  Per axis, a bound v maps to x = (v - origin) * inv, with origin the smallest finite
 // lower bound of all leaves and inv = 65535 / (largest finite upper bound - origin); lower bounds take
 // floor(x), upper bounds ceil(x), both clamped to [0, 65535], NaN to the full range.  Correctly rounded
 // subtraction and multiplication are monotone, and so are floor, ceil and the clamps, so overlapping
 // boxes keep overlapping (a.hi >= b.lo gives q(a.hi) >= q(b.lo)): the quantised test only ever keeps
-// more, and the FP64 leaf test decides.  Values outside the range (a refit whose mesh moved) clamp,
-// which stays conservative.
-struct __align__(16) NodeRec {
-    uint16_t b[NB];
-    uint32_t child;
-    uint32_t esc;
+// more, and the FP64 leaf test decides.  Values outside the range clamp, which stays conservative.
+constexpr int NWORD = 7;   // 32-bit words per side of a box
+struct __align__(16) BoxRec {
+    uint32_t lo[NWORD];
+    uint32_t hi[NWORD];
+    uint32_t face;   // a leaf's face id (0 at the upper levels)
+    uint32_t pad;
 };
+static_assert(sizeof(BoxRec) == 64, "box records are 64 bytes");
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2 as_halves(uint32_t x) { return __builtin_bit_cast(u16x2, x); }
+__device__ __forceinline__ uint32_t as_word(u16x2 x) { return __builtin_bit_cast(uint32_t, x); }
+// The halves of a that exceed those of b, as a nonzero value.
+__device__ __forceinline__ uint32_t exceeds(uint32_t a, uint32_t b)
+{
+    return as_word(__builtin_elementwise_sub_sat(as_halves(a), as_halves(b)));
+}
+__device__ __forceinline__ uint32_t halves_min(uint32_t a, uint32_t b)
+{
+    return as_word(__builtin_elementwise_min(as_halves(a), as_halves(b)));
+}
+__device__ __forceinline__ uint32_t halves_max(uint32_t a, uint32_t b)
+{
+    return as_word(__builtin_elementwise_max(as_halves(a), as_halves(b)));
+}
+struct Box16 {
+    uint32_t lo[NWORD], hi[NWORD];
+};
+__device__ __forceinline__ void load_box(const BoxRec *__restrict__ recs, int64_t n, Box16 &b)
+{
+    const uint4 *p = reinterpret_cast<const uint4 *>(recs + n);
+    const uint4 w0 = p[0], w1 = p[1], w2 = p[2], w3 = p[3];
+    b.lo[0] = w0.x, b.lo[1] = w0.y, b.lo[2] = w0.z, b.lo[3] = w0.w, b.lo[4] = w1.x, b.lo[5] = w1.y, b.lo[6] = w1.z;
+    b.hi[0] = w1.w, b.hi[1] = w2.x, b.hi[2] = w2.y, b.hi[3] = w2.z, b.hi[4] = w2.w, b.hi[5] = w3.x, b.hi[6] = w3.y;
+}
+__device__ __forceinline__ bool boxes_meet(const Box16 &a, const Box16 &b)
+{
+    uint32_t sep = 0;
+#pragma unroll
+    for (int w = 0; w < NWORD; w++) sep |= exceeds(a.lo[w], b.hi[w]) | exceeds(b.lo[w], a.hi[w]);
+    return sep == 0;
+}
+// The union of the 64 lanes' boxes, in every lane.
+__device__ __forceinline__ void wave_union(Box16 &b)
+{
+#pragma unroll
+    for (int w = 0; w < NWORD; w++) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            b.lo[w] = halves_min(b.lo[w], __shfl_xor(b.lo[w], d));
+            b.hi[w] = halves_max(b.hi[w], __shfl_xor(b.hi[w], d));
+        }
+    }
+}
+__device__ __forceinline__ void store_box(BoxRec *__restrict__ recs, int64_t n, const Box16 &b, uint32_t face)
+{
+    uint4 *p = reinterpret_cast<uint4 *>(recs + n);
+    p[0] = make_uint4(b.lo[0], b.lo[1], b.lo[2], b.lo[3]);
+    p[1] = make_uint4(b.lo[4], b.lo[5], b.lo[6], b.hi[0]);
+    p[2] = make_uint4(b.hi[1], b.hi[2], b.hi[3], b.hi[4]);
+    p[3] = make_uint4(b.hi[5], b.hi[6], face, 0u);
+}
 constexpr double QMAX = 65535.0;
 __device__ __forceinline__ uint16_t quant_lo(double v, double o, double inv)
 {
@@ -433,13 +428,13 @@ __global__ __launch_bounds__(64) void k_qrange_final(const double *__restrict__ 
     qparam[KAX + k] = ok ? QMAX / ext : 0.0;
 }
 
-// Leaf records in sorted order, and the FP64 bounds and vertex triples in sorted order.
+// Leaf records in sorted order with the record of each wavefront's cluster, and the FP64 bounds and
+// vertex triples in sorted order.
 __global__ __launch_bounds__(256) void k_leaf_records(const int32_t *__restrict__ order,
                                                       const double *__restrict__ dop64,
                                                       const int32_t *__restrict__ faces, int64_t F,
-                                                      const uint32_t *__restrict__ escape,
-                                                      const double *__restrict__ qparam,
-                                                      NodeRec *__restrict__ nodes, double *__restrict__ sdop64,
+                                                      const double *__restrict__ qparam, BoxRec *__restrict__ leaves,
+                                                      BoxRec *__restrict__ clusters, double *__restrict__ sdop64,
                                                       int4 *__restrict__ sfaces, int32_t *__restrict__ rank)
 {
     const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -456,139 +451,52 @@ __global__ __launch_bounds__(256) void k_leaf_records(const int32_t *__restrict_
         const int64_t fr = __shfl(f, rr);
         if (rr < nrow) sdop64[NB * j0 + e] = dop64[NB * fr + c];
     }
-    if (!active) return;
-    rank[f] = (int32_t)j;
-    const double *src = dop64 + NB * f;
-    NodeRec r;
+    Box16 r;
 #pragma unroll
-    for (int k = 0; k < KAX; k++) {
-        r.b[k] = quant_lo(src[k], qparam[k], qparam[KAX + k]);
-        r.b[KAX + k] = quant_hi(src[KAX + k], qparam[k], qparam[KAX + k]);
+    for (int w = 0; w < NWORD; w++) {   // the empty box: neutral in the cluster's union
+        r.lo[w] = 0xffffffffu;
+        r.hi[w] = 0u;
     }
-    r.child = (uint32_t)j;
-    r.esc = escape[F - 1 + j];
-    nodes[F - 1 + j] = r;
-    sfaces[j] = make_int4(faces[3 * f], faces[3 * f + 1], faces[3 * f + 2], (int)f);
-}
-
-// 4. Bottom-up refit: a lane per leaf climbs while it is the second child to arrive at a node.
-__global__ __launch_bounds__(256) void k_refit(int64_t F, const uint32_t *__restrict__ parent,
-                                               const uint32_t *__restrict__ left, const uint32_t *__restrict__ escape,
-                                               NodeRec *nodes, unsigned int *arrivals)
-{
-    int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (j >= F) return;
-    uint32_t node = parent[F - 1 + j];
-    while (true) {
-        __threadfence();   // release this lane's child bounds before announcing the arrival
-        unsigned int prior = atomicAdd(&arrivals[node], 1u);
-        if (prior == 0) return;   // the sibling subtree is not finished yet; its lane continues
-        __threadfence();          // acquire the sibling's bounds
-        uint32_t lc = left[node];
-        // The right child is the node after the left child's subtree, i.e. its escape link.
-        uint32_t rc = escape[lc];
-        NodeRec a = nodes[lc];
-        NodeRec b = nodes[rc];
-        NodeRec r;
+    if (active) {
+        const double *src = dop64 + NB * f;
 #pragma unroll
-        for (int k = 0; k < KAX; k++) {
-            r.b[k] = a.b[k] < b.b[k] ? a.b[k] : b.b[k];
-            r.b[KAX + k] = a.b[KAX + k] > b.b[KAX + k] ? a.b[KAX + k] : b.b[KAX + k];
+        for (int w = 0; w < NWORD; w++) {
+            const int k = 2 * w;
+            uint32_t lo = quant_lo(src[k], qparam[k], qparam[KAX + k]);
+            uint32_t hi = quant_hi(src[KAX + k], qparam[k], qparam[KAX + k]);
+            if (k + 1 < KAX) {
+                lo |= (uint32_t)quant_lo(src[k + 1], qparam[k + 1], qparam[KAX + k + 1]) << 16;
+                hi |= (uint32_t)quant_hi(src[KAX + k + 1], qparam[k + 1], qparam[KAX + k + 1]) << 16;
+            } else {
+                hi |= 0xffff0000u;   // the padding axis
+            }
+            r.lo[w] = lo;
+            r.hi[w] = hi;
         }
-        r.child = lc;
-        r.esc = escape[node];
-        nodes[node] = r;
-        if (node == 0) return;
-        node = parent[node];
+        store_box(leaves, j, r, (uint32_t)f);
+        rank[f] = (int32_t)j;
+        sfaces[j] = make_int4(faces[3 * f], faces[3 * f + 1], faces[3 * f + 2], (int)f);
     }
+    wave_union(r);
+    if (lane == 0) store_box(clusters, j0 >> 6, r, 0u);
 }
 
-// Level-synchronous refit for large trees.  The arrival-counter refit above needs a device-wide fence
-// per node, which writes back and invalidates the L2 of the lane's XCD; with millions of nodes those
-// fences serialise.  Instead each internal node's depth is found once per build by pointer jumping
-// over the parent links (8 rounds: exact up to depth 256, and a Karras tree over 63-bit keys with an
-// index tie-break is at most 97 deep, one level per distinct split bit), and the refit then runs one
-// launch per depth, deepest first: a kernel boundary orders each level's writes before the next
-// level's reads, with no fence inside.  Launches for depths past the tree's maximum return at once.
-constexpr int MAX_TREE_DEPTH = 128;
-constexpr int DEPTH_ROUNDS = 8;
-constexpr int64_t LEVEL_REFIT_MIN_FACES = 1 << 16;
-
-__global__ __launch_bounds__(256) void k_depth_init(int64_t F, const uint32_t *__restrict__ parent,
-                                                    uint32_t *__restrict__ jump, uint32_t *__restrict__ dist,
-                                                    uint32_t *__restrict__ maxd)
+// The records one level up: each wavefront the union of 64 records.
+__global__ __launch_bounds__(256) void k_group_records(const BoxRec *__restrict__ in, int64_t n,
+                                                       BoxRec *__restrict__ out)
 {
-    int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (n == 0) *maxd = 0;
-    if (n >= F - 1) return;
-    jump[n] = n == 0 ? NIL : parent[n];
-    dist[n] = n == 0 ? 0u : 1u;
-}
-
-__global__ __launch_bounds__(256) void k_depth_jump(int64_t F, const uint32_t *__restrict__ jin,
-                                                    const uint32_t *__restrict__ din, uint32_t *__restrict__ jout,
-                                                    uint32_t *__restrict__ dout)
-{
-    int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (n >= F - 1) return;
-    const uint32_t j = jin[n];
-    if (j == NIL) {
-        jout[n] = NIL;
-        dout[n] = din[n];
-    } else {
-        jout[n] = jin[j];
-        dout[n] = din[n] + din[j];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_depth_max(int64_t F, const uint32_t *__restrict__ depth,
-                                                   uint32_t *__restrict__ maxd)
-{
-    uint32_t m = 0;
-    for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < F - 1; n += (int64_t)gridDim.x * blockDim.x)
-        m = depth[n] > m ? depth[n] : m;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-        const uint32_t o = __shfl_xor(m, d);
-        m = o > m ? o : m;
-    }
-    if (__lane_id() == 0) atomicMax(maxd, m);
-}
-
-__global__ __launch_bounds__(256) void k_refit_level(int64_t F, uint32_t level, const uint32_t *__restrict__ depth,
-                                                     const uint32_t *__restrict__ maxd,
-                                                     const uint32_t *__restrict__ left,
-                                                     const uint32_t *__restrict__ escape, NodeRec *__restrict__ nodes)
-{
-    if (level > *maxd) return;
-    for (int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; n < F - 1; n += (int64_t)gridDim.x * blockDim.x) {
-        if (depth[n] != level) continue;
-        const uint32_t lc = left[n];
-        const uint32_t rc = escape[lc];   // the node after the left child's subtree
-        const NodeRec a = nodes[lc];
-        const NodeRec b = nodes[rc];
-        NodeRec r;
-#pragma unroll
-        for (int k = 0; k < KAX; k++) {
-            r.b[k] = a.b[k] < b.b[k] ? a.b[k] : b.b[k];
-            r.b[KAX + k] = a.b[KAX + k] > b.b[KAX + k] ? a.b[KAX + k] : b.b[KAX + k];
-        }
-        r.child = lc;
-        r.esc = escape[n];
-        nodes[n] = r;
-    }
+    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int lane = __lane_id();
+    if (j - lane >= n) return;
+    Box16 r;
+    load_box(in, j < n ? j : n - 1, r);   // the last record again: the union does not change
+    wave_union(r);
+    if (lane == 0) store_box(out, j >> 6, r, 0u);
 }
 
 // ------------------------------------------------------------------------------------------------
-// 6. Traversal: unordered overlapping non-neighbouring face pairs.
+// 4. Unordered overlapping non-neighbouring face pairs
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ bool overlap16(const uint16_t *q, const uint16_t *b)
-{
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < KAX; k++) ok = ok && !(q[KAX + k] < b[k] || b[KAX + k] < q[k]);
-    return ok;
-}
 // KDOPBroadPhase.cpp:132-137: disjoint iff some axis separates them strictly.
 __device__ __forceinline__ bool overlap64(const double *__restrict__ a, const double *__restrict__ b)
 {
@@ -603,167 +511,233 @@ __device__ __forceinline__ bool neighbours(int4 a, int4 b)   // Mesh.cpp:13-20
            a.z == b.y || a.z == b.z;
 }
 
-// inst_end: for batched instances, the sorted index one past the query's instance (its faces are the
-// sorted range [inst_off[k], inst_off[k+1])), else null (one instance).  An escape link always leads
-// to a node whose first leaf is its index (internal) or its leaf number: once that reaches inst_end
-// the walk has left the instance's subtree and stops.
-// Pairs are queued per lane (QN face ids in registers) and written when some lane's queue is full or
-// the traversal ends: one atomic per wavefront and flush, positions by a wavefront prefix sum.  A
-// single counter claimed by every wavefront on every iteration that emits serialises the device.
-// The query's FP64 bounds are read from memory only for the leaves that pass the FP32 test, which
-// keeps the lane's registers to its FP32 bounds and its queue.
-constexpr int TRAVERSE_QN = 8;
-__device__ __forceinline__ void traverse_flush(int me, const int (&q)[TRAVERSE_QN], int n, int2 *__restrict__ pairs,
-                                               int64_t cap, unsigned long long *counter)
+// One wavefront finds the pairs of one cluster's 64 sorted leaves (one per lane) with the leaves that
+// follow them: it looks for the clusters its cluster's box meets, 64 records per step (one per lane),
+// and tests each such cluster as a 64 x 64 tile.  In a tile, each lane first tests its own leaf of the
+// target cluster against the query cluster's box; the leaves that pass are broadcast one by one
+// (readlane) and tested against all 64 queries at once.  So every step of the search decides 64 box tests
+// from one load, and no step waits for the one before it but for the ballot: a tree walk by one
+// wavefront is a chain of dependent record loads (1.05 ms on the 256^2 cloth, 25.6 ms on a 1024^2 sheet with
+// 64 leaves per wavefront; here 0.34 and 15.6 ms, and 0.05 instead of 0.48 ms on a 97^2 cloth).
+//
+// The pairs that pass are queued in LDS and finished 64 at a time, so that the FP64 test runs with full
+// wavefronts: the shared-vertex test (Mesh.cpp:13-20), then the reference's 13-axis test (touching
+// counts).  Where every axis overlaps by two quanta or more the FP64 bounds are not read: with
+// qhi = ceil(x) > x - and so x > qhi - 1 -, qlo = floor(y) and so y < qlo + 1, qhi - 1 >= qlo + 1 gives
+// x > y, and the map to x is monotone, so the FP64 bounds overlap as well (the clamps keep this: a
+// clamped qhi = 65535 has x >= 65535, a clamped qlo = 0 has y < 1, a NaN bound never separates, and
+// the other clamps fail the test).  Accepted pairs wait in LDS too; a claim on the output counter covers
+// several hundred (one counter claimed per 64 pairs would serialise the device).
+//
+// Small meshes have few clusters; `slices` wavefronts then share one, each taking every slices-th of the
+// target clusters.
+// For batched instances a query pairs only with leaves before its instance's end (face_inst /
+// inst_off; its faces are the sorted range [inst_off[k], inst_off[k + 1])).
+constexpr int PAIR_BLOCK = 256;
+constexpr int PAIR_QUEUE = 128;   // quantised hits waiting for the exact test (below 64 after a flush)
+constexpr int PAIR_OUT = 512;     // accepted pairs waiting to be written
+struct PairLds {
+    int2 queue[PAIR_QUEUE];   // (query lane, target leaf)
+    int2 out[PAIR_OUT];
+};
+
+// Orders a wavefront's LDS accesses (its own region; one wavefront's LDS instructions execute in order,
+// so this only stops the compiler from moving them across).
+__device__ __forceinline__ void wave_lds_order()
 {
-    const int lane = __lane_id();
-    int incl = n;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
-    }
-    const int total = __shfl(incl, 63);
-    unsigned long long base = 0;
-    if (lane == 0 && total) base = atomicAdd(counter, (unsigned long long)total);
-    base = __shfl(base, 0);
-    const int64_t pos = (int64_t)base + (incl - n);
-#pragma unroll
-    for (int k = 0; k < TRAVERSE_QN; k++) {
-        if (k < n && pos + k < cap) {
-            const int b = q[k];
-            pairs[pos + k] = me < b ? make_int2(me, b) : make_int2(b, me);
-        }
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Packet traversal: one wavefront walks the tree once for its 64 consecutive sorted leaves.  The walk
-// starts at the escape link of the wavefront's first leaf i0 (the subtrees holding the leaves after
-// i0, which hold every leaf any lane pairs with) and follows child links into a subtree when some
-// lane's query overlaps it and the subtree holds a leaf in that lane's range (after its own leaf,
-// before its instance's end), escape links otherwise, until it passes the last instance end of the
-// wavefront.  The node index is the same in every lane, so a node record is one scalar load for the
-// whole wavefront, where 64 lanes walking their own paths fetched up to 64 different records per
-// step.  A lane tests the leaves the walk reaches that overlap its query in the quantised bounds and
-// lie in its range; every pair in a lane's range whose FP64 boxes overlap is reached (the quantised
-// bounds of its leaf and of that leaf's ancestors contain the FP64 ones), so each lane finds exactly
-// the pairs of a walk of its own.
-// The FP64 leaf test issues all its loads together and evaluates every comparison (an early-exit
-// test waits for one load after another: per leaf, up to 26 memory latencies in a row).  Loading the
-// child and escape records of each node ahead of the test was measured slower (the extra registers
-// halve the resident wavefronts).
-struct NodeWords {
-    uint4 w[4];   // a NodeRec as four 16-byte words: bounds in w[0..3] (26 halves), child w[3].y, escape w[3].z
+struct PairOut {
+    int2 *__restrict__ pairs;
+    int64_t cap;
+    unsigned long long *counter;
 };
-static_assert(sizeof(NodeRec) == 64, "node records are 64 bytes");
-__device__ __forceinline__ void load_node(const uint4 *__restrict__ recs, uint32_t n, NodeWords &r)
+__device__ __forceinline__ void pairs_write(PairLds &L, int n, const PairOut &o)
 {
-    const uint4 *p = recs + 4 * (int64_t)n;
-#pragma unroll
-    for (int k = 0; k < 4; k++) r.w[k] = p[k];
+    const int lane = __lane_id();
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(o.counter, (unsigned long long)n);
+    base = __shfl(base, 0);
+    for (int k = lane; k < n; k += 64)
+        if ((int64_t)base + k < o.cap) o.pairs[base + k] = L.out[k];
 }
-// Bound k (0 <= k < 26) of a record: 16-bit half k % 2 of 32-bit word k / 2.
-__device__ __forceinline__ uint32_t node_bound(const NodeWords &r, int k)
+
+// Certainly overlapping: two quanta or more on every axis.
+__device__ __forceinline__ bool boxes_meet_surely(const Box16 &a, const Box16 &b)
 {
-    const int wd = k >> 1;
-    const uint4 v = r.w[wd >> 2];
-    const uint32_t x = (wd & 3) == 0 ? v.x : ((wd & 3) == 1 ? v.y : ((wd & 3) == 2 ? v.z : v.w));
-    return (k & 1) ? (x >> 16) : (x & 0xffffu);
-}
-// overlap64 with every comparison evaluated (no early exit: the loads issue together).
-__device__ __forceinline__ bool overlap64_all(const double *__restrict__ a, const double *__restrict__ b)
-{
-    double av[NB], bv[NB];
-#pragma unroll
-    for (int k = 0; k < NB; k++) {
-        av[k] = a[k];
-        bv[k] = b[k];
-    }
     bool ok = true;
 #pragma unroll
-    for (int k = 0; k < KAX; k++) ok = ok & !((av[KAX + k] < bv[k]) | (bv[KAX + k] < av[k]));
+    for (int k = 0; k < KAX; k++) {
+        const int sh = (k & 1) * 16, w = k >> 1;
+        const int al = (a.lo[w] >> sh) & 0xffff, ah = (a.hi[w] >> sh) & 0xffff;
+        const int bl = (b.lo[w] >> sh) & 0xffff, bh = (b.hi[w] >> sh) & 0xffff;
+        ok = ok & (ah - bl >= 2) & (bh - al >= 2);
+    }
+    return ok;
+}
+// overlap64 with every comparison evaluated (no early exit: the loads of a part issue together).  Two
+// parts: all 52 doubles at once would take 159 registers, three wavefronts per SIMD.
+__device__ __forceinline__ bool overlap64_all(const double *__restrict__ a, const double *__restrict__ b)
+{
+    bool ok = true;
+#pragma nounroll
+    for (int part = 0; part < KAX && ok; part += 7) {
+        double al[7], ah[7], bl[7], bh[7];
+#pragma unroll
+        for (int u = 0; u < 7; u++) {
+            const int k = part + u < KAX ? part + u : KAX - 1;
+            al[u] = a[k];
+            ah[u] = a[KAX + k];
+            bl[u] = b[k];
+            bh[u] = b[KAX + k];
+        }
+#pragma unroll
+        for (int u = 0; u < 7; u++) ok = ok & !((ah[u] < bl[u]) | (bh[u] < al[u]));
+    }
     return ok;
 }
 
-__global__ __launch_bounds__(256) void k_traverse(int64_t F, const NodeRec *__restrict__ nodes,
-                                                  const double *__restrict__ sdop64,
-                                                  const int4 *__restrict__ sfaces, const int32_t *__restrict__ face_inst,
-                                                  const int64_t *__restrict__ inst_off, int2 *__restrict__ pairs,
-                                                  int64_t cap, unsigned long long *counter)
+// The exact test of queue[from .. from + n), n <= 64; accepted pairs are appended to out.
+__device__ __forceinline__ void pairs_test(PairLds &L, int from, int n, int64_t i0, const BoxRec *__restrict__ leaves,
+                                           const double *__restrict__ sdop64, const int4 *__restrict__ sfaces, int &nout,
+                                           const PairOut &o)
 {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const int64_t i0 = blockIdx.x * (int64_t)blockDim.x + (threadIdx.x & ~63);   // the wavefront's first leaf
-    if (i0 >= F || F < 2) return;   // the whole wavefront (lane 0 included) is past the leaves
-    const uint4 *__restrict__ recs = reinterpret_cast<const uint4 *>(nodes);
-    const bool active = i < F;
-    uint32_t q16[NB];
-    const double *q64 = sdop64 + NB * (active ? i : 0);
-    int4 qf = make_int4(0, 0, 0, 0);
-    int64_t iend = 0;   // inactive lanes accept no leaf
-    {
-        NodeWords me;
-        load_node(recs, (uint32_t)(F - 1 + (active ? i : i0)), me);
-#pragma unroll
-        for (int k = 0; k < NB; k++) q16[k] = node_bound(me, k);
+    const int lane = __lane_id();
+    bool ok = lane < n;
+    int2 pr = make_int2(0, 0);
+    if (ok) {
+        const int2 e = L.queue[from + lane];
+        const int64_t i = i0 + e.x, j = e.y;
+        const int4 qf = sfaces[i], of = sfaces[j];
+        pr = qf.w < of.w ? make_int2(qf.w, of.w) : make_int2(of.w, qf.w);
+        ok = !neighbours(qf, of);
+        if (ok) {
+            Box16 a, b;
+            load_box(leaves, i, a);
+            load_box(leaves, j, b);
+            if (!boxes_meet_surely(a, b)) ok = overlap64_all(sdop64 + NB * i, sdop64 + NB * j);
+        }
     }
-    if (active) {
-        qf = sfaces[i];
-        iend = face_inst ? inst_off[face_inst[qf.w] + 1] : F;
+    const uint64_t m = __ballot(ok);
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    if (nout + __popcll(m) > PAIR_OUT) {
+        wave_lds_order();
+        pairs_write(L, nout, o);
+        wave_lds_order();
+        nout = 0;
     }
-    // The last instance end of the wavefront's lanes.
-    int64_t jmax = iend;
+    if (ok) L.out[nout + __popcll(m & lt)] = pr;
+    nout += __popcll(m);
+}
+
+struct PairLevels {
+    const BoxRec *rec[4];   // leaves, clusters, groups, level 3 (levels above `top` unused)
+    int64_t n[4];
+    int top;                // the level scanned from end to end
+};
+
+__global__ __launch_bounds__(PAIR_BLOCK) void k_pairs(PairLevels lv, int slices, const double *__restrict__ sdop64,
+                                                      const int4 *__restrict__ sfaces,
+                                                      const int32_t *__restrict__ face_inst,
+                                                      const int64_t *__restrict__ inst_off, PairOut o)
+{
+    __shared__ PairLds s_lds[PAIR_BLOCK / 64];
+    PairLds &L = s_lds[threadIdx.x >> 6];
+    const int lane = __lane_id();
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const int F = (int)lv.n[0];   // below 2^30
+    const int64_t wave = blockIdx.x * (int64_t)(PAIR_BLOCK / 64) + (threadIdx.x >> 6);
+    const int c = __builtin_amdgcn_readfirstlane((int)(wave / slices));   // the query cluster
+    const int slice = __builtin_amdgcn_readfirstlane((int)(wave % slices));
+    if (c >= lv.n[1]) return;   // the whole wavefront
+    const BoxRec *__restrict__ leaves = lv.rec[0];
+    const int i0 = c * 64, i = i0 + lane;
+    Box16 q, cb;
+    load_box(leaves, i < F ? i : F - 1, q);
+    load_box(lv.rec[1], c, cb);
+    int iend = 0;   // lanes past the leaves accept none
+    if (i < F) iend = face_inst ? (int)inst_off[face_inst[sfaces[i].w] + 1] : F;
+    int jmax = iend;
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) {
-        const int64_t o = __shfl_xor(jmax, d);
-        jmax = o > jmax ? o : jmax;
+        const int x = __shfl_xor(jmax, d);
+        jmax = x > jmax ? x : jmax;
     }
-    const uint32_t nint = (uint32_t)(F - 1);
-    // The walk: node (uniform), its record, and the first leaf of its subtree.
-    uint32_t node = nodes[F - 1 + i0].esc;
-    int64_t fl = i0 + 1;
-    if (fl >= jmax) node = NIL;
-    node = __builtin_amdgcn_readfirstlane(node);
-    NodeWords cur;
-    if (node != NIL) load_node(recs, node, cur);
-    int q[TRAVERSE_QN] = {};
-    int nq = 0;
-    while (node != NIL) {
-        const uint32_t child = __builtin_amdgcn_readfirstlane(cur.w[3].y);
-        const uint32_t esc = __builtin_amdgcn_readfirstlane(cur.w[3].z);
-        const bool internal = node < nint;
-        // The subtree's leaves are [fl, r1): r1 is the first leaf of the node after it.
-        const int64_t r1 = esc == NIL ? F : (esc < nint ? (int64_t)esc : (int64_t)(esc - nint));
-        bool ov = true;
+    jmax = __builtin_amdgcn_readfirstlane(jmax);
+    const int tlast = (jmax - 1) >> 6;   // the last cluster any lane pairs with (jmax > i0 >= 0)
+    int nq = 0, nout = 0, turn = 0;
+
+    auto tile = [&](int t) {
+        const int j = t * 64 + lane;
+        Box16 b;
+        load_box(leaves, j < F ? j : F - 1, b);
+        for (uint64_t m = __ballot(j < jmax && boxes_meet(b, cb)); m; m &= m - 1) {
+            const int s = __ffsll((unsigned long long)m) - 1;
+            const int js = t * 64 + s;
+            uint32_t sep = 0;
 #pragma unroll
-        for (int k = 0; k < KAX; k++)
-            ov = ov & !((q16[KAX + k] < node_bound(cur, k)) | (node_bound(cur, KAX + k) < q16[k]));
-        const bool lane_ok = (r1 - 1 > i) & (fl < iend) & ov;
-        bool descend = false;
-        if (internal) {
-            descend = __ballot(lane_ok) != 0;
-        } else if (lane_ok) {
-            // leaf: child is its sorted index (== fl)
-            const int4 of = sfaces[child];
-            if (overlap64_all(q64, sdop64 + NB * (int64_t)child) && !neighbours(qf, of)) {
-#pragma unroll
-                for (int k = 0; k < TRAVERSE_QN; k++)
-                    if (k == nq) q[k] = of.w;
-                nq++;
+            for (int w = 0; w < NWORD; w++) {
+                const uint32_t tlo = __builtin_amdgcn_readlane(b.lo[w], s), thi = __builtin_amdgcn_readlane(b.hi[w], s);
+                sep |= exceeds(tlo, q.hi[w]) | exceeds(q.lo[w], thi);
+            }
+            const bool hit = (sep == 0) & (js > i) & (js < iend);
+            const uint64_t h = __ballot(hit);
+            if (h == 0) continue;
+            if (hit) L.queue[nq + __popcll(h & lt)] = make_int2(lane, js);
+            nq += __popcll(h);
+            if (nq >= 64) {
+                wave_lds_order();
+                pairs_test(L, nq - 64, 64, i0, leaves, sdop64, sfaces, nout, o);
+                wave_lds_order();
+                nq -= 64;
             }
         }
-        if (descend) {
-            node = child;   // the left child: its subtree starts at the same leaf
-            load_node(recs, node, cur);
-        } else {
-            node = esc;
-            fl = r1;
-            if (fl >= jmax) node = NIL;
-            if (node != NIL) load_node(recs, node, cur);
+    };
+    // The clusters of the 64 records [base, base + 64) of level 1 that the query cluster's box meets.
+    auto scan1 = [&](int base) {
+        const int t = base + lane;
+        Box16 b;
+        load_box(lv.rec[1], t < lv.n[1] ? t : lv.n[1] - 1, b);
+        for (uint64_t m = __ballot(t >= c && t <= tlast && boxes_meet(b, cb)); m; m &= m - 1) {
+            const int tt = base + __ffsll((unsigned long long)m) - 1;
+            if (turn == slice) tile(tt);
+            turn = turn + 1 == slices ? 0 : turn + 1;
         }
-        if (__ballot(nq == TRAVERSE_QN) || node == NIL) {
-            traverse_flush(qf.w, q, nq, pairs, cap, counter);
-            nq = 0;
-        }
+    };
+    auto scan2 = [&](int base) {
+        const int t = base + lane;
+        Box16 b;
+        load_box(lv.rec[2], t < lv.n[2] ? t : lv.n[2] - 1, b);
+        for (uint64_t m = __ballot(t >= (c >> 6) && t <= (tlast >> 6) && boxes_meet(b, cb)); m; m &= m - 1)
+            scan1((base + __ffsll((unsigned long long)m) - 1) << 6);
+    };
+    auto scan3 = [&](int base) {
+        const int t = base + lane;
+        Box16 b;
+        load_box(lv.rec[3], t < lv.n[3] ? t : lv.n[3] - 1, b);
+        for (uint64_t m = __ballot(t >= (c >> 12) && t <= (tlast >> 12) && boxes_meet(b, cb)); m; m &= m - 1)
+            scan2((base + __ffsll((unsigned long long)m) - 1) << 6);
+    };
+    const int up = 6 * (lv.top - 1);
+    const int last = tlast >> up;
+    for (int base = (c >> up) & ~63; base <= last; base += 64) {
+        if (lv.top == 1)
+            scan1(base);
+        else if (lv.top == 2)
+            scan2(base);
+        else
+            scan3(base);
+    }
+    if (nq) {
+        wave_lds_order();
+        pairs_test(L, 0, nq, i0, leaves, sdop64, sfaces, nout, o);
+    }
+    if (nout) {
+        wave_lds_order();
+        pairs_write(L, nout, o);
     }
 }
 
@@ -837,7 +811,7 @@ __global__ __launch_bounds__(256) void k_edge_opp(const int32_t *__restrict__ fa
 }
 
 // ------------------------------------------------------------------------------------------------
-// 7. Stencil expansion with owner-computes deduplication
+// 5. Stencil expansion with owner-computes deduplication
 // ------------------------------------------------------------------------------------------------
 struct MeshView {
     const int32_t *faces;
@@ -1620,8 +1594,7 @@ struct BPBufs {
     double *qpartial, *qparam;   // node quantisation: per-block partial ranges, origin[13] + inv[13]
     uint64_t *keys, *keys2;
     int32_t *vals, *order, *face_inst;
-    uint32_t *left, *rf, *rl, *parent, *escape, *arrivals;
-    NodeRec *nodes;
+    BoxRec *boxes;   // leaf records, then the levels above (level_offsets)
     int4 *sfaces;
     void *sort_tmp;
     int32_t *adj_cnt = nullptr, *adj_off = nullptr, *adj = nullptr;   // related-face table (null if too large)
@@ -1632,10 +1605,25 @@ struct BPBufs {
     int4 *vfk, *eek;
     int32_t *opp;    // edge -> opposite face, 3F (kept with the vertex -> face table for refits)
     int32_t *rank;   // face id -> Morton-sorted position
-    // level-synchronous refit (large trees): depth of every internal node, its pointer-jumping
-    // scratch, and the maximum depth
-    uint32_t *tdepth = nullptr, *tdepth2 = nullptr, *tjump = nullptr, *tjump2 = nullptr, *tmaxd = nullptr;
 };
+// Where each level's records start in BPBufs::boxes, and their number: level 0 the leaves, each level
+// above a 64th of the one below (rounded up).
+struct LevelOffsets {
+    int64_t at[4], n[4], total;
+};
+static LevelOffsets level_offsets(int64_t F)
+{
+    LevelOffsets l;
+    int64_t at = 0, n = F;
+    for (int k = 0; k < 4; k++) {
+        l.at[k] = at;
+        l.n[k] = n;
+        at += n;
+        n = (n + 63) >> 6;
+    }
+    l.total = at;
+    return l;
+}
 constexpr int NPARTS = 512;
 constexpr int QPARTS = 4096;   // blocks of the quantisation range pass (enough to fill the GPU)
 
@@ -1651,13 +1639,7 @@ static int bp_buffers(ccd_ctx *ctx, int64_t F, int64_t V, bool batched, BPBufs &
     b.vals = (int32_t *)buffer(ctx, "mvals", (size_t)F * 4);
     b.order = (int32_t *)buffer(ctx, "order", (size_t)F * 4);
     b.face_inst = batched ? (int32_t *)buffer(ctx, "face_inst", (size_t)F * 4) : nullptr;
-    b.left = (uint32_t *)buffer(ctx, "left", (size_t)F * 4);
-    b.rf = (uint32_t *)buffer(ctx, "rfirst", (size_t)F * 4);
-    b.rl = (uint32_t *)buffer(ctx, "rlast", (size_t)F * 4);
-    b.parent = (uint32_t *)buffer(ctx, "parent", (size_t)(2 * F) * 4);
-    b.escape = (uint32_t *)buffer(ctx, "escape", (size_t)(2 * F) * 4);
-    b.arrivals = (uint32_t *)buffer(ctx, "arrivals", (size_t)F * 4);
-    b.nodes = (NodeRec *)buffer(ctx, "nodes", (size_t)(2 * F) * sizeof(NodeRec));
+    b.boxes = (BoxRec *)buffer(ctx, "boxes", (size_t)level_offsets(F).total * sizeof(BoxRec));
     b.sdop64 = (double *)buffer(ctx, "sdop64", (size_t)F * NB * 8);
     b.sfaces = (int4 *)buffer(ctx, "sfaces", (size_t)F * 16);
     b.sort_tmp = buffer(ctx, "radix_tmp", radix_sort_temp_bytes(F));
@@ -1666,14 +1648,6 @@ static int bp_buffers(ccd_ctx *ctx, int64_t F, int64_t V, bool batched, BPBufs &
     b.eek = (int4 *)buffer(ctx, "ee_keys", (size_t)ctx->cap_ee * 16);
     b.opp = (int32_t *)buffer(ctx, "edge_opp", (size_t)(3 * F + 1) * 4);
     b.rank = (int32_t *)buffer(ctx, "face_rank", (size_t)F * 4);
-    if (F >= LEVEL_REFIT_MIN_FACES) {
-        b.tdepth = (uint32_t *)buffer(ctx, "tree_depth", (size_t)F * 4);
-        b.tdepth2 = (uint32_t *)buffer(ctx, "tree_depth2", (size_t)F * 4);
-        b.tjump = (uint32_t *)buffer(ctx, "tree_jump", (size_t)F * 4);
-        b.tjump2 = (uint32_t *)buffer(ctx, "tree_jump2", (size_t)F * 4);
-        b.tmaxd = (uint32_t *)buffer(ctx, "tree_maxd", 256);
-        if (!b.tdepth || !b.tdepth2 || !b.tjump || !b.tjump2 || !b.tmaxd) return CCD_E_OOM;
-    }
     if (2 * ctx->cap_pairs < ((int64_t)1 << 31) - 1) {   // int32 row offsets
         b.adj_cnt = (int32_t *)buffer(ctx, "adj_cnt", (size_t)(F + 1) * 4);
         b.adj_off = (int32_t *)buffer(ctx, "adj_off", (size_t)(F + 1) * 4);
@@ -1686,8 +1660,7 @@ static int bp_buffers(ccd_ctx *ctx, int64_t F, int64_t V, bool batched, BPBufs &
             return CCD_E_OOM;
     }
     if (!b.dop64 || !b.centre || !b.partial || !b.qpartial || !b.qparam || !b.keys || !b.keys2 || !b.vals || !b.order ||
-        (batched && !b.face_inst) || !b.left || !b.rf || !b.rl || !b.parent || !b.escape || !b.arrivals ||
-        !b.nodes || !b.sdop64 || !b.sfaces || !b.sort_tmp || !b.pairs || !b.vfk || !b.eek || !b.opp || !b.rank)
+        (batched && !b.face_inst) || !b.boxes || !b.sdop64 || !b.sfaces || !b.sort_tmp || !b.pairs || !b.vfk || !b.eek || !b.opp || !b.rank)
         return CCD_E_OOM;
     return CCD_OK;
 }
@@ -1724,39 +1697,39 @@ static int launch_qrange(ccd_ctx *ctx, const BPBufs &b, int64_t F)
     return CCD_OK;
 }
 
-// Interior bounds of the tree from its leaf records: the arrival-counter refit for small trees, the
-// level-synchronous one for large trees (new_topology: the tree was just built, so its depths are
-// computed first; a refit of the same tree keeps them).
-static int refit_tree(ccd_ctx *ctx, const BPBufs &b, int64_t F, bool new_topology)
+// The box records of every level, and the pair search over them.  The search scans the lowest level of at
+// most SCAN_MAX records from end to end (64 records a step), and descends from there.
+constexpr int64_t SCAN_MAX = 2048;
+static int launch_boxes(ccd_ctx *ctx, const BPBufs &b, const int32_t *order, const int32_t *faces, int64_t F)
 {
-    hipStream_t st = ctx->stream;
-    if (F < LEVEL_REFIT_MIN_FACES) {
-        int rc = fill_u32(ctx, b.arrivals, F, 0);
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_refit, dim3(blocks_for(F, 256)), dim3(256), 0, st, F, b.parent, b.left, b.escape,
-                           b.nodes, b.arrivals);
-        CCD_LAUNCH_CHECK(ctx);
-        return CCD_OK;
-    }
-    const unsigned g = blocks_for(F - 1, 256);
-    if (new_topology) {
-        hipLaunchKernelGGL(k_depth_init, dim3(g), dim3(256), 0, st, F, b.parent, b.tjump, b.tdepth, b.tmaxd);
-        CCD_LAUNCH_CHECK(ctx);
-        for (int r = 0; r < DEPTH_ROUNDS; r++) {   // an even count: the result ends in (tjump, tdepth)
-            const bool even = (r & 1) == 0;
-            hipLaunchKernelGGL(k_depth_jump, dim3(g), dim3(256), 0, st, F, even ? b.tjump : b.tjump2,
-                               even ? b.tdepth : b.tdepth2, even ? b.tjump2 : b.tjump, even ? b.tdepth2 : b.tdepth);
-            CCD_LAUNCH_CHECK(ctx);
-        }
-        hipLaunchKernelGGL(k_depth_max, dim3(std::min<unsigned>(g, 1024)), dim3(256), 0, st, F, b.tdepth, b.tmaxd);
+    const LevelOffsets l = level_offsets(F);
+    hipLaunchKernelGGL(k_leaf_records, dim3(blocks_for(F, 256)), dim3(256), 0, ctx->stream, order, b.dop64, faces, F,
+                       b.qparam, b.boxes, b.boxes + l.at[1], b.sdop64, b.sfaces, b.rank);
+    CCD_LAUNCH_CHECK(ctx);
+    for (int k = 1; k < 3 && l.n[k] > SCAN_MAX; k++) {
+        hipLaunchKernelGGL(k_group_records, dim3(blocks_for(l.n[k], 256)), dim3(256), 0, ctx->stream, b.boxes + l.at[k],
+                           l.n[k], b.boxes + l.at[k + 1]);
         CCD_LAUNCH_CHECK(ctx);
     }
-    const unsigned gl = std::min<unsigned>(g, 2048);
-    for (int level = MAX_TREE_DEPTH - 1; level >= 0; level--) {
-        hipLaunchKernelGGL(k_refit_level, dim3(gl), dim3(256), 0, st, F, (uint32_t)level, b.tdepth, b.tmaxd, b.left,
-                           b.escape, b.nodes);
-        CCD_LAUNCH_CHECK(ctx);
+    return CCD_OK;
+}
+static int launch_pairs(ccd_ctx *ctx, const BPBufs &b, int64_t F, const int64_t *inst_off)
+{
+    const LevelOffsets l = level_offsets(F);
+    PairLevels lv;
+    lv.top = 1;
+    for (int k = 0; k < 4; k++) {
+        lv.rec[k] = b.boxes + l.at[k];
+        lv.n[k] = l.n[k];
     }
+    while (lv.top < 3 && l.n[lv.top] > SCAN_MAX) lv.top++;
+    // Several wavefronts to a cluster while the clusters alone do not fill the chip.
+    const int64_t want = (int64_t)ctx->num_cus * 32;
+    const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(16, want / l.n[1]));
+    PairOut o{b.pairs, ctx->cap_pairs, (unsigned long long *)ctx->d_counts + C_PAIRS};
+    hipLaunchKernelGGL(k_pairs, dim3(blocks_for(l.n[1] * slices, PAIR_BLOCK / 64)), dim3(PAIR_BLOCK), 0, ctx->stream, lv,
+                       slices, b.sdop64, b.sfaces, b.face_inst, inst_off, o);
+    CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }
 
@@ -1846,23 +1819,14 @@ int broadphase_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const doubl
     bool in_alt = false;
     rc = radix_sort_pairs(ctx, b.keys, b.vals, b.keys2, b.order, F, 63, b.sort_tmp, in_alt);
     if (rc) return rc;
-    const uint64_t *skeys = in_alt ? b.keys2 : b.keys;
     const int32_t *order = in_alt ? b.order : b.vals;
     ctx->tree_order = order;
     prof_end(ctx, CCD_T_SORT);
 
     prof_begin(ctx, CCD_T_BUILD);
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(F - 1, 256)), dim3(256), 0, st, skeys, F, b.left, b.rf, b.rl,
-                       b.parent);
-    CCD_LAUNCH_CHECK(ctx);
-    hipLaunchKernelGGL(k_escape, dim3(blocks_for(2 * F - 1, 256)), dim3(256), 0, st, b.rf, b.rl, F, b.escape);
-    CCD_LAUNCH_CHECK(ctx);
     rc = launch_qrange(ctx, b, F);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_leaf_records, dim3(blocks_for(F, 256)), dim3(256), 0, st, order, b.dop64, faces, F,
-                       b.escape, b.qparam, b.nodes, b.sdop64, b.sfaces, b.rank);
-    CCD_LAUNCH_CHECK(ctx);
-    rc = refit_tree(ctx, b, F, true);
+    rc = launch_boxes(ctx, b, order, faces, F);
     if (rc) return rc;
     prof_end(ctx, CCD_T_BUILD);
 
@@ -1878,10 +1842,8 @@ int broadphase_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const doubl
     prof_end(ctx, CCD_T_TABLES);
 
     prof_begin(ctx, CCD_T_TRAVERSE);
-    hipLaunchKernelGGL(k_traverse, dim3(blocks_for(F, 256)), dim3(256), 0, st, F, b.nodes, b.sdop64, b.sfaces,
-                       batched ? b.face_inst : (const int32_t *)nullptr, inst_off, b.pairs, ctx->cap_pairs,
-                       c + C_PAIRS);
-    CCD_LAUNCH_CHECK(ctx);
+    rc = launch_pairs(ctx, b, F, inst_off);
+    if (rc) return rc;
     prof_end(ctx, CCD_T_TRAVERSE);
 
     prof_begin(ctx, CCD_T_EXPAND);
@@ -1899,16 +1861,15 @@ int broadphase_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const doubl
     return CCD_OK;
 }
 
-// Refit: the tree of the last full build on this context (same faces, same instance layout) with new
-// positions -- new leaf bounds and records, then the bottom-up refit; the Morton order, the radix tree,
-// the escape links and the vertex->face table are kept.  Candidate sets do not depend on the tree's
-// shape, so this is exact; only culling efficiency depends on how far the mesh moved since the build.
+// Refit: the sorted order of the last full build on this context (same faces, same instance layout) with
+// new positions -- new leaf bounds and records; the Morton order and the vertex->face table are kept.
+// Candidate sets do not depend on the order, so this is exact; only culling efficiency depends on how
+// far the mesh moved since the build.
 int broadphase_refit_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const double *qs, const double *qe,
                             int64_t V, double eta, const uint8_t *fixed, const int64_t *inst_off, int ninst)
 {
     hipStream_t st = ctx->stream;
     int64_t *cnt = ctx->d_counts;
-    unsigned long long *c = (unsigned long long *)cnt;
     int rc = fill_u64(ctx, (uint64_t *)cnt, NCOUNTERS, 0);
     if (rc) return rc;
     if (F < 2) return CCD_OK;
@@ -1925,19 +1886,14 @@ int broadphase_refit_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const
     prof_begin(ctx, CCD_T_BUILD);
     rc = launch_qrange(ctx, b, F);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_leaf_records, dim3(blocks_for(F, 256)), dim3(256), 0, st, ctx->tree_order, b.dop64, faces,
-                       F, b.escape, b.qparam, b.nodes, b.sdop64, b.sfaces, b.rank);
-    CCD_LAUNCH_CHECK(ctx);
-    rc = refit_tree(ctx, b, F, false);
+    rc = launch_boxes(ctx, b, ctx->tree_order, faces, F);
     if (rc) return rc;
     prof_end(ctx, CCD_T_BUILD);
     const int32_t *voff = nullptr, *vlist = nullptr;
     vertex_face_table(ctx, &voff, &vlist);
     prof_begin(ctx, CCD_T_TRAVERSE);
-    hipLaunchKernelGGL(k_traverse, dim3(blocks_for(F, 256)), dim3(256), 0, st, F, b.nodes, b.sdop64, b.sfaces,
-                       batched ? b.face_inst : (const int32_t *)nullptr, inst_off, b.pairs, ctx->cap_pairs,
-                       c + C_PAIRS);
-    CCD_LAUNCH_CHECK(ctx);
+    rc = launch_pairs(ctx, b, F, inst_off);
+    if (rc) return rc;
     prof_end(ctx, CCD_T_TRAVERSE);
     prof_begin(ctx, CCD_T_EXPAND);
     MeshView mv{faces, voff, vlist, b.dop64, fixed};
