@@ -1,4 +1,5 @@
 // C ABI of libccd_amd.so (declarations and contracts in include/ccd_amd.h).
+#include <algorithm>
 #include <cstdarg>
 #include <cstring>
 #include <mutex>
@@ -146,7 +147,7 @@ extern "C" {
 // only a stand-in for the symbol): it looks up each device's own address once, at set-up, and passes
 // that.  Layout for up to CCD_NOALLOC_MAX_STENCILS stencils (one stencil kind at a time):
 //   [0, 256)    the invalid-key counter (uint64)
-//   then sig, sig2 (uint64 per stencil), idx, idx2 (int32 per stencil), the radix sort's temporary.
+//   then the screening passes' lists (open_list_bytes).
 // ------------------------------------------------------------------------------------------------
 namespace {
 constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)26 << 20;
@@ -173,7 +174,6 @@ int scratch_address(int device, unsigned char **out)
     return CCD_OK;
 }
 
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 }   // namespace
 
 int ccd_create(ccd_ctx **out, int device)
@@ -315,20 +315,10 @@ int ccd_ctcd_narrowphase_noalloc(ccd_ctx *ctx, const double *qstart, const doubl
     unsigned char *base = nullptr;
     if (scratch_address(ctx->device, &base) != CCD_OK)
         return set_error(ctx, CCD_E_HIP, "no address for the device scratch array");
-    const size_t n = (size_t)CCD_NOALLOC_MAX_STENCILS;
-    OrderScratch os;
-    size_t o = 256;
-    os.sig = (uint64_t *)(base + o);
-    o = align256(o + 8 * n);
-    os.sig2 = (uint64_t *)(base + o);
-    o = align256(o + 8 * n);
-    os.idx = (int32_t *)(base + o);
-    o = align256(o + 4 * n);
-    os.idx2 = (int32_t *)(base + o);
-    o = align256(o + 4 * n);
-    os.tmp = base + o;
-    o += radix_sort_temp_bytes((int64_t)n);
-    if (o > NOALLOC_SCRATCH_BYTES) return set_error(ctx, CCD_E_INVALID, "scratch layout exceeds the array");
+    // The screening passes' lists, for one kind's stencils at a time.
+    void *list = base + 256;
+    if (256 + open_list_bytes(CCD_NOALLOC_MAX_STENCILS) > (int64_t)NOALLOC_SCRATCH_BYTES)
+        return set_error(ctx, CCD_E_INVALID, "scratch layout exceeds the array");
     // Key validation into the scratch counter (cleared by a fill kernel; the array keeps the last
     // call's contents), read back through the context's pinned mailbox.
     int64_t *bad = (int64_t *)base;
@@ -341,11 +331,10 @@ int ccd_ctcd_narrowphase_noalloc(ccd_ctx *ctx, const double *qstart, const doubl
     if (ctx->h_counts[C_BAD] != 0)
         return set_error(ctx, CCD_E_INVALID, "%lld stencil keys reference vertices outside [0, nverts)",
                          (long long)ctx->h_counts[C_BAD]);
-    // Both kinds reuse the same ordering buffers: the edge-edge launches follow the vertex-face ones on
-    // the stream.
-    rc = launch_narrow2(ctx, true, qstart, qend, vf_keys, vf_eta, eta_scalar, nvf, vf_hit, vf_t, vf_sub, &os);
+    // Both kinds reuse the same lists: the edge-edge launches follow the vertex-face ones on the stream.
+    rc = launch_narrow2(ctx, true, qstart, qend, vf_keys, vf_eta, eta_scalar, nvf, vf_hit, vf_t, vf_sub, list);
     if (rc) return rc;
-    return launch_narrow2(ctx, false, qstart, qend, ee_keys, ee_eta, eta_scalar, nee, ee_hit, ee_t, ee_sub, &os);
+    return launch_narrow2(ctx, false, qstart, qend, ee_keys, ee_eta, eta_scalar, nee, ee_hit, ee_t, ee_sub, list);
 }
 
 int ccd_ctcd_narrowphase_history(ccd_ctx *ctx, const int64_t *hist_off, const double *hist_t,
@@ -504,41 +493,27 @@ struct DetectArgs {
     int64_t ee_cap;
 };
 
-// The narrowphase half: counters reset by fill kernels, then the two persistent queue kernels.  Pure
-// launches (capturable).  n_max bounds the grids: the stencil counts are read on the device.
-// exact: nvf_max / nee_max are this call's stencil counts (the synchronous path), so the stencils can
-// be grouped by their vertex-edge signature first; the captured path passes capacities instead.
-static int narrow_launches(ccd_ctx *ctx, const DetectArgs &a, int64_t nvf_max, int64_t nee_max, bool exact)
+// The narrowphase half: counters reset by fill kernels, then each kind's passes.  Pure launches
+// (capturable).  n_max bounds the grids: the stencil counts are read on the device.  The two kinds share
+// the lists of the screening passes, one after the other on the stream.
+static int narrow_launches(ccd_ctx *ctx, const DetectArgs &a, int64_t nvf_max, int64_t nee_max)
 {
-    // work[0..1]: the two queues; work[2..3]: the edge-edge deferral list's counter and second queue.
-    unsigned long long *work = (unsigned long long *)buffer(ctx, "queue_work", 48);
+    unsigned long long *work = (unsigned long long *)buffer(ctx, "queue_work", 16);   // the one-pass form's queues
     if (!work) return CCD_E_OOM;
     int rc = fill_u64(ctx, (uint64_t *)(ctx->d_counts + C_VF_HITS), 2, 0);
-    if (!rc) rc = fill_u64(ctx, (uint64_t *)work, 4, 0);
+    if (!rc) rc = fill_u64(ctx, (uint64_t *)work, 2, 0);
     if (rc) return rc;
-    const EeDeferral def = ee_deferral(ctx, nee_max, work + 2);
-    const int32_t *vfk = (const int32_t *)ctx->bufs["vf_keys"].ptr;
-    const int32_t *eek = (const int32_t *)ctx->bufs["ee_keys"].ptr;
-    // The stage timers include the grouping.  Without exact host counts (a captured pipeline) the
-    // signature pass reads the device counts and sorts the unused capacity last.
-    const bool group_vf = ctx->group_stencils && ctx->vf_shape.group;
-    const bool group_ee = ctx->group_stencils && ctx->ee_shape.group;
+    void *list = open_list(ctx, std::min<int64_t>(std::max(nvf_max, nee_max), 0x7fffffffll));
     prof_begin(ctx, CCD_T_NARROW_VF);
-    if (group_vf) {
-        rc = group_by_signature(ctx, true, a.qs, a.qe, vfk, nvf_max, a.eta, exact ? nullptr : ctx->d_counts + C_VF, &vfk);
-        if (rc) return rc;
-    }
-    rc = launch_narrow2_queue(ctx, true, a.qs, a.qe, vfk, ctx->d_counts + C_VF, nvf_max, a.eta, a.vf_hits, a.vf_toi,
-                              a.vf_cap, ctx->d_counts + C_VF_HITS, work, ctx->vf_shape);
+    rc = launch_narrow2_queue(ctx, true, a.qs, a.qe, (const int32_t *)ctx->bufs["vf_keys"].ptr, ctx->d_counts + C_VF,
+                              nvf_max, a.eta, a.vf_hits, a.vf_toi, a.vf_cap, ctx->d_counts + C_VF_HITS, work,
+                              ctx->vf_shape, list);
     if (rc) return rc;
     prof_end(ctx, CCD_T_NARROW_VF);
     prof_begin(ctx, CCD_T_NARROW_EE);
-    if (group_ee) {
-        rc = group_by_signature(ctx, false, a.qs, a.qe, eek, nee_max, a.eta, exact ? nullptr : ctx->d_counts + C_EE, &eek);
-        if (rc) return rc;
-    }
-    rc = launch_narrow2_queue(ctx, false, a.qs, a.qe, eek, ctx->d_counts + C_EE, nee_max, a.eta, a.ee_hits, a.ee_toi,
-                              a.ee_cap, ctx->d_counts + C_EE_HITS, work + 1, ctx->ee_shape, &def);
+    rc = launch_narrow2_queue(ctx, false, a.qs, a.qe, (const int32_t *)ctx->bufs["ee_keys"].ptr, ctx->d_counts + C_EE,
+                              nee_max, a.eta, a.ee_hits, a.ee_toi, a.ee_cap, ctx->d_counts + C_EE_HITS, work + 1,
+                              ctx->ee_shape, ctx->ee_split ? list : nullptr);
     if (rc) return rc;
     prof_end(ctx, CCD_T_NARROW_EE);
     return CCD_OK;
@@ -555,7 +530,7 @@ static int detect_sync(ccd_ctx *ctx, const DetectArgs &a)
     ctx->last_ee = c.ee;
     ctx->last_nvf = c.nvf;
     ctx->last_nee = c.nee;
-    rc = narrow_launches(ctx, a, c.nvf, c.nee, true);
+    rc = narrow_launches(ctx, a, c.nvf, c.nee);
     if (rc) return rc;
     CCD_HIP_CHECK(ctx, hipMemcpyAsync(ctx->h_counts, ctx->d_counts, sizeof(int64_t) * NCOUNTERS, hipMemcpyDeviceToHost,
                                       ctx->stream));
@@ -612,15 +587,10 @@ static int detect_graph(ccd_ctx *ctx, const DetectArgs &a)
     memcpy(saved, ctx->h_counts, sizeof(saved));
     // Capture with the capacities the synchronous run settled on; buffers used inside the capture are
     // sized for them first (nothing can be allocated while capturing).
-    if (ctx->group_stencils && (ctx->vf_shape.group || ctx->ee_shape.group)) {
-        rc = reserve_grouping(ctx, ctx->cap_vf, ctx->cap_ee);
-        if (rc) return rc;
-    }
-    if (!buffer(ctx, "queue_work", 48)) return CCD_E_OOM;
-    if (ctx->ee_split && ctx->cap_ee <= 0x7fffffffll) {
-        const int64_t cd = ee_deferral_capacity(ctx, ctx->cap_ee);
-        if (!buffer(ctx, "ee_def_idx", (size_t)cd * 4) || !buffer(ctx, "ee_def_sub", (size_t)cd)) return CCD_E_OOM;
-    }
+    if (!buffer(ctx, "queue_work", 16)) return CCD_E_OOM;
+    if (std::max(ctx->cap_vf, ctx->cap_ee) > 0 &&
+        !open_list(ctx, std::min<int64_t>(std::max(ctx->cap_vf, ctx->cap_ee), 0x7fffffffll)))
+        return CCD_E_OOM;
     int64_t caps2[3] = {ctx->cap_pairs, ctx->cap_vf, ctx->cap_ee};
     memcpy(key + sizeof(DetectArgs), caps2, sizeof(caps2));
     ctx->capturing = true;
@@ -631,7 +601,7 @@ static int detect_graph(ccd_ctx *ctx, const DetectArgs &a)
     }
     rc = broadphase_launch(ctx, a.faces, a.F, a.qs, a.qe, nullptr, nullptr, a.V, a.outer_eta, a.fixed, false,
                            a.inst_off, (int)a.ninst);
-    if (!rc) rc = narrow_launches(ctx, a, ctx->cap_vf, ctx->cap_ee, false);
+    if (!rc) rc = narrow_launches(ctx, a, ctx->cap_vf, ctx->cap_ee);
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(ctx->stream, &g);
     ctx->capturing = false;
@@ -755,7 +725,7 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
     const int32_t *keys[2] = {ctx->last_vf, ctx->last_ee};
     int32_t *sink = (int32_t *)buffer(ctx, "tune_sink", 16 * 4096 + 64);
     double *sink_t = (double *)buffer(ctx, "tune_sink_t", 8 * 4096 + 64);
-    unsigned long long *work = (unsigned long long *)buffer(ctx, "tune_work", 32);   // queue; [2..3] deferral
+    unsigned long long *work = (unsigned long long *)buffer(ctx, "tune_work", 16);
     int64_t *cnt = (int64_t *)buffer(ctx, "tune_cnt", 16);
     int64_t *ndev = (int64_t *)buffer(ctx, "tune_n", 16);
     if (!sink || !sink_t || !work || !cnt || !ndev) return CCD_E_OOM;
@@ -774,15 +744,15 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
         }
         return CCD_OK;
     };
-    // Edge-edge shapes are timed as the pipeline runs them (two passes unless switched off).
-    const EeDeferral tdef = ee_deferral(ctx, nmax[1], work + 2);
+    // Shapes are timed as the pipeline runs them (edge-edge in one pass when that is switched off).
+    void *list = open_list(ctx, std::min<int64_t>(std::max(nmax[0], nmax[1]), 0x7fffffffll));
     auto queue = [&](int kind, const int32_t *k, const QueueShape &s) {
         return [&, kind, k, s]() -> int {
-            int rc = fill_u64(ctx, (uint64_t *)work, 4, 0);
+            int rc = fill_u64(ctx, (uint64_t *)work, 1, 0);
             if (!rc) rc = fill_u64(ctx, (uint64_t *)cnt, 1, 0);
             if (!rc)
                 rc = launch_narrow2_queue(ctx, kind == 0, qstart, qend, k, ndev, nmax[kind], eta, sink, sink_t, 0, cnt,
-                                          work, s, kind == 1 ? &tdef : nullptr);
+                                          work, s, kind == 0 || ctx->ee_split ? list : nullptr);
             return rc;
         };
     };
@@ -790,15 +760,6 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
     for (int kind = 0; kind < 2; kind++) {
         if (nmax[kind] == 0) continue;
         CCD_HIP_CHECK(ctx, hipMemcpyAsync(ndev, &nmax[kind], 8, hipMemcpyHostToDevice, st));
-        // The grouping as the pipeline runs it (signature pass, sort, gather), timed; the queue shapes
-        // on the grouped order; then the best shape on the stored order.  Grouping stays on only when
-        // it pays for itself.
-        const int32_t *grouped = keys[kind];
-        float t_group = 0.f;
-        int rc = timed(
-            [&]() { return group_by_signature(ctx, kind == 0, qstart, qend, keys[kind], nmax[kind], eta, nullptr, &grouped); },
-            t_group);
-        if (rc) return rc;
         float best_ms = 1e30f;
         for (int b : blocks)
             for (int t : tiles)
@@ -808,17 +769,13 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
                     s.tile = t;
                     s.waves_per_cu = w;
                     float ms = 0.f;
-                    rc = timed(queue(kind, grouped, s), ms);
+                    int rc = timed(queue(kind, keys[kind], s), ms);
                     if (rc) return rc;
                     if (ms < best_ms) {
                         best_ms = ms;
                         best[kind] = s;
                     }
                 }
-        float t_plain = 0.f;
-        rc = timed(queue(kind, keys[kind], best[kind]), t_plain);
-        if (rc) return rc;
-        best[kind].group = (grouped != keys[kind] && t_group + best_ms <= t_plain) ? 1 : 0;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);

@@ -101,6 +101,7 @@ CCD_FHD V3 mk(double x, double y, double z)
 }
 CCD_FHD V3 operator-(V3 a, V3 b) { return mk(a.x - b.x, a.y - b.y, a.z - b.z); }
 CCD_FHD V3 operator+(V3 a, V3 b) { return mk(a.x + b.x, a.y + b.y, a.z + b.z); }
+CCD_FHD V3 operator-(V3 a) { return mk(-a.x, -a.y, -a.z); }
 CCD_FHD V3 operator*(double s, V3 a) { return mk(s * a.x, s * a.y, s * a.z); }
 CCD_FHD double dot(V3 a, V3 b) { return (a.x * b.x + a.y * b.y) + a.z * b.z; }
 CCD_FHD V3 cross(V3 a, V3 b) { return mk(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x); }
@@ -1362,6 +1363,536 @@ CCD_HD int check_ee_window(const V3 *s, const V3 *e, double eta, double &t, C &&
     if (vertex_vertex(s[1], s[2], e[1], e[2], eta, t, cnt)) return 7;
     if (vertex_vertex(s[1], s[3], e[1], e[3], eta, t, cnt)) return 8;
     return -1;
+}
+
+// ------------------------------------------------------------------------------------------------
+// Screening.  screen_vf_window / screen_ee_window say which of a window's sub-tests may hit, without
+// solving, dividing or branching: a sub-test whose bit is clear returns false in the cascade above.  Most
+// stencils of a moving mesh come out with no bit set (97-100% vertex-face and 87-94% edge-edge on rigidly
+// moving instances and on crumpled sheets, half of both on a cloth whose noise is as large as its
+// edges), and only the rest need a root solver.
+//
+// Why a cleared sub-test is false.  Its answer needs a point of [0, 1] in an interval of each of its
+// lists, so one empty list decides it, in whichever order the lists are computed.  find_intervals
+// leaves a list empty when its polynomial has the rejected sign on all of [0, 1] by a margin far above
+// rounding: couldHaveRoots returns at once, or no root is isolated (every sign the isolator evaluates is
+// the same) or the closed forms' roots cut [0, 1] into pieces whose midpoints all have the rejected sign.
+// On [0, 1] a polynomial lies between the smallest and the largest of its Bernstein coefficients.
+//   * The polynomials are the cascade's own, coefficient for coefficient: dot(a, b) = dot(b, a) and
+//     dot(-a, b) = -dot(a, b) hold bit for bit, so the four barycentric quartics and the four
+//     vertex-edge tests of a stencil share their dot products (54 where they are written out with 144).
+//   * The margin, 2e-13 of the largest coefficient (plus 1e-300 against underflow), covers the rounding
+//     of the conversion (below 6e-15) and of normalising, evaluating and solving.
+//   * The coplanar-distance sextic is d(t)^2 - eta^2 |n(t)|^2 with d a cubic and n a quadratic vector,
+//     so it is positive when d's Bernstein coefficients have one sign and the smallest squared exceeds
+//     eta^2 times the largest |n|^2 of n's Bernstein vectors, by 1e-12 of the sum of the terms that the
+//     sextic's coefficients are made of (their rounding is below 1e-14 of it).
+//   * The vertex-vertex quadratic is evaluated on differences of positions, where the cascade expands
+//     |q1|^2 + |q2|^2 - 2 q1.q2: the two differ by the rounding of terms as large as the squared
+//     coordinates, below 2e-13 of 27 w^2 with w the largest coordinate; the margin is 4e-12 w^2.
+// Comparisons fail on NaN, and coordinates of 1e40 and more (whose products overflow) clear nothing.
+// ------------------------------------------------------------------------------------------------
+constexpr double SCREEN_TOL = 2e-13, SCREEN_TINY = 1e-300, SCREEN_MAX_COORD = 1e40;
+CCD_FHD double fmax2(double a, double b) { return __builtin_fmax(a, b); }
+CCD_FHD double fmin2(double a, double b) { return __builtin_fmin(a, b); }
+
+// The quadratic g(t) = c0 + c1 t + c2 t^2.
+struct Quad {
+    double c0, c1, c2;
+};
+CCD_FHD Quad operator-(Quad q) { return Quad{-q.c0, -q.c1, -q.c2}; }
+
+// A product of two moving vectors a + t va and b + t vb, in the cascade's order of operations.
+CCD_FHD Quad moving_dot(V3 a, V3 va, V3 b, V3 vb) { return Quad{dot(a, b), dot(a, vb) + dot(va, b), dot(va, vb)}; }
+CCD_FHD Quad moving_square(V3 a, V3 va) { return Quad{dot(a, a), 2 * dot(a, va), dot(va, va)}; }
+
+// g < 0 on [0, 1] by the margin.  (The largest of the coefficients ignores NaN; b2 holds every one.)
+CCD_FHD bool surely_negative(Quad q)
+{
+    const double tol = dfma(SCREEN_TOL, fmax2(fmax2(dabs(q.c0), dabs(q.c1)), dabs(q.c2)), SCREEN_TINY);
+    const double b1 = dfma(0.5, q.c1, q.c0), b2 = (q.c0 + q.c1) + q.c2;
+    return (fmax2(q.c0, b1) < -tol) & (b2 < -tol);
+}
+// op (descending powers, degree 4) < 0 on [0, 1] by the margin.
+CCD_FHD bool surely_negative4(double o0, double o1, double o2, double o3, double o4)
+{
+    const double m = fmax2(fmax2(fmax2(dabs(o0), dabs(o1)), fmax2(dabs(o2), dabs(o3))), dabs(o4));
+    const double tol = dfma(SCREEN_TOL, m, SCREEN_TINY);
+    const double b1 = dfma(0.25, o3, o4);
+    const double b2 = dfma(1.0 / 6.0, o2, dfma(0.5, o3, o4));
+    const double b3 = dfma(0.25, o1, dfma(0.5, o2, dfma(0.75, o3, o4)));
+    const double b4 = (((o4 + o3) + o2) + o1) + o0;
+    return (fmax2(fmax2(o4, b1), fmax2(b2, b3)) < -tol) & (b4 < -tol);
+}
+CCD_FHD bool surely_negative3(double o0, double o1, double o2, double o3)
+{
+    const double m = fmax2(fmax2(dabs(o0), dabs(o1)), fmax2(dabs(o2), dabs(o3)));
+    const double tol = dfma(SCREEN_TOL, m, SCREEN_TINY);
+    const double b1 = dfma(1.0 / 3.0, o2, o3);
+    const double b2 = dfma(1.0 / 3.0, o1, dfma(2.0 / 3.0, o2, o3));
+    const double b3 = ((o3 + o2) + o1) + o0;
+    return (fmax2(fmax2(o3, b1), b2) < -tol) & (b3 < -tol);
+}
+
+// A polynomial of degree D, coefficients in ascending powers.
+template <int D>
+struct Poly {
+    double c[D + 1];
+};
+CCD_FHD bool surely_negative(Poly<4> p) { return surely_negative4(p.c[4], p.c[3], p.c[2], p.c[1], p.c[0]); }
+CCD_FHD bool surely_negative(Poly<3> p) { return surely_negative3(p.c[3], p.c[2], p.c[1], p.c[0]); }
+
+// barycentric_poly's quartic from its quadratics: abc = x10.x10, def = x20.x10, ghi = x30.x20, jkl = x30.x10.
+CCD_FHD Poly<4> barycentric_quartic(Quad abc, Quad def, Quad ghi, Quad jkl)
+{
+    const double A = abc.c0, B = abc.c1, C = abc.c2, D = def.c0, E = def.c1, F = def.c2;
+    const double G = ghi.c0, H = ghi.c1, I = ghi.c2, J = jkl.c0, K = jkl.c1, L = jkl.c2;
+    return Poly<4>{{D * J - A * G, D * K + E * J - A * H - B * G, F * J + D * L + E * K - C * G - A * I - B * H,
+                    F * K + E * L - C * H - B * I, F * L - C * I}};
+}
+// plane_poly's cubic.
+CCD_FHD Poly<3> plane_cubic(V3 x10, V3 x20, V3 x30, V3 v10, V3 v20, V3 v30)
+{
+    const V3 v23 = cross(v20, v30), x2v3 = cross(x20, v30), v2x3 = cross(v20, x30), x23 = cross(x20, x30);
+    return Poly<3>{{dot(x10, x23), dot(x10, x2v3) + dot(x10, v2x3) + dot(v10, x23),
+                    dot(x10, v23) + dot(v10, x2v3) + dot(v10, v2x3), dot(v10, v23)}};
+}
+// distance_poly's sextic: positive on [0, 1] by the margin.
+CCD_FHD bool distance_positive(V3 x10, V3 x20, V3 x30, V3 v10, V3 v20, V3 v30, double minD)
+{
+    const V3 G = cross(v20, v30), x2v3 = cross(x20, v30), v2x3 = cross(v20, x30), E = cross(x20, x30);
+    const double A = dot(v10, G);
+    const double B = dot(x10, G) + dot(v10, x2v3) + dot(v10, v2x3);
+    const double C = dot(x10, x2v3) + dot(x10, v2x3) + dot(v10, E);
+    const double D = dot(x10, E);
+    const V3 F = x2v3 + v2x3;
+    const double b1 = dfma(1.0 / 3.0, C, D), b2 = dfma(1.0 / 3.0, B, dfma(2.0 / 3.0, C, D)), b3 = ((D + C) + B) + A;
+    const double hi = fmax2(fmax2(D, b1), fmax2(b2, b3)), lo = fmin2(fmin2(D, b1), fmin2(b2, b3));
+    const double d = fmax2(lo, -hi);   // the distance of the coefficients' range from zero, if positive
+    const V3 n1 = mk(dfma(0.5, F.x, E.x), dfma(0.5, F.y, E.y), dfma(0.5, F.z, E.z)), n2 = (E + F) + G;
+    const double nn = fmax2(fmax2(dot(E, E), dot(n1, n1)), dot(n2, n2));
+    const double S = (dabs(A) + dabs(B)) + (dabs(C) + dabs(D));
+    const double T = ((dabs(E.x) + dabs(E.y)) + (dabs(E.z) + dabs(F.x))) + ((dabs(F.y) + dabs(F.z)) + (dabs(G.x) + dabs(G.y))) +
+                     dabs(G.z);
+    // (S and T hold every coefficient, so a NaN fails the comparison)
+    return (d > 0.0) & (d * d - minD * nn > dfma(1e-12, S * S + minD * (T * T), SCREEN_TINY));
+}
+// vertex_edge's colinear-distance quartic, negated (its list keeps the negative pieces).
+CCD_FHD Poly<4> minus_colinear_quartic(Quad ab2, Quad ac2, Quad e1, double minD)
+{
+    const double A = ab2.c0, B = ab2.c1, C = ab2.c2, D = ac2.c0, E = ac2.c1, F = ac2.c2, G = e1.c0, H = e1.c1, I = e1.c2;
+    return Poly<4>{{-(A * D - G * G - minD * A), -(B * D + A * E - 2 * G * H - minD * B),
+                    -(B * E + A * F + C * D - H * H - 2 * G * I - minD * C), -(B * F + C * E - 2 * H * I),
+                    -(C * F - I * I)}};
+}
+// vertex_edge for a vertex at ac from the edge's first end: ab2 = ab.ab, ac2 = ac.ac, e1 = ab.ac and
+// e2 = ab.cb (the two side quadratics).
+CCD_FHD bool vertex_edge_cleared(Quad ab2, Quad ac2, Quad e1, Quad e2, double minD)
+{
+    return surely_negative(e1) | surely_negative(e2) | surely_negative(minus_colinear_quartic(ab2, ac2, e1, minD));
+}
+// vertex_vertex for two vertices whose difference squared is d2; margin as above.
+CCD_FHD bool vertex_vertex_cleared(Quad d2, double minD, double margin)
+{
+    const double b0 = d2.c0 - minD, b1 = dfma(0.5, d2.c1, b0), b2 = (b0 + d2.c1) + d2.c2;
+    return (fmin2(b0, b1) > margin) & (b2 > margin);
+}
+CCD_FHD double max_coord(const V3 *s, const V3 *e)
+{
+    double w = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        w = fmax2(w, fmax2(fmax2(dabs(s[j].x), dabs(s[j].y)), dabs(s[j].z)));
+        w = fmax2(w, fmax2(fmax2(dabs(e[j].x), dabs(e[j].y)), dabs(e[j].z)));
+    }
+    return w;
+}
+
+// Bits of a screen's result: the face or edge-edge test, its vertex-edge tests in order (three or four),
+// and the vertex-vertex tests together.
+constexpr unsigned SCREEN_PRIMARY = 1u, SCREEN_VE = 2u, SCREEN_VV = 32u;
+
+CCD_HD unsigned screen_vf_window(const V3 *s, const V3 *e, double eta)
+{
+    const double minD = eta * eta, w = max_coord(s, e), vv = 4e-12 * (w * w);
+    const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
+    const V3 a = s[2] - s[1], b = s[3] - s[1], c = s[3] - s[2], va = v2 - v1, vb = v3 - v1, vc = v3 - v2;
+    const V3 p1 = s[0] - s[1], p2 = s[0] - s[2], p3 = s[0] - s[3], vp1 = v0 - v1, vp2 = v0 - v2, vp3 = v0 - v3;
+    bool primary = !distance_positive(p1, a, b, vp1, va, vb, minD);
+    // x20 of the second and third plane, cross(-a, c) and cross(-c, -b), are -cross(a, c) and cross(c, b)
+    // bit for bit
+    primary = primary & !surely_negative(plane_cubic(p1, cross(b, a), b, vp1, cross(vb, va), vb));
+    primary = primary & !surely_negative(plane_cubic(p2, -cross(a, c), -a, vp2, -cross(va, vc), -va));
+    primary = primary & !surely_negative(plane_cubic(p3, cross(c, b), -c, vp3, cross(vc, vb), -vc));
+    unsigned m = primary ? SCREEN_PRIMARY : 0u;
+    const Quad d1 = moving_square(p1, vp1), d2 = moving_square(p2, vp2), d3 = moving_square(p3, vp3);
+    // (0; 1, 2): ab = a, ac = p1, cb = -p2;  (0; 2, 3): c, p2, -p3;  (0; 3, 1): -b, p3, -p1
+    if (!vertex_edge_cleared(moving_square(a, va), d1, moving_dot(p1, vp1, a, va), -moving_dot(p2, vp2, a, va), minD))
+        m |= SCREEN_VE;
+    if (!vertex_edge_cleared(moving_square(c, vc), d2, moving_dot(p2, vp2, c, vc), -moving_dot(p3, vp3, c, vc), minD))
+        m |= SCREEN_VE << 1;
+    if (!vertex_edge_cleared(moving_square(b, vb), d3, -moving_dot(p3, vp3, b, vb), moving_dot(p1, vp1, b, vb), minD))
+        m |= SCREEN_VE << 2;
+    if (!(vertex_vertex_cleared(d1, minD, vv) & vertex_vertex_cleared(d2, minD, vv) & vertex_vertex_cleared(d3, minD, vv)))
+        m |= SCREEN_VV;
+    return w < SCREEN_MAX_COORD ? m : SCREEN_PRIMARY | SCREEN_VE * 7u | SCREEN_VV;
+}
+
+CCD_HD unsigned screen_ee_window(const V3 *s, const V3 *e, double eta)
+{
+    const double minD = eta * eta, w = max_coord(s, e), vv = 4e-12 * (w * w);
+    const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
+    const V3 d1 = s[1] - s[0], d2 = s[3] - s[2], vd1 = v1 - v0, vd2 = v3 - v2;
+    bool primary = !distance_positive(s[1] - s[3], d1, d2, v1 - v3, vd1, vd2, minD);
+    const V3 r = s[0] - s[2], r1 = s[1] - s[2], r3 = s[3] - s[0], r4 = s[3] - s[1];
+    const V3 vr = v0 - v2, vr1 = v1 - v2, vr3 = v3 - v0, vr4 = v3 - v1;
+    const Quad l1 = moving_square(d1, vd1), l2 = moving_square(d2, vd2), x = moving_dot(d1, vd1, d2, vd2);
+    const Quad rd1 = moving_dot(r, vr, d1, vd1), rd2 = moving_dot(r, vr, d2, vd2);
+    const Quad r1d1 = moving_dot(r1, vr1, d1, vd1), r1d2 = moving_dot(r1, vr1, d2, vd2);
+    const Quad r3d1 = moving_dot(r3, vr3, d1, vd1), r3d2 = moving_dot(r3, vr3, d2, vd2);
+    const Quad r4d1 = moving_dot(r4, vr4, d1, vd1), r4d2 = moving_dot(r4, vr4, d2, vd2);
+    // edge_edge's four barycentric quartics, in its order
+    primary = primary & !surely_negative(barycentric_quartic(l2, x, rd1, rd2));
+    primary = primary & !surely_negative(barycentric_quartic(l2, -x, -r1d1, r1d2));
+    primary = primary & !surely_negative(barycentric_quartic(l1, x, -rd2, -rd1));
+    primary = primary & !surely_negative(barycentric_quartic(l1, -x, -r3d2, r3d1));
+    unsigned m = primary ? SCREEN_PRIMARY : 0u;
+    const Quad q = moving_square(r, vr), q1 = moving_square(r1, vr1), q3 = moving_square(r3, vr3),
+               q4 = moving_square(r4, vr4);
+    // (0; 2, 3): ab = d2, ac = r, cb = r3;  (1; 2, 3): d2, r1, r4;  (2; 0, 1): d1, -r, r1;  (3; 0, 1): d1, r3, -r4
+    if (!vertex_edge_cleared(l2, q, rd2, r3d2, minD)) m |= SCREEN_VE;
+    if (!vertex_edge_cleared(l2, q1, r1d2, r4d2, minD)) m |= SCREEN_VE << 1;
+    if (!vertex_edge_cleared(l1, q, -rd1, r1d1, minD)) m |= SCREEN_VE << 2;
+    if (!vertex_edge_cleared(l1, q3, r3d1, -r4d1, minD)) m |= SCREEN_VE << 3;
+    if (!(vertex_vertex_cleared(q, minD, vv) & vertex_vertex_cleared(q1, minD, vv) & vertex_vertex_cleared(q3, minD, vv) &
+          vertex_vertex_cleared(q4, minD, vv)))
+        m |= SCREEN_VV;
+    return w < SCREEN_MAX_COORD ? m : SCREEN_PRIMARY | SCREEN_VE * 15u | SCREEN_VV;
+}
+
+// ------------------------------------------------------------------------------------------------
+// Refinement of a screen: the same question on REFINE_LEAVES equal parts of [0, 1].  A sub-test hits only
+// at a time that lies in an interval of each of its lists; if on every part some list's polynomial is
+// rejected, no such time exists.
+//
+// With one list per part this needs more than the sign of the polynomials: the interval lists are computed,
+// and a list could hold a time at which its polynomial is clearly rejected, if the isolator missed a
+// root (a pair of roots so close that their polynomial's sign between them drowns in rounding) and the
+// piece's midpoint, by whose sign the whole piece is kept, fell on just that spot.  So a list's rejected
+// parts count only when its polynomial is clean on all of [0, 1]: on every part it has one sign by a
+// margin, or is strictly monotone (its Bernstein coefficients increase or decrease) with clear signs at
+// the part's ends, that is, it crosses zero once.  Then its true roots are simple and far from any
+// extremum near zero; the isolator compares signs at the critical points it finds, of which those whose
+// sign is uncertain can only lie at a crossing, so it finds every crossing, and every piece that extends
+// beyond the rounding zone of a crossing has the sign of its midpoint throughout.  The distance sextic
+// d^2 - eta^2 |n|^2 is clean on a part where it is positive by a margin, or where d is strictly
+// monotone from a clear sign to the other and eta^2 |n|^2 stays above the rounding of the sextic: it then
+// dips below zero once, by more than rounding, around d's root.  A list rejected on all parts is empty,
+// clean or not.  The vertex-vertex test has one quadratic, convex, whose smallest value decides.
+//
+// Of 200,000 stencils each, left open by the screen and then by 16 parts: a 200^2 cloth 49% -> 1.6%
+// vertex-face, 58% -> 9.2% edge-edge; a 330^2 sheet 2.5% -> 0.05%, 13% -> 3.2%.
+// ------------------------------------------------------------------------------------------------
+constexpr int REFINE_LEAVES = 16;
+constexpr unsigned REFINE_ALL = (1u << REFINE_LEAVES) - 1u;
+constexpr double REFINE_TOL = 1e-10, REFINE_SLOPE_TOL = 1e-13, REFINE_DISTANCE_TOL = 1e-12;
+
+struct Rejected {
+    unsigned parts = 0, unclean = 0;   // bit per part
+    // The parts on which the list can be relied on to hold no time.
+    CCD_FHD unsigned usable() const { return unclean == 0 || parts == REFINE_ALL ? parts : 0u; }
+};
+
+// Bernstein coefficients of p on [a, a + h].
+template <int D>
+CCD_FHD void bernstein_on(const Poly<D> &p, double a, double h, double (&b)[D + 1])
+{
+    double s[D + 1];
+#pragma unroll
+    for (int i = 0; i <= D; i++) s[i] = p.c[i];
+#pragma unroll
+    for (int i = 0; i < D; i++)
+#pragma unroll
+        for (int j = D - 1; j >= i; j--) s[j] = dfma(a, s[j + 1], s[j]);
+    double hp = h;
+#pragma unroll
+    for (int i = 1; i <= D; i++) {
+        s[i] *= hp;
+        hp *= h;
+    }
+#pragma unroll
+    for (int k = 0; k <= D; k++) {
+        b[k] = s[0];
+#pragma unroll
+        for (int i = 1; i <= k; i++) b[k] = dfma(binom(k, i) / binom(D, i), s[i], b[k]);
+    }
+}
+template <int N>
+CCD_FHD double max_of(const double (&b)[N])
+{
+    double m = b[0];
+#pragma unroll
+    for (int i = 1; i < N; i++) m = fmax2(m, b[i]);
+    return m;
+}
+template <int N>
+CCD_FHD double min_of(const double (&b)[N])
+{
+    double m = b[0];
+#pragma unroll
+    for (int i = 1; i < N; i++) m = fmin2(m, b[i]);
+    return m;
+}
+template <int N>
+CCD_FHD bool strictly_monotone(const double (&b)[N], double tol)
+{
+    double d[N - 1];
+#pragma unroll
+    for (int i = 0; i + 1 < N; i++) d[i] = b[i + 1] - b[i];
+    return (min_of(d) > tol) | (max_of(d) < -tol);
+}
+template <int D>
+CCD_FHD double largest(const Poly<D> &p)
+{
+    double m = 0.0;
+#pragma unroll
+    for (int i = 0; i <= D; i++) m = fmax2(m, dabs(p.c[i]));
+    return m;
+}
+// One part of a list that keeps p >= 0; m is p's largest coefficient.  (A NaN coefficient makes every b
+// NaN, so nothing is rejected and the part is unclean.)
+template <int D>
+CCD_FHD void refine_part(const Poly<D> &p, double m, double a, double h, unsigned bit, Rejected &r)
+{
+    double b[D + 1];
+    bernstein_on(p, a, h, b);
+    const double tol = dfma(REFINE_TOL, m, SCREEN_TINY), slope = dfma(REFINE_SLOPE_TOL, m, SCREEN_TINY);
+    const bool neg = max_of(b) < -tol;
+    const bool clean = (min_of(b) > tol) | (strictly_monotone(b, slope) & (dabs(b[0]) > tol) & (dabs(b[D]) > tol));
+    r.parts |= neg ? bit : 0u;
+    r.unclean |= neg | clean ? 0u : bit;
+}
+
+// The distance sextic as its cubic d, |n|^2 and the size of the terms of its coefficients.
+struct DistancePoly {
+    Poly<3> d;
+    Poly<4> nn;
+    double terms;
+};
+CCD_FHD DistancePoly distance_parts(V3 x10, V3 x20, V3 x30, V3 v10, V3 v20, V3 v30, double minD)
+{
+    const V3 G = cross(v20, v30), x2v3 = cross(x20, v30), v2x3 = cross(v20, x30), E = cross(x20, x30);
+    const V3 F = x2v3 + v2x3;
+    DistancePoly p;
+    p.d.c[3] = dot(v10, G);
+    p.d.c[2] = dot(x10, G) + dot(v10, x2v3) + dot(v10, v2x3);
+    p.d.c[1] = dot(x10, x2v3) + dot(x10, v2x3) + dot(v10, E);
+    p.d.c[0] = dot(x10, E);
+    p.nn = Poly<4>{{dot(E, E), 2 * dot(E, F), 2 * dot(E, G) + dot(F, F), 2 * dot(F, G), dot(G, G)}};
+    const double S = (dabs(p.d.c[0]) + dabs(p.d.c[1])) + (dabs(p.d.c[2]) + dabs(p.d.c[3]));
+    const double T = ((dabs(E.x) + dabs(E.y)) + (dabs(E.z) + dabs(F.x))) + ((dabs(F.y) + dabs(F.z)) + (dabs(G.x) + dabs(G.y))) +
+                     dabs(G.z);
+    p.terms = S * S + minD * (T * T);
+    return p;
+}
+CCD_FHD void refine_part(const DistancePoly &p, double minD, double a, double h, unsigned bit, Rejected &r)
+{
+    double b[4], g[5];
+    bernstein_on(p.d, a, h, b);
+    bernstein_on(p.nn, a, h, g);
+    const double tol = dfma(REFINE_DISTANCE_TOL, p.terms, SCREEN_TINY), far = dfma(minD, max_of(g), tol);
+    const double dist = fmax2(min_of(b), -max_of(b));
+    const bool positive = (dist > 0.0) & (dist * dist > far);
+    const double slope = REFINE_SLOPE_TOL * largest(p.d) + SCREEN_TINY;
+    const bool dips = strictly_monotone(b, slope) & ((b[0] < 0.0) != (b[3] < 0.0)) & (b[0] * b[0] > far) & (b[3] * b[3] > far) &
+                      (minD * min_of(g) > tol);
+    r.parts |= positive ? bit : 0u;
+    r.unclean |= positive | dips ? 0u : bit;
+}
+
+// Whether a stencil's face or edge-edge test cannot hit.
+CCD_HD bool refine_vertex_face(const V3 *s, const V3 *e, double eta)
+{
+    const double minD = eta * eta;
+    const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
+    const V3 a = s[2] - s[1], b = s[3] - s[1], c = s[3] - s[2], va = v2 - v1, vb = v3 - v1, vc = v3 - v2;
+    const V3 p1 = s[0] - s[1], p2 = s[0] - s[2], p3 = s[0] - s[3], vp1 = v0 - v1, vp2 = v0 - v2, vp3 = v0 - v3;
+    const DistancePoly dp = distance_parts(p1, a, b, vp1, va, vb, minD);
+    const Poly<3> f[3] = {plane_cubic(p1, cross(b, a), b, vp1, cross(vb, va), vb),
+                          plane_cubic(p2, -cross(a, c), -a, vp2, -cross(va, vc), -va),
+                          plane_cubic(p3, cross(c, b), -c, vp3, cross(vc, vb), -vc)};
+    const double m[3] = {largest(f[0]), largest(f[1]), largest(f[2])};
+    Rejected rd, r[3];
+    constexpr double h = 1.0 / REFINE_LEAVES;
+#pragma nounroll
+    for (int k = 0; k < REFINE_LEAVES; k++) {
+        const double at = k * h;
+        const unsigned bit = 1u << k;
+        refine_part(dp, minD, at, h, bit, rd);
+#pragma unroll
+        for (int j = 0; j < 3; j++) refine_part(f[j], m[j], at, h, bit, r[j]);
+    }
+    return (rd.usable() | r[0].usable() | r[1].usable() | r[2].usable()) == REFINE_ALL && max_coord(s, e) < SCREEN_MAX_COORD;
+}
+CCD_HD bool refine_edge_edge(const V3 *s, const V3 *e, double eta)
+{
+    const double minD = eta * eta;
+    const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
+    const V3 d1 = s[1] - s[0], d2 = s[3] - s[2], vd1 = v1 - v0, vd2 = v3 - v2;
+    const V3 x0 = s[0] - s[2], x1 = s[1] - s[2], x3 = s[3] - s[0], vx0 = v0 - v2, vx1 = v1 - v2, vx3 = v3 - v0;
+    const DistancePoly dp = distance_parts(s[1] - s[3], d1, d2, v1 - v3, vd1, vd2, minD);
+    const Quad l1 = moving_square(d1, vd1), l2 = moving_square(d2, vd2), x = moving_dot(d1, vd1, d2, vd2);
+    const Quad rd1 = moving_dot(x0, vx0, d1, vd1), rd2 = moving_dot(x0, vx0, d2, vd2);
+    const Poly<4> f[4] = {
+        barycentric_quartic(l2, x, rd1, rd2),
+        barycentric_quartic(l2, -x, -moving_dot(x1, vx1, d1, vd1), moving_dot(x1, vx1, d2, vd2)),
+        barycentric_quartic(l1, x, -rd2, -rd1),
+        barycentric_quartic(l1, -x, -moving_dot(x3, vx3, d2, vd2), moving_dot(x3, vx3, d1, vd1))};
+    const double m[4] = {largest(f[0]), largest(f[1]), largest(f[2]), largest(f[3])};
+    Rejected rd, r[4];
+    constexpr double h = 1.0 / REFINE_LEAVES;
+#pragma nounroll
+    for (int k = 0; k < REFINE_LEAVES; k++) {
+        const double at = k * h;
+        const unsigned bit = 1u << k;
+        refine_part(dp, minD, at, h, bit, rd);
+#pragma unroll
+        for (int j = 0; j < 4; j++) refine_part(f[j], m[j], at, h, bit, r[j]);
+    }
+    return (rd.usable() | r[0].usable() | r[1].usable() | r[2].usable() | r[3].usable()) == REFINE_ALL &&
+           max_coord(s, e) < SCREEN_MAX_COORD;
+}
+// Whether vertex_edge(q0, q1, q2) cannot hit.
+CCD_HD bool refine_vertex_edge(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, double eta)
+{
+    const V3 v0 = q0e - q0s, v1 = q1e - q1s, v2 = q2e - q2s;
+    const V3 ab = q2s - q1s, ac = q0s - q1s, cb = q2s - q0s, vab = v2 - v1, vac = v0 - v1, vcb = v2 - v0;
+    const Quad e1 = moving_dot(ac, vac, ab, vab), e2 = moving_dot(cb, vcb, ab, vab);
+    const Poly<2> f[2] = {Poly<2>{{e1.c0, e1.c1, e1.c2}}, Poly<2>{{e2.c0, e2.c1, e2.c2}}};
+    const Poly<4> g = minus_colinear_quartic(moving_square(ab, vab), moving_square(ac, vac), e1, eta * eta);
+    const double m[3] = {largest(f[0]), largest(f[1]), largest(g)};
+    Rejected r[3];
+    constexpr double h = 1.0 / REFINE_LEAVES;
+#pragma nounroll
+    for (int k = 0; k < REFINE_LEAVES; k++) {
+        const double at = k * h;
+        const unsigned bit = 1u << k;
+        refine_part(f[0], m[0], at, h, bit, r[0]);
+        refine_part(f[1], m[1], at, h, bit, r[1]);
+        refine_part(g, m[2], at, h, bit, r[2]);
+    }
+    const double w = fmax2(fmax2(m[0], m[1]), m[2]);
+    return (r[0].usable() | r[1].usable() | r[2].usable()) == REFINE_ALL && w < 1e150;
+}
+// Whether vertex_vertex cannot hit, for vertices whose coordinates stay below w.
+CCD_HD bool refine_vertex_vertex(V3 q1s, V3 q2s, V3 q1e, V3 q2e, double eta, double w)
+{
+    const V3 r = q1s - q2s, v = (q1e - q1s) - (q2e - q2s);
+    const Quad q = moving_square(r, v);
+    const double minD = eta * eta, margin = 4e-12 * (w * w);
+    double t = q.c2 > 0.0 ? -0.5 * q.c1 / q.c2 : 0.0;
+    t = smin(1.0, smax(t, 0.0));
+    const double at_t = dfma(dfma(q.c2, t, q.c1), t, q.c0), at_1 = (q.c0 + q.c1) + q.c2;
+    return (fmin2(fmin2(q.c0, at_1), at_t) - minD > margin) & (at_1 - minD > margin) & (w < SCREEN_MAX_COORD);
+}
+
+// The vertices of a stencil's sub-tests in the cascade's order: test j of the vertex-edge tests is
+// (vertex a; edge b, c), of the vertex-vertex tests (a, b).
+template <bool VF>
+CCD_FHD void vertex_edge_vertices(int j, int &a, int &b, int &c)
+{
+    if (VF) {   // (0; 1, 2), (0; 2, 3), (0; 3, 1)
+        a = 0;
+        b = j + 1;
+        c = j == 2 ? 1 : j + 2;
+    } else {    // (0; 2, 3), (1; 2, 3), (2; 0, 1), (3; 0, 1)
+        a = j;
+        b = j < 2 ? 2 : 0;
+        c = b + 1;
+    }
+}
+template <bool VF>
+CCD_FHD void vertex_vertex_vertices(int j, int &a, int &b)
+{
+    a = VF ? 0 : j >> 1;                // (0, 1), (0, 2), (0, 3)
+    b = VF ? j + 1 : 2 + (j & 1);       // (0, 2), (0, 3), (1, 2), (1, 3)
+}
+
+// A screen's mask after the refinement of the face or edge-edge test, and of the others.  `at` gives a
+// vertex's window positions by its place in the stencil (0..3), which is a runtime index.
+template <bool VF>
+CCD_HD unsigned refine_primary(const V3 *s, const V3 *e, double eta, unsigned m)
+{
+    if ((m & SCREEN_PRIMARY) && (VF ? refine_vertex_face(s, e, eta) : refine_edge_edge(s, e, eta))) m &= ~SCREEN_PRIMARY;
+    return m;
+}
+template <bool VF, class At>
+CCD_HD unsigned refine_others(const V3 *s, const V3 *e, double eta, unsigned m, At &&at)
+{
+    for (unsigned open = m & (15u * SCREEN_VE); open; open &= open - 1) {
+        const unsigned bit = open & (0u - open);
+        int a, b, c;
+        vertex_edge_vertices<VF>(low_bit(open) - 1, a, b, c);
+        V3 as, ae, bs, be, cs, ce;
+        at(a, as, ae);
+        at(b, bs, be);
+        at(c, cs, ce);
+        if (refine_vertex_edge(as, bs, cs, ae, be, ce, eta)) m &= ~bit;
+    }
+    if (m & SCREEN_VV) {
+        const double w = max_coord(s, e);
+        bool clear = true;
+#pragma unroll
+        for (int j = 0; j < (VF ? 3 : 4); j++) {
+            int a, b;
+            vertex_vertex_vertices<VF>(j, a, b);
+            clear = clear & refine_vertex_vertex(s[a], s[b], e[a], e[b], eta, w);
+        }
+        if (clear) m &= ~SCREEN_VV;
+    }
+    return m;
+}
+
+// The sub-tests left open (mask), in the cascade's order: the first that hits, or -1.  check_others leaves
+// the face or edge-edge test out.
+template <bool VF, class At, class C = NoCount>
+CCD_HD int check_others(double eta, double &t, unsigned m, At &&at, C &&cnt = C())
+{
+    for (unsigned open = m & (15u * SCREEN_VE); open; open &= open - 1) {
+        const int j = low_bit(open) - 1;
+        int a, b, c;
+        vertex_edge_vertices<VF>(j, a, b, c);
+        V3 as, ae, bs, be, cs, ce;
+        at(a, as, ae);
+        at(b, bs, be);
+        at(c, cs, ce);
+        if (vertex_edge(as, bs, cs, ae, be, ce, eta, t, cnt)) return 1 + j;
+    }
+    if (m & SCREEN_VV) {
+        constexpr int n = VF ? 3 : 4;
+#if defined(__HIPCC__)
+#pragma nounroll
+#endif
+        for (int j = 0; j < n; j++) {
+            int a, b;
+            vertex_vertex_vertices<VF>(j, a, b);
+            V3 as, ae, bs, be;
+            at(a, as, ae);
+            at(b, bs, be);
+            if (vertex_vertex(as, bs, ae, be, eta, t, cnt)) return 1 + n + j;
+        }
+    }
+    return -1;
+}
+template <bool VF, class At, class C = NoCount>
+CCD_HD int check_masked(const V3 *s, const V3 *e, double eta, double &t, unsigned m, At &&at, C &&cnt = C())
+{
+    if (m & SCREEN_PRIMARY) {
+        if (VF ? vertex_face(s[0], s[1], s[2], s[3], e[0], e[1], e[2], e[3], eta, t, cnt)
+               : edge_edge(s[0], s[1], s[2], s[3], e[0], e[1], e[2], e[3], eta, t, cnt))
+            return 0;
+    }
+    return check_others<VF>(eta, t, m, at, cnt);
 }
 
 // ------------------------------------------------------------------------------------------------

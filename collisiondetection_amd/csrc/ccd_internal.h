@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -10,21 +11,21 @@
 
 #include "../../include/ccd_amd.h"
 
-// Launch shape of the persistent work-queue narrowphase (tuned by ccd_autotune).
+// Launch shape of the narrowphase (tuned by ccd_autotune).  The screening form uses the tile; block and
+// waves_per_cu shape the persistent grid of the one-pass form.
 struct QueueShape {
     int block = 256;       // threads per block: 64, 128 or 256
-    int tile = 64;         // stencils a wavefront takes per atomic
-    int waves_per_cu = 12; // resident wavefronts per compute unit in the persistent grid (three per SIMD)
-    int group = 1;         // order the stencils by their sub-test signature first (1) or not (0)
+    int tile = 1024;       // stencils a wavefront takes at a time (fewer on short lists)
+    int waves_per_cu = 8;  // resident wavefronts per compute unit in the persistent grid (two per SIMD)
+    int group = 0;         // accepted and reported, without effect (0 or 1)
 };
 
 struct ccd_ctx {
     int device = 0;
     int num_cus = 256;
-    bool group_stencils = true;   // group stencils by vertex-edge signature before the narrowphase
-    bool ee_split = true;         // edge-edge narrowphase in two passes (deferred sextic recursions)
+    bool ee_split = true;         // edge-edge narrowphase screened, else in one pass
     QueueShape vf_shape;
-    QueueShape ee_shape{256, 64, 16, 1};   // the screening pass holds four wavefronts per SIMD
+    QueueShape ee_shape;
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     std::string err;
@@ -99,57 +100,44 @@ void *buffer(ccd_ctx *ctx, const char *name, size_t bytes);
 namespace ccdi {
 int launch_primitives(ccd_ctx *ctx, int kind, const double *q, const double *eta, double eta_s, int64_t n,
                       uint8_t *hit, double *t);
-// Buffers for ordering n stencils by signature before the narrowphase: sig, sig2 (n uint64), idx, idx2
-// (n int32) and tmp (radix_sort_temp_bytes(n) bytes).
-struct OrderScratch {
-    uint64_t *sig = nullptr, *sig2 = nullptr;
-    int32_t *idx = nullptr, *idx2 = nullptr;
-    void *tmp = nullptr;
+// Where a narrowphase's results go: appended to a hit list (PER_STENCIL false), or at each stencil's own
+// index, with a thickness per stencil (PER_STENCIL true).
+struct NarrowOut {
+    int4 *out_keys = nullptr;
+    double *out_toi = nullptr;
+    int64_t cap = 0;
+    unsigned long long *counter = nullptr;
+    const double *eta = nullptr;   // per stencil, or null
+    uint8_t *hit = nullptr;
+    double *t = nullptr;
+    uint8_t *sub = nullptr;
 };
+// The screening narrowphase (screened.hip) over n stencils (or the device count n_dev, if smaller), n < 2^31.
+// list: open_list_bytes of device memory for at least n stencils, uninitialised; tile: stencils that a
+// wavefront takes at a time on long lists.  open_list: the context's buffer, or null for n >= 2^31.
+int launch_screened(ccd_ctx *ctx, bool vf, bool per_stencil, const double *qs, const double *qe, const int32_t *keys,
+                    const int64_t *n_dev, int64_t n, double eta, const NarrowOut &o, int tile, void *list);
+int64_t open_list_bytes(int64_t n);
+void *open_list(ccd_ctx *ctx, int64_t n);
+// One result per stencil.  list: the caller's, for these n stencils, else the context's own.
 int launch_narrow2(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys,
                    const double *eta, double eta_s, int64_t n, uint8_t *hit, double *t, uint8_t *sub,
-                   const OrderScratch *order_scratch = nullptr);
+                   void *list = nullptr);
 // wave: one wavefront per stencil sharing the stitched windows (for long histories), else one lane.
 int launch_narrow_hist(ccd_ctx *ctx, bool vf, const int64_t *off, const double *ht, const double *hp,
                        const int32_t *keys, const double *eta, double eta_s, int64_t n, uint8_t *hit, double *t,
                        uint8_t *sub, int32_t *win, bool wave);
-// Narrowphase over a stencil list, compacting the colliding stencils (keys + toi) into out_keys /
-// out_toi with a device counter at counters[slot]; at most cap are written.
-int launch_narrow2_compact(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys,
-                           const int64_t *n_dev, int64_t n_max, double eta, int32_t *out_keys, double *out_toi,
-                           int64_t cap, int64_t *counter);
-// The deferred-stencil list of the two-pass edge-edge narrowphase: positions (idx) and first-pass
-// vertex-edge / vertex-vertex results (sub) of up to cap stencils, the list's device counter and the
-// second pass's queue counter (both zero before the launch).
-struct EeDeferral {
-    uint32_t *idx = nullptr;
-    uint8_t *sub = nullptr;
-    unsigned long long *count = nullptr;
-    unsigned long long *work = nullptr;
-    int64_t cap = 0;
-};
-// The context's deferral list for up to n stencils (grow-only buffers "ee_def_idx", "ee_def_sub"; counters
-// at count_and_work[0..1]), or an empty one when the context runs edge-edge in one pass.
-EeDeferral ee_deferral(ccd_ctx *ctx, int64_t n, unsigned long long *count_and_work);
-// The list slots the two-pass narrowphase needs for n stored stencils (the list is filled in blocks).
-int64_t ee_deferral_capacity(const ccd_ctx *ctx, int64_t n);
-// Persistent work-queue narrowphase; *work must be zero before the launch.  Edge-edge runs in two
-// passes when def holds a list for n_max stencils (n_max < 2^31), else in one.
+// Narrowphase over a stencil list, appending the colliding stencils (keys and times) to out_keys / out_toi
+// with a device counter; at most cap are written.  Screened when `list` (for at least n_max stencils) is
+// given, else the whole cascade on a persistent work queue, whose counter *work must be zero.
 int launch_narrow2_queue(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys,
                          const int64_t *n_dev, int64_t n_max, double eta, int32_t *out_keys, double *out_toi,
                          int64_t cap, int64_t *counter, unsigned long long *work, const QueueShape &shape,
-                         const EeDeferral *def = nullptr);
+                         void *list = nullptr);
 // Work accounting: per-stage execution counts (ccd::Stage order) summed over the stencils into counts.
 int launch_narrow2_count(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys,
                          int64_t n, double eta, unsigned long long *counts);
 // Validation: counts keys outside [0, nverts) into *bad.
-// The n stencils (device keys, n exact on the host) reordered by their vertex-edge signature
-// (ccd::ve_signature; stable) into a context buffer; *grouped receives it (or keys when n < 2).  With
-// n_dev (the stored count on the device, for captured pipelines) the n slots past it sort last.
-int reserve_grouping(ccd_ctx *ctx, int64_t nvf, int64_t nee);
-int group_by_signature(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys, int64_t n,
-                       double eta, const int64_t *n_dev,
-                       const int32_t **grouped);
 // Separating-plane narrowphase over a CSR history: launch_min_gap writes History::computeMinimumGap's
 // value (as bits) to *gap_bits on the device; launch_separating_plane reads it (eps = gap / 4).
 int launch_min_gap(ccd_ctx *ctx, const int64_t *off, const double *ht, int64_t nverts, uint64_t *gap_bits);

@@ -177,11 +177,11 @@ using namespace ccdi;
 int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
 
 // A request's transient device memory: face pairs, the related-face table and its emission masks
-// (two entries per pair), the stencil keys, the edge-edge deferred list (cd slots) and the hit lists.
-int64_t workspace_bytes(int64_t cp, int64_t cv, int64_t ce, int64_t cd, int64_t ch)
+// (two entries per pair), the stencil keys, the screening passes' lists and the hit lists.
+int64_t workspace_bytes(int64_t cp, int64_t cv, int64_t ce, int64_t ch)
 {
     return align256(cp * 8) + align256((2 * cp + 1) * 4) + align256((2 * cp + 1) * 2) + align256(cv * 16) +
-           align256(ce * 16) + align256(cd * 4) + align256(cd) + 2 * (align256(ch * 16) + align256(ch * 8)) + 256;
+           align256(ce * 16) + align256(open_list_bytes(std::max(cv, ce))) + 2 * (align256(ch * 16) + align256(ch * 8)) + 256;
 }
 
 // Point the session context's transient buffers at a slice of the pool.
@@ -200,9 +200,7 @@ void bind_workspace(ccd_server *S, Session &s, InFlight &f)
     put("adj_mask", (2 * f.cap_pairs + 1) * 2);
     put("vf_keys", f.cap_vf * 16);
     put("ee_keys", f.cap_ee * 16);
-    const int64_t cd = ee_deferral_capacity(s.ctx, f.cap_ee);   // the edge-edge deferred list
-    put("ee_def_idx", cd * 4);
-    put("ee_def_sub", cd);
+    put("open_list", open_list_bytes(std::max(f.cap_vf, f.cap_ee)));   // the screening passes' lists
     const int64_t kb = align256(f.cap_hits * 16), tb = align256(f.cap_hits * 8);
     f.hit_vk = (int32_t *)p;
     f.hit_vt = (double *)(p + kb);
@@ -223,20 +221,20 @@ int launch_request(ccd_server *S, Session &s, InFlight &f)
     CCD_HIP_CHECK(ctx, hipMemcpyAsync(end, f.req.qend.data(), (size_t)s.V * 24, hipMemcpyHostToDevice, st));
     int rc = broadphase_refit_launch(ctx, s.faces, s.F, start, end, s.V, s.outer_eta, nullptr, nullptr, 1);
     if (rc) return rc;
-    // work[0..1]: the two queues; [2..3]: the hit checksums; [4..5]: the edge-edge deferral list.
-    unsigned long long *work = (unsigned long long *)buffer(ctx, "queue_work", 48);
+    // work[0..1]: the one-pass form's queues; [2..3]: the hit checksums.
+    unsigned long long *work = (unsigned long long *)buffer(ctx, "queue_work", 32);
     if (!work) return CCD_E_OOM;
     rc = fill_u64(ctx, (uint64_t *)(ctx->d_counts + C_VF_HITS), 2, 0);
-    if (!rc) rc = fill_u64(ctx, (uint64_t *)work, 6, 0);
+    if (!rc) rc = fill_u64(ctx, (uint64_t *)work, 4, 0);
     if (rc) return rc;
-    const EeDeferral def = ee_deferral(ctx, f.cap_ee, work + 4);
+    void *list = open_list(ctx, std::min<int64_t>(std::max(f.cap_vf, f.cap_ee), 0x7fffffffll));
     rc = launch_narrow2_queue(ctx, true, start, end, (const int32_t *)ctx->bufs["vf_keys"].ptr, ctx->d_counts + C_VF,
                               f.cap_vf, s.eta, f.hit_vk, f.hit_vt, f.cap_hits, ctx->d_counts + C_VF_HITS, work,
-                              ctx->vf_shape);
+                              ctx->vf_shape, list);
     if (rc) return rc;
     rc = launch_narrow2_queue(ctx, false, start, end, (const int32_t *)ctx->bufs["ee_keys"].ptr, ctx->d_counts + C_EE,
                               f.cap_ee, s.eta, f.hit_ek, f.hit_et, f.cap_hits, ctx->d_counts + C_EE_HITS, work + 1,
-                              ctx->ee_shape, &def);
+                              ctx->ee_shape, list);
     if (rc) return rc;
     unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks_for(2 * f.cap_hits, 256), 1024));
     hipLaunchKernelGGL(k_hit_checksum, dim3(g), dim3(256), 0, st, (const int4 *)f.hit_vk, f.hit_vt,
@@ -345,8 +343,7 @@ void worker_loop(ccd_server *S)
             f.cap_vf = mul * s.last_vf + s.F + 4096;
             f.cap_ee = mul * s.last_ee + 2 * s.F + 4096;
             f.cap_hits = mul * s.last_hits + s.F / 16 + 4096;
-            f.pool_bytes = workspace_bytes(f.cap_pairs, f.cap_vf, f.cap_ee, ee_deferral_capacity(s.ctx, f.cap_ee),
-                                           f.cap_hits);
+            f.pool_bytes = workspace_bytes(f.cap_pairs, f.cap_vf, f.cap_ee, f.cap_hits);
             if (f.pool_bytes > S->pool.size) {   // can never be admitted: fail it rather than wait forever
                 ccd_request_result r{};
                 r.request_id = it->id;
@@ -508,7 +505,7 @@ int ccd_server_open_session(ccd_server *S, const int32_t *faces, int64_t nfaces,
     s.last_ee = nec;
     s.last_hits = std::max(nvh, neh);
     // The transient buffers come from the pool per request: release the context's own copies.
-    for (const char *name : {"pairs", "adj", "adj_mask", "vf_keys", "ee_keys", "ee_def_idx", "ee_def_sub"}) {
+    for (const char *name : {"pairs", "adj", "adj_mask", "vf_keys", "ee_keys", "open_list"}) {
         ccd_ctx::Buf &b = ctx->bufs[name];
         if (b.ptr && !b.external) {
             (void)hipFree(b.ptr);
@@ -616,7 +613,7 @@ int ccd_server_destroy(ccd_server *S)
     if (S->worker.joinable()) S->worker.join();
     (void)hipSetDevice(S->device);
     for (Session &s : S->sessions) {
-        for (const char *name : {"pairs", "adj", "adj_mask", "vf_keys", "ee_keys", "ee_def_idx", "ee_def_sub"}) s.ctx->bufs[name] = ccd_ctx::Buf();
+        for (const char *name : {"pairs", "adj", "adj_mask", "vf_keys", "ee_keys", "open_list"}) s.ctx->bufs[name] = ccd_ctx::Buf();
         (void)hipFree(s.faces);
         (void)hipFree(s.pos[0]);
         (void)hipFree(s.pos[1]);

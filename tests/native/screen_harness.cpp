@@ -1,0 +1,47 @@
+// Test-only: the screening and refining passes of the core beside the cascade they screen, on the host.  Per
+// stencil: the screen's mask, the refined mask, the cascade's sub-test and time, the masked cascade's (on
+// the refined mask), and a mask of the sub-tests that hit when each is run by itself.
+#include "../../collisiondetection_amd/csrc/ccd_core.h"
+
+using ccd::V3;
+
+template <bool VF>
+static void run(const double *qs, const double *qe, const int32_t *keys, int64_t n, double eta, uint32_t *mask,
+                uint32_t *refined, int32_t *sub, double *t, int32_t *sub_masked, double *t_masked, uint32_t *hits)
+{
+#pragma omp parallel for schedule(dynamic, 256)
+    for (int64_t i = 0; i < n; i++) {
+        V3 s[4], e[4];
+        for (int j = 0; j < 4; j++) {
+            const double *a = qs + 3 * (int64_t)keys[4 * i + j], *b = qe + 3 * (int64_t)keys[4 * i + j];
+            s[j] = ccd::mk(ccd::stitch0(a[0], b[0]), ccd::stitch0(a[1], b[1]), ccd::stitch0(a[2], b[2]));
+            e[j] = ccd::mk(b[0], b[1], b[2]);
+        }
+        auto at = [&](int j, V3 &x, V3 &y) {
+            x = s[j];
+            y = e[j];
+        };
+        mask[i] = VF ? ccd::screen_vf_window(s, e, eta) : ccd::screen_ee_window(s, e, eta);
+        refined[i] = ccd::refine_others<VF>(s, e, eta, ccd::refine_primary<VF>(s, e, eta, mask[i]), at);
+        t[i] = t_masked[i] = 0.0;
+        sub[i] = VF ? ccd::check_vf_window(s, e, eta, t[i]) : ccd::check_ee_window(s, e, eta, t[i]);
+        sub_masked[i] = ccd::check_masked<VF>(s, e, eta, t_masked[i], refined[i], at);
+        uint32_t h = 0;
+        for (int b = 0; b < 6; b++) {
+            double tt = 0.0;
+            if (VF && b == 4) continue;   // vertex-face has three vertex-edge tests
+            if (ccd::check_masked<VF>(s, e, eta, tt, 1u << b, at) >= 0) h |= 1u << b;
+        }
+        hits[i] = h;
+    }
+}
+
+extern "C" void screen_stencils(const double *qs, const double *qe, const int32_t *keys, int64_t n, int is_ee, double eta,
+                                uint32_t *mask, uint32_t *refined, int32_t *sub, double *t, int32_t *sub_masked,
+                                double *t_masked, uint32_t *hits)
+{
+    if (is_ee)
+        run<false>(qs, qe, keys, n, eta, mask, refined, sub, t, sub_masked, t_masked, hits);
+    else
+        run<true>(qs, qe, keys, n, eta, mask, refined, sub, t, sub_masked, t_masked, hits);
+}

@@ -1,0 +1,84 @@
+"""The narrowphase's screening and refining passes: a sub-test they clear never hits, and what they leave open
+gives the cascade's own answer, bit for bit (host build of the core)."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+import oracle
+from collisiondetection_amd import scenes
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def harness(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("screen") / "screen_harness.so")
+    subprocess.run(["g++", "-O2", "-ffp-contract=off", "-fno-fast-math", "-std=c++17", "-fPIC", "-shared", "-fopenmp",
+                    "-Wno-unknown-pragmas", "-o", out, os.path.join(ROOT, "tests", "native", "screen_harness.cpp")],
+                   check=True)
+    return ctypes.CDLL(out)
+
+
+def _run(H, qs, qe, keys, is_ee, eta):
+    qs, qe = np.ascontiguousarray(qs, np.float64), np.ascontiguousarray(qe, np.float64)
+    keys = np.ascontiguousarray(keys, np.int32)
+    n = len(keys)
+    mask, refined, hits = np.zeros(n, np.uint32), np.zeros(n, np.uint32), np.zeros(n, np.uint32)
+    sub, subm = np.zeros(n, np.int32), np.zeros(n, np.int32)
+    t, tm = np.zeros(n), np.zeros(n)
+    p = lambda a: a.ctypes.data_as(ctypes.c_void_p)   # noqa: E731
+    H.screen_stencils(p(qs), p(qe), p(keys), ctypes.c_int64(n), int(is_ee), ctypes.c_double(eta), p(mask), p(refined), p(sub), p(t),
+                      p(subm), p(tm), p(hits))
+    assert not (refined & ~mask).any() and not (hits & ~refined).any()
+    np.testing.assert_array_equal(sub, subm)
+    np.testing.assert_array_equal(t.view(np.int64), tm.view(np.int64))
+    return mask, refined
+
+
+SCENES = {
+    "cloth": lambda: scenes.cloth(48), "sheet": lambda: scenes.crumpled_sheet(48, eta=1e-3),
+    "spheres": lambda: scenes.converging_spheres(levels=2), "still": lambda: dict(scenes.cloth(24), qend=scenes.cloth(24)["qstart"]),
+    "thick": lambda: dict(scenes.cloth(32), eta=0.01),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SCENES))
+@pytest.mark.parametrize("shift,scale", [(0.0, 1.0), (1e4, 1.0), (0.0, 1e-60), (0.0, 1e45)])
+def test_screen_scenes(harness, name, shift, scale):
+    s = SCENES[name]()
+    qs, qe = (s["qstart"] + shift) * scale, (s["qend"] + shift) * scale
+    vf, ee = oracle.candidates(s["faces"], oracle.Hist.two_entry(s["qstart"], s["qend"]), s["eta"], method="tree")
+    for keys, is_ee in ((vf, False), (ee, True)):
+        mask, refined = _run(harness, qs, qe, keys, is_ee, s["eta"] * scale)
+        if scale == 1e45:
+            assert mask.all()
+        elif shift == 0.0 and scale == 1.0 and name == "sheet":
+            assert (mask == 0).mean() > 0.7   # the screen clears most of a smoothly moving sheet
+        elif shift == 0.0 and scale == 1.0 and name == "cloth":
+            assert (refined == 0).sum() > (mask == 0).sum()
+
+
+@pytest.mark.parametrize("is_ee", [False, True])
+@pytest.mark.parametrize("kind", ["random", "lattice", "collapsing", "touching", "nonfinite"])
+def test_screen_awkward_stencils(harness, is_ee, kind):
+    """Small-integer lattices (exact zeros, reduced degrees, parallel and degenerate features), features that
+    shrink to nothing within the step, pairs exactly eta apart, NaN and infinite positions."""
+    rng = np.random.default_rng(5)
+    n = 60000
+    q = rng.normal(size=(2, 4 * n, 3))
+    eta = 0.05
+    if kind == "lattice":
+        q = rng.integers(-1, 2, size=q.shape).astype(np.float64)
+        eta = 0.5
+    elif kind == "collapsing":
+        q[1] = np.repeat(q[1][::4], 4, axis=0) + 1e-9 * rng.normal(size=q[1].shape)
+    elif kind == "touching":
+        q[0, :, 2] = np.tile([0.0, eta, eta, eta] if not is_ee else [0.0, 0.0, eta, eta], n)
+        q[1] = q[0] + rng.integers(-1, 2, size=(n, 1, 3)).repeat(4, axis=1).reshape(-1, 3)
+    elif kind == "nonfinite":
+        bad = rng.integers(0, q.size, size=n)
+        q.reshape(-1)[bad] = rng.choice([np.nan, np.inf, -np.inf, 1e300, -1e300, 1e-310], size=n)
+    _run(harness, q[0], q[1], np.arange(4 * n, dtype=np.int32).reshape(n, 4), is_ee, eta)
