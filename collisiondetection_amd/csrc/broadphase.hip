@@ -406,9 +406,11 @@ __global__ __launch_bounds__(256) void k_qrange_partial(const double *__restrict
 }
 
 __global__ __launch_bounds__(64) void k_qrange_final(const double *__restrict__ partial, int nparts,
-                                                     double *__restrict__ qparam)
+                                                     double *__restrict__ qparam, unsigned long long *__restrict__ zero,
+                                                     int nzero)
 {
     const int k = blockIdx.x;   // one wavefront per axis
+    for (int z = k * 64 + threadIdx.x; z < nzero; z += 64 * gridDim.x) zero[z] = 0;   // counters of later kernels
     double lo = __builtin_inf(), hi = -__builtin_inf();
     for (int p = threadIdx.x; p < nparts; p += 64) {
         const double a = partial[NB * p + k], b = partial[NB * p + KAX + k];
@@ -497,28 +499,23 @@ __global__ __launch_bounds__(256) void k_group_records(const BoxRec *__restrict_
 // ------------------------------------------------------------------------------------------------
 // 4. Unordered overlapping non-neighbouring face pairs
 // ------------------------------------------------------------------------------------------------
-// KDOPBroadPhase.cpp:132-137: disjoint iff some axis separates them strictly.
-__device__ __forceinline__ bool overlap64(const double *__restrict__ a, const double *__restrict__ b)
-{
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < KAX; k++) ok = ok && !(a[KAX + k] < b[k] || b[KAX + k] < a[k]);
-    return ok;
-}
 __device__ __forceinline__ bool neighbours(int4 a, int4 b)   // Mesh.cpp:13-20
 {
     return a.x == b.x || a.x == b.y || a.x == b.z || a.y == b.x || a.y == b.y || a.y == b.z || a.z == b.x ||
            a.z == b.y || a.z == b.z;
 }
 
-// One wavefront finds the pairs of one cluster's 64 sorted leaves (one per lane) with the leaves that
-// follow them: it looks for the clusters its cluster's box meets, 64 records per step (one per lane),
-// and tests each such cluster as a 64 x 64 tile.  In a tile, each lane first tests its own leaf of the
-// target cluster against the query cluster's box; the leaves that pass are broadcast one by one
-// (readlane) and tested against all 64 queries at once.  So every step of the search decides 64 box tests
-// from one load, and no step waits for the one before it but for the ballot: a tree walk by one
-// wavefront is a chain of dependent record loads (1.05 ms on the 256^2 cloth, 25.6 ms on a 1024^2 sheet with
-// 64 leaves per wavefront; here 0.34 and 15.6 ms, and 0.05 instead of 0.48 ms on a 97^2 cloth).
+// The related faces of every face, as rows (CSR) in sorted leaf order: row i describes the sorted leaves j
+// that overlap leaf i without sharing a vertex with it (both directions of every pair), as tiles: a
+// cluster's number and the 64-bit mask of its related leaves.  A tile holds several related faces, and
+// the union of rows is an OR of masks.
+//
+// One wavefront finds the rows of one cluster's 64 sorted leaves (one per lane): it looks for the clusters
+// its cluster's box meets, 64 records per step (one per lane), and tests each such cluster as a 64 x 64
+// tile.  In a tile, each lane first tests its own leaf of the target cluster against the query cluster's
+// box; the leaves that pass are broadcast one by one (readlane) and tested against all 64 queries at
+// once.  So every step of the search decides 64 box tests from one load, and no step waits for the one
+// before it but for the ballot: a tree walk by one wavefront is a chain of dependent record loads.
 //
 // The pairs that pass are queued in LDS and finished 64 at a time, so that the FP64 test runs with full
 // wavefronts: the shared-vertex test (Mesh.cpp:13-20), then the reference's 13-axis test (touching
@@ -526,19 +523,24 @@ __device__ __forceinline__ bool neighbours(int4 a, int4 b)   // Mesh.cpp:13-20
 // qhi = ceil(x) > x - and so x > qhi - 1 -, qlo = floor(y) and so y < qlo + 1, qhi - 1 >= qlo + 1 gives
 // x > y, and the map to x is monotone, so the FP64 bounds overlap as well (the clamps keep this: a
 // clamped qhi = 65535 has x >= 65535, a clamped qlo = 0 has y < 1, a NaN bound never separates, and
-// the other clamps fail the test).  Accepted pairs wait in LDS too; a claim on the output counter covers
-// several hundred (one counter claimed per 64 pairs would serialise the device).
+// the other clamps fail the test).
 //
-// Small meshes have few clusters; `slices` wavefronts then share one, each taking every slices-th of the
-// target clusters.
-// For batched instances a query pairs only with leaves before its instance's end (face_inst /
-// inst_off; its faces are the sorted range [inst_off[k], inst_off[k + 1])).
-constexpr int PAIR_BLOCK = 256;
-constexpr int PAIR_QUEUE = 128;   // quantised hits waiting for the exact test (below 64 after a flush)
-constexpr int PAIR_OUT = 512;     // accepted pairs waiting to be written
-struct PairLds {
-    int2 queue[PAIR_QUEUE];   // (query lane, target leaf)
-    int2 out[PAIR_OUT];
+// The search keeps the tiles it finds in the order it finds them, and counts them by row; after a scan of
+// the counts a second run puts them into their rows.  A row belongs to one wavefront, or to the `slices`
+// wavefronts that share its cluster, each taking every slices-th of the target clusters with a count and a
+// part of the row of its own: no counter in memory is shared.  Writing each pair once, from its lower leaf, and building the rows from the pairs afterwards
+// took two atomics per pair and pass and a claim on one counter per wavefront (about 10 ns each, one after
+// another): 76 ms on a 1024^2 sheet with 31M tiles, and 7.7 ms on 128 instances with 3.8M; here 14.3 and
+// 1.75 ms, of which placing the tiles is 0.6 and 0.14 (searching a second time instead: 13.4 and 1.5).
+// For batched instances a query pairs only with leaves of its instance (face_inst / inst_off; its faces
+// are the sorted range [inst_off[k], inst_off[k + 1])).
+constexpr int ROW_BLOCK = 256;
+constexpr int ROW_QUEUE = 128;   // quantised hits waiting for the exact test (below 64 after a flush)
+struct RowLds {
+    unsigned long long mask[64];   // each query's related leaves of the tile
+    ulonglong2 staged[128];        // records waiting to be written
+    int count[64];                 // tiles placed so far, by query
+    uint16_t queue[ROW_QUEUE];     // query lane + 64 * target lane
 };
 
 // Orders a wavefront's LDS accesses (its own region; one wavefront's LDS instructions execute in order,
@@ -550,19 +552,18 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-struct PairOut {
-    int2 *__restrict__ pairs;
-    int64_t cap;
-    unsigned long long *counter;
-};
-__device__ __forceinline__ void pairs_write(PairLds &L, int n, const PairOut &o)
+__device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ int64_t read_lane(int64_t v, int l)
 {
-    const int lane = __lane_id();
-    unsigned long long base = 0;
-    if (lane == 0) base = atomicAdd(o.counter, (unsigned long long)n);
-    base = __shfl(base, 0);
-    for (int k = lane; k < n; k += 64)
-        if ((int64_t)base + k < o.cap) o.pairs[base + k] = L.out[k];
+    return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)v, l) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32);
+}
+
+__device__ __forceinline__ int64_t wave_sum(int64_t v)
+{
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
+    return v;
 }
 
 // Certainly overlapping: two quanta or more on every axis.
@@ -578,7 +579,8 @@ __device__ __forceinline__ bool boxes_meet_surely(const Box16 &a, const Box16 &b
     }
     return ok;
 }
-// overlap64 with every comparison evaluated (no early exit: the loads of a part issue together).  Two
+// Disjoint iff some axis separates them strictly (KDOPBroadPhase.cpp:132-137), with every comparison of a
+// part evaluated (no early exit: the loads of a part issue together).  Two
 // parts: all 52 doubles at once would take 159 registers, three wavefronts per SIMD.
 __device__ __forceinline__ bool overlap64_all(const double *__restrict__ a, const double *__restrict__ b)
 {
@@ -600,56 +602,49 @@ __device__ __forceinline__ bool overlap64_all(const double *__restrict__ a, cons
     return ok;
 }
 
-// The exact test of queue[from .. from + n), n <= 64; accepted pairs are appended to out.
-__device__ __forceinline__ void pairs_test(PairLds &L, int from, int n, int64_t i0, const BoxRec *__restrict__ leaves,
-                                           const double *__restrict__ sdop64, const int4 *__restrict__ sfaces, int &nout,
-                                           const PairOut &o)
-{
-    const int lane = __lane_id();
-    bool ok = lane < n;
-    int2 pr = make_int2(0, 0);
-    if (ok) {
-        const int2 e = L.queue[from + lane];
-        const int64_t i = i0 + e.x, j = e.y;
-        const int4 qf = sfaces[i], of = sfaces[j];
-        pr = qf.w < of.w ? make_int2(qf.w, of.w) : make_int2(of.w, qf.w);
-        ok = !neighbours(qf, of);
-        if (ok) {
-            Box16 a, b;
-            load_box(leaves, i, a);
-            load_box(leaves, j, b);
-            if (!boxes_meet_surely(a, b)) ok = overlap64_all(sdop64 + NB * i, sdop64 + NB * j);
-        }
-    }
-    const uint64_t m = __ballot(ok);
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    if (nout + __popcll(m) > PAIR_OUT) {
-        wave_lds_order();
-        pairs_write(L, nout, o);
-        wave_lds_order();
-        nout = 0;
-    }
-    if (ok) L.out[nout + __popcll(m & lt)] = pr;
-    nout += __popcll(m);
-}
-
-struct PairLevels {
+// The rows' tiles.
+struct Rows {
+    uint64_t *mask;
+    int32_t *cluster;
+    int64_t cap;
+};
+// What the first run finds, kept for the second one: segments of records, the last one of a wavefront known
+// by its head and each holding the place of the one before it.  They lie in the edge-edge keys' buffer,
+// which nothing writes before the rows are complete; each shard of it has a counter of its own (one counter:
+// about 10 ns per claim, one after another).  A wavefront whose shard is used up keeps nothing and searches
+// again.
+constexpr int REC_SHARDS = 64, REC_STRIDE = 8;   // (a counter per 64 bytes)
+constexpr unsigned long long REC_NONE = ~0ull, REC_LOST = ~1ull;
+struct RowRecords {
+    ulonglong2 *rec;               // mask, cluster | query lane << 32; first of a segment: the one before it
+    ulonglong2 *head;              // [wavefronts] last segment: its place (or REC_NONE, REC_LOST), its records
+    unsigned long long *claimed;   // [shards * REC_STRIDE]
+    int64_t per_shard;
+};
+struct RowLevels {
     const BoxRec *rec[4];   // leaves, clusters, groups, level 3 (levels above `top` unused)
     int64_t n[4];
     int top;                // the level scanned from end to end
 };
 
-__global__ __launch_bounds__(PAIR_BLOCK) void k_pairs(PairLevels lv, int slices, const double *__restrict__ sdop64,
-                                                      const int4 *__restrict__ sfaces,
-                                                      const int32_t *__restrict__ face_inst,
-                                                      const int64_t *__restrict__ inst_off, PairOut o)
+// off: [leaf * slices + slice], the tiles in the parts of the rows, or (FILL) their starts; pairs (may be
+// null): the related faces in them that come after their row's own.
+template <bool FILL>
+__global__ __launch_bounds__(ROW_BLOCK, 4) void k_rows(RowLevels lv, int slices, const double *__restrict__ sdop64,
+                                                    const int4 *__restrict__ sfaces,
+                                                    const int32_t *__restrict__ face_inst,
+                                                    const int64_t *__restrict__ inst_off, int64_t *__restrict__ off,
+                                                    int32_t *__restrict__ pairs, Rows rows, RowRecords kept)
 {
-    __shared__ PairLds s_lds[PAIR_BLOCK / 64];
-    PairLds &L = s_lds[threadIdx.x >> 6];
+    __shared__ RowLds s_lds[ROW_BLOCK / 64];
+    RowLds &L = s_lds[threadIdx.x >> 6];
     const int lane = __lane_id();
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     const int F = (int)lv.n[0];   // below 2^30
-    const int64_t wave = blockIdx.x * (int64_t)(PAIR_BLOCK / 64) + (threadIdx.x >> 6);
+    // (consecutive blocks run on different XCDs: each gets a contiguous part of the clusters)
+    const int64_t nb = gridDim.x >> 3;
+    const int64_t block = blockIdx.x < 8 * nb ? (blockIdx.x & 7) * nb + (blockIdx.x >> 3) : blockIdx.x;
+    const int64_t wave = block * (ROW_BLOCK / 64) + (threadIdx.x >> 6);
     const int c = __builtin_amdgcn_readfirstlane((int)(wave / slices));   // the query cluster
     const int slice = __builtin_amdgcn_readfirstlane((int)(wave % slices));
     if (c >= lv.n[1]) return;   // the whole wavefront
@@ -658,23 +653,96 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_pairs(PairLevels lv, int slices,
     Box16 q, cb;
     load_box(leaves, i < F ? i : F - 1, q);
     load_box(lv.rec[1], c, cb);
-    int iend = 0;   // lanes past the leaves accept none
-    if (i < F) iend = face_inst ? (int)inst_off[face_inst[sfaces[i].w] + 1] : F;
-    int jmax = iend;
+    int ibeg = 0x7fffffff, iend = 0;   // lanes past the leaves accept none
+    if (i < F) {
+        ibeg = 0;
+        iend = F;
+        if (face_inst) {
+            const int k = face_inst[sfaces[i].w];
+            ibeg = (int)inst_off[k];
+            iend = (int)inst_off[k + 1];
+        }
+    }
+    int jmin = ibeg, jmax = iend;
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) {
-        const int x = __shfl_xor(jmax, d);
-        jmax = x > jmax ? x : jmax;
+        const int x = __shfl_xor(jmin, d), y = __shfl_xor(jmax, d);
+        jmin = x < jmin ? x : jmin;
+        jmax = y > jmax ? y : jmax;
     }
+    jmin = __builtin_amdgcn_readfirstlane(jmin);
     jmax = __builtin_amdgcn_readfirstlane(jmax);
-    const int tlast = (jmax - 1) >> 6;   // the last cluster any lane pairs with (jmax > i0 >= 0)
-    int nq = 0, nout = 0, turn = 0;
+    const int tfirst = jmin >> 6, tlast = (jmax - 1) >> 6;   // the clusters any lane pairs with
+    int64_t row = 0;   // FILL: where this lane's part of the row starts
+    if (FILL && i < F) row = off[(int64_t)i * slices + slice];
+    int ntiles = 0, npairs = 0, turn = 0;
+    if (FILL) {
+        ulonglong2 seg = kept.head[wave];
+        if (seg.x != REC_LOST) {   // the tiles that the first run kept
+            L.count[lane] = 0;
+            wave_lds_order();
+            while (seg.x != REC_NONE) {
+                const ulonglong2 *r = kept.rec + seg.x;
+                const int n = (int)seg.y;
+                seg = r[0];
+                for (int k = lane; k < n; k += 64) {
+                    const ulonglong2 e = r[1 + k];
+                    const int ql = (int)(e.y >> 32);
+                    const int64_t at = off[(int64_t)(i0 + ql) * slices + slice] + atomicAdd(&L.count[ql], 1);
+                    if (at < rows.cap) {
+                        rows.mask[at] = e.x;
+                        rows.cluster[at] = (int32_t)e.y;
+                    }
+                }
+            }
+            return;
+        }
+    }
+    // !FILL: the last segment written, and the records waiting.
+    unsigned long long last = REC_NONE;
+    int last_n = 0, staged = 0;
+    auto write_segment = [&]() {
+        wave_lds_order();
+        const int shard = (int)(wave & (REC_SHARDS - 1));
+        unsigned long long got = 0;
+        if (lane == 0) got = atomicAdd(&kept.claimed[shard * REC_STRIDE], (unsigned long long)staged + 1);
+        got = (unsigned long long)read_lane((int64_t)got, 0);
+        if ((int64_t)got + staged + 1 <= kept.per_shard) {
+            ulonglong2 *r = kept.rec + shard * kept.per_shard + got;
+            if (lane == 0) r[0] = make_ulonglong2(last, last_n);
+            for (int k = lane; k < staged; k += 64) r[1 + k] = L.staged[k];
+            last = shard * kept.per_shard + got;
+            last_n = staged;
+        } else {
+            last = REC_LOST;
+        }
+        staged = 0;
+        wave_lds_order();
+    };
+    L.mask[lane] = 0;
 
+    // The exact test of queue[from .. from + n), n <= 64.
+    auto test = [&](int t, int from, int n) {
+        wave_lds_order();
+        if (lane < n) {
+            const int e = L.queue[from + lane], ql = e & 63, iq = i0 + ql, j = t * 64 + (e >> 6);
+            bool ok = !neighbours(sfaces[iq], sfaces[j]);
+            if (ok) {
+                Box16 x, y;
+                load_box(leaves, iq, x);
+                load_box(leaves, j, y);
+                if (!boxes_meet_surely(x, y)) ok = overlap64_all(sdop64 + NB * (int64_t)iq, sdop64 + NB * (int64_t)j);
+            }
+            if (ok) atomicOr(&L.mask[ql], 1ull << (e >> 6));
+        }
+        wave_lds_order();
+    };
     auto tile = [&](int t) {
         const int j = t * 64 + lane;
         Box16 b;
         load_box(leaves, j < F ? j : F - 1, b);
-        for (uint64_t m = __ballot(j < jmax && boxes_meet(b, cb)); m; m &= m - 1) {
+        int nq = 0;
+        for (uint64_t m = __ballot(j >= jmin && j < jmax && boxes_meet(b, cb)); m; m &= m - 1) {
             const int s = __ffsll((unsigned long long)m) - 1;
             const int js = t * 64 + s;
             uint32_t sep = 0;
@@ -683,61 +751,76 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_pairs(PairLevels lv, int slices,
                 const uint32_t tlo = __builtin_amdgcn_readlane(b.lo[w], s), thi = __builtin_amdgcn_readlane(b.hi[w], s);
                 sep |= exceeds(tlo, q.hi[w]) | exceeds(q.lo[w], thi);
             }
-            const bool hit = (sep == 0) & (js > i) & (js < iend);
+            const bool hit = (sep == 0) & (js != i) & (js >= ibeg) & (js < iend);
             const uint64_t h = __ballot(hit);
             if (h == 0) continue;
-            if (hit) L.queue[nq + __popcll(h & lt)] = make_int2(lane, js);
+            if (hit) L.queue[nq + __popcll(h & lt)] = (uint16_t)(lane | s << 6);
             nq += __popcll(h);
             if (nq >= 64) {
-                wave_lds_order();
-                pairs_test(L, nq - 64, 64, i0, leaves, sdop64, sfaces, nout, o);
-                wave_lds_order();
+                test(t, nq - 64, 64);
                 nq -= 64;
             }
         }
+        if (nq) test(t, 0, nq);
+        const uint64_t mine = L.mask[lane];
+        if (!FILL && last != REC_LOST) {
+            const uint64_t some = __ballot(mine != 0);
+            if (mine) L.staged[staged + __popcll(some & lt)] = make_ulonglong2(mine, (uint32_t)t | (uint64_t)lane << 32);
+            staged += __popcll(some);
+            if (staged >= 64) write_segment();
+        }
+        if (mine) {
+            L.mask[lane] = 0;
+            if (FILL && row + ntiles < rows.cap) {
+                rows.mask[row + ntiles] = mine;
+                rows.cluster[row + ntiles] = t;
+            }
+            ntiles++;
+            if (pairs) npairs += __popcll(t > c ? mine : (t == c ? mine & ~(lt << 1 | 1ull) : 0ull));   // j > i
+        }
+        wave_lds_order();
     };
     // The clusters of the 64 records [base, base + 64) of level 1 that the query cluster's box meets.
     auto scan1 = [&](int base) {
         const int t = base + lane;
         Box16 b;
         load_box(lv.rec[1], t < lv.n[1] ? t : lv.n[1] - 1, b);
-        for (uint64_t m = __ballot(t >= c && t <= tlast && boxes_meet(b, cb)); m; m &= m - 1) {
+        for (uint64_t m = __ballot(t >= tfirst && t <= tlast && boxes_meet(b, cb)); m; m &= m - 1) {
             const int tt = base + __ffsll((unsigned long long)m) - 1;
             if (turn == slice) tile(tt);
             turn = turn + 1 == slices ? 0 : turn + 1;
         }
     };
-    auto scan2 = [&](int base) {
-        const int t = base + lane;
-        Box16 b;
-        load_box(lv.rec[2], t < lv.n[2] ? t : lv.n[2] - 1, b);
-        for (uint64_t m = __ballot(t >= (c >> 6) && t <= (tlast >> 6) && boxes_meet(b, cb)); m; m &= m - 1)
-            scan1((base + __ffsll((unsigned long long)m) - 1) << 6);
-    };
-    auto scan3 = [&](int base) {
-        const int t = base + lane;
-        Box16 b;
-        load_box(lv.rec[3], t < lv.n[3] ? t : lv.n[3] - 1, b);
-        for (uint64_t m = __ballot(t >= (c >> 12) && t <= (tlast >> 12) && boxes_meet(b, cb)); m; m &= m - 1)
-            scan2((base + __ffsll((unsigned long long)m) - 1) << 6);
-    };
+    // Level `lv.top` from end to end, then down to level 1 below the records that the box meets.
     const int up = 6 * (lv.top - 1);
-    const int last = tlast >> up;
-    for (int base = (c >> up) & ~63; base <= last; base += 64) {
-        if (lv.top == 1)
+    for (int base = (tfirst >> up) & ~63; base <= (tlast >> up); base += 64) {
+        if (lv.top == 1) {
             scan1(base);
-        else if (lv.top == 2)
-            scan2(base);
-        else
-            scan3(base);
+            continue;
+        }
+        const int t = base + lane;
+        Box16 b;
+        load_box(lv.rec[lv.top], t < lv.n[lv.top] ? t : lv.n[lv.top] - 1, b);
+        for (uint64_t m = __ballot(t >= (tfirst >> up) && t <= (tlast >> up) && boxes_meet(b, cb)); m; m &= m - 1) {
+            const int t2 = base + __ffsll((unsigned long long)m) - 1;
+            if (lv.top == 2) {
+                scan1(t2 << 6);
+                continue;
+            }
+            const int u = (t2 << 6) + lane;
+            Box16 b2;
+            load_box(lv.rec[2], u < lv.n[2] ? u : lv.n[2] - 1, b2);
+            for (uint64_t m2 = __ballot(u >= (tfirst >> 6) && u <= (tlast >> 6) && boxes_meet(b2, cb)); m2; m2 &= m2 - 1)
+                scan1(((t2 << 6) + __ffsll((unsigned long long)m2) - 1) << 6);
+        }
     }
-    if (nq) {
-        wave_lds_order();
-        pairs_test(L, 0, nq, i0, leaves, sdop64, sfaces, nout, o);
+    if (!FILL) {
+        if (staged) write_segment();
+        if (lane == 0) kept.head[wave] = make_ulonglong2(last, last_n);
     }
-    if (nout) {
-        wave_lds_order();
-        pairs_write(L, nout, o);
+    if (!FILL && i < F) {
+        off[(int64_t)i * slices + slice] = ntiles;
+        if (pairs) pairs[(int64_t)i * slices + slice] = npairs;
     }
 }
 
@@ -786,166 +869,88 @@ __global__ void k_mesh_check(const int32_t *__restrict__ faces, int64_t F, const
     if (bad) atomicAdd(flag, 1ull);
 }
 
-// Edge -> opposite face: opp[3f + s] is the other face on edge (v[s], v[s+1]) of face f, -1 on a
-// boundary edge, -2 on an edge shared by more than two faces (the expansion then scans the vertex ->
-// face table for that pair, as it does for every pair without this table).
-__global__ __launch_bounds__(256) void k_edge_opp(const int32_t *__restrict__ faces, int64_t F,
-                                                  const int32_t *__restrict__ off, const int32_t *__restrict__ list,
-                                                  int32_t *__restrict__ opp)
+// Edges of the mesh, faces by their rows (sorted leaves): half-edge 3i + s is edge (v[s], v[s+1]) of face i.
+// edge: the edge's number, the smallest of its half-edges; other: the other face on it, -1 on a boundary
+// edge, -2 where there are more.
+struct FaceEdges {
+    uint32_t edge[3];
+    int32_t other[3];
+    int32_t pad[2];
+};
+__global__ __launch_bounds__(256) void k_edges(const int4 *__restrict__ sfaces, int64_t F, const int32_t *__restrict__ faces,
+                                               const int32_t *__restrict__ off, const int32_t *__restrict__ list,
+                                               const int32_t *__restrict__ rank, FaceEdges *__restrict__ edges)
 {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= 3 * F) return;
-    int64_t f = i / 3;
-    int s = (int)(i - 3 * f);
-    int a = faces[i], b = faces[3 * f + (s + 1) % 3];
+    const int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (x >= 3 * F) return;
+    const int i = (int)(x / 3), s = (int)(x - 3 * (int64_t)i);
+    const int4 A = sfaces[i];
+    const int a = s == 0 ? A.x : (s == 1 ? A.y : A.z), b = s == 0 ? A.y : (s == 1 ? A.z : A.x);
     int found = -1, n = 0;
+    uint32_t c = (uint32_t)x;   // (half-edge numbers need 32 bits: 3 * 2^30)
     for (int k = off[a]; k < off[a + 1]; k++) {
-        int h = list[k];
-        if (h == (int)f) continue;
-        if (faces[3 * h] == b || faces[3 * h + 1] == b || faces[3 * h + 2] == b) {
-            found = h;
-            n++;
+        const int h = list[k];
+        if (h == A.w) continue;
+        const int32_t *v = faces + 3 * (int64_t)h;
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            const int p = v[e], q = v[(e + 1) % 3];
+            if ((p == a && q == b) || (p == b && q == a)) {
+                found = rank[h];
+                n++;
+                const uint32_t g = (uint32_t)(3 * (int64_t)found + e);
+                c = g < c ? g : c;
+            }
         }
     }
-    opp[i] = n > 1 ? -2 : found;
+    edges[i].edge[s] = c;
+    edges[i].other[s] = n > 1 ? -2 : found;
 }
 
 // ------------------------------------------------------------------------------------------------
-// 5. Stencil expansion with owner-computes deduplication
+// 5. Stencil expansion: unions of rows
 // ------------------------------------------------------------------------------------------------
+// The pair of faces {a, b} generates the six vertex-face stencils (a's vertices, b) and (b's vertices, a)
+// and the nine edge-edge stencils (KDOPBroadPhase.cpp:150-184); different pairs generate the same ones.
+// Gathered by feature instead, each comes out once:
+//   * vertex p has the stencils (p, g) for the faces g in the union of the rows of the faces around p;
+//   * edge u has the stencils (u, w) for the edges w of the faces in the union of the rows of the faces on
+//     u; both u and w see each other, so the one with the smaller number has the stencil.  An edge w of two
+//     faces of the union counts at the one that gives it its number.
+// (Faces in a row share no vertex with its face, so g does not hold p, and w shares no vertex with u.)
+// One wavefront takes a vertex or an edge and ORs its rows' tiles into a table in LDS, by cluster; the set
+// bits, numbered across the table, are then shared out over the lanes.  Counts, a scan, and a second run
+// that writes the keys: no shared counter.
+//
+// Deciding for each pair by itself which of its fifteen stencils no smaller pair generates takes up to 39
+// membership tests in other faces' sorted rows: 99.5 ms on a 1024^2 sheet with 1.15G stencils, 4.5 ms on 128
+// instances with 92M (and minutes where rows of more than 2,048 faces were searched linearly); here 29 ms
+// and 3.9 ms.  Writing the keys is 18 GB at 1.2 TB/s on the sheet: the instructions around it bound it, about
+// 300 a feature.
+//
+// A feature whose rows name more clusters than the table takes goes through it several times, each time
+// with one class of the clusters, by the upper bits of a hash.  The edge rule asks for faces of other
+// classes, so such an edge looks them up in its rows instead of the table.
+constexpr int UNION_BLOCK = 256;
+constexpr int TABLE_SLOTS = 512;
+struct UnionTable {
+    unsigned long long mask[TABLE_SLOTS];
+    uint32_t cluster[TABLE_SLOTS];   // ~0u: empty
+    int list[128];                   // faces waiting to be written (below 64 after a batch)
+};
 struct MeshView {
     const int32_t *faces;
     const int32_t *vf_off;
     const int32_t *vf_list;
-    const double *dop64;   // by original face id
     const uint8_t *fixed;
-    const int32_t *adj_off = nullptr;   // [F + 1] related-face table rows, or null (no table)
-    const int32_t *adj = nullptr;       // [2 * pairs]
-    const int32_t *opp = nullptr;       // [3F] edge -> opposite face (k_edge_opp), or null
-    const int32_t *rank = nullptr;      // [F] face id -> Morton-sorted position
-    const double *sdop64 = nullptr;     // FP64 bounds in Morton order
-    const int4 *sfaces = nullptr;       // vertex triples and face id in Morton order
+    const FaceEdges *edges;   // by row
+    const int32_t *rank;      // [F] face -> its row
+    const int4 *sfaces;       // vertices and face id by row
+    const int64_t *off;       // [F * slices + 1] parts of the rows
+    Rows rows;
+    int slices;
 };
-
-__global__ __launch_bounds__(256) void k_adj_count(const int2 *__restrict__ pairs,
-                                                   const unsigned long long *__restrict__ np_dev, int64_t cap,
-                                                   int64_t F, int32_t *__restrict__ cnt)
-{
-    int64_t np = (int64_t)*np_dev;
-    if (np > cap) np = cap;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < np; i += (int64_t)gridDim.x * blockDim.x) {
-        int2 p = pairs[i];
-        atomicAdd(&cnt[p.x], 1);
-        atomicAdd(&cnt[p.y], 1);
-    }
-}
-
-// cnt holds the row lengths on entry and is counted back down to zero.
-__global__ __launch_bounds__(256) void k_adj_fill(const int2 *__restrict__ pairs,
-                                                  const unsigned long long *__restrict__ np_dev, int64_t cap, int64_t F,
-                                                  const int32_t *__restrict__ off, int32_t *__restrict__ cnt,
-                                                  int32_t *__restrict__ adj)
-{
-    int64_t np = (int64_t)*np_dev;
-    if (np > cap) np = cap;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < np; i += (int64_t)gridDim.x * blockDim.x) {
-        int2 p = pairs[i];
-        adj[off[p.x] + atomicSub(&cnt[p.x], 1) - 1] = p.y;
-        adj[off[p.y] + atomicSub(&cnt[p.y], 1) - 1] = p.x;
-    }
-}
-
-__device__ __forceinline__ int4 face3(const MeshView &m, int f)
-{
-    return make_int4(m.faces[3 * f], m.faces[3 * f + 1], m.faces[3 * f + 2], f);
-}
-// Rows of the related-face table up to this length are sorted (k_row_sort); longer ones stay in fill
-// order and are searched linearly.
-constexpr int ROW_SORT_CAP = 2048;
-
-// Related faces: overlapping swept k-DOPs and no shared vertex, i.e. exactly the face pairs the
-// traversal found.  ROWS: b is in a's row of the related-face table (binary search in the sorted row);
-// otherwise the FP64 test is repeated on the two faces' bounds (when there is no table).
-template <bool ROWS>
-__device__ __forceinline__ bool related(const MeshView &m, int a, int b)
-{
-    if (ROWS) {
-        const int end = m.adj_off[a + 1];
-        int lo = m.adj_off[a], hi = end;
-        if (hi - lo > ROW_SORT_CAP) {
-            for (int k = lo; k < hi; k++)
-                if (m.adj[k] == b) return true;
-            return false;
-        }
-        while (lo < hi) {   // first entry not below b
-            const int mid = (lo + hi) >> 1;
-            if (m.adj[mid] < b)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        return lo < end && m.adj[lo] == b;
-    }
-    if (m.rank) {   // the Morton-ordered copies: spatially close faces share cache lines
-        int ra = m.rank[a], rb = m.rank[b];
-        return !neighbours(m.sfaces[ra], m.sfaces[rb]) &&
-               overlap64(m.sdop64 + NB * (int64_t)ra, m.sdop64 + NB * (int64_t)rb);
-    }
-    return !neighbours(face3(m, a), face3(m, b)) && overlap64(m.dop64 + NB * (int64_t)a, m.dop64 + NB * (int64_t)b);
-}
-__device__ __forceinline__ bool has_vertex(const MeshView &m, int f, int v)
-{
-    return m.faces[3 * f] == v || m.faces[3 * f + 1] == v || m.faces[3 * f + 2] == v;
-}
 __device__ __forceinline__ bool is_fixed(const MeshView &m, int v) { return m.fixed && m.fixed[v]; }
-
-// VF stencil (p, face h) generated by pair {a, h} for every face a containing p with a related to h;
-// the owner is the smallest such a.  `mine` is the a of the current pair.
-template <bool ROWS>
-__device__ __forceinline__ bool vf_owner(const MeshView &m, int p, int h, int mine)
-{
-    for (int k = m.vf_off[p]; k < m.vf_off[p + 1]; k++) {
-        int a = m.vf_list[k];
-        if (a < mine && related<ROWS>(m, a, h)) return false;
-    }
-    return true;
-}
-
-// EE stencil (edge (u0,u1), edge (w0,w1)) generated by pairs {a, b}, a containing both u's and b both
-// w's, a related to b; the owner is the smallest (min(a,b), max(a,b)).  The current pair is (f < g).
-template <bool ROWS>
-__device__ __forceinline__ bool ee_owner(const MeshView &m, int u0, int u1, int w0, int w1, int f, int g)
-{
-    for (int ka = m.vf_off[u0]; ka < m.vf_off[u0 + 1]; ka++) {
-        int a = m.vf_list[ka];
-        if (!has_vertex(m, a, u1)) continue;
-        for (int kb = m.vf_off[w0]; kb < m.vf_off[w0 + 1]; kb++) {
-            int b = m.vf_list[kb];
-            if (!has_vertex(m, b, w1)) continue;
-            int lo = a < b ? a : b, hi = a < b ? b : a;
-            if (lo < f || (lo == f && hi < g)) {
-                if (related<ROWS>(m, a, b)) return false;
-            }
-        }
-    }
-    return true;
-}
-
-// The same rule from the edge table: the faces on edge u are f and oa, those on edge w are g and ob
-// (-1: none), so the other generating pairs are (f, ob), (oa, g) and (oa, ob).
-__device__ __forceinline__ bool precedes(int a, int b, int f, int g)
-{
-    int lo = a < b ? a : b, hi = a < b ? b : a;
-    return lo < f || (lo == f && hi < g);
-}
-template <bool ROWS>
-__device__ __forceinline__ bool ee_owner_opp(const MeshView &m, int oa, int ob, int f, int g)
-{
-    if (ob >= 0 && precedes(f, ob, f, g) && related<ROWS>(m, f, ob)) return false;
-    if (oa >= 0 && precedes(oa, g, f, g) && related<ROWS>(m, oa, g)) return false;
-    if (oa >= 0 && ob >= 0 && precedes(oa, ob, f, g) && related<ROWS>(m, oa, ob)) return false;
-    return true;
-}
 
 __device__ __forceinline__ int4 vf_key(int p, int a, int b, int c)   // Stencils.h:13-57
 {
@@ -962,530 +967,360 @@ __device__ __forceinline__ int4 ee_key(int a, int b, int c, int d)   // Stencils
     return make_int4(p0, p1, q0, q1);
 }
 
-// Per-pair expansion, for the two cases the row expansion below does not cover: raw emission and meshes
-// whose related-face table does not fit int32 offsets (rows_path false; the owner tests then repeat the
-// FP64 bounds test).  raw_dev: the mesh check's count of degenerate or duplicate faces; nonzero
-// switches every lane to raw emission (all 15 stencils of a pair), deduplicated afterwards by sorting.
+// A bijection of 32-bit words (xor-shifts and odd multipliers).
+__device__ __forceinline__ uint32_t hash32(uint32_t x)
+{
+    x ^= x >> 16;
+    x *= 0x9E3779B1u;
+    x ^= x >> 15;
+    x *= 0x85EBCA6Bu;
+    return x ^ (x >> 16);
+}
+// ORs a tile into a table of `last` + 1 slots (a power of two); false when there is no room.
+__device__ __forceinline__ bool table_or(UnionTable &T, uint32_t last, uint32_t cluster, uint64_t mask)
+{
+    uint32_t h = hash32(cluster) & last;
+    for (uint32_t probe = 0; probe <= last; probe++) {
+        const uint32_t old = atomicCAS(&T.cluster[h], ~0u, cluster);
+        if (old == ~0u || old == cluster) {
+            atomicOr(&T.mask[h], (unsigned long long)mask);
+            return true;
+        }
+        h = (h + 1) & last;
+    }
+    return false;
+}
+__device__ __forceinline__ bool table_has(const UnionTable &T, uint32_t last, int j)
+{
+    const uint32_t cluster = (uint32_t)j >> 6;
+    uint32_t h = hash32(cluster) & last;
+    for (uint32_t probe = 0; probe <= last; probe++) {
+        const uint32_t at = T.cluster[h];
+        if (at == ~0u) return false;
+        if (at == cluster) return (T.mask[h] >> (j & 63)) & 1ull;
+        h = (h + 1) & last;
+    }
+    return false;
+}
+// Inclusive sum over the wavefront's lanes (DPP row shifts and broadcasts: no LDS round trips).
+__device__ __forceinline__ int wave_scan(int x)
+{
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return x;
+}
+// Tiles [start, start + len) of row r.
+__device__ __forceinline__ void row_range(const MeshView &m, int r, int64_t &start, int &len)
+{
+    int64_t z = m.off[(int64_t)(r + 1) * m.slices];
+    start = m.off[(int64_t)r * m.slices];
+    z = z < m.rows.cap ? z : m.rows.cap;
+    len = start < z ? (int)(z - start) : 0;
+}
+// j in the rows of the faces f0 and f1, or (f1 -2) of those around u0 that hold u1, by search (edges whose
+// clusters do not fit the table).
+__device__ bool rows_have(const MeshView &m, int f0, int f1, int u0, int u1, int j)
+{
+    const int star = m.vf_off[u0], n = f1 == -2 ? m.vf_off[u0 + 1] - star : (f1 == -1 ? 1 : 2);
+    for (int k = 0; k < n; k++) {
+        int r = k == 0 ? f0 : f1;
+        if (f1 == -2) {
+            const int f = m.vf_list[star + k];
+            const int32_t *v = m.faces + 3 * (int64_t)f;
+            if (v[0] != u1 && v[1] != u1 && v[2] != u1) continue;
+            r = m.rank[f];
+        }
+        int64_t start;
+        int len;
+        row_range(m, r, start, len);
+        for (int64_t e = start; e < start + len; e++)
+            if (m.rows.cluster[e] == j >> 6 && ((m.rows.mask[e] >> (j & 63)) & 1ull)) return true;
+    }
+    return false;
+}
+
+// Feature x < V is vertex x; V + h the edge of half-edge h (nothing for a half-edge that is not its edge's
+// number).  counts[x]: its stencils (first run) or their offsets (WRITE): vertex-face ones from 0, edge-edge
+// ones from counts[V].  Nothing for meshes with degenerate or duplicate faces (raw emission).
 //
-// Output slots are claimed per block, not per wavefront: each lane first decides which of its 15
-// stencils it emits (two bit masks), the block scans the counts through LDS and one lane claims the
-// block's range with a single atomic per stencil kind.  The counters are single words that every block
-// hits, so per-wavefront claims (15 per wavefront and pass) made their serialisation the bottleneck.
-// The grid-stride loop bound is uniform across a block, so every lane reaches the barriers.
-constexpr int EXPAND_BLOCK = 256;
-__global__ __launch_bounds__(EXPAND_BLOCK) void k_expand(MeshView m, bool rows_path, const int2 *__restrict__ pairs,
-                                                         const unsigned long long *__restrict__ npairs_dev,
-                                                         int64_t pairs_cap, const unsigned long long *__restrict__ raw_dev,
-                                                         int4 *__restrict__ vf_out, int64_t vf_cap,
-                                                         unsigned long long *vf_counter, int4 *__restrict__ ee_out,
-                                                         int64_t ee_cap, unsigned long long *ee_counter)
+// A wavefront takes `chunk` features one after another; what leads to their rows (five dependent loads) is
+// read for all of them at once, one feature or one face around a vertex per lane.
+constexpr int UNION_CHUNK = 16;   // at most
+template <bool WRITE>
+__global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, int64_t V, int chunk,
+                                                       const unsigned long long *__restrict__ raw_dev,
+                                                       int64_t *__restrict__ counts, int4 *__restrict__ vf_out,
+                                                       int64_t vf_cap, int4 *__restrict__ ee_out, int64_t ee_cap)
 {
-    constexpr int NW = EXPAND_BLOCK / 64;
-    __shared__ unsigned s_off[2][NW];
-    __shared__ unsigned long long s_base[2];
-    const bool OWNER = *raw_dev == 0;
-    if (OWNER && rows_path) return;   // the row expansion has it
-    int64_t np = (int64_t)*npairs_dev;
-    if (np > pairs_cap) np = pairs_cap;
-    const int lane = __lane_id(), wave = threadIdx.x >> 6;
-    for (int64_t base = blockIdx.x * (int64_t)EXPAND_BLOCK; base < np; base += (int64_t)gridDim.x * EXPAND_BLOCK) {
-        int64_t i = base + threadIdx.x;
-        bool valid = i < np;
-        int2 pr = valid ? pairs[i] : make_int2(0, 0);
-        int f = pr.x, g = pr.y;
-        int4 F0 = valid ? face3(m, f) : make_int4(0, 0, 0, 0);
-        int4 G0 = valid ? face3(m, g) : make_int4(0, 0, 0, 0);
-        int fv[3] = {F0.x, F0.y, F0.z};
-        int gv[3] = {G0.x, G0.y, G0.z};
-        bool ffix = valid && is_fixed(m, fv[0]) && is_fixed(m, fv[1]) && is_fixed(m, fv[2]);
-        bool gfix = valid && is_fixed(m, gv[0]) && is_fixed(m, gv[1]) && is_fixed(m, gv[2]);
-        int fo[3] = {-2, -2, -2}, go[3] = {-2, -2, -2};
-        if (valid && m.opp) {
-#pragma unroll
-            for (int s = 0; s < 3; s++) {
-                fo[s] = m.opp[3 * (int64_t)f + s];
-                go[s] = m.opp[3 * (int64_t)g + s];
-            }
-        }
-        // 6 vertex-face stencils (KDOPBroadPhase.cpp:157-175): bit 2s for (fv[s], g), 2s+1 for (gv[s], f)
-        unsigned vmask = 0, emask = 0;
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-            int p = fv[s];
-            bool want = valid && !(is_fixed(m, p) && gfix);
-            if (OWNER && want) want = vf_owner<false>(m, p, g, f);
-            if (want) vmask |= 1u << (2 * s);
-            int q = gv[s];
-            want = valid && !(is_fixed(m, q) && ffix);
-            if (OWNER && want) want = vf_owner<false>(m, q, f, g);
-            if (want) vmask |= 1u << (2 * s + 1);
-        }
-        // 9 edge-edge stencils (KDOPBroadPhase.cpp:176-183): bit 3s+r for edges (s, r)
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-            int u0 = fv[s], u1 = fv[(s + 1) % 3];
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                int w0 = gv[r], w1 = gv[(r + 1) % 3];
-                bool want = valid && !(is_fixed(m, u0) && is_fixed(m, u1) && is_fixed(m, w0) && is_fixed(m, w1));
-                if (OWNER && want) {
-                    if (fo[s] != -2 && go[r] != -2)
-                        want = ee_owner_opp<false>(m, fo[s], go[r], f, g);
-                    else
-                        want = ee_owner<false>(m, u0, u1, w0, w1, f, g);
-                }
-                if (want) emask |= 1u << (3 * s + r);
-            }
-        }
-        // Block-wide exclusive offsets: wavefront inclusive scans, then the wavefront totals in LDS.
-        const unsigned nv = __popc(vmask), ne = __popc(emask);
-        unsigned pv = nv, pe = ne;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            unsigned tv = __shfl_up(pv, d), te = __shfl_up(pe, d);
-            if (lane >= d) {
-                pv += tv;
-                pe += te;
-            }
-        }
-        if (lane == 63) {
-            s_off[0][wave] = pv;
-            s_off[1][wave] = pe;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned tv = 0, te = 0;
-#pragma unroll
-            for (int w = 0; w < NW; w++) {
-                unsigned a = s_off[0][w], b = s_off[1][w];
-                s_off[0][w] = tv;
-                s_off[1][w] = te;
-                tv += a;
-                te += b;
-            }
-            s_base[0] = tv ? atomicAdd(vf_counter, (unsigned long long)tv) : 0ull;
-            s_base[1] = te ? atomicAdd(ee_counter, (unsigned long long)te) : 0ull;
-        }
-        __syncthreads();
-        int64_t pos_v = (int64_t)(s_base[0] + s_off[0][wave] + (pv - nv));
-        int64_t pos_e = (int64_t)(s_base[1] + s_off[1][wave] + (pe - ne));
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-            if (vmask & (1u << (2 * s))) {
-                if (pos_v < vf_cap) vf_out[pos_v] = vf_key(fv[s], gv[0], gv[1], gv[2]);
-                pos_v++;
-            }
-            if (vmask & (1u << (2 * s + 1))) {
-                if (pos_v < vf_cap) vf_out[pos_v] = vf_key(gv[s], fv[0], fv[1], fv[2]);
-                pos_v++;
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                if (emask & (1u << (3 * s + r))) {
-                    if (pos_e < ee_cap) ee_out[pos_e] = ee_key(fv[s], fv[(s + 1) % 3], gv[r], gv[(r + 1) % 3]);
-                    pos_e++;
-                }
-            }
-        }
-        __syncthreads();   // s_off / s_base are rewritten by the next pass
-    }
-}
-
-// ---- Row expansion -----------------------------------------------------------------------------
-// The stencils of every face pair, deduplicated by the same owner rule, organised by face: one
-// wavefront per face f walks f's row of the related-face table.  For each related face g it emits the
-// three vertex-face stencils (f's vertices against g) that f owns, and for g > f the nine edge-edge
-// stencils that the pair (f, g) owns.  Every unordered pair is visited from both sides, so each side
-// emits its own vertices' stencils.  The owner tests become membership tests in sorted rows:
-//   - f's own row (related(f, ob));
-//   - the rows of the faces around f's vertices and across f's edges, which every lane of the
-//     wavefront shares (they stay in cache).
-// The per-pair form instead re-reads two 208-byte FP64 bounds per test.  Output slots come from a
-// count pass, an exclusive scan over faces and a write pass that recomputes nothing: the count pass
-// stores each entry's 12-bit emission mask beside the row.  No atomics; the order is deterministic
-// (by face, then by related face).
-//
-// Rows of at most ROW_SORT_CAP entries, sorted ascending in LDS by one wavefront (bitonic network).
-__global__ __launch_bounds__(64) void k_row_sort(const unsigned long long *__restrict__ raw_dev, int64_t F,
-                                                 const int32_t *__restrict__ off, int32_t *__restrict__ adj)
-{
-    __shared__ int32_t s[ROW_SORT_CAP];
-    if (*raw_dev != 0) return;
-    for (int64_t a = blockIdx.x; a < F; a += gridDim.x) {
-        const int lo = off[a], len = off[a + 1] - lo;
-        if (len < 2 || len > ROW_SORT_CAP) continue;   // uniform across the block
-        if (len <= 64) {
-            // One element per lane, the same bitonic network in registers (no LDS round trips or
-            // barriers): lane i and its partner i ^ j keep the smaller value in the lower lane of an
-            // ascending run, the larger in a descending one.
-            const int lane = threadIdx.x;
-            int x = lane < len ? adj[lo + lane] : INT32_MAX;
-#pragma unroll
-            for (int k = 2; k <= 64; k <<= 1) {
-#pragma unroll
-                for (int j = k >> 1; j > 0; j >>= 1) {
-                    const int y = __shfl_xor(x, j);
-                    const bool lower = (lane & j) == 0, up = (lane & k) == 0;
-                    x = (lower == up) ? (x < y ? x : y) : (x < y ? y : x);
-                }
-            }
-            if (lane < len) adj[lo + lane] = x;
-            continue;
-        }
-        int n2 = 2;
-        while (n2 < len) n2 <<= 1;
-        for (int i = threadIdx.x; i < n2; i += 64) s[i] = i < len ? adj[lo + i] : INT32_MAX;
-        __syncthreads();
-        for (int k = 2; k <= n2; k <<= 1) {
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int i = threadIdx.x; i < n2; i += 64) {
-                    const int l = i ^ j;
-                    if (l > i) {
-                        const int x = s[i], y = s[l];
-                        if ((x > y) == ((i & k) == 0)) {
-                            s[i] = y;
-                            s[l] = x;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        for (int i = threadIdx.x; i < len; i += 64) adj[lo + i] = s[i];
-        __syncthreads();   // s is rewritten for the next row
-    }
-}
-
-__device__ __forceinline__ int64_t wave_sum(int64_t v)
-{
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d);
-    return v;
-}
-
-// Write pass of the row expansion: the keys of each entry's emission mask, at the exclusive offsets the
-// scan left in cnt_vf / cnt_ee.  Returns at once for raw emission.
-constexpr int ROWS_BLOCK = 256;
-__global__ __launch_bounds__(ROWS_BLOCK) void k_expand_rows_write(MeshView m, int64_t F,
-                                                                  const unsigned long long *__restrict__ raw_dev,
-                                                                  const uint16_t *__restrict__ mask,
-                                                                  const int64_t *__restrict__ cnt_vf,
-                                                                  const int64_t *__restrict__ cnt_ee,
-                                                                  int4 *__restrict__ vf_out, int64_t vf_cap,
-                                                                  int4 *__restrict__ ee_out, int64_t ee_cap)
-{
-    if (*raw_dev != 0) return;
+    __shared__ UnionTable s_table[UNION_BLOCK / 64];
+    UnionTable &T = s_table[threadIdx.x >> 6];
     const int lane = __lane_id();
-    const int64_t nwaves = (int64_t)gridDim.x * (ROWS_BLOCK / 64);
-    for (int64_t fw = blockIdx.x * (int64_t)(ROWS_BLOCK / 64) + (threadIdx.x >> 6); fw < F; fw += nwaves) {
-        const int f = __builtin_amdgcn_readfirstlane((int)fw);
-        const int lo = m.adj_off[f], hi = m.adj_off[f + 1];
-        const int4 F0 = face3(m, f);
-        const int fv[3] = {F0.x, F0.y, F0.z};
-        int64_t pos_v = cnt_vf[f], pos_e = cnt_ee[f];
-        {
-            for (int base = lo; base < hi; base += 64) {
-                const int k = base + lane;
-                const bool valid = k < hi;
-                const unsigned msk = valid ? mask[k] : 0u;
-                const int4 G0 = valid && msk ? face3(m, m.adj[k]) : make_int4(0, 0, 0, 0);
-                const unsigned nv = __popc(msk & 7u), ne = __popc(msk >> 3);
-                unsigned pv = nv, pe = ne;   // inclusive prefix over the wavefront
-#pragma unroll
-                for (int d = 1; d < 64; d <<= 1) {
-                    const unsigned tv = __shfl_up(pv, d), te = __shfl_up(pe, d);
-                    if (lane >= d) {
-                        pv += tv;
-                        pe += te;
-                    }
-                }
-                int64_t v = pos_v + (pv - nv), e = pos_e + (pe - ne);
-                const int gv[3] = {G0.x, G0.y, G0.z};
-#pragma unroll
-                for (int s = 0; s < 3; s++) {
-                    if (msk & (1u << s)) {
-                        if (v < vf_cap) vf_out[v] = vf_key(fv[s], gv[0], gv[1], gv[2]);
-                        v++;
-                    }
-                }
-#pragma unroll
-                for (int s = 0; s < 3; s++) {
-#pragma unroll
-                    for (int r = 0; r < 3; r++) {
-                        if (msk & (1u << (3 + 3 * s + r))) {
-                            if (e < ee_cap) ee_out[e] = ee_key(fv[s], fv[(s + 1) % 3], gv[r], gv[(r + 1) % 3]);
-                            e++;
-                        }
-                    }
-                }
-                pos_v += __shfl(pv, 63);
-                pos_e += __shfl(pe, 63);
-            }
-        }
-    }
-}
+    const int64_t total = V + 3 * F;
+    const int64_t nb = gridDim.x >> 3;   // (contiguous features per XCD, as in k_rows)
+    const int64_t block = blockIdx.x < 8 * nb ? (blockIdx.x & 7) * nb + (blockIdx.x >> 3) : blockIdx.x;
+    const int64_t x0 = (block * (UNION_BLOCK / 64) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * chunk;
+    if (x0 >= total) return;   // the whole wavefront
 
-// Count pass of the row expansion with the rows its owner tests read cached in LDS: f's own row and
-// those of the faces around f's vertices that precede f.  Every lane of the wavefront searches the same
-// few rows, so they are loaded once, coalesced, and searched in LDS instead of with dependent global
-// loads.  A directory of cached rows sits one entry per lane (face, LDS offset, length); lookups of a
-// face run in converged code with a ballot.  The tests that read other rows (the pair across both
-// edges when f's neighbour follows f; the generic rule for non-manifold edges) and rows that do not
-// fit use the table in global memory.
-constexpr int ROWS_LDS_PER_WAVE = 1536;   // int32 entries per wavefront
-
-struct RowDir {
-    const int32_t *lds;
-    int face = -1;   // this lane's directory entry (-1: none)
-    int off = 0, len = -1;   // its row in lds (len < 0: not cached)
-};
-
-// Directory lookup of a face (wave-uniform `a`, all lanes active): the row's LDS offset and length,
-// or false when the face is not cached.
-__device__ __forceinline__ bool dir_find(const RowDir &d, int a, int &off, int &len)
-{
-    const uint64_t hit = __ballot(d.face == a);
-    if (!hit) return false;
-    const int j = __ffsll((unsigned long long)hit) - 1;
-    off = __shfl(d.off, j);
-    len = __shfl(d.len, j);
-    return len >= 0;
-}
-
-// b in a sorted LDS row.
-__device__ __forceinline__ bool lds_row_has(const int32_t *lds, int off, int len, int b)
-{
-    int lo = off, hi = off + len;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (lds[mid] < b)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo < off + len && lds[lo] == b;
-}
-
-// related(a, b) with a's row from the directory when it is cached (cached: the lookup's result).
-__device__ __forceinline__ bool related_dir(const MeshView &m, const int32_t *lds, bool cached, int off, int len, int a,
-                                           int b)
-{
-    return cached ? lds_row_has(lds, off, len, b) : related<true>(m, a, b);
-}
-
-__global__ __launch_bounds__(ROWS_BLOCK) void k_expand_rows_count(MeshView m, int64_t F,
-                                                                  const unsigned long long *__restrict__ raw_dev,
-                                                                  uint16_t *__restrict__ mask,
-                                                                  int64_t *__restrict__ cnt_vf,
-                                                                  int64_t *__restrict__ cnt_ee)
-{
-    __shared__ int32_t s_rows[ROWS_BLOCK / 64][ROWS_LDS_PER_WAVE];
-    const bool raw = *raw_dev != 0;
-    const int lane = __lane_id();
-    int32_t *lds = s_rows[threadIdx.x >> 6];
-    const int64_t nwaves = (int64_t)gridDim.x * (ROWS_BLOCK / 64);
-    for (int64_t fw = blockIdx.x * (int64_t)(ROWS_BLOCK / 64) + (threadIdx.x >> 6); fw < F; fw += nwaves) {
-        const int f = __builtin_amdgcn_readfirstlane((int)fw);
-        if (raw) {
-            if (lane == 0) cnt_vf[f] = cnt_ee[f] = 0;
-            continue;
-        }
-        const int lo = m.adj_off[f], hi = m.adj_off[f + 1];
-        const int4 F0 = face3(m, f);
-        const int fv[3] = {F0.x, F0.y, F0.z};
-        int fo[3] = {-2, -2, -2};
-        if (m.opp) {
-#pragma unroll
-            for (int s = 0; s < 3; s++) fo[s] = m.opp[3 * (int64_t)f + s];
-        }
-        // Directory: f, then the faces around f's vertices that precede f, each once.
-        RowDir d;
-        d.lds = lds;
-        int nd = 0;
-        auto add = [&](int a) {
-            if (nd < 64 && __ballot(d.face == a) == 0) {
-                if (lane == nd) d.face = a;
-                nd++;
-            }
-        };
-        add(f);
-        // The three stars are loaded lane-parallel (64 entries per load, all three in flight together)
-        // and walked in registers, in the same order as one entry at a time.
-        int sb[3], se[3], sa[3];
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-            sb[s] = m.vf_off[fv[s]];
-            se[s] = m.vf_off[fv[s] + 1];
-        }
-#pragma unroll
-        for (int s = 0; s < 3; s++) sa[s] = sb[s] + lane < se[s] ? m.vf_list[sb[s] + lane] : 0x7fffffff;
-#pragma unroll
-        for (int s = 0; s < 3; s++) {
-            for (int base = sb[s]; base < se[s]; base += 64) {
-                const int a = base == sb[s] ? sa[s] : (base + lane < se[s] ? m.vf_list[base + lane] : 0x7fffffff);
-                const int cnt = se[s] - base < 64 ? se[s] - base : 64;
-                for (int j = 0; j < cnt; j++) {
-                    const int aj = __shfl(a, j);
-                    if (aj < f) add(aj);
-                }
-            }
-        }
-        // The directory holds every face around f's vertices that precedes f unless it overflowed.
-        const bool complete = nd < 64;
-        // Then the faces across f's edges that follow f: the edge-edge owner tests search their rows too
-        // (after the completeness test above, which concerns the faces that precede f).
-#pragma unroll
-        for (int s = 0; s < 3; s++)
-            if (fo[s] > f) add(fo[s]);
-        // Per directory entry: its row in the table, and which of f's vertices it holds (bit s: fv[s];
-        // only for the faces that precede f, the ones the vertex-face owner tests walk).
-        int rlen = 0, src = 0;
-        unsigned vbits = 0;
-        if (lane < nd) {
-            src = m.adj_off[d.face];
-            rlen = m.adj_off[d.face + 1] - src;
-            if (lane > 0 && d.face < f) {
-#pragma unroll
-                for (int s = 0; s < 3; s++)
-                    if (has_vertex(m, d.face, fv[s])) vbits |= 1u << s;
-            }
-        }
-        int incl = rlen;
-#pragma unroll
-        for (int dd = 1; dd < 64; dd <<= 1) {
-            const int t = __shfl_up(incl, dd);
-            if (lane >= dd) incl += t;
-        }
-        if (lane < nd) {
-            d.off = incl - rlen;
-            d.len = (incl <= ROWS_LDS_PER_WAVE && rlen <= ROW_SORT_CAP) ? rlen : -1;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();   // the previous face's reads of lds are done
-        // Row copies four entries at a time: their first 64 elements load together.
-        for (int j0 = 0; j0 < nd; j0 += 4) {
-            int val[4], dst[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int j = (j0 + u) & 63;
-                const int off = __shfl(d.off, j), len = __shfl(d.len, j), from = __shfl(src, j);
-                const bool ok = j0 + u < nd && lane < len;
-                val[u] = ok ? m.adj[from + lane] : 0;
-                dst[u] = ok ? off + lane : -1;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (dst[u] >= 0) lds[dst[u]] = val[u];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int j = (j0 + u) & 63;
-                const int off = __shfl(d.off, j), len = __shfl(d.len, j), from = __shfl(src, j);
-                if (j0 + u < nd)
-                    for (int i = 64 + lane; i < len; i += 64) lds[off + i] = m.adj[from + i];
-            }
-        }
-        unsigned long long star[3];   // directory entries around fv[s] (f excluded)
-#pragma unroll
-        for (int s = 0; s < 3; s++) star[s] = __ballot((vbits >> s) & 1u);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        int f_off = 0, f_len = 0;
-        const bool f_cached = dir_find(d, f, f_off, f_len);
-        int64_t nv = 0, ne = 0;
-        for (int base = lo; base < hi; base += 64) {
-            const int k = base + lane;
-            const bool valid = k < hi;
-            const int g = valid ? m.adj[k] : 0;
-            const int4 G0 = valid ? face3(m, g) : make_int4(0, 0, 0, 0);
-            const int gv[3] = {G0.x, G0.y, G0.z};
-            const bool gfix = valid && is_fixed(m, gv[0]) && is_fixed(m, gv[1]) && is_fixed(m, gv[2]);
-            // KDOPBroadPhase.cpp:157-175 (this side's three): owned unless a face around fv[s] that
-            // precedes f is related to g.
-            unsigned vmask = 0;
-#pragma unroll
-            for (int s = 0; s < 3; s++) {
-                bool own = valid && !(is_fixed(m, fv[s]) && gfix);
-                if (complete) {
-                    for (unsigned long long st = star[s]; st; st &= st - 1) {
-                        const int j = __ffsll(st) - 1;
-                        const int a = __shfl(d.face, j), off = __shfl(d.off, j), len = __shfl(d.len, j);
-                        if (own && related_dir(m, lds, len >= 0, off, len, a, g)) own = false;
-                    }
+    // One feature per lane: its end or ends; the faces around it as part [star, star + n) of the vertex ->
+    // face table, or (an edge of up to two faces) as the tiles of their rows.
+    const int64_t x = x0 + lane;
+    int u0 = 0, u1 = -1, f0 = -1, f1 = -2, star = 0, n = 0, len0 = 0, len1 = 0;
+    int64_t start0 = 0, start1 = 0, out = 0, result = 0;
+    if (lane < chunk && x < total && *raw_dev == 0) {
+        if (WRITE) out = counts[x];
+        bool star_needed = true;
+        if (x < V) {
+            u0 = (int)x;
+        } else {
+            const int64_t h = x - V;
+            f0 = (int)(h / 3);
+            const int s = (int)(h - 3 * (int64_t)f0);
+            star_needed = false;
+            if ((int64_t)m.edges[f0].edge[s] == h) {
+                const int4 A = m.sfaces[f0];
+                u0 = s == 0 ? A.x : (s == 1 ? A.y : A.z);
+                u1 = s == 0 ? A.y : (s == 1 ? A.z : A.x);
+                f1 = m.edges[f0].other[s];
+                if (f1 == -2) {
+                    star_needed = true;
                 } else {
-                    for (int kk = m.vf_off[fv[s]]; kk < m.vf_off[fv[s] + 1]; kk++) {
-                        const int a = m.vf_list[kk];
-                        if (a >= f) continue;
-                        int off = 0, len = 0;
-                        const bool cached = dir_find(d, a, off, len);
-                        if (own && related_dir(m, lds, cached, off, len, a, g)) own = false;
-                    }
-                }
-                if (own) vmask |= 1u << s;
-            }
-            // KDOPBroadPhase.cpp:176-183, for g > f
-            unsigned emask = 0;
-            const bool ee = valid && g > f;
-            int go[3] = {-2, -2, -2};
-            if (ee && m.opp) {
-#pragma unroll
-                for (int r = 0; r < 3; r++) go[r] = m.opp[3 * (int64_t)g + r];
-            }
-            // ee_owner_opp's first two tests depend on one edge each: (f, ob) on g's edge r, (oa, g) on f's
-            // edge s.  Each is evaluated once here, not once per edge pair.
-            bool t_fob[3], t_oag[3];
-#pragma unroll
-            for (int r = 0; r < 3; r++) {
-                const int ob = go[r];
-                t_fob[r] = ee && ob >= 0 && precedes(f, ob, f, g) &&
-                           related_dir(m, lds, f_cached, f_off, f_len, f, ob);
-            }
-            int oa_off[3] = {0, 0, 0}, oa_len[3] = {0, 0, 0};
-            bool oa_cached[3];
-#pragma unroll
-            for (int s = 0; s < 3; s++) {
-                const int oa = fo[s];
-                oa_cached[s] = oa >= 0 && dir_find(d, oa, oa_off[s], oa_len[s]);
-                t_oag[s] = ee && oa >= 0 && precedes(oa, g, f, g) &&
-                           related_dir(m, lds, oa_cached[s], oa_off[s], oa_len[s], oa, g);
-            }
-#pragma unroll
-            for (int s = 0; s < 3; s++) {
-                const int u0 = fv[s], u1 = fv[(s + 1) % 3];
-                const bool ufix = is_fixed(m, u0) && is_fixed(m, u1);
-                const int oa = fo[s];
-#pragma unroll
-                for (int r = 0; r < 3; r++) {
-                    const int w0 = gv[r], w1 = gv[(r + 1) % 3];
-                    if (!ee || (ufix && is_fixed(m, w0) && is_fixed(m, w1))) continue;
-                    const int ob = go[r];
-                    bool own;
-                    if (oa != -2 && ob != -2) {
-                        // ee_owner_opp with the cached rows: the other generating pairs (f, ob),
-                        // (oa, g) and (oa, ob)
-                        own = !t_fob[r] && !t_oag[s];
-                        if (own && oa >= 0 && ob >= 0 && precedes(oa, ob, f, g) &&
-                            related_dir(m, lds, oa_cached[s], oa_off[s], oa_len[s], oa, ob))
-                            own = false;
-                    } else {
-                        own = ee_owner<true>(m, u0, u1, w0, w1, f, g);
-                    }
-                    if (own) emask |= 1u << (3 * s + r);
+                    row_range(m, f0, start0, len0);
+                    if (f1 >= 0) row_range(m, f1, start1, len1);
                 }
             }
-            const unsigned msk = vmask | (emask << 3);
-            if (valid) mask[k] = (uint16_t)msk;
-            nv += __popc(vmask);
-            ne += __popc(emask);
         }
-        nv = wave_sum(nv);
-        ne = wave_sum(ne);
-        if (lane == 0) {
-            cnt_vf[f] = nv;
-            cnt_ee[f] = ne;
+        if (star_needed) {
+            star = m.vf_off[u0];
+            n = m.vf_off[u0 + 1] - star;
+        }
+    }
+    const bool fixed_end = m.fixed && lane < chunk && m.fixed[u0] && (u1 < 0 || m.fixed[u1]);
+    const uint64_t fixed_features = __ballot(fixed_end);
+
+    const int64_t ee_base = WRITE ? counts[V] : 0;
+
+    // Entries [wbase, wbase + 64) of the vertex -> face table, with the faces' rows.
+    int wbase = -128, wlen = 0;
+    int64_t wstart = 0;
+
+    for (uint64_t todo = __ballot(n > 0 || len0 + len1 > 0); todo; todo &= todo - 1) {
+        const int s = __ffsll((unsigned long long)todo) - 1;
+        const bool edge = x0 + s >= V, ufix = (fixed_features >> s) & 1ull;
+        const uint32_t h = edge ? (uint32_t)(x0 + s - V) : 0;
+        const int a0 = read_lane(u0, s), a1 = read_lane(u1, s), fn = read_lane(n, s), fstar = read_lane(star, s);
+        const int l0 = read_lane(len0, s), l1 = read_lane(len1, s);
+        const int64_t s0 = read_lane(start0, s), s1 = read_lane(start1, s);
+        const int64_t first = WRITE ? read_lane(out, s) - (edge ? ee_base : 0) : 0;
+        int64_t room = (edge ? ee_cap : vf_cap) - first;
+        room = room > 0 ? room : 0;
+        int4 *const keys = (edge ? ee_out : vf_out) + first;
+        int64_t found = 0;   // stencils so far
+        int bits = 0;        // classes of clusters: 2^bits, by the hash's upper bits
+        uint32_t slots = TABLE_SLOTS;
+        for (uint32_t cls = 0; cls < (1u << bits); cls++) {
+            bool over = false;
+            auto clear = [&](int entries) {
+                slots = 64;
+                while (slots < TABLE_SLOTS && slots < 2u * (uint32_t)entries) slots <<= 1;
+                if (bits) slots = TABLE_SLOTS;
+                for (uint32_t q = lane; q < slots; q += 64) {
+                    T.cluster[q] = ~0u;
+                    T.mask[q] = 0ull;
+                }
+                wave_lds_order();
+            };
+            auto add = [&](int64_t at) {
+                const uint32_t t = (uint32_t)m.rows.cluster[at];
+                const uint64_t mask = m.rows.mask[at];
+                if (bits == 0 || hash32(t) >> (32 - bits) == cls) over |= !table_or(T, slots - 1, t, mask);
+            };
+            if (fn == 0) {
+                clear(l0 + l1);
+                for (int e = lane; e < l0 + l1; e += 64) add(e < l0 ? s0 + e : s1 + (e - l0));
+            } else {
+                if (fn > 64) clear(TABLE_SLOTS);
+                for (int k0 = 0; k0 < fn; k0 += 64) {
+                    const int at0 = fstar + k0, k = fn - k0 < 64 ? fn - k0 : 64;
+                    if (at0 < wbase || at0 + k > wbase + 64) {
+                        wbase = at0;
+                        wlen = 0;
+                        if ((int64_t)wbase + lane < 3 * F) row_range(m, m.rank[m.vf_list[wbase + lane]], wstart, wlen);
+                    }
+                    const int a = at0 - wbase;
+                    int len = lane >= a && lane < a + k ? wlen : 0;
+                    if (edge && len) {   // those around a0 that hold a1
+                        const int32_t *v = m.faces + 3 * (int64_t)m.vf_list[wbase + lane];
+                        if (v[0] != a1 && v[1] != a1 && v[2] != a1) len = 0;
+                    }
+                    const int incl = wave_scan(len);
+                    const int all = read_lane(incl, 63);
+                    if (fn <= 64) clear(all);
+                    int steps = 1;
+                    while (steps < k) steps <<= 1;
+                    for (int e0 = 0; e0 < all; e0 += 64) {
+                        const int e = e0 + lane;
+                        int row = a;   // the row that holds entry e: the first whose inclusive sum exceeds it
+                        for (int d = steps >> 1; d > 0; d >>= 1) {
+                            const int probe = row + d - 1;
+                            if (__shfl(incl, probe < 63 ? probe : 63) <= e) row += d;
+                        }
+                        row = row < 63 ? row : 63;
+                        const int before = __shfl(incl - len, row);
+                        const int64_t at = __shfl(wstart, row) + (e - before);
+                        if (e < all) add(at);
+                    }
+                }
+            }
+            wave_lds_order();
+            if (__ballot(over)) {   // start again with twice the classes (2^23 of them have at most 512 clusters each)
+                bits++;
+                found = 0;
+                cls = ~0u;
+                continue;
+            }
+            // The faces of the table, 64 at a time.
+            auto batch = [&](int from, int cnt) {
+                const bool valid = lane < cnt;
+                wave_lds_order();
+                const int g = valid ? T.list[from + lane] : 0;
+                const int4 G = m.sfaces[g];
+                auto emit = [&](bool mine, int4 key) {
+                    const uint64_t b = __ballot(mine);
+                    if (WRITE && mine) {
+                        const int64_t pos = found + __builtin_amdgcn_mbcnt_hi((int)(b >> 32), __builtin_amdgcn_mbcnt_lo((int)b, 0));
+                        if (pos < room) keys[pos] = key;
+                    }
+                    found += __popcll(b);
+                };
+                if (!edge) {
+                    emit(valid && !(ufix && m.fixed[G.x] && m.fixed[G.y] && m.fixed[G.z]), vf_key(a0, G.x, G.y, G.z));
+                    return;
+                }
+                const FaceEdges E = m.edges[g];
+#pragma unroll
+                for (int w = 0; w < 3; w++) {
+                    const int w0 = w == 0 ? G.x : (w == 1 ? G.y : G.z), w1 = w == 0 ? G.y : (w == 1 ? G.z : G.x);
+                    bool mine = valid && E.edge[w] > h && !(ufix && m.fixed[w0] && m.fixed[w1]);
+                    if (mine && E.edge[w] != (uint32_t)g * 3u + (uint32_t)w) {
+                        // The number comes from another face: it has the edge if it is in the union.
+                        const int owner = (int)(E.edge[w] / 3u);
+                        auto has = [&](int j) {
+                            return bits == 0 ? table_has(T, slots - 1, j)
+                                             : rows_have(m, (int)(h / 3u), m.edges[h / 3u].other[h % 3u], a0, a1, j);
+                        };
+                        bool in = has(owner);
+                        if (!in && E.other[w] == -2) {
+                            // Several faces: the first of them in the union, by row, has it.
+                            for (int k = m.vf_off[w0]; k < m.vf_off[w0 + 1] && !in; k++) {
+                                const int f = m.vf_list[k], r = m.rank[f];
+                                const int32_t *v = m.faces + 3 * (int64_t)f;
+                                if (r < g && (v[0] == w1 || v[1] == w1 || v[2] == w1)) in = has(r);
+                            }
+                        }
+                        mine = !in;
+                    }
+                    emit(mine, ee_key(a0, a1, w0, w1));
+                }
+            };
+            int waiting = 0;
+            for (uint32_t q0 = 0; q0 < slots; q0 += 64) {
+                const int t = (int)T.cluster[q0 + lane];
+                const int64_t mask = (int64_t)T.mask[q0 + lane];
+                for (uint64_t b = __ballot(mask != 0); b; b &= b - 1) {
+                    const int q = __ffsll((unsigned long long)b) - 1;
+                    const uint64_t mk = (uint64_t)read_lane(mask, q);
+                    if (!WRITE && !edge && !ufix) {
+                        found += __popcll(mk);
+                        continue;
+                    }
+                    if ((mk >> lane) & 1ull)
+                        T.list[waiting + __builtin_amdgcn_mbcnt_hi((int)(mk >> 32), __builtin_amdgcn_mbcnt_lo((int)mk, 0))] =
+                            read_lane(t, q) * 64 + lane;
+                    waiting += __popcll(mk);
+                    if (waiting >= 64) {
+                        batch(waiting - 64, 64);
+                        waiting -= 64;
+                    }
+                }
+            }
+            if (waiting) batch(0, waiting);
+            wave_lds_order();
+        }
+        if (!WRITE && lane == s) result = found;
+    }
+    if (!WRITE && lane < chunk && x < total) counts[x] = result;
+}
+
+// The counters after the scans: the rows' tiles and the stencils.
+__global__ void k_expand_counts(const int64_t *__restrict__ row_total, const int64_t *__restrict__ counts, int64_t V,
+                                const int64_t *__restrict__ total, unsigned long long *c)
+{
+    c[ccdi::C_ROWS] = (unsigned long long)*row_total;
+    if (c[ccdi::C_BAD] == 0) {
+        c[ccdi::C_VF] = (unsigned long long)counts[V];
+        c[ccdi::C_EE] = (unsigned long long)(*total - counts[V]);
+    }
+}
+// Face pairs, from what the parts of the rows hold of them.
+__global__ __launch_bounds__(256) void k_pair_total(const int32_t *__restrict__ pairs, int64_t n, unsigned long long *c)
+{
+    __shared__ int64_t s[4];
+    int64_t v = 0;
+    for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) v += pairs[i];
+    v = wave_sum(v);
+    if (__lane_id() == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(&c[ccdi::C_PAIRS], (unsigned long long)(s[0] + s[1] + s[2] + s[3]));
+}
+
+// Raw emission, for meshes with degenerate or duplicate faces: all fifteen stencils of every pair (but those
+// of fixed vertices), deduplicated afterwards by sorting.  One wavefront per face over its row's later
+// faces; slots claimed with one atomic per stencil kind and step.
+__global__ __launch_bounds__(256) void k_expand_raw(MeshView m, int64_t F, const unsigned long long *__restrict__ raw_dev,
+                                                    int4 *__restrict__ vf_out, int64_t vf_cap,
+                                                    unsigned long long *vf_counter, int4 *__restrict__ ee_out,
+                                                    int64_t ee_cap, unsigned long long *ee_counter)
+{
+    if (*raw_dev == 0) return;
+    const int lane = __lane_id();
+    const int64_t nwaves = (int64_t)gridDim.x * 4;
+    for (int64_t i = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); i < F; i += nwaves) {
+        const int64_t lo = m.off[i * m.slices];
+        int64_t hi = m.off[(i + 1) * m.slices];
+        hi = hi < m.rows.cap ? hi : m.rows.cap;
+        const int4 A = m.sfaces[i];
+        const int fv[3] = {A.x, A.y, A.z};
+        const bool ffix = is_fixed(m, A.x) && is_fixed(m, A.y) && is_fixed(m, A.z);
+        for (int64_t e = lo; e < hi; e++) {   // a tile: one of its leaves per lane
+            const int64_t j = (int64_t)m.rows.cluster[e] * 64 + lane;
+            const bool valid = j > i && ((m.rows.mask[e] >> lane) & 1ull);
+            const int4 B = m.sfaces[valid ? j : 0];
+            const int gv[3] = {B.x, B.y, B.z};
+            const bool gfix = is_fixed(m, B.x) && is_fixed(m, B.y) && is_fixed(m, B.z);
+            auto emit = [&](bool want, int4 key, int4 *out, int64_t cap, unsigned long long *counter) {
+                const uint64_t b = __ballot(want);
+                if (b == 0) return;
+                unsigned long long at = 0;
+                if (lane == 0) at = atomicAdd(counter, (unsigned long long)__popcll(b));
+                at = __shfl(at, 0);
+                const int64_t pos = (int64_t)at + __popcll(b & ((1ull << lane) - 1ull));
+                if (want && pos < cap) out[pos] = key;
+            };
+#pragma unroll
+            for (int s = 0; s < 3; s++) {
+                emit(valid && !(is_fixed(m, fv[s]) && gfix), vf_key(fv[s], gv[0], gv[1], gv[2]), vf_out, vf_cap, vf_counter);
+                emit(valid && !(is_fixed(m, gv[s]) && ffix), vf_key(gv[s], fv[0], fv[1], fv[2]), vf_out, vf_cap, vf_counter);
+#pragma unroll
+                for (int t = 0; t < 3; t++) {
+                    const int a0 = fv[s], a1 = fv[(s + 1) % 3], b0 = gv[t], b1 = gv[(t + 1) % 3];
+                    emit(valid && !(is_fixed(m, a0) && is_fixed(m, a1) && is_fixed(m, b0) && is_fixed(m, b1)),
+                         ee_key(a0, a1, b0, b1), ee_out, ee_cap, ee_counter);
+                }
+            }
         }
     }
 }
@@ -1597,13 +1432,15 @@ struct BPBufs {
     BoxRec *boxes;   // leaf records, then the levels above (level_offsets)
     int4 *sfaces;
     void *sort_tmp;
-    int32_t *adj_cnt = nullptr, *adj_off = nullptr, *adj = nullptr;   // related-face table (null if too large)
-    void *adj_tmp = nullptr;
-    uint16_t *adj_mask = nullptr;                  // per table entry: the row expansion's emission mask
-    int64_t *exp_vf = nullptr, *exp_ee = nullptr;   // per face: stencil counts, then output offsets
-    int2 *pairs;
+    int64_t *row_off;    // parts of the related-face rows: tiles, then starts
+    Rows rows;           // their tiles
+    RowRecords kept;     // the first run's finds
+    int32_t *row_pairs;  // related faces in them (null unless the pairs are counted)
+    int64_t *counts;     // stencils per vertex and half-edge: counts, then offsets
+    int64_t *totals;     // their sum
+    void *scan_tmp;
     int4 *vfk, *eek;
-    int32_t *opp;    // edge -> opposite face, 3F (kept with the vertex -> face table for refits)
+    FaceEdges *edges;   // by row (kept with the vertex -> face table for refits)
     int32_t *rank;   // face id -> Morton-sorted position
 };
 // Where each level's records start in BPBufs::boxes, and their number: level 0 the leaves, each level
@@ -1627,6 +1464,19 @@ static LevelOffsets level_offsets(int64_t F)
 constexpr int NPARTS = 512;
 constexpr int QPARTS = 4096;   // blocks of the quantisation range pass (enough to fill the GPU)
 
+// Wavefronts that share a cluster in the row search: a power of two up to 16 (each of them scans the upper
+// levels by itself), and up to 512 wavefronts per CU, since work per cluster is very uneven.  Measured with
+// 64, 128, 512 and 1024 per CU: 436, 400, 366 and 355 us on 2,033 clusters, 4580, 2540, 1614 and 1970 us on
+// 14,294, and 29, 29, 13.6 and 13.2 ms on 32,705; with up to 32 in a cluster 57 and 27 us on 288 and 3
+// clusters become 61 and 27, and placing the tiles 6 and 4 become 8 and 23.
+static int row_slices(const ccd_ctx *ctx, int64_t F)
+{
+    const int64_t clusters = (F + 63) / 64, want = (int64_t)ctx->num_cus * 512;
+    int s = 1;
+    while (s < 16 && 2 * s * clusters <= want) s *= 2;
+    return s;
+}
+
 static int bp_buffers(ccd_ctx *ctx, int64_t F, int64_t V, bool batched, BPBufs &b)
 {
     b.dop64 = (double *)buffer(ctx, "dop64", (size_t)F * NB * 8);
@@ -1643,46 +1493,29 @@ static int bp_buffers(ccd_ctx *ctx, int64_t F, int64_t V, bool batched, BPBufs &
     b.sdop64 = (double *)buffer(ctx, "sdop64", (size_t)F * NB * 8);
     b.sfaces = (int4 *)buffer(ctx, "sfaces", (size_t)F * 16);
     b.sort_tmp = buffer(ctx, "radix_tmp", radix_sort_temp_bytes(F));
-    b.pairs = (int2 *)buffer(ctx, "pairs", (size_t)ctx->cap_pairs * 8);
     b.vfk = (int4 *)buffer(ctx, "vf_keys", (size_t)ctx->cap_vf * 16);
     b.eek = (int4 *)buffer(ctx, "ee_keys", (size_t)ctx->cap_ee * 16);
-    b.opp = (int32_t *)buffer(ctx, "edge_opp", (size_t)(3 * F + 1) * 4);
+    b.edges = (FaceEdges *)buffer(ctx, "face_edges", (size_t)F * sizeof(FaceEdges));
     b.rank = (int32_t *)buffer(ctx, "face_rank", (size_t)F * 4);
-    if (2 * ctx->cap_pairs < ((int64_t)1 << 31) - 1) {   // int32 row offsets
-        b.adj_cnt = (int32_t *)buffer(ctx, "adj_cnt", (size_t)(F + 1) * 4);
-        b.adj_off = (int32_t *)buffer(ctx, "adj_off", (size_t)(F + 1) * 4);
-        b.adj = (int32_t *)buffer(ctx, "adj", (size_t)(2 * ctx->cap_pairs + 1) * 4);
-        b.adj_tmp = buffer(ctx, "adj_scan_tmp", scan_temp_bytes(F + 1));
-        b.adj_mask = (uint16_t *)buffer(ctx, "adj_mask", (size_t)(2 * ctx->cap_pairs + 1) * 2);
-        b.exp_vf = (int64_t *)buffer(ctx, "exp_vf", (size_t)(F + 1) * 8);
-        b.exp_ee = (int64_t *)buffer(ctx, "exp_ee", (size_t)(F + 1) * 8);
-        if (!b.adj_cnt || !b.adj_off || !b.adj || !b.adj_tmp || !b.adj_mask || !b.exp_vf || !b.exp_ee)
-            return CCD_E_OOM;
-    }
+    const int64_t parts = (F + 1) * row_slices(ctx, F), feats = V + 3 * F + 1;
+    b.row_off = (int64_t *)buffer(ctx, "row_off", (size_t)parts * 8);
+    b.rows.mask = (uint64_t *)buffer(ctx, "row_mask", (size_t)ctx->cap_rows * 8);
+    b.rows.cluster = (int32_t *)buffer(ctx, "row_cluster", (size_t)ctx->cap_rows * 4);
+    b.rows.cap = ctx->cap_rows;
+    const int64_t waves = (F + 63) / 64 * row_slices(ctx, F);
+    b.kept.head = (ulonglong2 *)buffer(ctx, "row_heads", (size_t)waves * 16 + REC_SHARDS * REC_STRIDE * 8);
+    b.kept.claimed = (unsigned long long *)(b.kept.head + waves);
+    b.kept.rec = (ulonglong2 *)b.eek;
+    b.kept.per_shard = ctx->cap_ee / REC_SHARDS;
+    b.row_pairs = ctx->count_pairs ? (int32_t *)buffer(ctx, "row_pairs", (size_t)parts * 4) : nullptr;
+    b.counts = (int64_t *)buffer(ctx, "feature_counts", (size_t)feats * 8);
+    b.totals = (int64_t *)buffer(ctx, "expand_totals", 16);
+    b.scan_tmp = buffer(ctx, "expand_scan_tmp", scan_temp_bytes(std::max(parts, feats)));
     if (!b.dop64 || !b.centre || !b.partial || !b.qpartial || !b.qparam || !b.keys || !b.keys2 || !b.vals || !b.order ||
-        (batched && !b.face_inst) || !b.boxes || !b.sdop64 || !b.sfaces || !b.sort_tmp || !b.pairs || !b.vfk || !b.eek || !b.opp || !b.rank)
+        (batched && !b.face_inst) || !b.boxes || !b.sdop64 || !b.sfaces || !b.sort_tmp || !b.vfk || !b.eek || !b.edges ||
+        !b.rank || !b.row_off || !b.rows.mask || !b.rows.cluster || !b.kept.head || (ctx->count_pairs && !b.row_pairs) || !b.counts ||
+        !b.totals || !b.scan_tmp)
         return CCD_E_OOM;
-    return CCD_OK;
-}
-
-// Related-face table from the traversal's pairs (device-side count), rows in fill order.
-static int build_related_table(ccd_ctx *ctx, const BPBufs &b, int64_t F, MeshView &mv)
-{
-    if (!b.adj) return CCD_OK;
-    hipStream_t st = ctx->stream;
-    unsigned long long *c = (unsigned long long *)ctx->d_counts;
-    int rc = fill_u32(ctx, (uint32_t *)b.adj_cnt, F + 1, 0);
-    if (rc) return rc;
-    unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks_for(ctx->cap_pairs, 256), 8192));
-    hipLaunchKernelGGL(k_adj_count, dim3(grid), dim3(256), 0, st, b.pairs, c + C_PAIRS, ctx->cap_pairs, F, b.adj_cnt);
-    CCD_LAUNCH_CHECK(ctx);
-    rc = exclusive_scan_i32(ctx, b.adj_cnt, b.adj_off, F + 1, b.adj_tmp, nullptr);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_adj_fill, dim3(grid), dim3(256), 0, st, b.pairs, c + C_PAIRS, ctx->cap_pairs, F, b.adj_off,
-                       b.adj_cnt, b.adj);
-    CCD_LAUNCH_CHECK(ctx);
-    mv.adj_off = b.adj_off;
-    mv.adj = b.adj;
     return CCD_OK;
 }
 
@@ -1692,14 +1525,15 @@ static int launch_qrange(ccd_ctx *ctx, const BPBufs &b, int64_t F)
     const int nb = (int)std::min<int64_t>(QPARTS, blocks_for(F, 256));
     hipLaunchKernelGGL(k_qrange_partial, dim3(nb), dim3(256), 0, ctx->stream, b.dop64, F, b.qpartial);
     CCD_LAUNCH_CHECK(ctx);
-    hipLaunchKernelGGL(k_qrange_final, dim3(KAX), dim3(64), 0, ctx->stream, b.qpartial, nb, b.qparam);
+    hipLaunchKernelGGL(k_qrange_final, dim3(KAX), dim3(64), 0, ctx->stream, b.qpartial, nb, b.qparam,
+                       b.kept.claimed, REC_SHARDS * REC_STRIDE);
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }
 
 // The box records of every level, and the pair search over them.  The search scans the lowest level of at
 // most SCAN_MAX records from end to end (64 records a step), and descends from there.
-constexpr int64_t SCAN_MAX = 2048;
+constexpr int64_t SCAN_MAX = 512;   // (2,048: 476 us instead of 397 on 2,033 clusters)
 static int launch_boxes(ccd_ctx *ctx, const BPBufs &b, const int32_t *order, const int32_t *faces, int64_t F)
 {
     const LevelOffsets l = level_offsets(F);
@@ -1713,50 +1547,61 @@ static int launch_boxes(ccd_ctx *ctx, const BPBufs &b, const int32_t *order, con
     }
     return CCD_OK;
 }
-static int launch_pairs(ccd_ctx *ctx, const BPBufs &b, int64_t F, const int64_t *inst_off)
+// The related-face rows: count, scan, fill.  The rows' starts end up in b.row_off, (F + 1) * slices of them.
+static int launch_rows(ccd_ctx *ctx, const BPBufs &b, int64_t F, const int64_t *inst_off)
 {
     const LevelOffsets l = level_offsets(F);
-    PairLevels lv;
+    RowLevels lv;
     lv.top = 1;
     for (int k = 0; k < 4; k++) {
         lv.rec[k] = b.boxes + l.at[k];
         lv.n[k] = l.n[k];
     }
     while (lv.top < 3 && l.n[lv.top] > SCAN_MAX) lv.top++;
-    // Several wavefronts to a cluster while the clusters alone do not fill the chip.
-    const int64_t want = (int64_t)ctx->num_cus * 32;
-    const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(16, want / l.n[1]));
-    PairOut o{b.pairs, ctx->cap_pairs, (unsigned long long *)ctx->d_counts + C_PAIRS};
-    hipLaunchKernelGGL(k_pairs, dim3(blocks_for(l.n[1] * slices, PAIR_BLOCK / 64)), dim3(PAIR_BLOCK), 0, ctx->stream, lv,
-                       slices, b.sdop64, b.sfaces, b.face_inst, inst_off, o);
+    const int slices = row_slices(ctx, F);
+    const dim3 grid(blocks_for(l.n[1] * slices, ROW_BLOCK / 64));
+    hipLaunchKernelGGL(k_rows<false>, grid, dim3(ROW_BLOCK), 0, ctx->stream, lv, slices, b.sdop64, b.sfaces, b.face_inst,
+                       inst_off, b.row_off, b.row_pairs, b.rows, b.kept);
+    CCD_LAUNCH_CHECK(ctx);
+    // One scan over all parts; the entry past the last row's gets the total (what it held counts for nothing).
+    int rc = exclusive_scan_i64(ctx, b.row_off, b.row_off, F * slices + 1, b.scan_tmp, nullptr);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_rows<true>, grid, dim3(ROW_BLOCK), 0, ctx->stream, lv, slices, b.sdop64, b.sfaces, b.face_inst,
+                       inst_off, b.row_off, (int32_t *)nullptr, b.rows, b.kept);
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }
 
-// Expansion: with a related-face table, sort its rows and run the row expansion (count, scan, write;
-// the scans leave the unique stencil counts in the device counters); the per-pair kernel follows for
-// raw emission, or does everything when there is no table.
-static int launch_expand(ccd_ctx *ctx, const MeshView &mv, int64_t F, const BPBufs &b, unsigned grid)
+// The stencils from the rows: count, scan, write (or raw emission, by the device's own decision).
+static int launch_expand(ccd_ctx *ctx, const BPBufs &b, const int32_t *faces, int64_t F, int64_t V, const int32_t *voff,
+                         const int32_t *vlist, const uint8_t *fixed)
 {
     hipStream_t st = ctx->stream;
     unsigned long long *c = (unsigned long long *)ctx->d_counts;
-    const bool rows = mv.adj != nullptr;
-    if (rows) {
-        const unsigned gs = (unsigned)std::max<int64_t>(1, std::min<int64_t>(F, 65536));
-        hipLaunchKernelGGL(k_row_sort, dim3(gs), dim3(64), 0, st, c + C_BAD, F, mv.adj_off, b.adj);
-        CCD_LAUNCH_CHECK(ctx);
-        const unsigned gw = (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks_for(F, ROWS_BLOCK / 64), 65536));
-        hipLaunchKernelGGL(k_expand_rows_count, dim3(gw), dim3(ROWS_BLOCK), 0, st, mv, F, c + C_BAD, b.adj_mask,
-                           b.exp_vf, b.exp_ee);
-        CCD_LAUNCH_CHECK(ctx);
-        int rc = exclusive_scan_i64(ctx, b.exp_vf, b.exp_vf, F, b.adj_tmp, (int64_t *)(c + C_VF));
-        if (!rc) rc = exclusive_scan_i64(ctx, b.exp_ee, b.exp_ee, F, b.adj_tmp, (int64_t *)(c + C_EE));
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_expand_rows_write, dim3(gw), dim3(ROWS_BLOCK), 0, st, mv, F, c + C_BAD, b.adj_mask,
-                           b.exp_vf, b.exp_ee, b.vfk, ctx->cap_vf, b.eek, ctx->cap_ee);
+    const MeshView mv{faces, voff, vlist, fixed, b.edges, b.rank, b.sfaces, b.row_off, b.rows, row_slices(ctx, F)};
+    const int64_t feats = V + 3 * F;
+    // Fewer features to a wavefront where there are few: on 160 faces the two runs take 24 and 29 us with 16,
+    // 8 and 7 with 1; on 18,432 faces 43 and 52 with 16, 37 and 44 with 4, 40 and 45 with 2.
+    int chunk = UNION_CHUNK;
+    while (chunk > 1 && feats / chunk < (int64_t)ctx->num_cus * 48) chunk /= 2;
+    const dim3 grid(blocks_for(feats, chunk * (UNION_BLOCK / 64)));
+    hipLaunchKernelGGL(k_union<false>, grid, dim3(UNION_BLOCK), 0, st, mv, F, V, chunk, c + C_BAD, b.counts, b.vfk,
+                       (int64_t)0, b.eek, (int64_t)0);
+    CCD_LAUNCH_CHECK(ctx);
+    int rc = exclusive_scan_i64(ctx, b.counts, b.counts, feats, b.scan_tmp, b.totals);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_expand_counts, dim3(1), dim3(1), 0, st, b.row_off + F * mv.slices, b.counts, V, b.totals, c);
+    CCD_LAUNCH_CHECK(ctx);
+    if (b.row_pairs) {
+        const int64_t parts = F * mv.slices;
+        hipLaunchKernelGGL(k_pair_total, dim3((unsigned)std::min<int64_t>(blocks_for(parts, 1024), 256)), dim3(256), 0, st,
+                           b.row_pairs, parts, c);
         CCD_LAUNCH_CHECK(ctx);
     }
-    hipLaunchKernelGGL(k_expand, dim3(grid), dim3(EXPAND_BLOCK), 0, st, mv, rows, b.pairs, c + C_PAIRS, ctx->cap_pairs,
+    hipLaunchKernelGGL(k_union<true>, grid, dim3(UNION_BLOCK), 0, st, mv, F, V, chunk, c + C_BAD, b.counts, b.vfk, ctx->cap_vf,
+                       b.eek, ctx->cap_ee);
+    CCD_LAUNCH_CHECK(ctx);
+    hipLaunchKernelGGL(k_expand_raw, dim3((unsigned)std::min<int64_t>(blocks_for(F, 4), 4096)), dim3(256), 0, st, mv, F,
                        c + C_BAD, b.vfk, ctx->cap_vf, c + C_VF, b.eek, ctx->cap_ee, c + C_EE);
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
@@ -1764,9 +1609,9 @@ static int launch_expand(ccd_ctx *ctx, const MeshView &mv, int64_t F, const BPBu
 
 int broadphase_prepare(ccd_ctx *ctx, int64_t F, int64_t V, bool batched)
 {
-    // Capacities: grow-only, first guesses from the face count (the 256^2 cloth has 9.3 face pairs,
-    // 21 vertex-face and 38 edge-edge stencils per face); an overflow is detected after the run.
-    ctx->cap_pairs = std::max<int64_t>(ctx->cap_pairs, 16 * F + 1024);
+    // Capacities: grow-only, first guesses from the face count (the 256^2 cloth has 3.7 row tiles, 21
+    // vertex-face and 38 edge-edge stencils per face); an overflow is detected after the run.
+    ctx->cap_rows = std::max<int64_t>(ctx->cap_rows, 8 * F + 1024);
     ctx->cap_vf = std::max<int64_t>(ctx->cap_vf, 24 * F + 1024);
     ctx->cap_ee = std::max<int64_t>(ctx->cap_ee, 40 * F + 1024);
     BPBufs b;
@@ -1837,25 +1682,18 @@ int broadphase_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const doubl
     vertex_face_table(ctx, &voff, &vlist);
     hipLaunchKernelGGL(k_mesh_check, dim3(blocks_for(F, 256)), dim3(256), 0, st, faces, F, voff, vlist, c + C_BAD);
     CCD_LAUNCH_CHECK(ctx);
-    hipLaunchKernelGGL(k_edge_opp, dim3(blocks_for(3 * F, 256)), dim3(256), 0, st, faces, F, voff, vlist, b.opp);
+    hipLaunchKernelGGL(k_edges, dim3(blocks_for(3 * F, 256)), dim3(256), 0, st, b.sfaces, F, faces, voff, vlist, b.rank,
+                       b.edges);
     CCD_LAUNCH_CHECK(ctx);
     prof_end(ctx, CCD_T_TABLES);
 
     prof_begin(ctx, CCD_T_TRAVERSE);
-    rc = launch_pairs(ctx, b, F, inst_off);
+    rc = launch_rows(ctx, b, F, inst_off);
     if (rc) return rc;
     prof_end(ctx, CCD_T_TRAVERSE);
 
     prof_begin(ctx, CCD_T_EXPAND);
-    MeshView mv{faces, voff, vlist, b.dop64, fixed};
-    mv.opp = b.opp;
-    mv.rank = b.rank;
-    mv.sdop64 = b.sdop64;
-    mv.sfaces = b.sfaces;
-    rc = build_related_table(ctx, b, F, mv);
-    if (rc) return rc;
-    unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks_for(ctx->cap_pairs, 256), 16384));
-    rc = launch_expand(ctx, mv, F, b, grid);
+    rc = launch_expand(ctx, b, faces, F, V, voff, vlist, fixed);
     if (rc) return rc;
     prof_end(ctx, CCD_T_EXPAND);
     return CCD_OK;
@@ -1892,19 +1730,11 @@ int broadphase_refit_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const
     const int32_t *voff = nullptr, *vlist = nullptr;
     vertex_face_table(ctx, &voff, &vlist);
     prof_begin(ctx, CCD_T_TRAVERSE);
-    rc = launch_pairs(ctx, b, F, inst_off);
+    rc = launch_rows(ctx, b, F, inst_off);
     if (rc) return rc;
     prof_end(ctx, CCD_T_TRAVERSE);
     prof_begin(ctx, CCD_T_EXPAND);
-    MeshView mv{faces, voff, vlist, b.dop64, fixed};
-    mv.opp = b.opp;
-    mv.rank = b.rank;
-    mv.sdop64 = b.sdop64;
-    mv.sfaces = b.sfaces;
-    rc = build_related_table(ctx, b, F, mv);
-    if (rc) return rc;
-    unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks_for(ctx->cap_pairs, 256), 16384));
-    rc = launch_expand(ctx, mv, F, b, grid);
+    rc = launch_expand(ctx, b, faces, F, V, voff, vlist, fixed);
     if (rc) return rc;
     prof_end(ctx, CCD_T_EXPAND);
     return CCD_OK;
@@ -1924,17 +1754,16 @@ int broadphase(ccd_ctx *ctx, const int32_t *faces, int64_t F, const double *qs, 
         CCD_HIP_CHECK(ctx, hipMemcpyAsync(ctx->h_counts, ctx->d_counts, sizeof(int64_t) * NCOUNTERS,
                                           hipMemcpyDeviceToHost, st));
         CCD_HIP_CHECK(ctx, hipStreamSynchronize(st));
-        int64_t P = ctx->h_counts[C_PAIRS], nv = ctx->h_counts[C_VF], ne = ctx->h_counts[C_EE];
-        if (P <= ctx->cap_pairs && nv <= ctx->cap_vf && ne <= ctx->cap_ee) break;
-        // Too small: grow to the counts seen (the stencil counts are exact only once the pairs fit).
-        ctx->cap_pairs = std::max(ctx->cap_pairs, P + P / 8 + 1024);
+        int64_t P = ctx->h_counts[C_ROWS], nv = ctx->h_counts[C_VF], ne = ctx->h_counts[C_EE];
+        if (P <= ctx->cap_rows && nv <= ctx->cap_vf && ne <= ctx->cap_ee) break;
+        // Too small: grow to the counts seen (the stencil counts are exact only once the rows fit).
+        ctx->cap_rows = std::max(ctx->cap_rows, P + P / 8 + 1024);
         ctx->cap_vf = std::max(ctx->cap_vf, nv + nv / 8 + 1024);
         ctx->cap_ee = std::max(ctx->cap_ee, ne + ne / 8 + 1024);
         rc = broadphase_prepare(ctx, F, V, inst_off && ninst > 1);
         if (rc) return rc;
         if (attempt == 2) return set_error(ctx, CCD_E_CAPACITY, "broadphase buffers did not converge");
     }
-    out.npairs = ctx->h_counts[C_PAIRS];
     out.nvf = ctx->h_counts[C_VF];
     out.nee = ctx->h_counts[C_EE];
     out.vf = (int32_t *)ctx->bufs["vf_keys"].ptr;

@@ -555,7 +555,7 @@ static int detect_graph(ccd_ctx *ctx, const DetectArgs &a)
     unsigned char key[256] = {};
     static_assert(sizeof(DetectArgs) + 3 * sizeof(int64_t) <= sizeof(key), "graph key");
     memcpy(key, &a, sizeof(DetectArgs));
-    int64_t caps[3] = {ctx->cap_pairs, ctx->cap_vf, ctx->cap_ee};
+    int64_t caps[3] = {ctx->cap_rows, ctx->cap_vf, ctx->cap_ee};
     memcpy(key + sizeof(DetectArgs), caps, sizeof(caps));
     if (ctx->graph_valid && memcmp(key, ctx->graph_key, sizeof(key)) == 0) {
         if (ctx->profiling) (void)hipEventRecord(ctx->ev[2 * CCD_T_PIPELINE], ctx->stream);
@@ -570,7 +570,7 @@ static int detect_graph(ccd_ctx *ctx, const DetectArgs &a)
         prof_collect(ctx);
         ctx->graph_replays++;
         int64_t *h = ctx->h_counts;
-        if (h[C_PAIRS] <= ctx->cap_pairs && h[C_VF] <= ctx->cap_vf && h[C_EE] <= ctx->cap_ee && h[C_BAD] == 0) {
+        if (h[C_ROWS] <= ctx->cap_rows && h[C_VF] <= ctx->cap_vf && h[C_EE] <= ctx->cap_ee && h[C_BAD] == 0) {
             ctx->last_vf = (const int32_t *)ctx->bufs["vf_keys"].ptr;
             ctx->last_ee = (const int32_t *)ctx->bufs["ee_keys"].ptr;
             ctx->last_nvf = h[C_VF];
@@ -591,7 +591,7 @@ static int detect_graph(ccd_ctx *ctx, const DetectArgs &a)
     if (std::max(ctx->cap_vf, ctx->cap_ee) > 0 &&
         !open_list(ctx, std::min<int64_t>(std::max(ctx->cap_vf, ctx->cap_ee), 0x7fffffffll)))
         return CCD_E_OOM;
-    int64_t caps2[3] = {ctx->cap_pairs, ctx->cap_vf, ctx->cap_ee};
+    int64_t caps2[3] = {ctx->cap_rows, ctx->cap_vf, ctx->cap_ee};
     memcpy(key + sizeof(DetectArgs), caps2, sizeof(caps2));
     ctx->capturing = true;
     hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);

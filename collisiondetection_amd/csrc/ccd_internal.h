@@ -44,8 +44,9 @@ struct ccd_ctx {
     bool pending[CCD_NTIMERS] = {};
     double stage_ms[CCD_NTIMERS] = {};
     int64_t stage_calls[CCD_NTIMERS] = {};
-    // Grow-only capacities of the broadphase outputs (face pairs, stencils).
-    int64_t cap_pairs = 0, cap_vf = 0, cap_ee = 0;
+    // Grow-only capacities of the broadphase outputs (tiles of the related-face rows, stencils).
+    int64_t cap_rows = 0, cap_vf = 0, cap_ee = 0;
+    bool count_pairs = false;   // whether C_PAIRS is computed (a server reports it)
     // Sorted face order of the last full broadphase build (kept for refits).
     const int32_t *tree_order = nullptr;
     // Captured detection pipeline (ccd_batch_detect with CCD_GRAPH): replayed while its arguments match.
@@ -66,12 +67,13 @@ constexpr int NCOUNTERS = 16;
 
 // Counter slots in ctx->d_counts.
 enum Counter {
-    C_PAIRS = 0,    // overlapping non-neighbouring face pairs found by the traversal
+    C_PAIRS = 0,    // overlapping non-neighbouring face pairs (where count_pairs is set)
     C_VF = 1,       // unique vertex-face stencils
     C_EE = 2,       // unique edge-edge stencils
     C_VF_HITS = 3,  // colliding vertex-face stencils
     C_EE_HITS = 4,  // colliding edge-edge stencils
     C_BAD = 5,      // validation failures
+    C_ROWS = 6,     // tiles of the related-face rows
 };
 
 int set_error(ccd_ctx *ctx, int code, const char *fmt, ...);
@@ -156,7 +158,7 @@ int launch_validate_history(ccd_ctx *ctx, const int64_t *off, const double *ht, 
 struct Candidates {
     int32_t *vf = nullptr;
     int32_t *ee = nullptr;
-    int64_t nvf = 0, nee = 0, npairs = 0;
+    int64_t nvf = 0, nee = 0;
     int64_t vf_cap = 0, ee_cap = 0;
 };
 // aabb selects AABBBroadPhase's 3-axis bounds (used by the mesh self-distance), else the 13-axis k-DOP.

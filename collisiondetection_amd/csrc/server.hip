@@ -131,14 +131,14 @@ struct Session {
     int64_t resident = 0;
     bool busy = false;
     // workspace sizing from the last completed request
-    int64_t last_pairs = 0, last_vf = 0, last_ee = 0, last_hits = 0;
+    int64_t last_rows = 0, last_vf = 0, last_ee = 0, last_hits = 0;
     bool moved = false;   // a request has completed: the last counts come from a moving mesh
 };
 
 struct InFlight {
     ccd_request_rec req;
     int64_t pool_off = -1, pool_bytes = 0;
-    int64_t cap_pairs = 0, cap_vf = 0, cap_ee = 0, cap_hits = 0;
+    int64_t cap_rows = 0, cap_vf = 0, cap_ee = 0, cap_hits = 0;
     hipEvent_t done = nullptr;
     int64_t *h_rec = nullptr;   // pinned: NCOUNTERS counters + 2 checksums
     double t_start = 0;
@@ -176,11 +176,11 @@ using namespace ccdi;
 
 int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
 
-// A request's transient device memory: face pairs, the related-face table and its emission masks
-// (two entries per pair), the stencil keys, the screening passes' lists and the hit lists.
-int64_t workspace_bytes(int64_t cp, int64_t cv, int64_t ce, int64_t ch)
+// A request's transient device memory: the related-face rows' tiles, the stencil keys, the screening
+// passes' lists and the hit lists.
+int64_t workspace_bytes(int64_t cr, int64_t cv, int64_t ce, int64_t ch)
 {
-    return align256(cp * 8) + align256((2 * cp + 1) * 4) + align256((2 * cp + 1) * 2) + align256(cv * 16) +
+    return align256(cr * 8) + align256(cr * 4) + align256(cv * 16) +
            align256(ce * 16) + align256(open_list_bytes(std::max(cv, ce))) + 2 * (align256(ch * 16) + align256(ch * 8)) + 256;
 }
 
@@ -195,9 +195,8 @@ void bind_workspace(ccd_server *S, Session &s, InFlight &f)
         b.external = true;
         p += align256(bytes);
     };
-    put("pairs", f.cap_pairs * 8);
-    put("adj", (2 * f.cap_pairs + 1) * 4);
-    put("adj_mask", (2 * f.cap_pairs + 1) * 2);
+    put("row_mask", f.cap_rows * 8);
+    put("row_cluster", f.cap_rows * 4);
     put("vf_keys", f.cap_vf * 16);
     put("ee_keys", f.cap_ee * 16);
     put("open_list", open_list_bytes(std::max(f.cap_vf, f.cap_ee)));   // the screening passes' lists
@@ -207,7 +206,7 @@ void bind_workspace(ccd_server *S, Session &s, InFlight &f)
     p += kb + tb;
     f.hit_ek = (int32_t *)p;
     f.hit_et = (double *)(p + kb);
-    s.ctx->cap_pairs = f.cap_pairs;
+    s.ctx->cap_rows = f.cap_rows;
     s.ctx->cap_vf = f.cap_vf;
     s.ctx->cap_ee = f.cap_ee;
 }
@@ -261,9 +260,9 @@ void worker_loop(ccd_server *S)
             }
             Session &s = S->sessions[f.req.session];
             int64_t *h = f.h_rec;
-            bool overflow = h[C_PAIRS] > f.cap_pairs || h[C_VF] > f.cap_vf || h[C_EE] > f.cap_ee ||
+            bool overflow = h[C_ROWS] > f.cap_rows || h[C_VF] > f.cap_vf || h[C_EE] > f.cap_ee ||
                             h[C_VF_HITS] > f.cap_hits || h[C_EE_HITS] > f.cap_hits;
-            s.last_pairs = h[C_PAIRS];
+            s.last_rows = h[C_ROWS];
             s.last_vf = h[C_VF];
             s.last_ee = h[C_EE];
             s.last_hits = std::max(h[C_VF_HITS], h[C_EE_HITS]);
@@ -339,11 +338,11 @@ void worker_loop(ccd_server *S)
             // itself), and every overflow costs a rerun of the whole request; the headroom costs only
             // pool memory, about 60 bytes per face.
             const int64_t mul = s.moved ? 2 : 4;
-            f.cap_pairs = mul * s.last_pairs + s.F / 4 + 4096;
+            f.cap_rows = mul * s.last_rows + s.F / 4 + 4096;
             f.cap_vf = mul * s.last_vf + s.F + 4096;
             f.cap_ee = mul * s.last_ee + 2 * s.F + 4096;
             f.cap_hits = mul * s.last_hits + s.F / 16 + 4096;
-            f.pool_bytes = workspace_bytes(f.cap_pairs, f.cap_vf, f.cap_ee, f.cap_hits);
+            f.pool_bytes = workspace_bytes(f.cap_rows, f.cap_vf, f.cap_ee, f.cap_hits);
             if (f.pool_bytes > S->pool.size) {   // can never be admitted: fail it rather than wait forever
                 ccd_request_result r{};
                 r.request_id = it->id;
@@ -468,6 +467,7 @@ int ccd_server_open_session(ccd_server *S, const int32_t *faces, int64_t nfaces,
     Session s;
     int rc = ccd_create(&s.ctx, S->device);
     if (rc) return rc;
+    s.ctx->count_pairs = true;
     s.F = nfaces;
     s.V = nverts;
     s.outer_eta = outer_eta;
@@ -500,12 +500,12 @@ int ccd_server_open_session(ccd_server *S, const int32_t *faces, int64_t nfaces,
     if (rc && rc != CCD_E_CAPACITY) return fail(rc);
     if (ctx->h_counts[C_BAD] != 0) return fail(set_error(ctx, CCD_E_INVALID, "sessions need meshes without degenerate or duplicate faces"));
     s.cur = 1;   // the first request starts at qend
-    s.last_pairs = ctx->h_counts[C_PAIRS];
+    s.last_rows = ctx->h_counts[C_ROWS];
     s.last_vf = nvc;
     s.last_ee = nec;
     s.last_hits = std::max(nvh, neh);
     // The transient buffers come from the pool per request: release the context's own copies.
-    for (const char *name : {"pairs", "adj", "adj_mask", "vf_keys", "ee_keys", "open_list"}) {
+    for (const char *name : {"row_mask", "row_cluster", "vf_keys", "ee_keys", "open_list"}) {
         ccd_ctx::Buf &b = ctx->bufs[name];
         if (b.ptr && !b.external) {
             (void)hipFree(b.ptr);
@@ -613,7 +613,7 @@ int ccd_server_destroy(ccd_server *S)
     if (S->worker.joinable()) S->worker.join();
     (void)hipSetDevice(S->device);
     for (Session &s : S->sessions) {
-        for (const char *name : {"pairs", "adj", "adj_mask", "vf_keys", "ee_keys", "open_list"}) s.ctx->bufs[name] = ccd_ctx::Buf();
+        for (const char *name : {"row_mask", "row_cluster", "vf_keys", "ee_keys", "open_list"}) s.ctx->bufs[name] = ccd_ctx::Buf();
         (void)hipFree(s.faces);
         (void)hipFree(s.pos[0]);
         (void)hipFree(s.pos[1]);

@@ -81,3 +81,31 @@ def test_pairs_instances_within_a_cluster(sizes):
         vf, ee = oracle.candidates(f, oracle.Hist.two_entry(a, b), 1e-3, method="tree")
         nvf, nee = nvf + len(vf), nee + len(ee)
     assert (r["vf_candidates"], r["ee_candidates"]) == (nvf, nee) and nvf > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,fins", [(9, False), (90, False), (150, False), (150, True)])
+def test_stencils_of_a_face_over_many(n, fins):
+    """A triangle whose swept bounds hold a whole lattice: its stencils with every vertex, edge and face of
+    it, besides the lattice's own.  Its row has up to 793 clusters (more than the union's table holds);
+    with fins there are edges of three faces."""
+    v, f = scenes.grid(n)
+    if fins:
+        base = f[::7, :2]
+        apex = v[base].mean(axis=1) + [0.0, 0.0, 1e-4]
+        f = np.concatenate([f, np.column_stack([base, len(v) + np.arange(len(base))])]).astype(np.int32)
+        v = np.concatenate([v, apex])
+    eta = 1e-9
+    own_vf, own_ee = api.kdop_candidates(f, v, v, eta)
+    big, shift = np.array([[0.0, 0.0, 0.0], [1.0, 0.0, 0.0], [0.0, 1.0, 1.0]]), np.array([50.0, 60.0, 70.0])
+    nv = len(v)
+    vf, ee = api.kdop_candidates(np.concatenate([f, [[nv, nv + 1, nv + 2]]]).astype(np.int32),
+                                 np.concatenate([v, big - shift]), np.concatenate([v, big + shift]), eta)
+    fs = np.sort(f, axis=1)
+    edges = np.unique(np.sort(np.concatenate([f[:, [0, 1]], f[:, [1, 2]], f[:, [2, 0]]]), axis=1), axis=0)
+    want_vf = [own_vf, np.column_stack([np.arange(nv), np.tile([nv, nv + 1, nv + 2], (nv, 1))])]
+    want_vf += [np.column_stack([np.full(len(fs), nv + k), fs]) for k in range(3)]
+    want_ee = [own_ee] + [np.column_stack([edges, np.tile([nv + a, nv + b], (len(edges), 1))])
+                          for a, b in ((0, 1), (0, 2), (1, 2))]
+    np.testing.assert_array_equal(vf, np.unique(np.concatenate(want_vf), axis=0))
+    np.testing.assert_array_equal(ee, np.unique(np.concatenate(want_ee), axis=0))
