@@ -30,6 +30,13 @@ def test_pairs_at_cluster_edges(F):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("F", [2047, 2048, 2049, 262144, 262145])
+def test_pairs_at_sort_tiles(F):
+    """Around a sort tile (2,048 keys) and the most tiles that the scatter adds up by itself (128)."""
+    assert _check(*_loose_triangles(F, F, 0.3 / F ** (1 / 3)), 1e-4) > 0
+
+
+@pytest.mark.gpu
 def test_pairs_all_overlapping():
     """Every leaf meets every other: full tiles, the output queue written several times."""
     faces, qs, qe = _loose_triangles(200, 1, 3.0)
