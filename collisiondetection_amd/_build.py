@@ -11,7 +11,7 @@ CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libccd_amd.so")
 LOADGEN = os.path.join(PKG, "serve_loadgen")
 OBJDIR = os.path.join(PKG, "_build")
-SOURCES = ["narrowphase.hip", "screened.hip", "workcount.hip", "broadphase.hip", "distance.hip", "devprims.hip", "server.hip",
+SOURCES = ["narrowphase.hip", "screened.hip", "history.hip", "workcount.hip", "broadphase.hip", "distance.hip", "devprims.hip", "server.hip",
            "capi.hip", "velocity_filter.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 

@@ -356,14 +356,12 @@ int ccd_ctcd_narrowphase_history(ccd_ctx *ctx, const int64_t *hist_off, const do
     if (rc) return rc;
     rc = validate_keys(ctx, ee_keys, nee, nverts, "edge-edge keys reference vertices outside [0, nverts)");
     if (rc) return rc;
-    // Long histories (16 or more entries per vertex on average): one wavefront per stencil tests 64
-    // stitched windows at a time; short ones: one lane per stencil.
-    const bool wave = nentries >= 16 * nverts;
+    const int64_t entries = nentries / std::max<int64_t>(nverts, 1);
     rc = launch_narrow_hist(ctx, true, hist_off, hist_t, hist_pos, vf_keys, vf_eta, eta_scalar, nvf, vf_hit, vf_t,
-                            vf_sub, vf_win, wave);
+                            vf_sub, vf_win, entries);
     if (rc) return rc;
     return launch_narrow_hist(ctx, false, hist_off, hist_t, hist_pos, ee_keys, ee_eta, eta_scalar, nee, ee_hit, ee_t,
-                              ee_sub, ee_win, wave);
+                              ee_sub, ee_win, entries);
 }
 
 int ccd_separating_plane_narrowphase(ccd_ctx *ctx, const int64_t *hist_off, const double *hist_t,
@@ -392,14 +390,12 @@ int ccd_separating_plane_narrowphase(ccd_ctx *ctx, const int64_t *hist_off, cons
     if (rc) return rc;
     rc = launch_min_gap(ctx, hist_off, hist_t, nverts, dev);
     if (rc) return rc;
-    // Long histories (16 or more entries per vertex on average, as the velocity filter builds): one
-    // wavefront per stencil shares each trajectory scan; short ones: one lane per stencil.
-    const bool wave = nentries >= 16 * nverts;
+    const int64_t entries = nentries / std::max<int64_t>(nverts, 1);
     rc = launch_separating_plane(ctx, true, hist_off, hist_t, hist_pos, vf_keys, vf_eta, eta_scalar, nvf, dev,
-                                 vf_status, (int64_t *)(dev + 1), wave);
+                                 vf_status, (int64_t *)(dev + 1), entries);
     if (rc) return rc;
     rc = launch_separating_plane(ctx, false, hist_off, hist_t, hist_pos, ee_keys, ee_eta, eta_scalar, nee, dev,
-                                 ee_status, (int64_t *)(dev + 1), wave);
+                                 ee_status, (int64_t *)(dev + 1), entries);
     if (rc) return rc;
     int64_t und = 0;
     CCD_HIP_CHECK(ctx, hipMemcpyAsync(&und, dev + 1, 8, hipMemcpyDeviceToHost, ctx->stream));

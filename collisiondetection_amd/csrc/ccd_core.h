@@ -2113,129 +2113,144 @@ CCD_HD double plane_trajectory_intersect(const HistCSR &h, int v, int start, boo
 // at most halves the interval; only an interval closing in on a history entry time gets that deep).
 constexpr int SP_MAX_DEPTH = 160;
 
-// The trajectory scan one lane runs by itself.  A scanner with the same call operator may split the
-// scan over the lanes of a wavefront (every lane then runs the same check on the same stencil).
-struct SeqScan {
-    CCD_HD double operator()(const HistCSR &h, int v, int start, bool forward, V3 ppos, V3 pvel, V3 nrm, V3 ptstart,
-                             double tstart, double eta) const
+// One stencil's histories as the recursion reads them: positions at a time (with the entry before it), the step
+// from an entry to the next, and a node's eight trajectory scans (t_lo: the smallest backward result, t_hi: the
+// smallest forward one).  Lanes that share a stencil may hold them in another form.
+struct CsrHistory {
+    const HistCSR &h;
+    const int (&v)[4];
+    CCD_HD V3 pos(int j, double time, int &idx) const { return pos_at_time(h, v[j], time, idx); }
+    CCD_HD void step(int j, int idx, V3 &d, double &dt) const
     {
-        return plane_trajectory_intersect(h, v, start, forward, ppos, pvel, nrm, ptstart, tstart, eta);
+        const int64_t k = h.off[v[j]] + idx;
+        d = hist_pos(h, k + 1) - hist_pos(h, k);
+        dt = h.t[k + 1] - h.t[k];
+    }
+    template <bool VF>
+    CCD_HD void scan(const int (&mi)[4], V3 ppos, V3 pvel, V3 closest, const V3 (&mp)[4], double midt, double eta,
+                     double &t_lo, double &t_hi) const
+    {
+        for (int dir = 0; dir < 2; dir++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                double sign = (j == 0 || (j == 1 && !VF)) ? -1.0 : 1.0;
+                V3 nrm = sign * closest;
+                double &m = dir == 0 ? t_lo : t_hi;
+                m = smin(m, plane_trajectory_intersect(h, v[j], mi[j] + dir, dir == 1, ppos, pvel, nrm, mp[j], midt, eta));
+            }
     }
 };
 
+// The recursion.  window(s, e): a window within one history entry interval of every vertex; true if it
+// collides.  (A caller may test the windows later and let `window` return false: the result is then 1 if
+// one of them collides, whatever the recursion returned; it can only have gone on for nothing.)
 // max_nodes bounds the intervals examined: when more remain the result is 3 ("not decided yet"), which
 // a caller uses to sort stencils by how much work they need before running them in full.
-template <bool VF, class C = NoCount, class Scan = SeqScan>
-CCD_HD int separating_plane_check(const HistCSR &h, const int (&v)[4], double eta, double eps, C &&cnt = C(),
-                                  Scan scan = Scan(), int max_nodes = 0x7fffffff)
+template <bool VF, class Histories, class Window>
+CCD_HD int separating_plane_nodes(const Histories &hist, double eta, double eps, int max_nodes, Window &&window)
 {
     const double inf = bits_to_double(0x7ff0000000000000ll);
-    // pending intervals and their depths; a node at depth d leaves at most d pending uppers below it
+    // pending upper intervals and their depths; a node at depth d leaves at most d of them below it
     double st_lo[SP_MAX_DEPTH + 2], st_hi[SP_MAX_DEPTH + 2];
     int st_d[SP_MAX_DEPTH + 2];
-    st_lo[0] = 0.0;
-    st_hi[0] = 1.0;
-    st_d[0] = 0;
-    int top = 1;
-    while (top > 0) {
+    int top = 0;
+    double mint = 0.0, maxt = 1.0;
+    int depth = 0;
+    for (;;) {
         if (max_nodes-- <= 0) return 3;
-        top--;
-        CCD_INDEX_CHECK(top, SP_MAX_DEPTH + 2);
-        const double mint = st_lo[top], maxt = st_hi[top];
-        const int depth = st_d[top];
         if (depth > SP_MAX_DEPTH) return 2;
-        if (maxt < mint) continue;
-        if (maxt - mint < 3 * eps) {
+        bool leaf = maxt < mint;
+        if (!leaf && maxt - mint < 3 * eps) {
             V3 s[4], e[4];
             bool ok = true;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 int io = 0, in = 0;
-                s[j] = pos_at_time(h, v[j], mint, io);
-                e[j] = pos_at_time(h, v[j], maxt, in);
+                s[j] = hist.pos(j, mint, io);
+                e[j] = hist.pos(j, maxt, in);
                 if (io != in) ok = false;
             }
             if (ok) {
-                double t = 0.0;
-                int r = VF ? check_vf_window(s, e, eta, t, cnt) : check_ee_window(s, e, eta, t, cnt);
-                if (r >= 0) return 1;
-                continue;
+                if (window(s, e)) return 1;
+                leaf = true;
             }
         }
-        const double midt = 0.5 * (mint + maxt);
-        V3 mp[4];
-        int mi[4];
+        double t_lo = inf, t_hi = inf, midt = 0.0;
+        if (!leaf) {
+            midt = 0.5 * (mint + maxt);
+            V3 mp[4];
+            int mi[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) mp[j] = pos_at_time(h, v[j], midt, mi[j]);
-        double b1 = 0, b2 = 0, b3 = 0, b4 = 0;
-        V3 closest = VF ? vertex_face_distance(mp[0], mp[1], mp[2], mp[3], b1, b2, b3)
-                        : edge_edge_distance(mp[0], mp[1], mp[2], mp[3], b1, b2, b3, b4);
-        if (dot(closest, closest) < eta * eta) return 1;
-        // The separating plane: through the midpoint of the closest points, moving with their mean
-        // velocity over the current history windows (:162-185).
-        V3 dv[4];
-        double dts[4];
+            for (int j = 0; j < 4; j++) mp[j] = hist.pos(j, midt, mi[j]);
+            double b1 = 0, b2 = 0, b3 = 0, b4 = 0;
+            V3 closest = VF ? vertex_face_distance(mp[0], mp[1], mp[2], mp[3], b1, b2, b3)
+                            : edge_edge_distance(mp[0], mp[1], mp[2], mp[3], b1, b2, b3, b4);
+            if (dot(closest, closest) < eta * eta) return 1;
+            // The separating plane: through the midpoint of the closest points, moving with their mean
+            // velocity over the current history windows (:162-185).
+            V3 dv[4];
+            double dts[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int64_t k = h.off[v[j]] + mi[j];
-            V3 d = hist_pos(h, k + 1) - hist_pos(h, k);
-            dts[j] = h.t[k + 1] - h.t[k];
-            dv[j] = d;
-        }
-        V3 ppos, pvel;
-        if (VF) {
-            ppos = 0.5 * (((mp[0] + b1 * mp[1]) + b2 * mp[2]) + b3 * mp[3]);
-            V3 w0 = mk(dv[0].x / dts[0], dv[0].y / dts[0], dv[0].z / dts[0]);
-            V3 w1 = b1 * dv[1], w2 = b2 * dv[2], w3 = b3 * dv[3];
-            w1 = mk(w1.x / dts[1], w1.y / dts[1], w1.z / dts[1]);
-            w2 = mk(w2.x / dts[2], w2.y / dts[2], w2.z / dts[2]);
-            w3 = mk(w3.x / dts[3], w3.y / dts[3], w3.z / dts[3]);
-            pvel = 0.5 * (((w0 + w1) + w2) + w3);
-        } else {
-            ppos = 0.5 * (((b1 * mp[0] + b2 * mp[1]) + b3 * mp[2]) + b4 * mp[3]);
-            V3 w0 = b1 * dv[0], w1 = b2 * dv[1], w2 = b3 * dv[2], w3 = b4 * dv[3];
-            w0 = mk(w0.x / dts[0], w0.y / dts[0], w0.z / dts[0]);
-            w1 = mk(w1.x / dts[1], w1.y / dts[1], w1.z / dts[1]);
-            w2 = mk(w2.x / dts[2], w2.y / dts[2], w2.z / dts[2]);
-            w3 = mk(w3.x / dts[3], w3.y / dts[3], w3.z / dts[3]);
-            pvel = 0.5 * (((w0 + w1) + w2) + w3);
-        }
-        const double cn = norm(closest);
-        closest = mk(closest.x / cn, closest.y / cn, closest.z / cn);
-        double t_lo = inf, t_hi = inf;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            double sign = (j == 0 || (j == 1 && !VF)) ? -1.0 : 1.0;
-            V3 nrm = sign * closest;
-            t_lo = smin(t_lo, scan(h, v[j], mi[j], false, ppos, pvel, nrm, mp[j], midt, eta));
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            double sign = (j == 0 || (j == 1 && !VF)) ? -1.0 : 1.0;
-            V3 nrm = sign * closest;
-            t_hi = smin(t_hi, scan(h, v[j], mi[j] + 1, true, ppos, pvel, nrm, mp[j], midt, eta));
+            for (int j = 0; j < 4; j++) hist.step(j, mi[j], dv[j], dts[j]);
+            V3 ppos, pvel;
+            if (VF) {
+                ppos = 0.5 * (((mp[0] + b1 * mp[1]) + b2 * mp[2]) + b3 * mp[3]);
+                V3 w0 = mk(dv[0].x / dts[0], dv[0].y / dts[0], dv[0].z / dts[0]);
+                V3 w1 = b1 * dv[1], w2 = b2 * dv[2], w3 = b3 * dv[3];
+                w1 = mk(w1.x / dts[1], w1.y / dts[1], w1.z / dts[1]);
+                w2 = mk(w2.x / dts[2], w2.y / dts[2], w2.z / dts[2]);
+                w3 = mk(w3.x / dts[3], w3.y / dts[3], w3.z / dts[3]);
+                pvel = 0.5 * (((w0 + w1) + w2) + w3);
+            } else {
+                ppos = 0.5 * (((b1 * mp[0] + b2 * mp[1]) + b3 * mp[2]) + b4 * mp[3]);
+                V3 w0 = b1 * dv[0], w1 = b2 * dv[1], w2 = b3 * dv[2], w3 = b4 * dv[3];
+                w0 = mk(w0.x / dts[0], w0.y / dts[0], w0.z / dts[0]);
+                w1 = mk(w1.x / dts[1], w1.y / dts[1], w1.z / dts[1]);
+                w2 = mk(w2.x / dts[2], w2.y / dts[2], w2.z / dts[2]);
+                w3 = mk(w3.x / dts[3], w3.y / dts[3], w3.z / dts[3]);
+                pvel = 0.5 * (((w0 + w1) + w2) + w3);
+            }
+            const double cn = norm(closest);
+            closest = mk(closest.x / cn, closest.y / cn, closest.z / cn);
+            hist.template scan<VF>(mi, ppos, pvel, closest, mp, midt, eta, t_lo, t_hi);
         }
         // Depth first, lower sub-interval first: push the upper one underneath.  A child equal to its
         // node is undecided when it is reached (the upper one only if the lower subtree finds nothing).
-        if (t_hi < 1.0) {
-            const double lo = midt + smax(0.0, t_hi - eps);
-            CCD_INDEX_CHECK(top, SP_MAX_DEPTH + 2);
-            st_lo[top] = lo;
-            st_hi[top] = maxt;
-            st_d[top] = lo == mint ? SP_MAX_DEPTH + 1 : depth + 1;   // equal to this node: undecided if reached
-            top++;
-        }
-        if (t_lo < 1.0) {
-            const double hi = midt - smax(0.0, t_lo - eps);
+        const bool upper = !leaf && t_hi < 1.0, lower = !leaf && t_lo < 1.0;
+        const double lo = midt + smax(0.0, t_hi - eps), hi = midt - smax(0.0, t_lo - eps);
+        const int below = lo == mint ? SP_MAX_DEPTH + 1 : depth + 1;   // equal to this node: undecided if reached
+        if (lower) {
             if (hi == maxt) return 2;
+            if (upper) {
+                CCD_INDEX_CHECK(top, SP_MAX_DEPTH + 2);
+                st_lo[top] = lo;
+                st_hi[top] = maxt;
+                st_d[top] = below;
+                top++;
+            }
+            maxt = hi;
+            depth++;
+        } else if (upper) {
+            mint = lo;
+            depth = below;
+        } else {
+            if (top == 0) return 0;
+            top--;
             CCD_INDEX_CHECK(top, SP_MAX_DEPTH + 2);
-            st_lo[top] = mint;
-            st_hi[top] = hi;
-            st_d[top] = depth + 1;
-            top++;
+            mint = st_lo[top];
+            maxt = st_hi[top];
+            depth = st_d[top];
         }
     }
-    return 0;
+}
+
+template <bool VF, class C = NoCount>
+CCD_HD int separating_plane_check(const HistCSR &h, const int (&v)[4], double eta, double eps, C &&cnt = C())
+{
+    return separating_plane_nodes<VF>(CsrHistory{h, v}, eta, eps, 0x7fffffff, [&](const V3 (&s)[4], const V3 (&e)[4]) {
+        double t = 0.0;
+        return (VF ? check_vf_window(s, e, eta, t, cnt) : check_ee_window(s, e, eta, t, cnt)) >= 0;
+    });
 }
 
 }   // namespace ccd

@@ -119,16 +119,36 @@ struct NarrowOut {
 // wavefront takes at a time on long lists.  open_list: the context's buffer, or null for n >= 2^31.
 int launch_screened(ccd_ctx *ctx, bool vf, bool per_stencil, const double *qs, const double *qe, const int32_t *keys,
                     const int64_t *n_dev, int64_t n, double eta, const NarrowOut &o, int tile, void *list);
+// Windows of multi-entry histories that a kernel gathers for the screening narrowphase, in shards with a
+// counter each (claims on one counter take about 10 ns each, one after another).
+struct WindowPool {
+    static constexpr int SHARDS = 64, STRIDE = 8;   // (a counter per 64 bytes)
+    double *pos;        // [24 * capacity] four vertices at the window's start, four at its end
+    double *eta;
+    int32_t *owner;     // the stencil, -1: nothing here
+    uint32_t *place;    // the window among the stencil's
+    uint8_t *hit;       // results, as launch_narrow2's
+    uint8_t *sub;
+    double *t;
+    unsigned long long *claimed;   // [SHARDS * STRIDE]; may exceed per_shard
+    int64_t per_shard;             // a multiple of 64; at most 65,536 for all shards' regions of 64
+    __device__ __forceinline__ int64_t filled(int64_t shard) const
+    {
+        const int64_t c = (int64_t)claimed[shard * STRIDE];
+        return c < per_shard ? c : per_shard;
+    }
+};
+int launch_screened_pool(ccd_ctx *ctx, bool vf, const WindowPool &pool, void *list);
 int64_t open_list_bytes(int64_t n);
 void *open_list(ccd_ctx *ctx, int64_t n);
 // One result per stencil.  list: the caller's, for these n stencils, else the context's own.
 int launch_narrow2(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys,
                    const double *eta, double eta_s, int64_t n, uint8_t *hit, double *t, uint8_t *sub,
                    void *list = nullptr);
-// wave: one wavefront per stencil sharing the stitched windows (for long histories), else one lane.
+// entries: history entries per vertex on average.
 int launch_narrow_hist(ccd_ctx *ctx, bool vf, const int64_t *off, const double *ht, const double *hp,
                        const int32_t *keys, const double *eta, double eta_s, int64_t n, uint8_t *hit, double *t,
-                       uint8_t *sub, int32_t *win, bool wave);
+                       uint8_t *sub, int32_t *win, int64_t entries);
 // Narrowphase over a stencil list, appending the colliding stencils (keys and times) to out_keys / out_toi
 // with a device counter; at most cap are written.  Screened when `list` (for at least n_max stencils) is
 // given, else the whole cascade on a persistent work queue, whose counter *work must be zero.
@@ -143,10 +163,10 @@ int launch_narrow2_count(ccd_ctx *ctx, bool vf, const double *qs, const double *
 // Separating-plane narrowphase over a CSR history: launch_min_gap writes History::computeMinimumGap's
 // value (as bits) to *gap_bits on the device; launch_separating_plane reads it (eps = gap / 4).
 int launch_min_gap(ccd_ctx *ctx, const int64_t *off, const double *ht, int64_t nverts, uint64_t *gap_bits);
-// wave: one wavefront per stencil sharing the trajectory scans (for long histories), else one lane.
+// entries: history entries per vertex on average.
 int launch_separating_plane(ccd_ctx *ctx, bool vf, const int64_t *off, const double *ht, const double *hp,
                             const int32_t *keys, const double *eta, double eta_s, int64_t n, const uint64_t *gap_bits,
-                            uint8_t *status, int64_t *undecided, bool wave);
+                            uint8_t *status, int64_t *undecided, int64_t entries);
 int launch_validate_keys(ccd_ctx *ctx, const int32_t *keys, int64_t n4, int64_t nverts, int64_t *bad);
 int launch_validate_history(ccd_ctx *ctx, const int64_t *off, const double *ht, int64_t nverts, int64_t nentries,
                             int64_t *bad);

@@ -120,71 +120,6 @@ __global__ __launch_bounds__(256) CCD_TWO_WAVES void k_narrow2_queue(
     }
 }
 
-// Multi-entry histories: stitch on the fly (History.cpp:98-140) and test window by window.
-template <bool VF, class M>
-__global__ __launch_bounds__(256) CCD_TWO_WAVES void k_narrow_hist(const int64_t *__restrict__ off, const double *__restrict__ ht,
-                                                     const double *__restrict__ hp, const int4 *__restrict__ keys,
-                                                     const double *__restrict__ eta, double eta_s, int64_t n,
-                                                     uint8_t *__restrict__ hit, double *__restrict__ tout,
-                                                     uint8_t *__restrict__ sub, int32_t *__restrict__ win)
-{
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int4 k = keys[i];
-    int v[4] = {k.x, k.y, k.z, k.w};
-    double e = eta ? eta[i] : eta_s;
-    int64_t its[4], ends[4];
-    int64_t total = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        its[j] = off[v[j]];
-        ends[j] = off[v[j] + 1];
-        total += ends[j] - its[j];
-    }
-    V3 prev[4], cur[4];
-    double curtime = 0.0;
-    int w = -1;
-    int r = -1;
-    double t = 0.0;
-    // Each pass advances curtime strictly (entries at or before it are consumed), so the number of
-    // stitched entries is at most the total entry count; the bound also guards malformed input.
-    for (int64_t guard = 0; guard <= total && curtime <= 1.0; guard++) {
-        double newtime = __builtin_inf();
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            int64_t next = its[j] + 1;
-            while (next != ends[j] && ht[next] <= curtime) {
-                ++next;
-                ++its[j];
-            }
-            V3 oldp = ccd::mk(hp[3 * its[j]], hp[3 * its[j] + 1], hp[3 * its[j] + 2]);
-            if (next == ends[j]) {
-                cur[j] = oldp;
-            } else {
-                V3 newp = ccd::mk(hp[3 * next], hp[3 * next + 1], hp[3 * next + 2]);
-                double dt = ht[next] - ht[its[j]];
-                double a = curtime - ht[its[j]];
-                double b = ht[next] - curtime;
-                cur[j] = ccd::mk((b * oldp.x + a * newp.x) / dt, (b * oldp.y + a * newp.y) / dt,
-                                 (b * oldp.z + a * newp.z) / dt);
-                newtime = ccd::smin(newtime, ht[next]);
-            }
-        }
-        if (w >= 0) {
-            r = VF ? ccd::check_vf_window(prev, cur, e, t, M()) : ccd::check_ee_window(prev, cur, e, t, M());
-            if (r >= 0) break;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) prev[j] = cur[j];
-        w++;
-        curtime = newtime;
-    }
-    hit[i] = r >= 0 ? 1 : 0;
-    if (tout) tout[i] = r >= 0 ? t : 0.0;
-    if (sub) sub[i] = r >= 0 ? (uint8_t)r : (uint8_t)255;
-    if (win) win[i] = r >= 0 ? w : -1;
-}
-
 __global__ void k_validate_keys(const int32_t *__restrict__ keys, int64_t n4, int64_t nverts,
                                 unsigned long long *bad)
 {
@@ -234,234 +169,10 @@ __global__ __launch_bounds__(256) void k_min_gap(const int64_t *__restrict__ off
 }
 __global__ void k_set_bits(unsigned long long *p, unsigned long long v) { *p = v; }
 
-// SeparatingPlaneNarrowPhase (SeparatingPlaneNarrowPhase.cpp:9-278): one lane per stencil, status 1
-// (collision), 0 (none) or 2 (undecided: the reference's recursion would not end; counted in *undecided).
-template <bool VF, class M>
-__global__ __launch_bounds__(256) CCD_TWO_WAVES void k_separating_plane(
-    const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
-    const int4 *__restrict__ keys, const double *__restrict__ eta, double eta_s, int64_t n,
-    const unsigned long long *__restrict__ gap_bits, uint8_t *__restrict__ status, unsigned long long *undecided,
-    const int32_t *__restrict__ order)
-{
-    const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    int r = 0;
-    if (j < n) {
-        const int64_t i = order ? (int64_t)order[j] : j;   // lane j runs stencil order[j]
-        const double eps = ccd::bits_to_double((long long)*gap_bits) / 4.0;
-        int4 k = keys[i];
-        int v[4] = {k.x, k.y, k.z, k.w};
-        ccd::HistCSR h{off, ht, hp};
-        r = ccd::separating_plane_check<VF>(h, v, eta ? eta[i] : eta_s, eps, M());
-        status[i] = (uint8_t)r;
-    }
-    uint64_t m = __ballot(r == 2);
-    if (m && __lane_id() == __ffsll((unsigned long long)m) - 1) atomicAdd(undecided, (unsigned long long)__popcll(m));
-}
-
-// Sort key for the separating-plane narrowphase: 1 if a stencil's root interval [0, 1] does not decide
-// it (its recursion goes on; with two-entry histories that means one or two CTCD window tests), else 0.
-// Most stencils are decided at the root; grouping the others keeps a wavefront's lanes on the same path.
-template <bool VF>
-__global__ __launch_bounds__(256) void k_sp_order_key(const int64_t *__restrict__ off, const double *__restrict__ ht,
-                                                      const double *__restrict__ hp, const int4 *__restrict__ keys,
-                                                      const double *__restrict__ eta, double eta_s, int64_t n,
-                                                      const unsigned long long *__restrict__ gap_bits,
-                                                      uint64_t *__restrict__ key, int32_t *__restrict__ idx)
-{
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double eps = ccd::bits_to_double((long long)*gap_bits) / 4.0;
-    const int4 k = keys[i];
-    const int v[4] = {k.x, k.y, k.z, k.w};
-    ccd::HistCSR h{off, ht, hp};
-    const int r = ccd::separating_plane_check<VF>(h, v, eta ? eta[i] : eta_s, eps, ccd::FullCascade(), ccd::SeqScan(), 1);
-    key[i] = r == 3 ? 1u : 0u;
-    idx[i] = (int32_t)i;
-}
-
-// The narrowphase over stitched history windows (k_narrow_hist) with one wavefront per stencil, for
-// long histories.  The stitching (History.cpp:98-140) is a merge of the four vertices' timelines; every
-// lane runs the same merge (uniform control flow, identical values) 65 steps at a time and keeps the
-// stitched positions of two consecutive steps, so lane l holds window W0 + l of a 64-window chunk and
-// tests it.  The first window in order that collides (the lowest set bit of a ballot, in the first
-// chunk with any) gives the answer, as the sequential loop's early exit does.
-template <bool VF, class M>
-__global__ __launch_bounds__(64) CCD_TWO_WAVES void k_narrow_hist_wave(
-    const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
-    const int4 *__restrict__ keys, const double *__restrict__ eta, double eta_s, int64_t n, uint8_t *__restrict__ hit,
-    double *__restrict__ tout, uint8_t *__restrict__ sub, int32_t *__restrict__ win)
-{
-    using ccd::V3;
-    const int64_t i = blockIdx.x;
-    if (i >= n) return;
-    const int lane = (int)__lane_id();
-    const int4 k = keys[i];
-    const int v[4] = {k.x, k.y, k.z, k.w};
-    const double e = eta ? eta[i] : eta_s;
-    int64_t its[4], ends[4];
-    int64_t total = 0;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        its[j] = off[v[j]];
-        ends[j] = off[v[j] + 1];
-        total += ends[j] - its[j];
-    }
-    double curtime = 0.0;
-    int64_t g = 0;   // step index of the sequential loop (its guard); cur is evaluated at curtime
-    int r = -1, w = -1;
-    double t = 0.0;
-    bool alive = true;
-    while (alive) {
-        const int64_t w0 = g;   // this chunk: windows w0 .. w0 + 63, window w = (step w, step w + 1)
-        V3 pa[4], pb[4];
-        bool va = false, vb = false;
-        for (int s = 0; s <= 64; s++) {
-            alive = g <= total && curtime <= 1.0;
-            if (!alive) break;
-            V3 cur[4];
-            double newtime = __builtin_inf();
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                int64_t next = its[j] + 1;
-                while (next != ends[j] && ht[next] <= curtime) {
-                    ++next;
-                    ++its[j];
-                }
-                V3 oldp = ccd::mk(hp[3 * its[j]], hp[3 * its[j] + 1], hp[3 * its[j] + 2]);
-                if (next == ends[j]) {
-                    cur[j] = oldp;
-                } else {
-                    V3 newp = ccd::mk(hp[3 * next], hp[3 * next + 1], hp[3 * next + 2]);
-                    double dt = ht[next] - ht[its[j]];
-                    double a = curtime - ht[its[j]];
-                    double b = ht[next] - curtime;
-                    cur[j] = ccd::mk((b * oldp.x + a * newp.x) / dt, (b * oldp.y + a * newp.y) / dt,
-                                     (b * oldp.z + a * newp.z) / dt);
-                    newtime = ccd::smin(newtime, ht[next]);
-                }
-            }
-            if (s == lane) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) pa[j] = cur[j];
-                va = true;
-            }
-            if (s == lane + 1) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) pb[j] = cur[j];
-                vb = true;
-            }
-            if (s == 64) break;   // the next chunk starts by evaluating this step again (idempotent)
-            curtime = newtime;
-            g++;
-        }
-        bool h = false;
-        int rl = -1;
-        double tl = 0.0;
-        if (va && vb) {
-            rl = VF ? ccd::check_vf_window(pa, pb, e, tl, M()) : ccd::check_ee_window(pa, pb, e, tl, M());
-            h = rl >= 0;
-        }
-        const unsigned long long m = __ballot(h);
-        if (m) {
-            const int f = __ffsll(m) - 1;
-            r = __shfl(rl, f);
-            t = __shfl(tl, f);
-            w = (int)(w0 + f);
-            break;
-        }
-    }
-    if (lane == 0) {
-        hit[i] = r >= 0 ? 1 : 0;
-        if (tout) tout[i] = r >= 0 ? t : 0.0;
-        if (sub) sub[i] = r >= 0 ? (uint8_t)r : (uint8_t)255;
-        if (win) win[i] = r >= 0 ? w : -1;
-    }
-}
-
-// The trajectory scan of planeTrajectoryIntersect (SeparatingPlaneNarrowPhase.cpp:216-265) split over
-// the 64 lanes of a wavefront that all run the same stencil: each lane tests one history segment of a
-// 64-segment chunk, and the first segment in scan order that meets the plane (the lowest lane whose
-// test passes, in the first chunk with any) gives the result, computed by that lane with the
-// sequential scan's own expressions.  Needs the whole wavefront active and on the same call.
-struct WaveScan {
-    __device__ double operator()(const ccd::HistCSR &h, int v, int start, bool forward, ccd::V3 ppos, ccd::V3 pvel,
-                                 ccd::V3 nrm, ccd::V3 ptstart, double tstart, double eta) const
-    {
-        using ccd::V3;
-        const double inf = ccd::bits_to_double(0x7ff0000000000000ll);
-        const int64_t b = h.off[v];
-        const int n = (int)(h.off[v + 1] - b);
-        const double dt = forward ? h.t[b + start] - tstart : tstart - h.t[b + start];
-        const double t = ccd::plane_intersect(ppos, (forward ? 1.0 : -1.0) * pvel, nrm, ptstart,
-                                              ccd::hist_pos(h, b + start), dt, eta);
-        if (t >= 0 && t <= dt) return t;
-        const int lane = (int)__lane_id();
-        if (forward) {
-            // segments (i, i + 1) for i = start .. n - 2, in increasing i
-            for (int base = start; base < n - 1; base += 64) {
-                const int i = base + lane;
-                bool hit = false;
-                double r = 0.0;
-                if (i < n - 1) {
-                    V3 npp = ppos + (h.t[b + i] - tstart) * pvel;
-                    double d = h.t[b + i + 1] - h.t[b + i];
-                    double u = ccd::plane_intersect(npp, pvel, nrm, ccd::hist_pos(h, b + i), ccd::hist_pos(h, b + i + 1),
-                                                    d, eta);
-                    hit = u >= 0 && u <= d;
-                    r = h.t[b + i] + u - tstart;
-                }
-                const unsigned long long m = __ballot(hit);
-                if (m) return __shfl(r, __ffsll(m) - 1);
-            }
-        } else {
-            // segments (i, i - 1) for i = start .. 1, in decreasing i
-            for (int base = start; base >= 1; base -= 64) {
-                const int i = base - lane;
-                bool hit = false;
-                double r = 0.0;
-                if (i >= 1) {
-                    V3 npp = ppos - (tstart - h.t[b + i]) * pvel;
-                    double d = h.t[b + i] - h.t[b + i - 1];
-                    double u = ccd::plane_intersect(npp, -1.0 * pvel, nrm, ccd::hist_pos(h, b + i),
-                                                    ccd::hist_pos(h, b + i - 1), d, eta);
-                    hit = u >= 0 && u <= d;
-                    r = tstart - (h.t[b + i] - u);
-                }
-                const unsigned long long m = __ballot(hit);
-                if (m) return __shfl(r, __ffsll(m) - 1);
-            }
-        }
-        return inf;
-    }
-};
-
-// SeparatingPlaneNarrowPhase with one wavefront per stencil, for long histories: the lanes share the
-// trajectory scans (WaveScan) and otherwise compute the same values, so control flow stays uniform.
-template <bool VF, class M>
-__global__ __launch_bounds__(64) CCD_TWO_WAVES void k_separating_plane_wave(
-    const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
-    const int4 *__restrict__ keys, const double *__restrict__ eta, double eta_s, int64_t n,
-    const unsigned long long *__restrict__ gap_bits, uint8_t *__restrict__ status, unsigned long long *undecided)
-{
-    const int64_t i = blockIdx.x;
-    if (i >= n) return;
-    const double eps = ccd::bits_to_double((long long)*gap_bits) / 4.0;
-    const int4 k = keys[i];
-    const int v[4] = {k.x, k.y, k.z, k.w};
-    ccd::HistCSR h{off, ht, hp};
-    const int r = ccd::separating_plane_check<VF>(h, v, eta ? eta[i] : eta_s, eps, M(), WaveScan());
-    if (__lane_id() == 0) {
-        status[i] = (uint8_t)r;
-        if (r == 2) atomicAdd(undecided, 1ull);
-    }
-}
-
 inline unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// One wavefront per block for the kernels that give each lane one stencil of very uneven cost (the
-// separating-plane recursion, the plain narrowphases): a wavefront's slot is refilled as soon as it
-// finishes instead of when the slowest of its block's wavefronts does.  Separating plane on the 256^2
-// cloth candidates: 92 ms with 256-thread blocks, 73 ms with 64.
+// One wavefront per block for the kernels that give each lane one stencil of very uneven cost: a wavefront's
+// slot is refilled as soon as it finishes instead of when the slowest of its block's wavefronts does.
 constexpr int LANE_BLOCK = 64;
 
 }   // namespace
@@ -543,36 +254,6 @@ int launch_narrow2_queue(ccd_ctx *ctx, bool vf, const double *qs, const double *
     return CCD_OK;
 }
 
-int launch_narrow_hist(ccd_ctx *ctx, bool vf, const int64_t *off, const double *ht, const double *hp,
-                       const int32_t *keys, const double *eta, double eta_s, int64_t n, uint8_t *hit, double *t,
-                       uint8_t *sub, int32_t *win, bool wave)
-{
-    if (n == 0) return CCD_OK;
-    if (wave) {
-        if (n > 0x7fffffffll) return set_error(ctx, CCD_E_INVALID, "too many stencils for one launch");
-        if (vf)
-            CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_narrow_hist_wave<true, M>), dim3((unsigned)n), dim3(64), 0,
-                                                      ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n, hit,
-                                                      t, sub, win));
-        else
-            CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_narrow_hist_wave<false, M>), dim3((unsigned)n), dim3(64), 0,
-                                                      ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n, hit,
-                                                      t, sub, win));
-        CCD_LAUNCH_CHECK(ctx);
-        return CCD_OK;
-    }
-    if (vf)
-        CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_narrow_hist<true, M>), dim3(blocks_for(n, LANE_BLOCK)), dim3(LANE_BLOCK), 0,
-                                                  ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n, hit, t,
-                                                  sub, win));
-    else
-        CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_narrow_hist<false, M>), dim3(blocks_for(n, LANE_BLOCK)), dim3(LANE_BLOCK), 0,
-                                                  ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n, hit, t,
-                                                  sub, win));
-    CCD_LAUNCH_CHECK(ctx);
-    return CCD_OK;
-}
-
 int launch_min_gap(ccd_ctx *ctx, const int64_t *off, const double *ht, int64_t nverts, uint64_t *gap_bits)
 {
     hipLaunchKernelGGL(k_set_bits, dim3(1), dim3(1), 0, ctx->stream, (unsigned long long *)gap_bits,
@@ -582,60 +263,6 @@ int launch_min_gap(ccd_ctx *ctx, const int64_t *off, const double *ht, int64_t n
     unsigned grid = (unsigned)std::min<int64_t>(blocks_for(nverts, 256), 4096);
     hipLaunchKernelGGL(k_min_gap, dim3(grid), dim3(256), 0, ctx->stream, off, ht, nverts,
                        (unsigned long long *)gap_bits);
-    CCD_LAUNCH_CHECK(ctx);
-    return CCD_OK;
-}
-
-int launch_separating_plane(ccd_ctx *ctx, bool vf, const int64_t *off, const double *ht, const double *hp,
-                            const int32_t *keys, const double *eta, double eta_s, int64_t n, const uint64_t *gap_bits,
-                            uint8_t *status, int64_t *undecided, bool wave)
-{
-    if (n == 0) return CCD_OK;
-    auto gb = (const unsigned long long *)gap_bits;
-    auto und = (unsigned long long *)undecided;
-    if (wave) {
-        if (n > 0x7fffffffll) return set_error(ctx, CCD_E_INVALID, "too many stencils for one launch");
-        if (vf)
-            CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_separating_plane_wave<true, M>), dim3((unsigned)n), dim3(64),
-                                                      0, ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n,
-                                                      gb, status, und));
-        else
-            CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_separating_plane_wave<false, M>), dim3((unsigned)n),
-                                                      dim3(64), 0, ctx->stream, off, ht, hp, (const int4 *)keys, eta,
-                                                      eta_s, n, gb, status, und));
-        CCD_LAUNCH_CHECK(ctx);
-        return CCD_OK;
-    }
-    // Order the stencils so that those decided at the root run together (results are per stencil and
-    // land at the stencil's own index, so the order changes nothing else).
-    const int32_t *order = nullptr;
-    if (n >= 4096 && n <= 0x7fffffffll) {   // int32 order indices
-        uint64_t *key = (uint64_t *)buffer(ctx, "spo_key", (size_t)n * 8);
-        uint64_t *key2 = (uint64_t *)buffer(ctx, "spo_key2", (size_t)n * 8);
-        int32_t *idx = (int32_t *)buffer(ctx, "spo_idx", (size_t)n * 4);
-        int32_t *idx2 = (int32_t *)buffer(ctx, "spo_idx2", (size_t)n * 4);
-        void *tmp = buffer(ctx, "spo_tmp", radix_sort_temp_bytes(n));
-        if (!key || !key2 || !idx || !idx2 || !tmp) return CCD_E_OOM;
-        if (vf)
-            hipLaunchKernelGGL(k_sp_order_key<true>, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, off, ht, hp,
-                               (const int4 *)keys, eta, eta_s, n, gb, key, idx);
-        else
-            hipLaunchKernelGGL(k_sp_order_key<false>, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, off, ht, hp,
-                               (const int4 *)keys, eta, eta_s, n, gb, key, idx);
-        CCD_LAUNCH_CHECK(ctx);
-        bool in_alt = false;
-        int rc = radix_sort_pairs(ctx, key, idx, key2, idx2, n, 1, tmp, in_alt);   // one stable pass
-        if (rc) return rc;
-        order = in_alt ? idx2 : idx;
-    }
-    if (vf)
-        CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_separating_plane<true, M>), dim3(blocks_for(n, LANE_BLOCK)), dim3(LANE_BLOCK),
-                                                  0, ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n, gb,
-                                                  status, und, order));
-    else
-        CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_separating_plane<false, M>), dim3(blocks_for(n, LANE_BLOCK)), dim3(LANE_BLOCK),
-                                                  0, ctx->stream, off, ht, hp, (const int4 *)keys, eta, eta_s, n, gb,
-                                                  status, und, order));
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }

@@ -46,23 +46,57 @@ __device__ __forceinline__ int region_length(int64_t n, int regions)
 }
 __device__ __forceinline__ int region_of(int block, int regions) { return (block & 7) * (regions >> 3) + (block >> 3); }
 
-__device__ __forceinline__ void load_window(const double *__restrict__ qs, const double *__restrict__ qe, int4 k, V3 *s,
-                                            V3 *e)
-{
-    const int v[4] = {k.x, k.y, k.z, k.w};
-#pragma unroll
-    for (int q = 0; q < 4; q++) window_pos(qs, qe, v[q], s[q], e[q]);
-}
-// Vertices by their place in the stencil, a runtime index: read again, since selecting from arrays of
-// positions would keep those in scratch memory.
-struct VertexAt {
-    const double *qs, *qe;
-    int4 k;
-    __device__ __forceinline__ void operator()(int w, V3 &x, V3 &y) const
+// Where the stencils' windows come from.  at(i) gives the i-th stencil's vertices by their place in it, a
+// runtime index: read again, since selecting from arrays of positions would keep those in scratch memory.
+// extent: a region's first stencil and its length.
+struct KeyedWindows {   // two-entry histories, by the vertices' numbers
+    const double *__restrict__ qs, *__restrict__ qe;
+    const int4 *__restrict__ keys;
+    const int64_t *__restrict__ n_dev;   // may exceed n_max: an overflowing broadphase counts every stencil
+    int64_t n_max;
+    struct At {
+        const double *qs, *qe;
+        int4 k;
+        __device__ __forceinline__ void operator()(int w, V3 &x, V3 &y) const
+        {
+            window_pos(qs, qe, w == 0 ? k.x : (w == 1 ? k.y : (w == 2 ? k.z : k.w)), x, y);
+        }
+    };
+    __device__ __forceinline__ At at(int64_t i) const { return At{qs, qe, keys[i]}; }
+    __device__ __forceinline__ int4 key(int64_t i) const { return keys[i]; }
+    __device__ __forceinline__ int extent(int r, int regions, int64_t &begin) const
     {
-        window_pos(qs, qe, w == 0 ? k.x : (w == 1 ? k.y : (w == 2 ? k.z : k.w)), x, y);
+        const int64_t n = n_dev && *n_dev < n_max ? *n_dev : n_max;
+        const int len = region_length(n, regions);
+        begin = (int64_t)r * len;
+        return (int)(begin < n ? (n - begin < len ? n - begin : len) : 0);
     }
 };
+struct PooledWindows {   // a pool of windows with their positions: eight vertices each, four at the start, four at the end
+    ccdi::WindowPool pool;
+    struct At {
+        const double *p;
+        __device__ __forceinline__ void operator()(int w, V3 &x, V3 &y) const
+        {
+            x = ccd::mk(p[3 * w], p[3 * w + 1], p[3 * w + 2]);
+            y = ccd::mk(p[12 + 3 * w], p[13 + 3 * w], p[14 + 3 * w]);
+        }
+    };
+    __device__ __forceinline__ At at(int64_t i) const { return At{pool.pos + 24 * i}; }
+    __device__ __forceinline__ int4 key(int64_t) const { return make_int4(0, 0, 0, 0); }
+    __device__ __forceinline__ int extent(int r, int, int64_t &begin) const
+    {
+        begin = (int64_t)r * 64;
+        const int64_t shard = begin / pool.per_shard, left = pool.filled(shard) - (begin - shard * pool.per_shard);
+        return (int)(left < 0 ? 0 : (left < 64 ? left : 64));
+    }
+};
+template <class At>
+__device__ __forceinline__ void load_window(const At &at, V3 *s, V3 *e)
+{
+#pragma unroll
+    for (int q = 0; q < 4; q++) at(q, s[q], e[q]);
+}
 template <bool PER_STENCIL>
 __device__ __forceinline__ void store_result(const NarrowOut &o, int64_t i, int r, double t)
 {
@@ -76,17 +110,14 @@ __device__ __forceinline__ int rank_in(uint64_t mask) { return __popcll(mask & (
 
 // Without a solver the registers would allow three wavefronts per SIMD as well as two; the kernel is bound by
 // its FP64 instructions (about 1,270 for an edge-edge stencil).
-template <bool VF, bool PER_STENCIL>
+template <bool VF, bool PER_STENCIL, class Windows>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_screen(
-    const double *__restrict__ qs, const double *__restrict__ qe, const int4 *__restrict__ keys,
-    const int64_t *__restrict__ n_dev, int64_t n_max, double eta, NarrowOut o, OpenLists l)
+    Windows windows, double eta, NarrowOut o, OpenLists l)
 {
-    // The device count may exceed the stored keys (an overflowing broadphase counts every stencil).
-    const int64_t n = n_dev && *n_dev < n_max ? *n_dev : n_max;
     const int lane = __lane_id();
-    const int r = region_of(blockIdx.x, l.regions), len = region_length(n, l.regions);
-    const int64_t begin = (int64_t)r * len;
-    const int cnt = (int)(begin < n ? (n - begin < len ? n - begin : len) : 0);
+    const int r = region_of(blockIdx.x, l.regions);
+    int64_t begin;
+    const int cnt = windows.extent(r, l.regions, begin);
     int na = 0, nb = 0;
     for (int j0 = 0; j0 < cnt; j0 += 64) {
         const int j = j0 + lane;
@@ -94,7 +125,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         if (j < cnt) {
             const int64_t i = begin + j;
             V3 s[4], e[4];
-            load_window(qs, qe, keys[i], s, e);
+            load_window(windows.at(i), s, e);
             const double et = PER_STENCIL && o.eta ? o.eta[i] : eta;
             m = VF ? ccd::screen_vf_window(s, e, et) : ccd::screen_ee_window(s, e, et);
             store_result<PER_STENCIL>(o, i, -1, 0.0);   // a hit found later replaces it
@@ -117,16 +148,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 
 // One wavefront per region and list; a list is compacted in place (an entry moves only to where entries
 // were read before).
-template <bool VF, bool PER_STENCIL>
+template <bool VF, bool PER_STENCIL, class Windows>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_refine(
-    const double *__restrict__ qs, const double *__restrict__ qe, const int4 *__restrict__ keys,
-    const int64_t *__restrict__ n_dev, int64_t n_max, double eta, NarrowOut o, OpenLists l)
+    Windows windows, double eta, NarrowOut o, OpenLists l)
 {
-    const int64_t n = n_dev && *n_dev < n_max ? *n_dev : n_max;
     const int lane = __lane_id();
     const bool list_b = (int)blockIdx.x >= l.regions;
     const int r = region_of(list_b ? blockIdx.x - l.regions : blockIdx.x, l.regions);
-    const int64_t begin = (int64_t)r * region_length(n, l.regions);
+    int64_t begin;
+    windows.extent(r, l.regions, begin);
     int32_t *count = l.count + (list_b ? l.regions : 0) + r;
     const int cnt = *count;
     if (cnt == 0) return;
@@ -140,10 +170,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         if (j < cnt) {
             off = list[begin + j];
             const int64_t i = begin + off;
-            const VertexAt at{qs, qe, keys[i]};
+            const auto at = windows.at(i);
             const double et = PER_STENCIL && o.eta ? o.eta[i] : eta;
             V3 s[4], e[4];
-            load_window(qs, qe, at.k, s, e);
+            load_window(at, s, e);
             if (list_b) {
                 m = l.mask[begin + j];
                 m = ccd::refine_others<VF>(s, e, et, m, at);
@@ -164,16 +194,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 
 // Three wavefronts per SIMD (168 registers, a few spills): the root solves are chains of dependent FP64
 // operations, and a third wavefront hides more of their latency than the spills cost.
-template <bool VF, bool PER_STENCIL>
+template <bool VF, bool PER_STENCIL, class Windows>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_solve(
-    const double *__restrict__ qs, const double *__restrict__ qe, const int4 *__restrict__ keys,
-    const int64_t *__restrict__ n_dev, int64_t n_max, double eta, NarrowOut o, OpenLists l)
+    Windows windows, double eta, NarrowOut o, OpenLists l)
 {
-    const int64_t n = n_dev && *n_dev < n_max ? *n_dev : n_max;
     const int lane = __lane_id();
     const bool list_b = (int)blockIdx.x >= l.regions;
     const int r = region_of(list_b ? blockIdx.x - l.regions : blockIdx.x, l.regions);
-    const int64_t begin = (int64_t)r * region_length(n, l.regions);
+    int64_t begin;
+    windows.extent(r, l.regions, begin);
     const int cnt = l.count[(list_b ? l.regions : 0) + r];
     for (int j0 = 0; j0 < cnt; j0 += 64) {
         const int j = j0 + lane;
@@ -182,8 +211,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         int sub = -1;
         if (j < cnt) {
             const int64_t i = begin + (list_b ? l.b : l.a)[begin + j];
-            k = keys[i];
-            const VertexAt at{qs, qe, k};
+            k = windows.key(i);
+            const auto at = windows.at(i);
             const double et = PER_STENCIL && o.eta ? o.eta[i] : eta;
             unsigned m = list_b ? l.mask[begin + j] : ccd::SCREEN_PRIMARY;
             const bool also_a = list_b && (m & ccd::SCREEN_PRIMARY);
@@ -194,7 +223,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 int found = -1;
                 if (again || !list_b) {
                     V3 s[4], e[4];
-                    load_window(qs, qe, k, s, e);
+                    load_window(at, s, e);
                     found = ccd::check_masked<VF>(s, e, et, tt, ccd::SCREEN_PRIMARY, at, ccd::NoCount());
                 } else {
                     found = ccd::check_others<VF>(et, tt, m, at, ccd::NoCount());
@@ -239,24 +268,22 @@ void *open_list(ccd_ctx *ctx, int64_t n)
     return buffer(ctx, "open_list", (size_t)open_list_bytes(n));
 }
 
-template <bool VF, bool PER_STENCIL>
-static int launch_passes(ccd_ctx *ctx, const double *qs, const double *qe, const int32_t *keys, const int64_t *n_dev,
-                         int64_t n, double eta, const NarrowOut &o, int tile, void *list)
+template <bool VF, bool PER_STENCIL, class Windows>
+static int launch_passes(ccd_ctx *ctx, const Windows &w, double eta, const NarrowOut &o, int64_t len, int regions, void *list)
 {
-    const int64_t len = region_max_length(n, tile);
     OpenLists l;
-    l.regions = (int)(((n + len - 1) / len + 7) / 8 * 8);
-    const int64_t cap = l.regions * len;
+    l.regions = regions;
+    const int64_t cap = regions * len;
     l.count = (int32_t *)list;
     l.a = (uint16_t *)(l.count + 2 * (MAX_REGIONS + 8));
     l.b = l.a + cap;
     l.mask = (uint8_t *)(l.b + cap);
-    const dim3 one((unsigned)l.regions), both((unsigned)(2 * l.regions)), wave(64);
-    hipLaunchKernelGGL((k_screen<VF, PER_STENCIL>), one, wave, 0, ctx->stream, qs, qe, (const int4 *)keys, n_dev, n, eta, o, l);
+    const dim3 one((unsigned)regions), both((unsigned)(2 * regions)), wave(64);
+    hipLaunchKernelGGL((k_screen<VF, PER_STENCIL, Windows>), one, wave, 0, ctx->stream, w, eta, o, l);
     CCD_LAUNCH_CHECK(ctx);
-    hipLaunchKernelGGL((k_refine<VF, PER_STENCIL>), both, wave, 0, ctx->stream, qs, qe, (const int4 *)keys, n_dev, n, eta, o, l);
+    hipLaunchKernelGGL((k_refine<VF, PER_STENCIL, Windows>), both, wave, 0, ctx->stream, w, eta, o, l);
     CCD_LAUNCH_CHECK(ctx);
-    hipLaunchKernelGGL((k_solve<VF, PER_STENCIL>), both, wave, 0, ctx->stream, qs, qe, (const int4 *)keys, n_dev, n, eta, o, l);
+    hipLaunchKernelGGL((k_solve<VF, PER_STENCIL, Windows>), both, wave, 0, ctx->stream, w, eta, o, l);
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }
@@ -264,9 +291,24 @@ static int launch_passes(ccd_ctx *ctx, const double *qs, const double *qe, const
 int launch_screened(ccd_ctx *ctx, bool vf, bool per_stencil, const double *qs, const double *qe, const int32_t *keys,
                     const int64_t *n_dev, int64_t n, double eta, const NarrowOut &o, int tile, void *list)
 {
-    auto f = vf ? (per_stencil ? launch_passes<true, true> : launch_passes<true, false>)
-                : (per_stencil ? launch_passes<false, true> : launch_passes<false, false>);
-    return f(ctx, qs, qe, keys, n_dev, n, eta, o, tile, list);
+    const KeyedWindows w{qs, qe, (const int4 *)keys, n_dev, n};
+    const int64_t len = region_max_length(n, tile);
+    const int regions = (int)(((n + len - 1) / len + 7) / 8 * 8);
+    auto f = vf ? (per_stencil ? launch_passes<true, true, KeyedWindows> : launch_passes<true, false, KeyedWindows>)
+                : (per_stencil ? launch_passes<false, true, KeyedWindows> : launch_passes<false, false, KeyedWindows>);
+    return f(ctx, w, eta, o, len, regions, list);
+}
+
+// One chunk of 64 windows to a region: their positions lie side by side, so longer regions would gain nothing.
+int launch_screened_pool(ccd_ctx *ctx, bool vf, const WindowPool &pool, void *list)
+{
+    NarrowOut o;
+    o.eta = pool.eta;
+    o.hit = pool.hit;
+    o.t = pool.t;
+    o.sub = pool.sub;
+    auto f = vf ? launch_passes<true, true, PooledWindows> : launch_passes<false, true, PooledWindows>;
+    return f(ctx, PooledWindows{pool}, 0.0, o, 64, (int)(WindowPool::SHARDS * pool.per_shard / 64), list);
 }
 
 }   // namespace ccdi
