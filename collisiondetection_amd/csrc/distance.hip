@@ -18,7 +18,6 @@
 //      non-negative doubles, whose integer order is their numeric order.
 #include <cmath>
 #include <cstring>
-#include <vector>
 
 #include "ccd_core.h"
 #include "ccd_internal.h"
@@ -161,8 +160,51 @@ __global__ __launch_bounds__(256) void k_face_pair_bound(const double *__restric
     block_min_into(best, best_bits);
 }
 
-// Step 1b: cell keys.  Cell coordinates (21 bits each, clamped) of (x - lo) * inv, packed z, y, x so that
-// the three cells x-1, x, x+1 of one (y, z) row are consecutive keys.
+// The vertices' bounding box, one partial box per block (lo, hi): NaN coordinates count only in vertex 0, where
+// they make the box NaN and the caller does without a grid.  Read back instead of the vertices: 24 bytes
+// each, copied and compared by the host, took 150 us of a call on 40,401 vertices.
+constexpr int BOX_BLOCKS = 64;
+__global__ __launch_bounds__(256) void k_box(const double *__restrict__ v, int64_t V, double *__restrict__ partial)
+{
+    __shared__ double red[2][3][4];
+    double lo[3], hi[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) lo[k] = hi[k] = v[k];
+    for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < V; i += (int64_t)gridDim.x * 256)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const double x = v[3 * i + k];
+            lo[k] = x < lo[k] ? x : lo[k];
+            hi[k] = hi[k] < x ? x : hi[k];
+        }
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            const double a = __shfl_xor(lo[k], d), b = __shfl_xor(hi[k], d);
+            lo[k] = a < lo[k] ? a : lo[k];
+            hi[k] = hi[k] < b ? b : hi[k];
+        }
+        if ((threadIdx.x & 63) == 0) {
+            red[0][k][threadIdx.x >> 6] = lo[k];
+            red[1][k][threadIdx.x >> 6] = hi[k];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        const int k = threadIdx.x % 3, up = threadIdx.x / 3;
+        double x = red[up][k][0];
+        for (int w = 1; w < 4; w++) {
+            const double y = red[up][k][w];
+            x = up ? (x < y ? y : x) : (y < x ? y : x);
+        }
+        partial[6 * blockIdx.x + threadIdx.x] = x;
+    }
+}
+
+// Step 1b: cell keys.  Cell coordinates (clamped) of (x - lo) * inv, packed z, y, x so that the three cells
+// x-1, x, x+1 of one (y, z) row are consecutive keys.  x takes sx bits and y the next sy - sx: enough for
+// every coordinate and its neighbour, and few, since each 8 bits are a pass of the sort.
 constexpr uint64_t CELL_MAX = (1ull << 21) - 1;
 __device__ __forceinline__ uint64_t cell_coord(double x, double lo, double inv)
 {
@@ -172,20 +214,21 @@ __device__ __forceinline__ uint64_t cell_coord(double x, double lo, double inv)
     return (uint64_t)s;
 }
 __global__ __launch_bounds__(256) void k_cell_keys(const double *__restrict__ v, int64_t V, double lx, double ly,
-                                                   double lz, double inv, uint64_t *__restrict__ key,
-                                                   int32_t *__restrict__ idx)
+                                                   double lz, double inv, int sx, int sy,
+                                                   uint64_t *__restrict__ key, int32_t *__restrict__ idx)
 {
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= V) return;
     uint64_t cx = cell_coord(v[3 * i], lx, inv), cy = cell_coord(v[3 * i + 1], ly, inv),
              cz = cell_coord(v[3 * i + 2], lz, inv);
-    key[i] = (cz << 42) | (cy << 21) | cx;
+    key[i] = (cz << sy) | (cy << sx) | cx;
     idx[i] = (int32_t)i;
 }
 
 // Step 1c: each vertex against the vertices of its 27 surrounding cells (9 rows of 3 consecutive keys).
 __global__ __launch_bounds__(256) void k_grid_closest(const double *__restrict__ v, int64_t V, double lx, double ly,
-                                                      double lz, double inv, const uint64_t *__restrict__ key,
+                                                      double lz, double inv, int sx, int sy,
+                                                      const uint64_t *__restrict__ key,
                                                       const int32_t *__restrict__ idx,
                                                       const int32_t *__restrict__ faces,
                                                       const int32_t *__restrict__ voff,
@@ -203,7 +246,7 @@ __global__ __launch_bounds__(256) void k_grid_closest(const double *__restrict__
             for (int dy = -1; dy <= 1; dy++) {
                 const int64_t y = cy + dy, z = cz + dz;
                 if (y < 0 || z < 0 || y > (int64_t)CELL_MAX || z > (int64_t)CELL_MAX) continue;
-                const uint64_t row = ((uint64_t)z << 42) | ((uint64_t)y << 21);
+                const uint64_t row = ((uint64_t)z << sy) | ((uint64_t)y << sx);
                 const uint64_t k0 = row | (uint64_t)(cx > 0 ? cx - 1 : 0);
                 const uint64_t k1 = row | (uint64_t)(cx < (int64_t)CELL_MAX ? cx + 1 : CELL_MAX);
                 int64_t lo = 0, hi = V;   // first key >= k0
@@ -272,7 +315,7 @@ int mesh_self_distance(ccd_ctx *ctx, const double *verts, int64_t V, const int32
                        const uint8_t *fixed, double *out, int64_t *nvf, int64_t *nee)
 {
     hipStream_t st = ctx->stream;
-    unsigned long long *best = (unsigned long long *)buffer(ctx, "selfdist_best", 16);
+    unsigned long long *best = (unsigned long long *)buffer(ctx, "selfdist_best", 16 + BOX_BLOCKS * 6 * 8);
     if (!best) return CCD_E_OOM;
     const unsigned long long inf_bits = 0x7ff0000000000000ull;
     int rc = build_vertex_face_table(ctx, faces, F, V);
@@ -288,17 +331,21 @@ int mesh_self_distance(ccd_ctx *ctx, const double *verts, int64_t V, const int32
         unsigned g = (unsigned)std::min<int64_t>(blocks_for(F, 256), 4096);
         hipLaunchKernelGGL(k_face_pair_bound, dim3(g), dim3(256), 0, st, verts, faces, F, voff, vlist, best);
         CCD_LAUNCH_CHECK(ctx);
-        std::vector<double> hv((size_t)3 * V);
-        CCD_HIP_CHECK(ctx, hipMemcpyAsync(hv.data(), verts, (size_t)V * 24, hipMemcpyDeviceToHost, st));
-        unsigned long long b0 = inf_bits;
-        CCD_HIP_CHECK(ctx, hipMemcpyAsync(&b0, best, 8, hipMemcpyDeviceToHost, st));
+        const int nb = (int)std::min<int64_t>(BOX_BLOCKS, blocks_for(V, 256));
+        hipLaunchKernelGGL(k_box, dim3(nb), dim3(256), 0, st, verts, V, (double *)(best + 2));
+        CCD_LAUNCH_CHECK(ctx);
+        double h[2 + BOX_BLOCKS * 6];
+        CCD_HIP_CHECK(ctx, hipMemcpyAsync(h, best, (2 + 6 * (size_t)nb) * 8, hipMemcpyDeviceToHost, st));
         CCD_HIP_CHECK(ctx, hipStreamSynchronize(st));
-        memcpy(&r02, &b0, 8);
-        for (int k = 0; k < 3; k++) lo[k] = hi[k] = hv[k];
-        for (int64_t i = 1; i < V; i++)
+        r02 = h[0];
+        for (int k = 0; k < 3; k++) {
+            lo[k] = h[2 + k];
+            hi[k] = h[5 + k];
+        }
+        for (int i = 1; i < nb; i++)
             for (int k = 0; k < 3; k++) {
-                lo[k] = std::min(lo[k], hv[3 * i + k]);
-                hi[k] = std::max(hi[k], hv[3 * i + k]);
+                lo[k] = std::min(lo[k], h[2 + 6 * i + k]);
+                hi[k] = std::max(hi[k], h[5 + 6 * i + k]);
             }
     }
     // Cells at least r0 wide (with a relative margin that covers the rounding of the cell coordinates),
@@ -310,6 +357,12 @@ int mesh_self_distance(ccd_ctx *ctx, const double *verts, int64_t V, const int32
     if (grid) {
         // Step 1b/1c: vertices sorted by cell, each against its 27 surrounding cells.
         const double inv = 1.0 / cell;
+        int bits[3];
+        for (int k = 0; k < 3; k++) {   // (a coordinate is at most 2^20 + 1 here)
+            const uint64_t most = (uint64_t)((hi[k] - lo[k]) * inv) + 1;
+            for (bits[k] = 1; most >> bits[k];) bits[k]++;
+        }
+        const int sx = bits[0], sy = bits[0] + bits[1];
         uint64_t *key = (uint64_t *)buffer(ctx, "grid_key", (size_t)V * 8);
         uint64_t *key2 = (uint64_t *)buffer(ctx, "grid_key2", (size_t)V * 8);
         int32_t *idx = (int32_t *)buffer(ctx, "grid_idx", (size_t)V * 4);
@@ -317,13 +370,13 @@ int mesh_self_distance(ccd_ctx *ctx, const double *verts, int64_t V, const int32
         void *tmp = buffer(ctx, "grid_tmp", radix_sort_temp_bytes(V));
         if (!key || !key2 || !idx || !idx2 || !tmp) return CCD_E_OOM;
         hipLaunchKernelGGL(k_cell_keys, dim3(blocks_for(V, 256)), dim3(256), 0, st, verts, V, lo[0], lo[1], lo[2], inv,
-                           key, idx);
+                           sx, sy, key, idx);
         CCD_LAUNCH_CHECK(ctx);
         bool in_alt = false;
-        rc = radix_sort_pairs(ctx, key, idx, key2, idx2, V, 64, tmp, in_alt);
+        rc = radix_sort_pairs(ctx, key, idx, key2, idx2, V, sy + bits[2], tmp, in_alt);
         if (rc) return rc;
         hipLaunchKernelGGL(k_grid_closest, dim3(blocks_for(V, 256)), dim3(256), 0, st, verts, V, lo[0], lo[1], lo[2],
-                           inv, in_alt ? key2 : key, in_alt ? idx2 : idx, faces, voff, vlist, best);
+                           inv, sx, sy, in_alt ? key2 : key, in_alt ? idx2 : idx, faces, voff, vlist, best);
         CCD_LAUNCH_CHECK(ctx);
     } else if (V > 0 && F > 0 && r02 != 0.0) {
         int64_t slices = std::max<int64_t>(1, std::min<int64_t>(64, (int64_t)8192 / std::max<int64_t>(1, blocks_for(V, 256))));
