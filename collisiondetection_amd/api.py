@@ -224,6 +224,24 @@ def _fixed_mask(fixed, V, ctx):
     return to_device(m, torch.uint8, ctx)
 
 
+class _DeviceKeys:
+    """Stencil keys in memory that a context owns, for torch to copy."""
+
+    def __init__(self, ptr, n):
+        self.__cuda_array_interface__ = {"shape": (n, 4), "typestr": "<i4", "data": (ptr, False), "version": 2}
+
+
+def _last_candidates(ctx):
+    """Copies of the candidates of the context's last call, int32 tensors of shape (n, 4)."""
+    torch = _torch()
+    pv, pe = ctypes.c_void_p(), ctypes.c_void_p()
+    nv, ne = ctypes.c_int64(0), ctypes.c_int64(0)
+    ctx.check(N.lib().ccd_last_candidates(ctx.ptr, ctypes.byref(pv), ctypes.byref(nv), ctypes.byref(pe),
+                                          ctypes.byref(ne)))
+    return tuple(torch.as_tensor(_DeviceKeys(p.value, n.value), device=ctx.torch_device).clone() if n.value else
+                 torch.empty((0, 4), dtype=torch.int32, device=ctx.torch_device) for p, n in ((pv, nv), (pe, ne)))
+
+
 def kdop_candidates(faces, qstart, qend, outer_eta, fixed=None, sort=True, ctx: Context | None = None,
                     hist=None, as_numpy=True):
     """KDOPBroadPhase candidate sets -> (vf, ee) int32 arrays of shape (n, 4).
@@ -248,24 +266,19 @@ def kdop_candidates(faces, qstart, qend, outer_eta, fixed=None, sort=True, ctx: 
     fx = _fixed_mask(fixed, V, ctx)
     nv = ctypes.c_int64(0)
     ne = ctypes.c_int64(0)
-    cap_v, cap_e = 0, 0
-    for _ in range(2):
-        vf = torch.empty(max(cap_v, 1) * 4, dtype=torch.int32, device=ctx.torch_device)
-        ee = torch.empty(max(cap_e, 1) * 4, dtype=torch.int32, device=ctx.torch_device)
-        if hist is None:
-            rc = N.lib().ccd_kdop_candidates(ctx.ptr, _ptr(fd), F, _ptr(qs), _ptr(qe), V, float(outer_eta), _ptr(fx),
-                                             _ptr(vf), cap_v, ctypes.byref(nv), _ptr(ee), cap_e, ctypes.byref(ne), flags)
-        else:
-            rc = N.lib().ccd_kdop_candidates_history(ctx.ptr, _ptr(fd), F, _ptr(off), _ptr(hp), V, E,
-                                                     float(outer_eta), _ptr(fx), _ptr(vf), cap_v, ctypes.byref(nv),
-                                                     _ptr(ee), cap_e, ctypes.byref(ne), flags)
-        if rc == N.CCD_E_CAPACITY:
-            cap_v, cap_e = nv.value, ne.value
-            continue
+    # Without room for them the candidates stay in the context's buffers; they are copied from there, which
+    # needs their numbers first but no second broadphase.
+    if hist is None:
+        rc = N.lib().ccd_kdop_candidates(ctx.ptr, _ptr(fd), F, _ptr(qs), _ptr(qe), V, float(outer_eta), _ptr(fx),
+                                         None, 0, ctypes.byref(nv), None, 0, ctypes.byref(ne), flags)
+    else:
+        rc = N.lib().ccd_kdop_candidates_history(ctx.ptr, _ptr(fd), F, _ptr(off), _ptr(hp), V, E,
+                                                 float(outer_eta), _ptr(fx), None, 0, ctypes.byref(nv),
+                                                 None, 0, ctypes.byref(ne), flags)
+    if rc != N.CCD_E_CAPACITY:
         ctx.check(rc)
-        break
+    vf, ee = _last_candidates(ctx)
     torch.cuda.synchronize(ctx.torch_device)
-    vf, ee = vf[: 4 * nv.value].reshape(-1, 4), ee[: 4 * ne.value].reshape(-1, 4)
     if not as_numpy:
         return vf, ee
     return vf.cpu().numpy(), ee.cpu().numpy()
