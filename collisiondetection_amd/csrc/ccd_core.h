@@ -1593,14 +1593,13 @@ CCD_HD unsigned screen_ee_window(const V3 *s, const V3 *e, double eta)
 // Of 200,000 stencils each, left open by the screen and then by 16 parts: a 200^2 cloth 49% -> 1.6%
 // vertex-face, 58% -> 9.2% edge-edge; a 330^2 sheet 2.5% -> 0.05%, 13% -> 3.2%.
 // ------------------------------------------------------------------------------------------------
-constexpr int REFINE_LEAVES = 16;
-constexpr unsigned REFINE_ALL = (1u << REFINE_LEAVES) - 1u;
+constexpr int REFINE_LEAVES = 16;   // at most 32; a power of two, so that the parts' ends are exact
 constexpr double REFINE_TOL = 1e-10, REFINE_SLOPE_TOL = 1e-13, REFINE_DISTANCE_TOL = 1e-12;
 
 struct Rejected {
     unsigned parts = 0, unclean = 0;   // bit per part
     // The parts on which the list can be relied on to hold no time.
-    CCD_FHD unsigned usable() const { return unclean == 0 || parts == REFINE_ALL ? parts : 0u; }
+    CCD_FHD unsigned usable(unsigned all) const { return unclean == 0 || parts == all ? parts : 0u; }
 };
 
 // Bernstein coefficients of p on [a, a + h].
@@ -1711,7 +1710,7 @@ CCD_FHD void refine_part(const DistancePoly &p, double minD, double a, double h,
 }
 
 // Whether a stencil's face or edge-edge test cannot hit.
-CCD_HD bool refine_vertex_face(const V3 *s, const V3 *e, double eta)
+CCD_HD bool refine_vertex_face(const V3 *s, const V3 *e, double eta, int leaves = REFINE_LEAVES)
 {
     const double minD = eta * eta;
     const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
@@ -1723,18 +1722,19 @@ CCD_HD bool refine_vertex_face(const V3 *s, const V3 *e, double eta)
                           plane_cubic(p3, cross(c, b), -c, vp3, cross(vc, vb), -vc)};
     const double m[3] = {largest(f[0]), largest(f[1]), largest(f[2])};
     Rejected rd, r[3];
-    constexpr double h = 1.0 / REFINE_LEAVES;
+    const double h = 1.0 / leaves;
+    const unsigned all = ~0u >> (32 - leaves);
 #pragma nounroll
-    for (int k = 0; k < REFINE_LEAVES; k++) {
+    for (int k = 0; k < leaves; k++) {
         const double at = k * h;
         const unsigned bit = 1u << k;
         refine_part(dp, minD, at, h, bit, rd);
 #pragma unroll
         for (int j = 0; j < 3; j++) refine_part(f[j], m[j], at, h, bit, r[j]);
     }
-    return (rd.usable() | r[0].usable() | r[1].usable() | r[2].usable()) == REFINE_ALL && max_coord(s, e) < SCREEN_MAX_COORD;
+    return (rd.usable(all) | r[0].usable(all) | r[1].usable(all) | r[2].usable(all)) == all && max_coord(s, e) < SCREEN_MAX_COORD;
 }
-CCD_HD bool refine_edge_edge(const V3 *s, const V3 *e, double eta)
+CCD_HD bool refine_edge_edge(const V3 *s, const V3 *e, double eta, int leaves = REFINE_LEAVES)
 {
     const double minD = eta * eta;
     const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
@@ -1750,20 +1750,21 @@ CCD_HD bool refine_edge_edge(const V3 *s, const V3 *e, double eta)
         barycentric_quartic(l1, -x, -moving_dot(x3, vx3, d2, vd2), moving_dot(x3, vx3, d1, vd1))};
     const double m[4] = {largest(f[0]), largest(f[1]), largest(f[2]), largest(f[3])};
     Rejected rd, r[4];
-    constexpr double h = 1.0 / REFINE_LEAVES;
+    const double h = 1.0 / leaves;
+    const unsigned all = ~0u >> (32 - leaves);
 #pragma nounroll
-    for (int k = 0; k < REFINE_LEAVES; k++) {
+    for (int k = 0; k < leaves; k++) {
         const double at = k * h;
         const unsigned bit = 1u << k;
         refine_part(dp, minD, at, h, bit, rd);
 #pragma unroll
         for (int j = 0; j < 4; j++) refine_part(f[j], m[j], at, h, bit, r[j]);
     }
-    return (rd.usable() | r[0].usable() | r[1].usable() | r[2].usable() | r[3].usable()) == REFINE_ALL &&
+    return (rd.usable(all) | r[0].usable(all) | r[1].usable(all) | r[2].usable(all) | r[3].usable(all)) == all &&
            max_coord(s, e) < SCREEN_MAX_COORD;
 }
 // Whether vertex_edge(q0, q1, q2) cannot hit.
-CCD_HD bool refine_vertex_edge(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, double eta)
+CCD_HD bool refine_vertex_edge(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, double eta, int leaves = REFINE_LEAVES)
 {
     const V3 v0 = q0e - q0s, v1 = q1e - q1s, v2 = q2e - q2s;
     const V3 ab = q2s - q1s, ac = q0s - q1s, cb = q2s - q0s, vab = v2 - v1, vac = v0 - v1, vcb = v2 - v0;
@@ -1772,9 +1773,10 @@ CCD_HD bool refine_vertex_edge(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, d
     const Poly<4> g = minus_colinear_quartic(moving_square(ab, vab), moving_square(ac, vac), e1, eta * eta);
     const double m[3] = {largest(f[0]), largest(f[1]), largest(g)};
     Rejected r[3];
-    constexpr double h = 1.0 / REFINE_LEAVES;
+    const double h = 1.0 / leaves;
+    const unsigned all = ~0u >> (32 - leaves);
 #pragma nounroll
-    for (int k = 0; k < REFINE_LEAVES; k++) {
+    for (int k = 0; k < leaves; k++) {
         const double at = k * h;
         const unsigned bit = 1u << k;
         refine_part(f[0], m[0], at, h, bit, r[0]);
@@ -1782,7 +1784,7 @@ CCD_HD bool refine_vertex_edge(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, d
         refine_part(g, m[2], at, h, bit, r[2]);
     }
     const double w = fmax2(fmax2(m[0], m[1]), m[2]);
-    return (r[0].usable() | r[1].usable() | r[2].usable()) == REFINE_ALL && w < 1e150;
+    return (r[0].usable(all) | r[1].usable(all) | r[2].usable(all)) == all && w < 1e150;
 }
 // Whether vertex_vertex cannot hit, for vertices whose coordinates stay below w.
 CCD_HD bool refine_vertex_vertex(V3 q1s, V3 q2s, V3 q1e, V3 q2e, double eta, double w)
@@ -1821,13 +1823,14 @@ CCD_FHD void vertex_vertex_vertices(int j, int &a, int &b)
 // A screen's mask after the refinement of the face or edge-edge test, and of the others.  `at` gives a
 // vertex's window positions by its place in the stencil (0..3), which is a runtime index.
 template <bool VF>
-CCD_HD unsigned refine_primary(const V3 *s, const V3 *e, double eta, unsigned m)
+CCD_HD unsigned refine_primary(const V3 *s, const V3 *e, double eta, unsigned m, int leaves = REFINE_LEAVES)
 {
-    if ((m & SCREEN_PRIMARY) && (VF ? refine_vertex_face(s, e, eta) : refine_edge_edge(s, e, eta))) m &= ~SCREEN_PRIMARY;
+    if ((m & SCREEN_PRIMARY) && (VF ? refine_vertex_face(s, e, eta, leaves) : refine_edge_edge(s, e, eta, leaves)))
+        m &= ~SCREEN_PRIMARY;
     return m;
 }
 template <bool VF, class At>
-CCD_HD unsigned refine_others(const V3 *s, const V3 *e, double eta, unsigned m, At &&at)
+CCD_HD unsigned refine_others(const V3 *s, const V3 *e, double eta, unsigned m, At &&at, int leaves = REFINE_LEAVES)
 {
     for (unsigned open = m & (15u * SCREEN_VE); open; open &= open - 1) {
         const unsigned bit = open & (0u - open);
@@ -1837,7 +1840,7 @@ CCD_HD unsigned refine_others(const V3 *s, const V3 *e, double eta, unsigned m, 
         at(a, as, ae);
         at(b, bs, be);
         at(c, cs, ce);
-        if (refine_vertex_edge(as, bs, cs, ae, be, ce, eta)) m &= ~bit;
+        if (refine_vertex_edge(as, bs, cs, ae, be, ce, eta, leaves)) m &= ~bit;
     }
     if (m & SCREEN_VV) {
         const double w = max_coord(s, e);

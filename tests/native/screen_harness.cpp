@@ -45,3 +45,24 @@ extern "C" void screen_stencils(const double *qs, const double *qe, const int32_
     else
         run<true>(qs, qe, keys, n, eta, mask, refined, sub, t, sub_masked, t_masked, hits);
 }
+
+// The refined masks with another number of parts.
+extern "C" void refine_stencils(const double *qs, const double *qe, const int32_t *keys, int64_t n, int is_ee, double eta,
+                                int leaves, const uint32_t *mask, uint32_t *refined)
+{
+#pragma omp parallel for schedule(dynamic, 256)
+    for (int64_t i = 0; i < n; i++) {
+        V3 s[4], e[4];
+        for (int j = 0; j < 4; j++) {
+            const double *a = qs + 3 * (int64_t)keys[4 * i + j], *b = qe + 3 * (int64_t)keys[4 * i + j];
+            s[j] = ccd::mk(ccd::stitch0(a[0], b[0]), ccd::stitch0(a[1], b[1]), ccd::stitch0(a[2], b[2]));
+            e[j] = ccd::mk(b[0], b[1], b[2]);
+        }
+        auto at = [&](int j, V3 &x, V3 &y) {
+            x = s[j];
+            y = e[j];
+        };
+        refined[i] = is_ee ? ccd::refine_others<false>(s, e, eta, ccd::refine_primary<false>(s, e, eta, mask[i], leaves), at, leaves)
+                           : ccd::refine_others<true>(s, e, eta, ccd::refine_primary<true>(s, e, eta, mask[i], leaves), at, leaves);
+    }
+}

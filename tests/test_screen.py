@@ -82,3 +82,23 @@ def test_screen_awkward_stencils(harness, is_ee, kind):
         bad = rng.integers(0, q.size, size=n)
         q.reshape(-1)[bad] = rng.choice([np.nan, np.inf, -np.inf, 1e300, -1e300, 1e-310], size=n)
     _run(harness, q[0], q[1], np.arange(4 * n, dtype=np.int32).reshape(n, 4), is_ee, eta)
+
+
+@pytest.mark.parametrize("is_ee", [False, True])
+@pytest.mark.parametrize("leaves", [1, 4, 32])
+def test_refine_with_other_numbers_of_parts(harness, is_ee, leaves):
+    """No sub-test that hits is cleared, whatever the number of parts (4 is the first pass over long lists)."""
+    rng = np.random.default_rng(leaves)
+    n = 60000
+    q = np.concatenate([rng.integers(-1, 2, size=(2, 2 * n, 3)).astype(np.float64), rng.normal(size=(2, 2 * n, 3))], axis=1)
+    q = np.ascontiguousarray(q)
+    keys = np.arange(4 * n, dtype=np.int32).reshape(n, 4)
+    mask, refined, hits, parts = (np.zeros(n, np.uint32) for _ in range(4))
+    sub, subm, t, tm = np.zeros(n, np.int32), np.zeros(n, np.int32), np.zeros(n), np.zeros(n)
+    p = lambda a: a.ctypes.data_as(ctypes.c_void_p)   # noqa: E731
+    harness.screen_stencils(p(q[0]), p(q[1]), p(keys), ctypes.c_int64(n), int(is_ee), ctypes.c_double(0.3), p(mask), p(refined),
+                            p(sub), p(t), p(subm), p(tm), p(hits))
+    harness.refine_stencils(p(q[0]), p(q[1]), p(keys), ctypes.c_int64(n), int(is_ee), ctypes.c_double(0.3), leaves, p(mask),
+                            p(parts))
+    assert not (parts & ~mask).any() and not (hits & ~parts).any() and hits.any()
+    assert (parts == 0).sum() > (mask == 0).sum() or leaves == 1
