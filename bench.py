@@ -508,7 +508,7 @@ def main():
     workload = (f"batched: {b.ninst} two-mesh instances (icospheres / noisy grids, log-uniform 80-20,480 tris per "
                 f"mesh), {F} tris, rigid motion + N(0, 0.005^2), seed 2, eta 1e-6")
     log(f"workload: {workload}")
-    # Queue shape and stencil grouping per kind from the committed tuning cache for this workload shape
+    # Narrowphase shape per kind from the committed tuning cache for this workload shape
     # (tuned now, and stored, when the cache has no entry for this GPU and workload).
     shape, how = b.tune(ETA_BATCH, ETA_BATCH, cache=args.tune_cache)
     log(f"narrowphase shape ({how}): {shape}")
@@ -534,8 +534,8 @@ def main():
         json.dumps({k: round(v, 3) for k, v in stage_ms.items()}))
     prof = load_profile("batched512_counters.json", workload)
     dom = max(("narrow_vf", "narrow_ee"), key=stage_ms.get)
-    # The edge-edge stage is two kernels (first pass, then the deferred stencils): counted together.
-    kern = "k_narrow2_queue<VF>" if dom == "narrow_vf" else "k_narrow2_queue_ee_shared+k_ee_deferred"
+    # A stage is three kernels (screen, refine, solve): counted together.
+    kern = "k_screen+k_refine+k_solve " + ("vertex-face" if dom == "narrow_vf" else "edge-edge")
     roof = roofline(kern, stage_ms[dom], fv if dom == "narrow_vf" else fe, prof)
     roof["stage_ms"] = {k: round(v, 5) for k, v in stage_ms.items()}
     roof["narrowphase_tflops"] = {"vf": fv / max(stage_ms["narrow_vf"], 1e-9) / 1e9,

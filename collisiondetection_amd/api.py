@@ -621,7 +621,7 @@ class Batch:
         return np.searchsorted(self.vert_off, v, side="right") - 1
 
     def tune(self, outer_eta, eta, cache=None):
-        """Tune the persistent narrowphase (queue shape and stencil grouping per kind) on this batch's
+        """Tune the narrowphase (its shape per kind) on this batch's
         candidates and install the result on the batch's context.  With `cache` (a JSON file path) the
         shape stored there for this workload shape (GPU architecture and compute units, faces, vertices,
         instances) is installed
@@ -678,8 +678,8 @@ class Batch:
 
 
 def autotune(qstart, qend, eta, ctx: Context | None = None):
-    """Tune the persistent narrowphase on the last detection's candidates; returns the 8-int shape
-    (block, tile, waves/CU per kind, then the grouping flag per kind)."""
+    """Tune the narrowphase on the last detection's candidates; returns the 8-int shape
+    (block, tile, waves/CU per kind, then a grouping flag per kind, which has no effect)."""
     torch = _torch()
     ctx = ctx or default_context()
     ctx.bind_stream()

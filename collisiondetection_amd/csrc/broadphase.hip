@@ -7,19 +7,18 @@
 // file sorts the leaves along a Morton curve and searches 64-wide levels of boxes over that order:
 //   1. leaf bounds: per face, 13 axes x (3 vertices x history entries), min/max of pos.axis -/+ eta in
 //      FP64 exactly as KDOPBroadPhase.cpp:60-70 (bit-identical);
-//   2. 63-bit Morton codes of the leaf centres, radix-sorted (devprims.hip);
+//   2. Morton codes of the leaf centres, radix-sorted (devprims.hip);
 //   3. box records quantised to 16 bits per bound: one per leaf, one per 64 leaves (a cluster), one per
 //      64 clusters, and so on: the width of a wavefront;
 //   4. the pair search: one wavefront per cluster finds the clusters its box meets, 64 box tests at a
 //      time, and tests each as a 64 x 64 tile of leaves.  The quantised test culls; the leaf-leaf
 //      decision is the reference's FP64 13-axis test (touching overlaps) and the shared-vertex test
 //      (Mesh.cpp:13-20), run on full wavefronts from a queue in LDS;
-//   5. expansion of each face pair into its 6 vertex-face and 9 edge-edge stencils
-//      (KDOPBroadPhase.cpp:150-184) with owner-computes deduplication: a stencil is written only by
-//      the smallest face pair that generates it, which is decided from the face -> related faces table
-//      built from the search's pairs (rows sorted; one wavefront per face) and the vertex->face
-//      table, so the unique set comes out with no global sort.
-// Meshes with degenerate faces (a repeated vertex) or duplicate faces break the owner rule's
+//      Its finds become one row per face, of clusters with a mask of the related faces in each;
+//   5. the 6 vertex-face and 9 edge-edge stencils of each face pair (KDOPBroadPhase.cpp:150-184), each
+//      once: a vertex's or an edge's stencils are the union of the rows of the faces around it, an OR of
+//      masks, so the unique set comes out with no global sort.
+// Meshes with degenerate faces (a repeated vertex) or duplicate faces break the rule's
 // assumptions; for them the raw stencils are emitted and deduplicated by sorting.
 #include <cstring>
 #include <rocprim/device/device_merge_sort.hpp>
@@ -221,8 +220,8 @@ __device__ __forceinline__ uint64_t spread21(uint64_t x)
     return x;
 }
 
-// Keys are (instance id << (63 - inst_bits)) | Morton code with (63 - inst_bits) / 3 bits per axis:
-// sorting groups each instance's faces, so every instance owns one subtree of the radix tree.
+// Keys are (instance id << 3 * axis_bits) | Morton code with axis_bits bits per axis: sorting groups each
+// instance's faces, so every instance owns a contiguous range of the leaves.
 __global__ __launch_bounds__(256) void k_morton(const double *__restrict__ centre, int64_t F,
                                                 const double *__restrict__ box, const int32_t *__restrict__ face_inst,
                                                 int axis_bits, uint64_t *__restrict__ keys, int32_t *__restrict__ vals)

@@ -139,16 +139,13 @@ struct NoCount {
 struct FullCascade {
     CCD_FHD void operator()(int) const {}
 };
-// The product's counter type for the first pass of the two-pass edge-edge narrowphase: it screens the
-// coplanar-distance sextic and solves nothing.  find_intervals on the sextic decides only the case
+// A counter type for a screening run of the edge-edge test: it screens the coplanar-distance sextic and
+// solves nothing (the host's model of a two-pass schedule; the device screens with screen_ee_window).  find_intervals on the sextic decides only the case
 // "full degree, and no root in [0, 1] by the Bernstein test" (couldHaveRoots false, or no sign change
 // of the Bernstein coefficients with every one clear of zero), where the list is the one piece [0, 1]
 // or nothing, as the isolator gives it; any other sextic sets `deferred`.  edge_edge then returns
 // false at once, and also sets `deferred` when the sextic leaves a coplanar interval.  So a stencil
-// the screen does not defer has no edge-edge collision, exactly as the full test finds; the deferred
-// ones get the full test later, on a list that holds only them.  The first pass then carries no root
-// solver, no parallel check and no barycentric quartics for the edge-edge test (fewer registers: more
-// wavefronts per SIMD), and the stencils whose sextics need the solver run together.
+// the screen does not defer has no edge-edge collision, exactly as the full test finds.
 struct ScreenSextic {
     bool deferred = false;
     CCD_FHD void operator()(int) const {}
@@ -1143,8 +1140,7 @@ CCD_HD bool ve_sides(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, Ivls<3> &e1
 
 // Which vertex-edge sub-tests of a stencil's window would reach their quartic (both side quadratics
 // non-empty and overlapping): bit j for the j-th vertex-edge test in the reference's order.  Cheap
-// (closed-form quadratics only); the narrowphase groups stencils by it so that a wavefront's lanes
-// take the same quartic solves.
+// (closed-form quadratics only).
 struct SolverProbe {
     static constexpr bool stops_at_solver = true;
     bool called = false;

@@ -1,9 +1,9 @@
 // Serving runtime: device-resident CCD sessions driven by a continuous-batching request loop.
 //
 // A session owns one mesh (or a set of meshes packed as one, e.g. a mesh pair) on the device: faces,
-// two position buffers (the current end and the next end), its radix tree from a first full build, and
+// two position buffers (the current end and the next end), its Morton order from a first full build, and
 // a ccd_ctx with its own HIP stream.  A request supplies new end positions; the session's previous end
-// becomes the start, the tree is refit (not rebuilt), and the narrowphase runs on the candidates.
+// becomes the start, the order is kept (a refit), and the narrowphase runs on the candidates.
 //
 // The worker thread admits requests in arrival order as soon as (a) their session is idle -- requests
 // of one session are sequential because each starts where the last ended -- (b) an in-flight slot is

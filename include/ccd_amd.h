@@ -50,9 +50,9 @@ extern "C" {
 /* Stage timers (ccd_stage_times), in pipeline order. */
 #define CCD_T_BOUNDS 0    /* leaf k-DOPs, scene box, Morton codes */
 #define CCD_T_SORT 1      /* Morton radix sort */
-#define CCD_T_BUILD 2     /* radix tree, escape links, leaf records, bottom-up refit */
-#define CCD_T_TABLES 3    /* vertex -> face table and mesh checks */
-#define CCD_T_TRAVERSE 4  /* face-pair traversal */
+#define CCD_T_BUILD 2     /* box records of every level */
+#define CCD_T_TABLES 3    /* vertex -> face and edge tables, mesh checks */
+#define CCD_T_TRAVERSE 4  /* face-pair search: rows of related faces */
 #define CCD_T_EXPAND 5    /* stencil expansion with deduplication */
 #define CCD_T_NARROW_VF 6 /* vertex-face narrowphase */
 #define CCD_T_NARROW_EE 7 /* edge-edge narrowphase */
@@ -106,7 +106,7 @@ int ccd_ctcd_narrowphase(ccd_ctx *ctx, const double *qstart, const double *qend,
  * ccd_ctcd_narrowphase_noalloc: ccd_ctcd_narrowphase (same arguments, results and errors) without any
  * device allocation.  No counterpart in the reference: it is for callers that cannot allocate (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  Its working memory
- * (stencil ordering buffers, a validation counter) is one file-scope device array of 26 MiB per GPU,
+ * (lists of the narrowphase's passes, a validation counter) is one file-scope device array of 26 MiB per GPU,
  * held until the process ends, whose address ccd_create looks up once per device.  At most
  * CCD_NOALLOC_MAX_STENCILS stencils per kind and call: larger calls return CCD_E_CAPACITY.  Every call
  * on one GPU shares that GPU's array, so calls that overlap on one GPU (other threads, other streams)
@@ -279,8 +279,8 @@ int ccd_last_candidates(ccd_ctx *ctx, const int32_t **vf_keys, int64_t *nvf, con
  * inst_face_off[k] .. inst_face_off[k+1]-1 (inst_face_off: device, ninst+1 int64, starting at 0 and
  * ending at nfaces); faces hold global vertex indices and no vertex is shared between instances.  The
  * result is the union of ccd_detect over the instances -- no stencil pairs primitives of two
- * instances -- computed by one pipeline: one forest of radix trees (instance id in the high bits of
- * the sort keys), one traversal, one persistent work-queue narrowphase.  flags: CCD_GRAPH replays a
+ * instances -- computed by one pipeline: one order of the leaves (instance id in the high bits of the
+ * sort keys), one pair search, one narrowphase.  flags: CCD_GRAPH replays a
  * captured HIP graph of the whole pipeline on calls with the same arguments (after the first call has
  * sized every buffer); a capacity overflow found after a replay falls back to a fresh synchronous run.
  * Output and counts as ccd_detect.  Synchronous.  No counterpart in the reference (one mesh per call).
@@ -292,12 +292,12 @@ int ccd_batch_detect(ccd_ctx *ctx, int64_t ninst, const int64_t *inst_face_off, 
                      int64_t *ee_candidates, int flags);
 
 /*
- * Tuning of the persistent narrowphase: times the work-queue kernel on the candidates of the last
- * detection on this context over block sizes {64, 128, 256}, tiles {64, 128, ..., 4096} and
- * {4, 8, 12, 16} resident wavefronts per CU, on the stencils grouped by sub-test signature, and then
- * whether that grouping (its own passes included) beats the stored order; keeps the fastest per stencil kind
- * and returns it in shape[0..7] = {vf block, vf tile, vf waves/CU, ee block, ee tile, ee waves/CU,
- * vf grouping, ee grouping} (host, may be NULL; grouping 1 or 0).  ccd_set_queue_shape installs such
+ * Tuning of the narrowphase: times it on the candidates of the last detection on this context over
+ * block sizes {64, 128, 256}, tiles {64, 128, ..., 4096} and {4, 8, 12, 16} resident wavefronts per CU;
+ * keeps the fastest per stencil kind and returns it in shape[0..7] = {vf block, vf tile, vf waves/CU,
+ * ee block, ee tile, ee waves/CU, vf grouping, ee grouping} (host, may be NULL).  The tile bounds the
+ * stencils that a wavefront of the screening passes takes; block and waves/CU matter to the one-pass form
+ * only; grouping (1 or 0) is accepted and has no effect.  ccd_set_queue_shape installs such
  * a shape (e.g. one cached from an earlier tuning run).
  */
 int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double eta, int *shape);
@@ -305,11 +305,9 @@ int ccd_set_queue_shape(ccd_ctx *ctx, const int *shape);
 
 /*
  * ccd_set_edge_edge_split (no counterpart in the reference; a scheduling choice, same results): on (the
- * default), the persistent edge-edge narrowphase of ccd_detect / ccd_batch_detect / the server runs in
- * two passes: the first screens each stencil's coplanar-distance sextic and sets aside the stencils
- * whose sextic needs the root solver, the second finishes them.  The list of set-aside stencils takes
- * 4 + 1 bytes per slot, about 1.25 slots per stored edge-edge stencil plus 512 per resident wavefront.
- * Off, one pass.
+ * default), the edge-edge narrowphase of ccd_detect / ccd_batch_detect / the server runs in passes: a
+ * screen of every stencil without a root solver, a refinement of what it leaves open, and the solver on
+ * the rest.  The passes' lists take 5 bytes per stored stencil.  Off, one pass with the solver.
  */
 int ccd_set_edge_edge_split(ccd_ctx *ctx, int on);
 
@@ -317,14 +315,14 @@ int ccd_set_edge_edge_split(ccd_ctx *ctx, int on);
  * Serving (no counterpart in the reference): device-resident sessions and a continuous-batching loop.
  *
  * ccd_server_create: a server on `device` with an HBM pool of hbm_budget_bytes for the transient
- *   workspace of in-flight requests (face pairs, stencils, collisions) and at most max_inflight
+ *   workspace of in-flight requests (related-face rows, stencils, collisions) and at most max_inflight
  *   requests on the device at once.  A worker thread admits requests in arrival order when their
  *   session is idle, a slot is free and their workspace fits in the pool.
- * ccd_server_open_session: uploads a mesh (host arrays: faces 3F, qstart/qend 3V) and builds its tree
+ * ccd_server_open_session: uploads a mesh (host arrays: faces 3F, qstart/qend 3V) and builds its order
  *   (one full detection qstart -> qend).  Fails with CCD_E_BUDGET if less than 2 GiB of device
  *   memory would remain.  Synchronous; returns the session id.
  * ccd_server_submit: a request with new end positions (host, 3V, copied): the session's previous end
- *   becomes the start and its tree is refit, not rebuilt.  Asynchronous.
+ *   becomes the start and its order is kept, not rebuilt.  Asynchronous.
  * ccd_server_poll: completed requests (counts, checksums of the colliding stencils, timestamps).
  * ccd_server_drain: waits until every submitted request has completed.
  * ccd_server_stats: 10 int64 = {submitted, completed, pending, in flight, pool bytes in use, resident
