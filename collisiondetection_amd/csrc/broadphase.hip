@@ -26,6 +26,7 @@
 
 #include "ccd_core.h"
 #include "ccd_internal.h"
+#include "grids.h"
 
 namespace {
 
@@ -272,12 +273,7 @@ __global__ __launch_bounds__(256) void k_face_instance(const int64_t *__restrict
 // subtractions.  64 consecutive sorted leaves form a cluster (level 1), 64 clusters a group (level 2),
 // 64 groups a level-3 record; each record is the union of its children.
 //
-// Quantisation.  Per axis, a bound v maps to x = (v - origin) * inv, with origin the smallest finite
-// lower bound of all leaves and inv = 65535 / (largest finite upper bound - origin); lower bounds take
-// floor(x), upper bounds ceil(x), both clamped to [0, 65535], NaN to the full range.  Correctly rounded
-// subtraction and multiplication are monotone, and so are floor, ceil and the clamps, so overlapping
-// boxes keep overlapping (a.hi >= b.lo gives q(a.hi) >= q(b.lo)): the quantised test only ever keeps
-// more, and the FP64 leaf test decides.  Values outside the range clamp, which stays conservative.
+// The quantisation (ccd::quant_lo, ccd::quant_hi) only ever keeps more pairs; the FP64 leaf test decides.
 constexpr int NWORD = 7;   // 32-bit words per side of a box
 struct __align__(16) BoxRec {
     uint32_t lo[NWORD];
@@ -339,23 +335,6 @@ __device__ __forceinline__ void store_box(BoxRec *__restrict__ recs, int64_t n, 
     p[2] = make_uint4(b.hi[1], b.hi[2], b.hi[3], b.hi[4]);
     p[3] = make_uint4(b.hi[5], b.hi[6], face, 0u);
 }
-constexpr double QMAX = 65535.0;
-__device__ __forceinline__ uint16_t quant_lo(double v, double o, double inv)
-{
-    const double x = (v - o) * inv;
-    if (!(x >= 0.0)) return 0;   // below the range, -inf, NaN: the smallest
-    if (x >= QMAX) return (uint16_t)QMAX;
-    return (uint16_t)floor(x);
-}
-__device__ __forceinline__ uint16_t quant_hi(double v, double o, double inv)
-{
-    const double x = (v - o) * inv;
-    if (x != x) return (uint16_t)QMAX;   // NaN: the largest
-    if (x <= 0.0) return 0;
-    if (x >= QMAX) return (uint16_t)QMAX;
-    return (uint16_t)ceil(x);
-}
-
 // Quantisation parameters: per-block partial min of the finite lower and max of the finite upper
 // bounds per axis (wavefront shuffles, then LDS), then one block folds the partials into origin[13]
 // and inv[13] (qparam[0..12], qparam[13..25]).
@@ -422,10 +401,8 @@ __global__ __launch_bounds__(64) void k_qrange_final(const double *__restrict__ 
         hi = b > hi ? b : hi;
     }
     if (threadIdx.x != 0) return;
-    const double ext = hi - lo;
-    const bool ok = __builtin_isfinite(lo) && __builtin_isfinite(hi) && ext > 0.0 && __builtin_isfinite(QMAX / ext);
     qparam[k] = __builtin_isfinite(lo) ? lo : 0.0;
-    qparam[KAX + k] = ok ? QMAX / ext : 0.0;
+    qparam[KAX + k] = ccd::quant_scale(lo, hi);
 }
 
 // Leaf records in sorted order with the record of each wavefront's cluster, and the FP64 bounds and
@@ -462,11 +439,11 @@ __global__ __launch_bounds__(256) void k_leaf_records(const int32_t *__restrict_
 #pragma unroll
         for (int w = 0; w < NWORD; w++) {
             const int k = 2 * w;
-            uint32_t lo = quant_lo(src[k], qparam[k], qparam[KAX + k]);
-            uint32_t hi = quant_hi(src[KAX + k], qparam[k], qparam[KAX + k]);
+            uint32_t lo = ccd::quant_lo(src[k], qparam[k], qparam[KAX + k]);
+            uint32_t hi = ccd::quant_hi(src[KAX + k], qparam[k], qparam[KAX + k]);
             if (k + 1 < KAX) {
-                lo |= (uint32_t)quant_lo(src[k + 1], qparam[k + 1], qparam[KAX + k + 1]) << 16;
-                hi |= (uint32_t)quant_hi(src[KAX + k + 1], qparam[k + 1], qparam[KAX + k + 1]) << 16;
+                lo |= (uint32_t)ccd::quant_lo(src[k + 1], qparam[k + 1], qparam[KAX + k + 1]) << 16;
+                hi |= (uint32_t)ccd::quant_hi(src[KAX + k + 1], qparam[k + 1], qparam[KAX + k + 1]) << 16;
             } else {
                 hi |= 0xffff0000u;   // the padding axis
             }
@@ -517,11 +494,8 @@ __device__ __forceinline__ bool neighbours(int4 a, int4 b)   // Mesh.cpp:13-20
 //
 // The pairs that pass are queued in LDS and finished 64 at a time, so that the FP64 test runs with full
 // wavefronts: the shared-vertex test (Mesh.cpp:13-20), then the reference's 13-axis test (touching
-// counts).  Where every axis overlaps by two quanta or more the FP64 bounds are not read: with
-// qhi = ceil(x) > x - and so x > qhi - 1 -, qlo = floor(y) and so y < qlo + 1, qhi - 1 >= qlo + 1 gives
-// x > y, and the map to x is monotone, so the FP64 bounds overlap as well (the clamps keep this: a
-// clamped qhi = 65535 has x >= 65535, a clamped qlo = 0 has y < 1, a NaN bound never separates, and
-// the other clamps fail the test).
+// counts).  Where every axis overlaps by two quanta or more the FP64 bounds are not read, since they then
+// overlap as well (ccd::surely_reaches).
 //
 // The search keeps the tiles it finds in the order it finds them, and counts them by row; after a scan of
 // the counts a second run puts them into their rows.  A row belongs to one wavefront, or to the `slices`
@@ -573,7 +547,7 @@ __device__ __forceinline__ bool boxes_meet_surely(const Box16 &a, const Box16 &b
         const int sh = (k & 1) * 16, w = k >> 1;
         const int al = (a.lo[w] >> sh) & 0xffff, ah = (a.hi[w] >> sh) & 0xffff;
         const int bl = (b.lo[w] >> sh) & 0xffff, bh = (b.hi[w] >> sh) & 0xffff;
-        ok = ok & (ah - bl >= 2) & (bh - al >= 2);
+        ok = ok & ccd::surely_reaches(ah, bl) & ccd::surely_reaches(bh, al);
     }
     return ok;
 }

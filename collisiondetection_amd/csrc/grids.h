@@ -1,0 +1,49 @@
+// Integer grids that the broadphase puts boxes on: the rounding rules, for the device and for tests on the host.
+#pragma once
+
+#include "ccd_core.h"
+
+namespace ccd {
+
+// ------------------------------------------------------------------------------------------------
+// Bounds quantised to 16 bits
+// ------------------------------------------------------------------------------------------------
+// Per axis, a bound v maps to x = (v - origin) * inv, with origin the smallest finite lower bound of all leaves
+// and inv = 65535 / (largest finite upper bound - origin), or 0 where that is no finite positive number; lower
+// bounds take floor(x), upper bounds ceil(x), both clamped to [0, 65535].  Correctly rounded subtraction and
+// multiplication are monotone, and so are floor, ceil and the clamps, so overlapping boxes keep overlapping
+// (a.hi >= b.lo gives q(a.hi) >= q(b.lo)): the quantised test only ever keeps more.
+constexpr double QUANT_MAX = 65535.0;
+CCD_FHD double quant_scale(double lo, double hi)
+{
+    const double ext = hi - lo;
+    const bool ok = __builtin_isfinite(lo) && __builtin_isfinite(hi) && ext > 0.0 && __builtin_isfinite(QUANT_MAX / ext);
+    return ok ? QUANT_MAX / ext : 0.0;
+}
+CCD_FHD uint16_t quant_lo(double v, double o, double inv)
+{
+    const double x = (v - o) * inv;
+    if (!(x >= 0.0)) return 0;   // below the range, -inf, NaN: the smallest
+    if (x >= QUANT_MAX) return (uint16_t)QUANT_MAX;
+    return (uint16_t)__builtin_floor(x);
+}
+CCD_FHD uint16_t quant_hi(double v, double o, double inv)
+{
+    const double x = (v - o) * inv;
+    // No number: a bound that separates nothing (NaN, +inf) is the largest.  Any other comes from an axis without
+    // a scale (0 times a difference that overflows, or -inf): the smallest, where every lower bound is too, so
+    // that the quantised values decide nothing.
+    if (x != x) return v != v || v == __builtin_inf() ? (uint16_t)QUANT_MAX : 0;
+    if (x <= 0.0) return 0;
+    if (x >= QUANT_MAX) return (uint16_t)QUANT_MAX;
+    return (uint16_t)__builtin_ceil(x);
+}
+
+// The bounds a.hi >= b.lo hold for certain if their quantised values differ by two quanta or more: with
+// qhi = ceil(x) and so x > qhi - 1, qlo = floor(y) and so y < qlo + 1, qhi - 1 >= qlo + 1 gives x > y, and the
+// map to x is monotone.  (The clamps keep this: a clamped qhi = 65535 has x >= 65535 or is a bound that
+// separates nothing, a clamped qlo = 0 has y < 1 or is NaN, and the other clamps fail the test.  On an axis
+// without a scale only bounds that separate nothing differ from 0.)
+CCD_FHD bool surely_reaches(int qhi, int qlo) { return qhi - qlo >= 2; }
+
+}   // namespace ccd
