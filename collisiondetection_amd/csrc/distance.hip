@@ -21,6 +21,7 @@
 
 #include "ccd_core.h"
 #include "ccd_internal.h"
+#include "grids.h"
 
 namespace {
 
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(256) void k_face_pair_bound(const double *__restric
 }
 
 // The vertices' bounding box, one partial box per block (lo, hi): NaN coordinates count only in vertex 0, where
-// they make the box NaN and the caller does without a grid.  Read back instead of the vertices: 24 bytes
+// they make the box NaN on their axis: without a grid then for x, one layer of cells for y or z.  Read back instead of the vertices: 24 bytes
 // each, copied and compared by the host, took 150 us of a call on 40,401 vertices.
 constexpr int BOX_BLOCKS = 64;
 __global__ __launch_bounds__(256) void k_box(const double *__restrict__ v, int64_t V, double *__restrict__ partial)
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(256) void k_box(const double *__restrict__ v, int64
 // Step 1b: cell keys.  Cell coordinates (clamped) of (x - lo) * inv, packed z, y, x so that the three cells
 // x-1, x, x+1 of one (y, z) row are consecutive keys.  x takes sx bits and y the next sy - sx: enough for
 // every coordinate and its neighbour, and few, since each 8 bits are a pass of the sort.
-constexpr uint64_t CELL_MAX = (1ull << 21) - 1;
+constexpr uint64_t CELL_MAX = (1ull << ccd::CELL_BITS) - 1;
 __device__ __forceinline__ uint64_t cell_coord(double x, double lo, double inv)
 {
     double s = (x - lo) * inv;
@@ -357,12 +358,8 @@ int mesh_self_distance(ccd_ctx *ctx, const double *verts, int64_t V, const int32
     if (grid) {
         // Step 1b/1c: vertices sorted by cell, each against its 27 surrounding cells.
         const double inv = 1.0 / cell;
-        int bits[3];
-        for (int k = 0; k < 3; k++) {   // (a coordinate is at most 2^20 + 1 here)
-            const uint64_t most = (uint64_t)((hi[k] - lo[k]) * inv) + 1;
-            for (bits[k] = 1; most >> bits[k];) bits[k]++;
-        }
-        const int sx = bits[0], sy = bits[0] + bits[1];
+        const int sx = ccd::cell_bits(hi[0] - lo[0], inv), sy = sx + ccd::cell_bits(hi[1] - lo[1], inv);
+        const int key_bits = sy + ccd::cell_bits(hi[2] - lo[2], inv);
         uint64_t *key = (uint64_t *)buffer(ctx, "grid_key", (size_t)V * 8);
         uint64_t *key2 = (uint64_t *)buffer(ctx, "grid_key2", (size_t)V * 8);
         int32_t *idx = (int32_t *)buffer(ctx, "grid_idx", (size_t)V * 4);
@@ -373,7 +370,7 @@ int mesh_self_distance(ccd_ctx *ctx, const double *verts, int64_t V, const int32
                            sx, sy, key, idx);
         CCD_LAUNCH_CHECK(ctx);
         bool in_alt = false;
-        rc = radix_sort_pairs(ctx, key, idx, key2, idx2, V, sy + bits[2], tmp, in_alt);
+        rc = radix_sort_pairs(ctx, key, idx, key2, idx2, V, key_bits, tmp, in_alt);
         if (rc) return rc;
         hipLaunchKernelGGL(k_grid_closest, dim3(blocks_for(V, 256)), dim3(256), 0, st, verts, V, lo[0], lo[1], lo[2],
                            inv, sx, sy, in_alt ? key2 : key, in_alt ? idx2 : idx, faces, voff, vlist, best);

@@ -46,4 +46,20 @@ CCD_FHD uint16_t quant_hi(double v, double o, double inv)
 // without a scale only bounds that separate nothing differ from 0.)
 CCD_FHD bool surely_reaches(int qhi, int qlo) { return qhi - qlo >= 2; }
 
+
+// ------------------------------------------------------------------------------------------------
+// Cells of the closest-vertex search
+// ------------------------------------------------------------------------------------------------
+// Bits for the cell coordinates 0 .. extent * inv of an axis and the neighbour after the last.  An extent that is
+// no number (a NaN coordinate in the box, or all of them the same infinity) puts every vertex into cell 0.
+constexpr int CELL_BITS = 21;   // at most: three axes to a 64-bit key
+CCD_FHD int cell_bits(double extent, double inv)
+{
+    const double last = extent * inv;
+    if (!(last >= 1.0)) return 1;
+    int bits = 2;
+    while (bits < CELL_BITS && last + 1.0 >= (double)(1ll << bits)) bits++;
+    return bits;
+}
+
 }   // namespace ccd

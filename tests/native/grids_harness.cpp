@@ -16,3 +16,4 @@ extern "C" void quantise_axis(const double *lo, const double *hi, int64_t n, uin
     }
 }
 extern "C" int surely_reaches(int qhi, int qlo) { return ccd::surely_reaches(qhi, qlo); }
+extern "C" int cell_bits(double extent, double inv) { return ccd::cell_bits(extent, inv); }

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 import oracle
-from collisiondetection_amd import api
+from collisiondetection_amd import api, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -19,3 +19,33 @@ def test_candidates_at_the_largest_coordinates(places):
     np.testing.assert_array_equal(vf, ovf)
     np.testing.assert_array_equal(ee, oee)
     assert len(vf) == (6 if places[1] == places[2] else 0)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("vertex", ["first", "last"])
+def test_self_distance_with_a_vertex_nowhere(axis, value, vertex):
+    """A vertex of no face with a coordinate that is no number changes nothing."""
+    s = scenes.cloth(40)
+    v, f = s["qstart"], s["faces"]
+    want = oracle.mesh_self_distance(v, f)
+    nowhere = np.array([[0.5, 0.5, 0.0]])
+    nowhere[0, axis] = value
+    print("case: self distance, axis", axis, value, vertex, flush=True)
+    if vertex == "first":
+        got = api.mesh_self_distance(np.concatenate([nowhere, v]), f + 1)
+    else:
+        got = api.mesh_self_distance(np.concatenate([v, nowhere]), f)
+    assert tuple(got) == tuple(want)
+
+
+def test_self_distance_with_a_face_nowhere():
+    """The first vertex, in faces, with a NaN: the same result whichever coordinate it is in."""
+    s = scenes.cloth(40)
+    got = []
+    for axis in range(3):
+        v = s["qstart"].copy()
+        v[0, axis] = np.nan
+        print("case: self distance, a face with a NaN, axis", axis, flush=True)
+        got.append(api.mesh_self_distance(v, s["faces"])[0])
+    assert got[0] == got[1] == got[2] and np.isfinite(got[0])

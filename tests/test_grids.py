@@ -46,3 +46,16 @@ def test_quantised_boxes(grids, name, order):
     sure = np.array([[grids.surely_reaches(int(h), int(l)) for l in np.unique(ql)] for h in np.unique(qh)], bool)
     sure = sure[np.searchsorted(np.unique(qh), qh)][:, np.searchsorted(np.unique(ql), ql)]
     assert reaches[sure].all()
+
+
+def test_cell_bits(grids):
+    """Enough for every cell coordinate and the one after it, and no more; an extent that is no number ends too."""
+    f = grids.cell_bits
+    f.argtypes = [ctypes.c_double, ctypes.c_double]
+    rng = np.random.default_rng(0)
+    for n in [1, 2, 3, 4, 7, 8, 9, 1023, 1024, 2**20 - 1, 2**20] + rng.integers(1, 2**20, size=50).tolist():
+        for extent, inv in ((float(n), 1.0), (float(n) * 0.37, 1.0 / 0.37), (n - 1e-9, 1.0)):
+            assert f(extent, inv) == (int(extent * inv) + 1).bit_length()
+    for extent in (0.0, float("nan"), -1.0, 5e-324):
+        assert f(extent, 10.0) == 1
+    assert f(float("inf"), 1.0) == f(1e300, 1e10) == 21
