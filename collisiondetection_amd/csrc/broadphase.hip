@@ -901,8 +901,11 @@ __global__ __launch_bounds__(256) void k_edges(const int4 *__restrict__ sfaces, 
 // 300 a feature.
 //
 // A feature whose rows name more clusters than the table takes goes through it several times, each time
-// with one class of the clusters, by the upper bits of a hash.  The edge rule asks for faces of other
-// classes, so such an edge looks them up in its rows instead of the table.
+// with one class of the clusters, by the upper bits of a hash.  The edge rule may ask for a face of another
+// class; whether that is related to the edge's faces is decided again from the bounds.  (Looking it up in
+// their rows, which are as long as what they hold, and starting with one class took 1009 ms for a detection of a
+// 256^2 cloth over a ground of two triangles, quadratic in the faces; here 23 ms, 16 of them the ground's features,
+// 0.8 us for 64 faces.)
 constexpr int UNION_BLOCK = 256;
 constexpr int TABLE_SLOTS = 512;
 struct UnionTable {
@@ -918,6 +921,7 @@ struct MeshView {
     const FaceEdges *edges;   // by row
     const int32_t *rank;      // [F] face -> its row
     const int4 *sfaces;       // vertices and face id by row
+    const double *sdop64;     // bounds by row
     const int64_t *off;       // [F * slices + 1] parts of the rows
     Rows rows;
     int slices;
@@ -993,24 +997,24 @@ __device__ __forceinline__ void row_range(const MeshView &m, int r, int64_t &sta
     z = z < m.rows.cap ? z : m.rows.cap;
     len = start < z ? (int)(z - start) : 0;
 }
-// j in the rows of the faces f0 and f1, or (f1 -2) of those around u0 that hold u1, by search (edges whose
-// clusters do not fit the table).
-__device__ bool rows_have(const MeshView &m, int f0, int f1, int u0, int u1, int j)
+// Whether the leaves r and j are related, as the search decides it.
+__device__ __forceinline__ bool related(const MeshView &m, int r, int j)
 {
-    const int star = m.vf_off[u0], n = f1 == -2 ? m.vf_off[u0 + 1] - star : (f1 == -1 ? 1 : 2);
-    for (int k = 0; k < n; k++) {
-        int r = k == 0 ? f0 : f1;
-        if (f1 == -2) {
-            const int f = m.vf_list[star + k];
-            const int32_t *v = m.faces + 3 * (int64_t)f;
-            if (v[0] != u1 && v[1] != u1 && v[2] != u1) continue;
-            r = m.rank[f];
-        }
-        int64_t start;
-        int len;
-        row_range(m, r, start, len);
-        for (int64_t e = start; e < start + len; e++)
-            if (m.rows.cluster[e] == j >> 6 && ((m.rows.mask[e] >> (j & 63)) & 1ull)) return true;
+    if (neighbours(m.sfaces[r], m.sfaces[j])) return false;
+    const double *a = m.sdop64 + NB * (int64_t)r, *b = m.sdop64 + NB * (int64_t)j;
+    bool apart = false;
+#pragma unroll 3
+    for (int k = 0; k < KAX; k++) apart = apart | (a[KAX + k] < b[k]) | (b[KAX + k] < a[k]);
+    return !apart;
+}
+// j related to the leaf f0 or f1, or (f1 -2) to one of the faces around u0 that hold u1.
+__device__ bool edge_related(const MeshView &m, int f0, int f1, int u0, int u1, int j)
+{
+    if (f1 != -2) return related(m, f0, j) || (f1 >= 0 && related(m, f1, j));
+    for (int k = m.vf_off[u0]; k < m.vf_off[u0 + 1]; k++) {
+        const int f = m.vf_list[k];
+        const int32_t *v = m.faces + 3 * (int64_t)f;
+        if ((v[0] == u1 || v[1] == u1 || v[2] == u1) && related(m, m.rank[f], j)) return true;
     }
     return false;
 }
@@ -1091,7 +1095,10 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
         room = room > 0 ? room : 0;
         int4 *const keys = (edge ? ee_out : vf_out) + first;
         int64_t found = 0;   // stencils so far
-        int bits = 0;        // classes of clusters: 2^bits, by the hash's upper bits
+        // Classes of clusters: 2^bits, by the hash's upper bits.  (A row names a cluster once, so an edge has at least
+        // so many.)
+        int bits = 0;
+        while ((l0 > l1 ? l0 : l1) >> bits > TABLE_SLOTS * 3 / 4) bits++;
         uint32_t slots = TABLE_SLOTS;
         for (uint32_t cls = 0; cls < (1u << bits); cls++) {
             bool over = false;
@@ -1112,10 +1119,13 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
             };
             if (fn == 0) {
                 clear(l0 + l1);
-                for (int e = lane; e < l0 + l1; e += 64) add(e < l0 ? s0 + e : s1 + (e - l0));
+                for (int e0 = 0; e0 < l0 + l1 && !__ballot(over); e0 += 64) {
+                    const int e = e0 + lane;
+                    if (e < l0 + l1) add(e < l0 ? s0 + e : s1 + (e - l0));
+                }
             } else {
                 if (fn > 64) clear(TABLE_SLOTS);
-                for (int k0 = 0; k0 < fn; k0 += 64) {
+                for (int k0 = 0; k0 < fn && !__ballot(over); k0 += 64) {
                     const int at0 = fstar + k0, k = fn - k0 < 64 ? fn - k0 : 64;
                     if (at0 < wbase || at0 + k > wbase + 64) {
                         wbase = at0;
@@ -1133,7 +1143,7 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
                     if (fn <= 64) clear(all);
                     int steps = 1;
                     while (steps < k) steps <<= 1;
-                    for (int e0 = 0; e0 < all; e0 += 64) {
+                    for (int e0 = 0; e0 < all && !__ballot(over); e0 += 64) {
                         const int e = e0 + lane;
                         int row = a;   // the row that holds entry e: the first whose inclusive sum exceeds it
                         for (int d = steps >> 1; d > 0; d >>= 1) {
@@ -1181,8 +1191,8 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
                         // The number comes from another face: it has the edge if it is in the union.
                         const int owner = (int)(E.edge[w] / 3u);
                         auto has = [&](int j) {
-                            return bits == 0 ? table_has(T, slots - 1, j)
-                                             : rows_have(m, (int)(h / 3u), m.edges[h / 3u].other[h % 3u], a0, a1, j);
+                            if (bits == 0 || hash32((uint32_t)j >> 6) >> (32 - bits) == cls) return table_has(T, slots - 1, j);
+                            return edge_related(m, (int)(h / 3u), m.edges[h / 3u].other[h % 3u], a0, a1, j);
                         };
                         bool in = has(owner);
                         if (!in && E.other[w] == -2) {
@@ -1550,7 +1560,7 @@ static int launch_expand(ccd_ctx *ctx, const BPBufs &b, const int32_t *faces, in
 {
     hipStream_t st = ctx->stream;
     unsigned long long *c = (unsigned long long *)ctx->d_counts;
-    const MeshView mv{faces, voff, vlist, fixed, b.edges, b.rank, b.sfaces, b.row_off, b.rows, row_slices(ctx, F)};
+    const MeshView mv{faces, voff, vlist, fixed, b.edges, b.rank, b.sfaces, b.sdop64, b.row_off, b.rows, row_slices(ctx, F)};
     const int64_t feats = V + 3 * F;
     // Fewer features to a wavefront where there are few: on 160 faces the two runs take 24 and 29 us with 16,
     // 8 and 7 with 1; on 18,432 faces 43 and 52 with 16, 37 and 44 with 4, 40 and 45 with 2.
