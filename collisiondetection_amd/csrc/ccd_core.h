@@ -2111,6 +2111,7 @@ CCD_HD double plane_trajectory_intersect(const HistCSR &h, int v, int start, boo
 // recursion is a pure function of the interval) or one more than SP_MAX_DEPTH levels down (each level
 // at most halves the interval; only an interval closing in on a history entry time gets that deep).
 constexpr int SP_MAX_DEPTH = 160;
+constexpr int SP_LOST = 3, SP_RUN_AGAIN = 4;   // statuses between two passes over the same stencils
 
 // One stencil's histories as the recursion reads them: positions at a time (with the entry before it), the step
 // from an entry to the next, and a node's eight trajectory scans (t_lo: the smallest backward result, t_hi: the
@@ -2141,8 +2142,7 @@ struct CsrHistory {
 };
 
 // The recursion.  window(s, e): a window within one history entry interval of every vertex; true if it
-// collides.  (A caller may test the windows later and let `window` return false: the result is then 1 if
-// one of them collides, whatever the recursion returned; it can only have gone on for nothing.)
+// collides.  (A caller may test the windows later, with DeferredWindows.)
 // max_nodes bounds the intervals examined: when more remain the result is 3 ("not decided yet"), which
 // a caller uses to sort stencils by how much work they need before running them in full.
 template <bool VF, class Histories, class Window>
@@ -2242,6 +2242,38 @@ CCD_HD int separating_plane_nodes(const Histories &hist, double eta, double eps,
         }
     }
 }
+
+// Windows that are tested later, in full wavefronts: store(s, e) keeps one that the screen leaves open, or says
+// that there is no room.  Testing a window at once would end the recursion at the first that collides; here it
+// ends where the closest distance at a window's start, middle or end is below the thickness, since that window
+// should collide.  (Going on after every window: sheets resting a little above the thickness after a touch at the
+// start, 200 entries per vertex, up to 69 nodes a stencil instead of 9, and 2.79 ms a call of 7,361 stencils
+// instead of 0.85.)
+template <bool VF, class Store>
+struct DeferredWindows {
+    double eta;
+    Store store;
+    bool lost = false, ended = false;
+    CCD_HD DeferredWindows(double eta_, Store store_) : eta(eta_), store(store_) {}
+    CCD_HD bool operator()(const V3 (&s)[4], const V3 (&e)[4])
+    {
+        if (!(VF ? screen_vf_window(s, e, eta) : screen_ee_window(s, e, eta))) return false;
+        lost = !store(s, e);
+        ended = lost;
+        for (int k = 0; k < 3 && !ended; k++) {
+            V3 q[4];
+            for (int j = 0; j < 4; j++) q[j] = k == 0 ? s[j] : (k == 1 ? e[j] : 0.5 * (s[j] + e[j]));
+            double b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+            const V3 d = VF ? vertex_face_distance(q[0], q[1], q[2], q[3], b0, b1, b2)
+                            : edge_edge_distance(q[0], q[1], q[2], q[3], b0, b1, b2, b3);
+            ended = dot(d, d) < eta * eta;
+        }
+        return ended;
+    }
+    // From the recursion's result: a status that a stored window which collides changes to 1, or, if none does,
+    // SP_RUN_AGAIN (the recursion ended for a window) or SP_LOST (there was no room).
+    CCD_HD int status(int r) const { return lost ? SP_LOST : (ended ? SP_RUN_AGAIN : r); }
+};
 
 template <bool VF, class C = NoCount>
 CCD_HD int separating_plane_check(const HistCSR &h, const int (&v)[4], double eta, double eps, C &&cnt = C())

@@ -275,7 +275,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
 // ------------------------------------------------------------------------------------------------
 // Separating planes
 // ------------------------------------------------------------------------------------------------
-// Status 1 (collision), 0 (none) or 2 (undecided: the reference's recursion would not end).
+// Status 1 (collision), 0 (none) or 2 (undecided: the reference's recursion would not end); SP_LOST and
+// SP_RUN_AGAIN between the passes.
 
 // W lanes that all run the same stencil.
 template <int W>
@@ -456,8 +457,8 @@ __global__ __launch_bounds__(256) void k_sp_order_key(const int64_t *__restrict_
     if (r != 3) status[i] = (uint8_t)r;
 }
 
-// The recursions, their windows left to the pool.  Status 3: the pool had no room.  W lanes to a stencil; with an
-// order, group j runs stencil order[j] if open[j] is not 0.
+// The recursions, their windows left to the pool, their statuses as DeferredWindows gives them.  W lanes to a
+// stencil; with an order, group j runs stencil order[j] if open[j] is not 0.
 template <bool VF, int W>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_sp_nodes(
     const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
@@ -474,16 +475,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     ccd::HistCSR h{off, ht, hp};
     const ccd::CsrHistory csr{h, v};
     const bool writes = (__lane_id() & (W - 1)) == 0;
-    bool full = false;
-    auto window = [&](const V3 (&s)[4], const V3 (&e)[4]) {
-        if ((VF ? ccd::screen_vf_window(s, e, et) : ccd::screen_ee_window(s, e, et)) && !full) {
-            int64_t at = claim(pool, (int)(blockIdx.x & (WindowPool::SHARDS - 1)), writes ? 1 : 0);
-            at = __shfl(at, __lane_id() & ~(W - 1));
-            if (at < 0) full = true;
-            else if (writes) store_window(pool, at, i, 0, et, s, e);
-        }
-        return false;
+    auto store = [&](const V3 (&s)[4], const V3 (&e)[4]) {
+        int64_t at = claim(pool, (int)(blockIdx.x & (WindowPool::SHARDS - 1)), writes ? 1 : 0);
+        at = __shfl(at, __lane_id() & ~(W - 1));
+        if (at >= 0 && writes) store_window(pool, at, i, 0, et, s, e);
+        return at >= 0;
     };
+    ccd::DeferredWindows<VF, decltype(store) &> window(et, store);
     int r;
     if constexpr (W == 1) {
         r = ccd::separating_plane_nodes<VF>(csr, et, eps, 0x7fffffff, window);
@@ -499,7 +497,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
             r = ccd::separating_plane_nodes<VF>(shared, et, eps, 0x7fffffff, window);
         }
     }
-    if (writes) status[i] = full && r != 1 ? 3 : (uint8_t)r;
+    if (writes) status[i] = (uint8_t)window.status(r);
 }
 // A window that collides decides its stencil.
 __global__ __launch_bounds__(64) void k_sp_hits(WindowPool pool, uint8_t *__restrict__ status)
@@ -517,7 +515,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     const int64_t i0 = blockIdx.x * (int64_t)64, i = i0 + lane;
     int r = i < n ? status[i] : 0;
     const double eps = ccd::bits_to_double((long long)*gap_bits) / 4.0;
-    for (uint64_t lost = __ballot(r == 3); lost; lost &= lost - 1) {   // by the whole wavefront
+    for (uint64_t lost = __ballot(r == ccd::SP_LOST || r == ccd::SP_RUN_AGAIN); lost; lost &= lost - 1) {   // by the whole wavefront
         const int l = __ffsll((unsigned long long)lost) - 1;
         const int4 k = keys[i0 + l];
         const int v[4] = {k.x, k.y, k.z, k.w};
