@@ -494,7 +494,7 @@ struct DetectArgs {
 // the lists of the screening passes, one after the other on the stream.
 static int narrow_launches(ccd_ctx *ctx, const DetectArgs &a, int64_t nvf_max, int64_t nee_max)
 {
-    unsigned long long *work = (unsigned long long *)buffer(ctx, "queue_work", 16);   // the one-pass form's queues
+    unsigned long long *work = queue_work(ctx);
     if (!work) return CCD_E_OOM;
     int rc = fill_u64(ctx, (uint64_t *)(ctx->d_counts + C_VF_HITS), 2, 0);
     if (!rc) rc = fill_u64(ctx, (uint64_t *)work, 2, 0);
@@ -583,7 +583,7 @@ static int detect_graph(ccd_ctx *ctx, const DetectArgs &a)
     memcpy(saved, ctx->h_counts, sizeof(saved));
     // Capture with the capacities the synchronous run settled on; buffers used inside the capture are
     // sized for them first (nothing can be allocated while capturing).
-    if (!buffer(ctx, "queue_work", 16)) return CCD_E_OOM;
+    if (!queue_work(ctx)) return CCD_E_OOM;
     if (std::max(ctx->cap_vf, ctx->cap_ee) > 0 &&
         !open_list(ctx, std::min<int64_t>(std::max(ctx->cap_vf, ctx->cap_ee), 0x7fffffffll)))
         return CCD_E_OOM;

@@ -100,6 +100,11 @@ void *buffer(ccd_ctx *ctx, const char *name, size_t bytes);
 // Narrowphase launchers (narrowphase.hip)
 // ----------------------------------------------------------------------------------------------
 namespace ccdi {
+// The context's counters that a narrowphase works with, one buffer size for every caller (a request to grow it
+// frees and allocates, and so stalls the device): [0..1] the one-pass form's queues, [2..3] a server's checksums
+// of the hits.  Null without memory.
+constexpr int QUEUE_WORK = 4;
+inline unsigned long long *queue_work(ccd_ctx *ctx) { return (unsigned long long *)buffer(ctx, "queue_work", QUEUE_WORK * 8); }
 int launch_primitives(ccd_ctx *ctx, int kind, const double *q, const double *eta, double eta_s, int64_t n,
                       uint8_t *hit, double *t);
 // Where a narrowphase's results go: appended to a hit list (PER_STENCIL false), or at each stencil's own

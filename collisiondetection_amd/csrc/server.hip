@@ -128,7 +128,6 @@ struct Session {
     int cur = 0;
     int64_t F = 0, V = 0;
     double outer_eta = 0, eta = 0;
-    int64_t resident = 0;
     bool busy = false;
     // workspace sizing from the last completed request
     int64_t last_rows = 0, last_vf = 0, last_ee = 0, last_hits = 0;
@@ -156,7 +155,7 @@ struct ccd_server {
     std::deque<ccd_request_result> done;
     std::map<int64_t, std::vector<int32_t>> kept;   // request id -> colliding stencils (when keeping)
     bool keep_hits = false;
-    int64_t resident_bytes = 0, budget = 0;
+    int64_t budget = 0;
     std::mutex mu;
     std::condition_variable cv;
     std::thread worker;
@@ -175,6 +174,9 @@ namespace {
 using namespace ccdi;
 
 int64_t align256(int64_t x) { return (x + 255) & ~255ll; }
+
+// What a session holds on the device between requests.
+int64_t resident_bytes(const Session &s) { return ccd_device_bytes(s.ctx) + s.F * 12 + 2 * s.V * 24; }
 
 // A request's transient device memory: the related-face rows' tiles, the stencil keys, the screening
 // passes' lists and the hit lists.
@@ -220,11 +222,10 @@ int launch_request(ccd_server *S, Session &s, InFlight &f)
     CCD_HIP_CHECK(ctx, hipMemcpyAsync(end, f.req.qend.data(), (size_t)s.V * 24, hipMemcpyHostToDevice, st));
     int rc = broadphase_refit_launch(ctx, s.faces, s.F, start, end, s.V, s.outer_eta, nullptr, nullptr, 1);
     if (rc) return rc;
-    // work[0..1]: the one-pass form's queues; [2..3]: the hit checksums.
-    unsigned long long *work = (unsigned long long *)buffer(ctx, "queue_work", 32);
+    unsigned long long *work = queue_work(ctx);
     if (!work) return CCD_E_OOM;
     rc = fill_u64(ctx, (uint64_t *)(ctx->d_counts + C_VF_HITS), 2, 0);
-    if (!rc) rc = fill_u64(ctx, (uint64_t *)work, 4, 0);
+    if (!rc) rc = fill_u64(ctx, (uint64_t *)work, QUEUE_WORK, 0);
     if (rc) return rc;
     void *list = open_list(ctx, std::min<int64_t>(std::max(f.cap_vf, f.cap_ee), 0x7fffffffll));
     rc = launch_narrow2_queue(ctx, true, start, end, (const int32_t *)ctx->bufs["vf_keys"].ptr, ctx->d_counts + C_VF,
@@ -514,12 +515,10 @@ int ccd_server_open_session(ccd_server *S, const int32_t *faces, int64_t nfaces,
         b.ptr = nullptr;
         b.bytes = 0;
     }
-    s.resident = ccd_device_bytes(ctx) + (int64_t)nfaces * 12 + 2 * (int64_t)nverts * 24;
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < ((size_t)2 << 30))
         return fail(CCD_E_BUDGET);   // admission by HBM footprint: keep 2 GiB of headroom
     std::lock_guard<std::mutex> lk(S->mu);
-    S->resident_bytes += s.resident;
     S->sessions.push_back(s);
     *session = (int)S->sessions.size() - 1;
     return CCD_OK;
@@ -575,7 +574,8 @@ int ccd_server_stats(ccd_server *S, int64_t *stats)
     stats[2] = (int64_t)S->pending.size();
     stats[3] = (int64_t)S->inflight.size();
     stats[4] = S->pool.used;
-    stats[5] = S->resident_bytes;
+    stats[5] = 0;
+    for (const Session &s : S->sessions) stats[5] += resident_bytes(s);
     stats[6] = S->retries;
     stats[7] = (int64_t)S->sessions.size();
     stats[8] = S->mem_waits;
