@@ -1637,13 +1637,7 @@ int broadphase_launch(ccd_ctx *ctx, const int32_t *faces, int64_t F, const doubl
                            b.face_inst);
         CCD_LAUNCH_CHECK(ctx);
     }
-    // Cells per axis: 2^5 times what a surface of F faces takes (one outlying face 32 times as far away as the
-    // mesh is large leaves each face a cell of its own), in whole digits of the sort.  The order is only for
-    // tight boxes, and a digit is a pass of the sort: five on 18,432 faces, against eight with 63 bits.
-    int axis_bits = 5;
-    while ((1ll << 2 * (axis_bits - 5)) < F) axis_bits++;
-    const int sort_bits = std::min((inst_bits + 3 * axis_bits + 7) / 8 * 8, 63);
-    axis_bits = (sort_bits - inst_bits) / 3;
+    const int axis_bits = ccd::morton_axis_bits(inst_bits), sort_bits = inst_bits + 3 * axis_bits;
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(F, 256)), dim3(256), 0, st, b.centre, F, box,
                        batched ? b.face_inst : (const int32_t *)nullptr, axis_bits, b.keys, b.vals);
     CCD_LAUNCH_CHECK(ctx);

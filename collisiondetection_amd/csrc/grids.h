@@ -48,6 +48,16 @@ CCD_FHD bool surely_reaches(int qhi, int qlo) { return qhi - qlo >= 2; }
 
 
 // ------------------------------------------------------------------------------------------------
+// Cells of the Morton order
+// ------------------------------------------------------------------------------------------------
+// Bits per axis of a Morton code below inst_bits bits of an instance's number: all that a 63-bit key holds,
+// since a body far away makes the rest of the scene small.  (Only as many as 32 times what a surface of the mesh's
+// faces takes saved three of eight passes of the sort on 18,432 faces, 55 us of a 1.24 ms call; but with a
+// triangle 10^5 mesh sizes away the order of a shuffled sheet of 522,242 faces was its input order: a detection
+// took 673 ms, against 62 with all bits and 24 without the triangle.)
+CCD_FHD int morton_axis_bits(int inst_bits) { return (63 - inst_bits) / 3; }
+
+// ------------------------------------------------------------------------------------------------
 // Cells of the closest-vertex search
 // ------------------------------------------------------------------------------------------------
 // Bits for the cell coordinates 0 .. extent * inv of an axis and the neighbour after the last.  An extent that is

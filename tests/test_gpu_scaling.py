@@ -40,3 +40,21 @@ def test_expansion_over_a_ground_of_two_triangles():
         times.append(_stage_ms(ctx, N.TIMER_NAMES.index("expand"), lambda: api.kdop_candidates(faces, qs, qe, 1e-6, sort=False, ctx=ctx)))
         print("case: ground under a cloth", n, "expansion ms", times[-1], flush=True)
     assert times[1] < 12.0 * times[0]
+
+
+def test_search_with_a_body_far_away():
+    """A sheet whose faces are in no order, and with a triangle 10^5 times its size away.  21 bits per axis leave
+    the sheet 21 cells along each side: 18 clusters of faces in each, instead of one, at the places of the 9
+    around it.  A search that finds no order in the sheet meets all 8,160 clusters for each."""
+    ctx = api.Context()
+    s = scenes.crumpled_sheet(512)
+    faces = np.random.default_rng(1).permutation(s["faces"]).astype(np.int32)
+    nv = len(s["qstart"])
+    far = 1e5 * np.ones(3) + np.array([[0.0, 0.0, 0.0], [1.0, 0.0, 0.0], [0.0, 1.0, 0.0]])
+    times = []
+    for f, extra in ((faces, far[:0]), (np.concatenate([faces, [[nv, nv + 1, nv + 2]]]).astype(np.int32), far)):
+        qs, qe = np.concatenate([s["qstart"], extra]), np.concatenate([s["qend"], extra])
+        times.append(_stage_ms(ctx, N.TIMER_NAMES.index("traverse"),
+                               lambda: api.kdop_candidates(f, qs, qe, 1e-7, sort=False, as_numpy=False, ctx=ctx)))
+        print("case: a shuffled sheet,", len(extra) // 3, "bodies far away, search ms", times[-1], flush=True)
+    assert times[1] < 60.0 * times[0]
