@@ -2243,6 +2243,16 @@ CCD_HD int separating_plane_nodes(const Histories &hist, double eta, double eps,
     }
 }
 
+// Whether a stencil's features are closer than the thickness.
+template <bool VF>
+CCD_HD bool touching(const V3 (&q)[4], double eta)
+{
+    double b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+    const V3 d = VF ? vertex_face_distance(q[0], q[1], q[2], q[3], b0, b1, b2)
+                    : edge_edge_distance(q[0], q[1], q[2], q[3], b0, b1, b2, b3);
+    return dot(d, d) < eta * eta;
+}
+
 // Windows that are tested later, in full wavefronts: store(s, e) keeps one that the screen leaves open, or says
 // that there is no room.  Testing a window at once would end the recursion at the first that collides; here it
 // ends where the closest distance at a window's start, middle or end is below the thickness, since that window
@@ -2263,10 +2273,7 @@ struct DeferredWindows {
         for (int k = 0; k < 3 && !ended; k++) {
             V3 q[4];
             for (int j = 0; j < 4; j++) q[j] = k == 0 ? s[j] : (k == 1 ? e[j] : 0.5 * (s[j] + e[j]));
-            double b0 = 0, b1 = 0, b2 = 0, b3 = 0;
-            const V3 d = VF ? vertex_face_distance(q[0], q[1], q[2], q[3], b0, b1, b2)
-                            : edge_edge_distance(q[0], q[1], q[2], q[3], b0, b1, b2, b3);
-            ended = dot(d, d) < eta * eta;
+            ended = touching<VF>(q, eta);
         }
         return ended;
     }

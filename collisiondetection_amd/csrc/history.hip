@@ -12,7 +12,8 @@
 //     0.35 + 0.60 ms, 0.23 + 0.39 ms;
 //   separating plane, the cascade in the lane: 1.38 + 1.96 ms, 2.71 + 3.23 ms (a wavefront a stencil); here
 //     0.73 + 0.91 ms, 0.90 + 1.01 ms.
-// A pool that is too small costs time only: the last kernel runs its stencils from the start, a wavefront each.
+// A pool that is too small costs time only: the last kernel runs the stencils without room from the start, a
+// wavefront each.
 #include "narrow_common.h"
 #include <algorithm>
 
@@ -122,9 +123,14 @@ struct Stitch {
 };
 
 // A stencil's windows are walked through by 2^log_parts lanes, each those that start in one of as many equal spans
-// of time, 64 windows between two visits to the pool.  count[part]: its windows; best[stencil]: ~0, or 0 where
-// the pool had no room.
+// of time, 64 windows between two visits to the pool.  A lane stops after a window at whose end the features are
+// closer than the thickness: that window should collide, and later ones do not matter then.  (Walking on took
+// 24.8 ms, and testing the windows at once 2.2 ms, for 8,600 stencils of each kind over 60 entries that nearly all
+// collide; here 1.7.)
+// count[part]: its windows; best[stencil]: the least of ~0 and, where a part stopped or the pool had no room, the
+// place after which its windows are not known, with 0 for the place in the pool.
 constexpr int PLACE_BITS = 20;   // a window's place: part << PLACE_BITS | number in the part
+constexpr uint32_t LAST_PLACE = (1u << PLACE_BITS) - 1;
 template <bool VF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_hist_open(
     const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
@@ -146,25 +152,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         if (now < until && now <= 1.0) next = s.at(now, prev);
     }
     int w = 0;
-    bool lost = false;
-    while (__ballot(now < until && next <= 1.0)) {
+    bool stopped = false;
+    uint32_t unknown = 0;   // where `stopped`: the place from which the part's windows are not known
+    while (__ballot(!stopped && now < until && next <= 1.0)) {
         const double first = now;
         const int w0 = w;
         uint64_t open = 0;
-        for (; now < until && next <= 1.0 && w < w0 + 64; w++) {
+        for (; !stopped && now < until && next <= 1.0 && w < w0 + 64; w++) {
             const double after = s.at(next, cur);
-            if (VF ? ccd::screen_vf_window(prev, cur, et) : ccd::screen_ee_window(prev, cur, et)) open |= 1ull << (w - w0);
+            if (VF ? ccd::screen_vf_window(prev, cur, et) : ccd::screen_ee_window(prev, cur, et)) {
+                open |= 1ull << (w - w0);
+                stopped = ccd::touching<VF>(cur, et);
+                unknown = LAST_PLACE;
+            }
 #pragma unroll
             for (int j = 0; j < 4; j++) prev[j] = cur[j];
             now = next;
             next = after;
         }
-        if (w > 1 << PLACE_BITS) lost = true;
-        const int need = lost ? 0 : __popcll(open);
+        const bool room = w <= 1 << PLACE_BITS;
+        const int need = room ? __popcll(open) : 0;
         int64_t at = claim(pool, (int)(blockIdx.x & (WindowPool::SHARDS - 1)), need);
-        if (need == 0) continue;
-        if (at < 0) {
-            lost = true;
+        if (open == 0) continue;
+        if (at < 0 || !room) {
+            stopped = true;
+            unknown = (uint32_t)w0 < LAST_PLACE ? (uint32_t)w0 : LAST_PLACE;
             continue;
         }
         // Once more, to the windows to be kept.
@@ -182,7 +194,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     }
     if (!mine) return;
     count[x] = w;
-    if (lost) best[i] = 0;
+    if (stopped) atomicMin(&best[i], (unsigned long long)((uint32_t)g << PLACE_BITS | unknown) << 32);
 }
 // The first window, in time, that collides: its place and where it lies in the pool.
 __global__ __launch_bounds__(64) void k_hist_hits(WindowPool pool, unsigned long long *__restrict__ best)
@@ -237,15 +249,17 @@ template <bool VF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_hist_result(
     const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
     const int4 *__restrict__ keys, const double *__restrict__ eta, double eta_s, int64_t n, int log_parts,
-    const int32_t *__restrict__ count, const unsigned long long *__restrict__ best, WindowPool pool, uint8_t *__restrict__ hit,
-    double *__restrict__ tout, uint8_t *__restrict__ sub, int32_t *__restrict__ win)
+    const int32_t *__restrict__ count, const unsigned long long *__restrict__ best, WindowPool pool, int share,
+    uint8_t *__restrict__ hit, double *__restrict__ tout, uint8_t *__restrict__ sub, int32_t *__restrict__ win)
 {
     const int lane = __lane_id();
-    const int64_t i0 = blockIdx.x * (int64_t)64, i = i0 + lane;
-    const unsigned long long found = i < n ? best[i] : ~0ull;
+    const int64_t i0 = (int64_t)(blockIdx.x / share) * 64, i = i0 + lane;
+    const bool mine = i < n && lane % share == (int)(blockIdx.x % share);
+    const unsigned long long found = mine ? best[i] : ~0ull;
     int r = -1, w = 0;
     double t = 0.0;
-    if (found != ~0ull && (uint32_t)found != 0) {
+    const bool again = (uint32_t)found == 0;   // (a place in the pool is above 0, no window at all ~0)
+    if (found != ~0ull && !again) {
         const int64_t at = (int64_t)(uint32_t)found - 1;
         const uint32_t place = (uint32_t)(found >> 32);
         r = pool.sub[at];
@@ -254,7 +268,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
         if (win)
             for (uint32_t g = 0; g < place >> PLACE_BITS; g++) w += count[(i << log_parts) + g];
     }
-    for (uint64_t lost = __ballot(found == 0); lost; lost &= lost - 1) {
+    for (uint64_t lost = __ballot(again); lost; lost &= lost - 1) {
         const int l = __ffsll((unsigned long long)lost) - 1;
         int rr, ww = 0;
         double tt = 0.0;
@@ -265,7 +279,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
             w = ww;
         }
     }
-    if (i >= n) return;
+    if (!mine) return;
     hit[i] = r >= 0 ? 1 : 0;
     if (tout) tout[i] = r >= 0 ? t : 0.0;
     if (sub) sub[i] = r >= 0 ? (uint8_t)r : (uint8_t)255;
@@ -509,11 +523,11 @@ template <bool VF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_sp_result(
     const int64_t *__restrict__ off, const double *__restrict__ ht, const double *__restrict__ hp,
     const int4 *__restrict__ keys, const double *__restrict__ eta, double eta_s, int64_t n,
-    const unsigned long long *__restrict__ gap_bits, uint8_t *__restrict__ status, unsigned long long *undecided)
+    const unsigned long long *__restrict__ gap_bits, int share, uint8_t *__restrict__ status, unsigned long long *undecided)
 {
     const int lane = __lane_id();
-    const int64_t i0 = blockIdx.x * (int64_t)64, i = i0 + lane;
-    int r = i < n ? status[i] : 0;
+    const int64_t i0 = (int64_t)(blockIdx.x / share) * 64, i = i0 + lane;
+    int r = i < n && lane % share == (int)(blockIdx.x % share) ? status[i] : 0;
     const double eps = ccd::bits_to_double((long long)*gap_bits) / 4.0;
     for (uint64_t lost = __ballot(r == ccd::SP_LOST || r == ccd::SP_RUN_AGAIN); lost; lost &= lost - 1) {   // by the whole wavefront
         const int l = __ffsll((unsigned long long)lost) - 1;
@@ -563,6 +577,15 @@ static int window_pool(ccd_ctx *ctx, int64_t n, WindowPool &p, void *&list)
     return fill_u64(ctx, (uint64_t *)p.claimed, WindowPool::SHARDS * WindowPool::STRIDE, 0);
 }
 
+// Wavefronts that share 64 stencils in the last kernels, each its part of those to be run again: as many as there
+// are places for on the chip, since nearly all of a call's stencils may be such.
+static int result_share(int64_t n)
+{
+    int share = 64;
+    while (share > 1 && n * share > 1 << 18) share /= 2;
+    return share;
+}
+
 // Stencils to a set of launches: bounds the scratch memory and the grids.
 constexpr int64_t PIECE = 1 << 22;
 
@@ -594,8 +617,9 @@ static int narrow_hist_piece(ccd_ctx *ctx, bool vf, const int64_t *off, const do
                        best);
     CCD_LAUNCH_CHECK(ctx);
     auto k_result = vf ? k_hist_result<true> : k_hist_result<false>;
-    hipLaunchKernelGGL(k_result, dim3(blocks_for(n, 64)), dim3(64), 0, ctx->stream, off, ht, hp, (const int4 *)keys, eta,
-                       eta_s, n, log_parts, count, best, pool, hit, t, sub, win);
+    const int share = result_share(n);
+    hipLaunchKernelGGL(k_result, dim3(blocks_for(n, 64) * share), dim3(64), 0, ctx->stream, off, ht, hp, (const int4 *)keys, eta,
+                       eta_s, n, log_parts, count, best, pool, share, hit, t, sub, win);
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }
@@ -657,8 +681,9 @@ static int separating_plane_piece(ccd_ctx *ctx, bool vf, const int64_t *off, con
                        status);
     CCD_LAUNCH_CHECK(ctx);
     auto k_result = vf ? k_sp_result<true> : k_sp_result<false>;
-    hipLaunchKernelGGL(k_result, dim3(blocks_for(n, 64)), dim3(64), 0, ctx->stream, off, ht, hp, (const int4 *)keys, eta,
-                       eta_s, n, gb, status, (unsigned long long *)undecided);
+    const int share = result_share(n);
+    hipLaunchKernelGGL(k_result, dim3(blocks_for(n, 64) * share), dim3(64), 0, ctx->stream, off, ht, hp, (const int4 *)keys, eta,
+                       eta_s, n, gb, share, status, (unsigned long long *)undecided);
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }

@@ -58,3 +58,31 @@ def test_search_with_a_body_far_away():
                                lambda: api.kdop_candidates(f, qs, qe, 1e-7, sort=False, as_numpy=False, ctx=ctx)))
         print("case: a shuffled sheet,", len(extra) // 3, "bodies far away, search ms", times[-1], flush=True)
     assert times[1] < 60.0 * times[0]
+
+
+def test_histories_that_nearly_all_collide():
+    """Stencils that are closer than the thickness all the time take no more than a few times what those take that
+    hardly ever are: their first windows decide them."""
+    import time
+
+    import torch
+
+    rng = np.random.default_rng(3)
+    V, entries, n = 40, 60, 8600
+    t = [np.concatenate([[0], np.sort(rng.choice(np.arange(1, 1024), size=entries - 2, replace=False)), [1024]]) for _ in range(V)]
+    hist = [np.arange(V + 1, dtype=np.int64) * entries, np.concatenate(t) / 1024.0,
+            np.repeat(rng.uniform(size=(V, 3)), entries, axis=0) + rng.normal(0.0, 0.005, size=(V * entries, 3))]
+    keys = np.stack([rng.permutation(V)[:4] for _ in range(n)]).astype(np.int32)
+    args = [torch.from_numpy(a).cuda() for a in (*hist, keys, keys)]
+    times, hits = [], []
+    for eta in (1e-6, 2.0):
+        best = np.inf
+        for _ in range(4):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            r = api.narrowphase_history(*args, eta)
+            best = min(best, time.perf_counter() - t0)
+        times.append(best)
+        hits.append(r["vf_hit"].mean())
+        print("case: histories, thickness", eta, "ms", 1e3 * best, "collide", hits[-1], flush=True)
+    assert hits[0] < 0.05 and hits[1] > 0.95 and times[1] < 4.0 * times[0]
