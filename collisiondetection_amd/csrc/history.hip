@@ -556,15 +556,21 @@ inline unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) /
 
 namespace ccdi {
 
-// A pool for the windows of n stencils, and its lists.  One window per stencil, within limits: most stencils
-// need none, and the positions take 192 bytes a window.
-static int window_pool(ccd_ctx *ctx, int64_t n, WindowPool &p, void *&list)
+// A pool for the windows of n stencils, and its lists (223 bytes a window, and half a megabyte).  All the windows
+// of the stencils on short lists, one per stencil on long ones: most stencils need none.  Without memory for that,
+// half as many, and so on: the pool's size changes no result.
+static int window_pool(ccd_ctx *ctx, int64_t n, int64_t windows, WindowPool &p, void *&list)
 {
-    constexpr int64_t LEAST = 1 << 18, MOST = 1 << 22;
-    const int64_t cap = (std::min(std::max(n, LEAST), MOST) + 4095) / 4096 * 4096;
-    char *b = (char *)buffer(ctx, "window_pool", (size_t)cap * (192 + 8 + 8 + 4 + 4 + 1 + 1) + WindowPool::SHARDS * WindowPool::STRIDE * 8);
-    list = open_list(ctx, cap);
-    if (!b || !list) return CCD_E_OOM;
+    constexpr int64_t FEW = 1 << 14, ENOUGH = 1 << 19, MOST = 1 << 22, STEP = 4096;
+    int64_t cap = std::max(std::min(std::max(windows * n, FEW), ENOUGH), std::min(n, MOST));
+    char *b = nullptr;
+    for (;; cap /= 2) {
+        cap = (cap + STEP - 1) / STEP * STEP;
+        b = (char *)buffer(ctx, "window_pool", (size_t)cap * (192 + 8 + 8 + 4 + 4 + 1 + 1) + WindowPool::SHARDS * WindowPool::STRIDE * 8);
+        list = b ? open_list(ctx, cap) : nullptr;
+        if (list) break;
+        if (cap == STEP) return CCD_E_OOM;
+    }
     p.pos = (double *)b;
     p.eta = p.pos + 24 * cap;
     p.t = p.eta + cap;
@@ -600,7 +606,7 @@ static int narrow_hist_piece(ccd_ctx *ctx, bool vf, const int64_t *off, const do
     const int64_t nparts = n << log_parts;
     WindowPool pool;
     void *list;
-    int rc = window_pool(ctx, n, pool, list);
+    int rc = window_pool(ctx, n, 4 * entries, pool, list);
     if (rc) return rc;
     unsigned long long *best = (unsigned long long *)buffer(ctx, "hist_best", (size_t)n * 8);
     int32_t *count = (int32_t *)buffer(ctx, "hist_count", (size_t)nparts * 4);
@@ -649,7 +655,7 @@ static int separating_plane_piece(ccd_ctx *ctx, bool vf, const int64_t *off, con
     const int lanes = entries <= 2 ? 1 : (entries <= 8 ? 8 : 64);
     WindowPool pool;
     void *list;
-    int rc = window_pool(ctx, n, pool, list);
+    int rc = window_pool(ctx, n, 16, pool, list);   // (a recursion ends after a window or two)
     if (rc) return rc;
     const int32_t *order = nullptr;
     const uint64_t *open = nullptr;

@@ -125,6 +125,9 @@ int ccd_ctcd_narrowphase_noalloc(ccd_ctx *ctx, const double *qstart, const doubl
  * (device): vertex v owns entries hist_off[v] .. hist_off[v+1]-1 with times hist_t[] (the first 0,
  * the last 1, nondecreasing) and positions hist_pos[3*e ..].  t is local to the window that fired
  * (window index in win, may be NULL), as the reference's CTCD calls see it.
+ * This call and ccd_separating_plane_narrowphase gather windows in memory that the context keeps: 4 MB for few
+ * stencils, 0.12 GB for many windows, up to 0.94 GB from 4.2M stencils on, and a quarter more as headroom.  Where
+ * the device has less they do with less, down to 2 MB, and take longer.
  */
 int ccd_ctcd_narrowphase_history(ccd_ctx *ctx, const int64_t *hist_off, const double *hist_t,
                                  const double *hist_pos, int64_t nverts, int64_t nentries, const int32_t *vf_keys,
