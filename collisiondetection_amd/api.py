@@ -583,6 +583,9 @@ class VelocityFilter:
 # ------------------------------------------------------------------------------------------------
 # Batched instances
 # ------------------------------------------------------------------------------------------------
+TUNED_KERNELS = "screen+refine+solve"   # the narrowphase's form that a stored shape was tuned for
+
+
 class Batch:
     """Independent meshes packed for ccd_batch_detect: faces with global vertex indices, face offsets
     per instance and vertex offsets (to map results back)."""
@@ -623,16 +626,16 @@ class Batch:
     def tune(self, outer_eta, eta, cache=None):
         """Tune the narrowphase (its shape per kind) on this batch's
         candidates and install the result on the batch's context.  With `cache` (a JSON file path) the
-        shape stored there for this workload shape (GPU architecture and compute units, faces, vertices,
-        instances) is installed
-        instead, and a newly tuned shape is stored.  Returns (shape, 'cache' or 'tuned')."""
+        shape stored there for these kernels and this workload shape (GPU architecture and compute units, faces,
+        vertices, instances) is installed instead, and a newly tuned shape is stored.  Returns (shape, 'cache' or 'tuned')."""
         import json
         import os
 
         torch = _torch()
         props = torch.cuda.get_device_properties(self.ctx.torch_device)
         arch = (getattr(props, "gcnArchName", "") or props.name).split(":")[0]
-        key = f"{arch}|cus={props.multi_processor_count}|faces={self.F}|verts={self.V}|instances={self.ninst}"
+        key = (f"{TUNED_KERNELS}|{arch}|cus={props.multi_processor_count}|faces={self.F}|verts={self.V}|"
+               f"instances={self.ninst}")
         table = {}
         if cache and os.path.exists(cache):
             with open(cache) as fh:

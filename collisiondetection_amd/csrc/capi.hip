@@ -717,6 +717,7 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
     const int blocks[3] = {64, 128, 256};
     const int tiles[7] = {64, 128, 256, 512, 1024, 2048, 4096};
     const int waves[4] = {4, 8, 12, 16};
+    const QueueShape usual;
     int64_t nmax[2] = {ctx->last_nvf, ctx->last_nee};
     const int32_t *keys[2] = {ctx->last_vf, ctx->last_ee};
     int32_t *sink = (int32_t *)buffer(ctx, "tune_sink", 16 * 4096 + 64);
@@ -728,15 +729,18 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
     hipEvent_t e0, e1;
     CCD_HIP_CHECK(ctx, hipEventCreate(&e0));
     CCD_HIP_CHECK(ctx, hipEventCreate(&e1));
-    // Milliseconds of `launch` on the context's stream: the second of two runs (the first warms caches).
-    auto timed = [&](auto &&launch, float &ms) -> int {
-        for (int rep = 0; rep < 2; rep++) {
+    // Milliseconds of `launch` on the context's stream: the least of `reps` runs after one that warms caches.
+    auto timed = [&](auto &&launch, int reps, float &ms) -> int {
+        ms = 1e30f;
+        for (int rep = 0; rep <= reps; rep++) {
             CCD_HIP_CHECK(ctx, hipEventRecord(e0, st));
             int rc = launch();
             if (rc) return rc;
             CCD_HIP_CHECK(ctx, hipEventRecord(e1, st));
             CCD_HIP_CHECK(ctx, hipEventSynchronize(e1));
-            CCD_HIP_CHECK(ctx, hipEventElapsedTime(&ms, e0, e1));
+            float once = 0.f;
+            CCD_HIP_CHECK(ctx, hipEventElapsedTime(&once, e0, e1));
+            if (rep > 0) ms = std::min(ms, once);
         }
         return CCD_OK;
     };
@@ -757,15 +761,18 @@ int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double 
         if (nmax[kind] == 0) continue;
         CCD_HIP_CHECK(ctx, hipMemcpyAsync(ndev, &nmax[kind], 8, hipMemcpyHostToDevice, st));
         float best_ms = 1e30f;
+        // The screening form has a tile only; block and waves_per_cu stay as they are for the one-pass form then.
+        const bool screened = list && nmax[kind] <= 0x7fffffffll && (kind == 0 || ctx->ee_split);
         for (int b : blocks)
             for (int t : tiles)
                 for (int w : waves) {
+                    if (screened && (b != usual.block || w != usual.waves_per_cu)) continue;
                     QueueShape s;
                     s.block = b;
                     s.tile = t;
                     s.waves_per_cu = w;
                     float ms = 0.f;
-                    int rc = timed(queue(kind, keys[kind], s), ms);
+                    int rc = timed(queue(kind, keys[kind], s), screened ? 5 : 1, ms);
                     if (rc) return rc;
                     if (ms < best_ms) {
                         best_ms = ms;

@@ -296,12 +296,11 @@ int ccd_batch_detect(ccd_ctx *ctx, int64_t ninst, const int64_t *inst_face_off, 
 
 /*
  * Tuning of the narrowphase: times it on the candidates of the last detection on this context over
- * block sizes {64, 128, 256}, tiles {64, 128, ..., 4096} and {4, 8, 12, 16} resident wavefronts per CU;
- * keeps the fastest per stencil kind and returns it in shape[0..7] = {vf block, vf tile, vf waves/CU,
- * ee block, ee tile, ee waves/CU, vf grouping, ee grouping} (host, may be NULL).  The tile bounds the
- * stencils that a wavefront of the screening passes takes; block and waves/CU matter to the one-pass form
- * only; grouping (1 or 0) is accepted and has no effect.  ccd_set_queue_shape installs such
- * a shape (e.g. one cached from an earlier tuning run).
+ * tiles {64, 128, ..., 4096} and, where the one-pass form runs, block sizes {64, 128, 256} and {4, 8, 12, 16}
+ * resident wavefronts per CU; keeps the fastest per stencil kind and returns it in shape[0..7] = {vf block,
+ * vf tile, vf waves/CU, ee block, ee tile, ee waves/CU, vf grouping, ee grouping} (host, may be NULL).  The tile
+ * bounds the stencils that a wavefront of the screening passes takes; grouping (1 or 0) is accepted and has no
+ * effect.  ccd_set_queue_shape installs such a shape (e.g. one cached from an earlier tuning run).
  */
 int ccd_autotune(ccd_ctx *ctx, const double *qstart, const double *qend, double eta, int *shape);
 int ccd_set_queue_shape(ccd_ctx *ctx, const int *shape);
