@@ -903,9 +903,9 @@ __global__ __launch_bounds__(256) void k_edges(const int4 *__restrict__ sfaces, 
 // A feature whose rows name more clusters than the table takes goes through it several times, each time
 // with one class of the clusters, by the upper bits of a hash.  The edge rule may ask for a face of another
 // class; whether that is related to the edge's faces is decided again from the bounds.  (Looking it up in
-// their rows, which are as long as what they hold, and starting with one class took 1009 ms for a detection of a
-// 256^2 cloth over a ground of two triangles, quadratic in the faces; here 23 ms, 16 of them the ground's features,
-// 0.8 us for 64 faces.)
+// their rows, which are as long as what they hold, took 1009 ms for a detection of a 256^2 cloth over a ground
+// of two triangles, quadratic in the faces; here 26 ms, 20 of them the ground's features, about a microsecond for
+// 64 faces.)
 constexpr int UNION_BLOCK = 256;
 constexpr int TABLE_SLOTS = 512;
 struct UnionTable {
@@ -952,11 +952,13 @@ __device__ __forceinline__ uint32_t hash32(uint32_t x)
     x *= 0x85EBCA6Bu;
     return x ^ (x >> 16);
 }
-// ORs a tile into a table of `last` + 1 slots (a power of two); false when there is no room.
+// ORs a tile into a table of `last` + 1 slots (a power of two); false when there is no room near its place (a full
+// table searched from end to end by tile after tile took longer than the pass that fits).
+constexpr uint32_t MOST_PROBES = 128;
 __device__ __forceinline__ bool table_or(UnionTable &T, uint32_t last, uint32_t cluster, uint64_t mask)
 {
     uint32_t h = hash32(cluster) & last;
-    for (uint32_t probe = 0; probe <= last; probe++) {
+    for (uint32_t probe = 0; probe <= last && probe < MOST_PROBES; probe++) {
         const uint32_t old = atomicCAS(&T.cluster[h], ~0u, cluster);
         if (old == ~0u || old == cluster) {
             atomicOr(&T.mask[h], (unsigned long long)mask);
@@ -1010,11 +1012,16 @@ __device__ __forceinline__ bool related(const MeshView &m, int r, int j)
 // j related to the leaf f0 or f1, or (f1 -2) to one of the faces around u0 that hold u1.
 __device__ bool edge_related(const MeshView &m, int f0, int f1, int u0, int u1, int j)
 {
-    if (f1 != -2) return related(m, f0, j) || (f1 >= 0 && related(m, f1, j));
-    for (int k = m.vf_off[u0]; k < m.vf_off[u0 + 1]; k++) {
-        const int f = m.vf_list[k];
-        const int32_t *v = m.faces + 3 * (int64_t)f;
-        if ((v[0] == u1 || v[1] == u1 || v[2] == u1) && related(m, m.rank[f], j)) return true;
+    const int star = m.vf_off[u0], n = f1 == -2 ? m.vf_off[u0 + 1] - star : (f1 == -1 ? 1 : 2);
+    for (int k = 0; k < n; k++) {
+        int r = k == 0 ? f0 : f1;
+        if (f1 == -2) {
+            const int f = m.vf_list[star + k];
+            const int32_t *v = m.faces + 3 * (int64_t)f;
+            if (v[0] != u1 && v[1] != u1 && v[2] != u1) continue;
+            r = m.rank[f];
+        }
+        if (related(m, r, j)) return true;
     }
     return false;
 }
@@ -1095,10 +1102,7 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
         room = room > 0 ? room : 0;
         int4 *const keys = (edge ? ee_out : vf_out) + first;
         int64_t found = 0;   // stencils so far
-        // Classes of clusters: 2^bits, by the hash's upper bits.  (A row names a cluster once, so an edge has at least
-        // so many.)
-        int bits = 0;
-        while ((l0 > l1 ? l0 : l1) >> bits > TABLE_SLOTS * 3 / 4) bits++;
+        int bits = 0;        // classes of clusters: 2^bits, by the hash's upper bits
         uint32_t slots = TABLE_SLOTS;
         for (uint32_t cls = 0; cls < (1u << bits); cls++) {
             bool over = false;
@@ -1115,17 +1119,17 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
             auto add = [&](int64_t at) {
                 const uint32_t t = (uint32_t)m.rows.cluster[at];
                 const uint64_t mask = m.rows.mask[at];
-                if (bits == 0 || hash32(t) >> (32 - bits) == cls) over |= !table_or(T, slots - 1, t, mask);
+                if (!over && (bits == 0 || hash32(t) >> (32 - bits) == cls)) over = !table_or(T, slots - 1, t, mask);
             };
             if (fn == 0) {
                 clear(l0 + l1);
-                for (int e0 = 0; e0 < l0 + l1 && !__ballot(over); e0 += 64) {
+                for (int e0 = 0; e0 < l0 + l1; e0 += 64) {
                     const int e = e0 + lane;
                     if (e < l0 + l1) add(e < l0 ? s0 + e : s1 + (e - l0));
                 }
             } else {
                 if (fn > 64) clear(TABLE_SLOTS);
-                for (int k0 = 0; k0 < fn && !__ballot(over); k0 += 64) {
+                for (int k0 = 0; k0 < fn; k0 += 64) {
                     const int at0 = fstar + k0, k = fn - k0 < 64 ? fn - k0 : 64;
                     if (at0 < wbase || at0 + k > wbase + 64) {
                         wbase = at0;
@@ -1143,7 +1147,7 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
                     if (fn <= 64) clear(all);
                     int steps = 1;
                     while (steps < k) steps <<= 1;
-                    for (int e0 = 0; e0 < all && !__ballot(over); e0 += 64) {
+                    for (int e0 = 0; e0 < all; e0 += 64) {
                         const int e = e0 + lane;
                         int row = a;   // the row that holds entry e: the first whose inclusive sum exceeds it
                         for (int d = steps >> 1; d > 0; d >>= 1) {
@@ -1158,7 +1162,7 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
                 }
             }
             wave_lds_order();
-            if (__ballot(over)) {   // start again with twice the classes (2^23 of them have at most 512 clusters each)
+            if (__ballot(over)) {   // start again with twice the classes (the clusters of one of 2^23 have a slot each)
                 bits++;
                 found = 0;
                 cls = ~0u;
@@ -1191,7 +1195,7 @@ __global__ __launch_bounds__(UNION_BLOCK) void k_union(MeshView m, int64_t F, in
                         // The number comes from another face: it has the edge if it is in the union.
                         const int owner = (int)(E.edge[w] / 3u);
                         auto has = [&](int j) {
-                            if (bits == 0 || hash32((uint32_t)j >> 6) >> (32 - bits) == cls) return table_has(T, slots - 1, j);
+                            if (bits == 0) return table_has(T, slots - 1, j);
                             return edge_related(m, (int)(h / 3u), m.edges[h / 3u].other[h % 3u], a0, a1, j);
                         };
                         bool in = has(owner);
