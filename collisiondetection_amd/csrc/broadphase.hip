@@ -1328,8 +1328,6 @@ struct KeyEq {
     }
 };
 
-__global__ void k_copy_count(const unsigned long long *src, int64_t *dst) { *dst = (int64_t)*src; }
-
 }   // namespace
 
 namespace ccdi {

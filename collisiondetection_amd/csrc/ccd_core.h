@@ -139,13 +139,14 @@ struct NoCount {
 struct FullCascade {
     CCD_FHD void operator()(int) const {}
 };
-// A counter type for a screening run of the edge-edge test: it screens the coplanar-distance sextic and
-// solves nothing (the host's model of a two-pass schedule; the device screens with screen_ee_window).  find_intervals on the sextic decides only the case
-// "full degree, and no root in [0, 1] by the Bernstein test" (couldHaveRoots false, or no sign change
-// of the Bernstein coefficients with every one clear of zero), where the list is the one piece [0, 1]
-// or nothing, as the isolator gives it; any other sextic sets `deferred`.  edge_edge then returns
-// false at once, and also sets `deferred` when the sextic leaves a coplanar interval.  So a stencil
-// the screen does not defer has no edge-edge collision, exactly as the full test finds.
+// A counter type for a screening run of the edge-edge test by the sextic alone, a host's model of a two-pass
+// schedule with no use on the device (which screens with screen_ee_window): it screens the coplanar-distance
+// sextic and solves nothing.  find_intervals on the sextic decides only the case "full degree, and no root in
+// [0, 1] by the Bernstein test" (couldHaveRoots false, or no sign change of the Bernstein coefficients with every
+// one clear of zero), where the list is the one piece [0, 1] or nothing, as the isolator gives it; any other
+// sextic sets `deferred`.  edge_edge then returns false at once, and also sets `deferred` when the sextic leaves a
+// coplanar interval.  So a stencil the screen does not defer has no edge-edge collision, exactly as the full
+// test finds.
 struct ScreenSextic {
     bool deferred = false;
     CCD_FHD void operator()(int) const {}
@@ -155,14 +156,6 @@ struct prunes : std::integral_constant<bool, std::is_same<std::decay_t<C>, NoCou
                                                  std::is_same<std::decay_t<C>, ScreenSextic>::value> {};
 template <class C>
 struct screens_sextic : std::integral_constant<bool, std::is_same<std::decay_t<C>, ScreenSextic>::value> {};
-// A counter type whose `stops_at_solver` member is true makes find_intervals return, with no intervals,
-// where it would call the root solver.  SolverProbe records whether that point was reached; the
-// stencil-ordering pre-pass uses it to see which polynomials need the solver.
-template <class C, class = void>
-struct stops_at_solver : std::false_type {};
-template <class C>
-struct stops_at_solver<C, std::void_t<decltype(C::stops_at_solver)>> : std::integral_constant<bool, C::stops_at_solver> {};
-
 // A counter type whose `plain_roots` member is true isolates roots without the Bernstein shortcuts and
 // with plain safeguarded Newton (bisection fallback, plain Horner values): the work-accounting kernel.
 template <class C, class = void>
@@ -753,7 +746,6 @@ CCD_HD void find_intervals(double *op, Ivls<CAP> &out, bool pos, C &&cnt = C())
             return;
         }
         cnt(S_ISOLATE);
-        if constexpr (stops_at_solver<CT>::value) return;
         roots = isolate_roots<N, NT, plain_roots<CT>::value>(op, reduced, time);
         // Pieces between consecutive roots (all in [0,1], ascending) and the ends, as CTCD.cpp:160-176.
         set_cuts(roots);
@@ -1136,73 +1128,6 @@ CCD_HD bool ve_sides(V3 q0s, V3 q1s, V3 q2s, V3 q0e, V3 q1e, V3 q2e, Ivls<3> &e1
     cnt(S_VE_QUAD);
     find_intervals<2>(op, e2, true, cnt);
     return !e2.empty();
-}
-
-// Which vertex-edge sub-tests of a stencil's window would reach their quartic (both side quadratics
-// non-empty and overlapping): bit j for the j-th vertex-edge test in the reference's order.  Cheap
-// (closed-form quadratics only).
-struct SolverProbe {
-    static constexpr bool stops_at_solver = true;
-    bool called = false;
-    CCD_FHD void operator()(int stage)
-    {
-        if (stage == S_ISOLATE) called = true;
-    }
-};
-
-// Which of the polynomials of a window's face or edge-edge test would reach the root solver, each
-// evaluated whether or not the test would get that far (vertexFaceCTCD's / edgeEdgeCTCD's arguments for
-// check_vf_window's / check_ee_window's vertex order).  Vertex-face: the three edge-side cubics (bits
-// 0-2) and the coplanar-distance sextic (bit 3).  Edge-edge: the coplanar-distance sextic (bit 0) and
-// how many of the four barycentric quartics (bits 1-3).  A sort key only.
-CCD_HD unsigned first_phase_signature(bool vf, const V3 *s, const V3 *e, double eta)
-{
-    const V3 v0 = e[0] - s[0], v1 = e[1] - s[1], v2 = e[2] - s[2], v3 = e[3] - s[3];
-    if (vf) {
-        Ivls<4> iv;
-        Ivls<7> iv7;
-        SolverProbe p0, p1, p2, p3;
-        plane_poly(s[0] - s[1], cross(s[3] - s[1], s[2] - s[1]), s[3] - s[1], v0 - v1, cross(v3 - v1, v2 - v1), v3 - v1,
-                   iv, p0);
-        plane_poly(s[0] - s[2], cross(s[1] - s[2], s[3] - s[2]), s[1] - s[2], v0 - v2, cross(v1 - v2, v3 - v2), v1 - v2,
-                   iv, p1);
-        plane_poly(s[0] - s[3], cross(s[2] - s[3], s[1] - s[3]), s[2] - s[3], v0 - v3, cross(v2 - v3, v1 - v3), v2 - v3,
-                   iv, p2);
-        distance_poly(s[0] - s[1], s[2] - s[1], s[3] - s[1], v0 - v1, v2 - v1, v3 - v1, eta * eta, iv7, p3);
-        return (p0.called ? 1u : 0u) | (p1.called ? 2u : 0u) | (p2.called ? 4u : 0u) | (p3.called ? 8u : 0u);
-    }
-    // edgeEdgeCTCD(q0 = s[0], p0 = s[1], q1 = s[2], p1 = s[3])
-    Ivls<7> iv7;
-    Ivls<5> iv5;
-    SolverProbe pd, pa0, pa1, pb0, pb1;
-    distance_poly(s[1] - s[3], s[1] - s[0], s[3] - s[2], v1 - v3, v1 - v0, v3 - v2, eta * eta, iv7, pd);
-    barycentric_poly(s[3] - s[2], s[1] - s[0], s[0] - s[2], v3 - v2, v1 - v0, v0 - v2, iv5, pa0);
-    barycentric_poly(s[3] - s[2], s[0] - s[1], s[1] - s[2], v3 - v2, v0 - v1, v1 - v2, iv5, pa1);
-    barycentric_poly(s[1] - s[0], s[3] - s[2], s[2] - s[0], v1 - v0, v3 - v2, v2 - v0, iv5, pb0);
-    barycentric_poly(s[1] - s[0], s[2] - s[3], s[3] - s[0], v1 - v0, v2 - v3, v3 - v0, iv5, pb1);
-    const unsigned nb = (pa0.called ? 1u : 0u) + (pa1.called ? 1u : 0u) + (pb0.called ? 1u : 0u) + (pb1.called ? 1u : 0u);
-    return (pd.called ? 1u : 0u) | (nb << 1);
-}
-
-CCD_HD unsigned ve_signature(bool vf, const V3 *s, const V3 *e)
-{
-    unsigned sig = 0;
-    NoCount nc;
-    auto bit = [&](int j, int a, int b, int c) {
-        Ivls<3> e1, e2;
-        if (ve_sides(s[a], s[b], s[c], e[a], e[b], e[c], e1, e2, nc) && any_overlap(e1, ~0u, e2)) sig |= 1u << j;
-    };
-    if (vf) {   // check_vf_window's order
-        bit(0, 0, 1, 2);
-        bit(1, 0, 2, 3);
-        bit(2, 0, 3, 1);
-    } else {    // check_ee_window's order
-        bit(0, 0, 2, 3);
-        bit(1, 1, 2, 3);
-        bit(2, 2, 0, 1);
-        bit(3, 3, 0, 1);
-    }
-    return sig;
 }
 
 // vertexEdgeCTCD (CTCD.cpp:511-602): vertex q0 and edge (q1,q2).
@@ -1665,7 +1590,7 @@ CCD_FHD void refine_part(const Poly<D> &p, double m, double a, double h, unsigne
     const bool neg = max_of(b) < -tol;
     const bool clean = (min_of(b) > tol) | (strictly_monotone(b, slope) & (dabs(b[0]) > tol) & (dabs(b[D]) > tol));
     r.parts |= neg ? bit : 0u;
-    r.unclean |= neg | clean ? 0u : bit;
+    r.unclean |= (neg | clean) ? 0u : bit;
 }
 
 // The distance sextic as its cubic d, |n|^2 and the size of the terms of its coefficients.
@@ -1702,7 +1627,7 @@ CCD_FHD void refine_part(const DistancePoly &p, double minD, double a, double h,
     const bool dips = strictly_monotone(b, slope) & ((b[0] < 0.0) != (b[3] < 0.0)) & (b[0] * b[0] > far) & (b[3] * b[3] > far) &
                       (minD * min_of(g) > tol);
     r.parts |= positive ? bit : 0u;
-    r.unclean |= positive | dips ? 0u : bit;
+    r.unclean |= (positive | dips) ? 0u : bit;
 }
 
 // Whether a stencil's face or edge-edge test cannot hit.
