@@ -1,0 +1,90 @@
+"""Both sides of the sizes at which the detection changes its way: the levels of the pair search (512 records are
+scanned from end to end), the screened narrowphase (4,096 stencils), its coarse refinement (128 open stencils in a
+region)."""
+import numpy as np
+import pytest
+
+import oracle
+from collisiondetection_amd import api, scenes
+from tests.helpers import core_narrowphase
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("F", [511 * 64, 511 * 64 + 1, 512 * 64, 512 * 64 + 1])
+def test_pairs_at_the_second_level(F):
+    rng = np.random.default_rng(F)
+    size = 0.3 / F ** (1 / 3)
+    q = rng.uniform(size=(F, 1, 3)) + rng.uniform(-size, size, size=(F, 3, 3))
+    qs, qe = q.reshape(-1, 3), (q + rng.normal(0.0, 0.3 * size, size=q.shape)).reshape(-1, 3)
+    faces = np.arange(3 * F, dtype=np.int32).reshape(F, 3)
+    vf, ee = api.kdop_candidates(faces, qs, qe, 1e-4)
+    ovf, oee = oracle.candidates(faces, oracle.Hist.two_entry(qs, qe), 1e-4, method="tree")
+    np.testing.assert_array_equal(vf, ovf)
+    np.testing.assert_array_equal(ee, oee)
+    assert len(vf) > 0
+
+
+@pytest.mark.parametrize("F", [512 * 64 * 64, 512 * 64 * 64 + 1])
+def test_pairs_at_the_third_level(F):
+    """A lattice of far-apart small triangles with planted pairs, the last triangle in one of them."""
+    i = np.arange(F)
+    c = np.stack([i % 128, i // 128 % 128, i // 16384], axis=1).astype(np.float64)
+    q = c[:, None, :] + np.array([[0.0, 0.0, 0.0], [0.1, 0.0, 0.0], [0.0, 0.1, 0.05]])[None]
+    rng = np.random.default_rng(F)
+    a = rng.choice(F // 2, size=500, replace=False)
+    b = F // 2 + rng.choice(F // 2 - 1, size=500, replace=False)
+    b[0] = F - 1
+    q[b] = q[a] + 0.01
+    faces = np.arange(3 * F, dtype=np.int32).reshape(F, 3)
+    vf, _ = api.kdop_candidates(faces, q.reshape(-1, 3), q.reshape(-1, 3), 1e-6)
+    pairs = {(int(r[0]) // 3, int(r[1]) // 3) for r in vf}
+    assert pairs == {(int(x), int(y)) for x, y in zip(a, b)} | {(int(y), int(x)) for x, y in zip(a, b)}
+
+
+def _check(r, pre, hit, t, sub):
+    np.testing.assert_array_equal(r[pre + "_hit"], hit)
+    np.testing.assert_array_equal(r[pre + "_t"].view(np.int64), t.view(np.int64))
+    np.testing.assert_array_equal(np.where(hit, r[pre + "_sub"], 0), np.where(hit, sub, 0))
+
+
+@pytest.fixture(scope="module")
+def contact(core_harness):
+    """A cloth's candidates with what the host-built core finds: {is_ee: (keys, hit, t, sub)}."""
+    s = scenes.cloth(64, drop=0.05, noise=0.01)
+    eta = 2e-3
+    sets = oracle.candidates(s["faces"], oracle.Hist.two_entry(s["qstart"], s["qend"]), eta, method="tree")
+    return s, eta, {is_ee: (keys, *core_narrowphase(core_harness, s["qstart"], s["qend"], keys, is_ee, eta))
+                    for keys, is_ee in zip(sets, (False, True))}
+
+
+@pytest.mark.parametrize("n", [4095, 4096, 4097])
+def test_narrowphase_at_the_screen(contact, n):
+    s, eta, sets = contact
+    rng = np.random.default_rng(n)
+    pick = {is_ee: rng.choice(len(x[0]), size=n, replace=False) for is_ee, x in sets.items()}
+    r = api.narrowphase(s["qstart"], s["qend"], sets[False][0][pick[False]], sets[True][0][pick[True]], eta)
+    for is_ee, pre in ((False, "vf"), (True, "ee")):
+        _check(r, pre, *(x[pick[is_ee]] for x in sets[is_ee][1:]))
+        assert r[pre + "_hit"].any()
+
+
+@pytest.mark.parametrize("first_test", [True, False])
+def test_narrowphase_at_the_coarse_refinement(contact, first_test):
+    """2^20 stencils make regions of 256: each with 127, 128 or 129 that hit by their first sub-test (or by a later
+    one, which is open in the other list) among some that are far apart."""
+    s, eta, sets = contact
+    n, region = 1 << 20, 256
+    rng = np.random.default_rng(first_test)
+    far = np.concatenate([s["qstart"], s["qstart"] + 100.0]), np.concatenate([s["qend"], s["qend"] + 100.0])
+    pick, keys = {}, {}
+    opened = np.arange(region)[None, :] < (127 + np.arange(n // region) % 3)[:, None]
+    opened = rng.permuted(opened, axis=1).reshape(-1)
+    for is_ee, (k, hit, t, sub) in sets.items():
+        pick[is_ee] = rng.choice(np.nonzero(hit & ((sub == 0) == first_test))[0], size=n)
+        keys[is_ee] = k[pick[is_ee]].copy()
+        keys[is_ee][~opened, 2 if is_ee else 1:] += len(s["qstart"])   # the second feature goes far away
+    r = api.narrowphase(*far, keys[False], keys[True], eta)
+    for is_ee, pre in ((False, "vf"), (True, "ee")):
+        hit, t, sub = (x[pick[is_ee]] for x in sets[is_ee][1:])
+        _check(r, pre, hit & opened, np.where(opened, t, 0.0), sub)
