@@ -86,3 +86,17 @@ def test_histories_that_nearly_all_collide():
         hits.append(r["vf_hit"].mean())
         print("case: histories, thickness", eta, "ms", 1e3 * best, "collide", hits[-1], flush=True)
     assert hits[0] < 0.05 and hits[1] > 0.95 and times[1] < 4.0 * times[0]
+
+
+def test_expansion_of_a_mesh_with_a_degenerate_face():
+    """One degenerate face sends the whole mesh to the raw emission: fifteen stencils of every pair instead of each
+    stencil once, a few times the keys, and no more than ten times the time."""
+    ctx = api.Context()
+    s = scenes.cloth(256)
+    times = []
+    for faces in (s["faces"], np.concatenate([s["faces"], [[0, 0, 1]]]).astype(np.int32)):
+        times.append(_stage_ms(ctx, N.TIMER_NAMES.index("expand"),
+                               lambda: api.kdop_candidates(faces, s["qstart"], s["qend"], s["eta"], sort=False, as_numpy=False,
+                                                           ctx=ctx)))
+        print("case: cloth with", len(faces) - len(s["faces"]), "degenerate faces, expansion ms", times[-1], flush=True)
+    assert times[1] < 10.0 * times[0]
