@@ -11,8 +11,8 @@
 
 #include "../../include/ccd_amd.h"
 
-// Launch shape of the narrowphase (tuned by ccd_autotune).  The screening form uses the tile; block and
-// waves_per_cu shape the persistent grid of the one-pass form.
+// Launch shape of the narrowphase (tuned by ccd_autotune).  Both forms use the tile; block and waves_per_cu shape
+// the persistent grid of the one-pass form.
 struct QueueShape {
     int block = 256;       // threads per block: 64, 128 or 256
     int tile = 1024;       // stencils a wavefront takes at a time (fewer on short lists)

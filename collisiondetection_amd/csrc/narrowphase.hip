@@ -239,17 +239,21 @@ int launch_narrow2_queue(ccd_ctx *ctx, bool vf, const double *qs, const double *
         o.counter = (unsigned long long *)counter;
         return launch_screened(ctx, vf, false, qs, qe, keys, n_dev, n_max, eta, o, shape.tile, list);
     }
-    const int64_t need = (n_max + shape.tile - 1) / shape.tile;
-    const int64_t waves = std::max<int64_t>(1, std::min((int64_t)ctx->num_cus * shape.waves_per_cu, need));
+    // Sixteen turns of the queue for each resident wavefront if there are so many chunks of 64: a wavefront's turns are
+    // of very uneven length (87,000 edge-edge stencils by 1,024 at a time, 85 turns in all: 2.16 ms; by 64: 0.20).
+    const int64_t resident = (int64_t)ctx->num_cus * shape.waves_per_cu;
+    const int tile = (int)std::max<int64_t>(64, std::min<int64_t>(shape.tile, n_max / (16 * resident) / 64 * 64));
+    const int64_t need = (n_max + tile - 1) / tile;
+    const int64_t waves = std::max<int64_t>(1, std::min(resident, need));
     const unsigned grid = (unsigned)((waves * 64 + shape.block - 1) / shape.block);
     if (vf)
         CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_narrow2_queue<true, M>), dim3(grid), dim3(shape.block), 0, ctx->stream, qs,
                                               qe, (const int4 *)keys, n_dev, n_max, eta, (int4 *)out_keys, out_toi, cap,
-                                              (unsigned long long *)counter, work, shape.tile));
+                                              (unsigned long long *)counter, work, tile));
     else
         CCD_PRODUCT_LAUNCH(hipLaunchKernelGGL((k_narrow2_queue<false, M>), dim3(grid), dim3(shape.block), 0, ctx->stream, qs,
                                               qe, (const int4 *)keys, n_dev, n_max, eta, (int4 *)out_keys, out_toi, cap,
-                                              (unsigned long long *)counter, work, shape.tile));
+                                              (unsigned long long *)counter, work, tile));
     CCD_LAUNCH_CHECK(ctx);
     return CCD_OK;
 }

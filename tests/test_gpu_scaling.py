@@ -100,3 +100,17 @@ def test_expansion_of_a_mesh_with_a_degenerate_face():
                                                            ctx=ctx)))
         print("case: cloth with", len(faces) - len(s["faces"]), "degenerate faces, expansion ms", times[-1], flush=True)
     assert times[1] < 10.0 * times[0]
+
+
+def test_one_pass_narrowphase_of_a_short_list():
+    """87,000 edge-edge stencils in one pass with the solver, on all wavefronts: no more than four times the three
+    passes, which run the solver on a tenth of them."""
+    s = scenes.cloth(97)
+    times = []
+    for on in (True, False):
+        ctx = api.Context()
+        api.set_edge_edge_split(on, ctx)
+        times.append(_stage_ms(ctx, N.TIMER_NAMES.index("narrow_ee"),
+                               lambda: api.detect(s["faces"], s["qstart"], s["qend"], s["eta"], s["eta"], ctx=ctx)))
+        print("case: edge-edge narrowphase,", "three passes" if on else "one pass", "ms", times[-1], flush=True)
+    assert times[1] < 4.0 * times[0]
