@@ -197,14 +197,19 @@ int launch_primitives(ccd_ctx *ctx, int kind, const double *q, const double *eta
     return CCD_OK;
 }
 
-// Stencils from which the per-stencil narrowphase is screened: below, one lane per stencil in one launch.
-constexpr int64_t SCREEN_MIN = 4096;
+// The per-stencil narrowphase is screened where its stencils are more than the lanes that k_narrow2 keeps resident
+// (two wavefronts per SIMD: 131,072 on 256 compute units).  Below, all of them run at once, and the launch takes as long
+// as its slowest lane, with or without a screen before it.  One launch against three, vertex-face / edge-edge, us:
+//   256^2 cloth: 139 / 209 against 124 / 182 for 4,096 stencils, 152 / 228 against 171 / 246 for 65,536, 177 / 281 against
+//     202 / 308 for 131,072, 317 / 483 against 254 / 424 for 262,144;
+//   256^2 sheet: 24 / 95 against 39 / 104, 59 / 103 against 69 / 131, 67 / 132 against 95 / 181, 88 / 232 against 93 / 233.
+constexpr int64_t RESIDENT_LANES_PER_CU = 4 * 2 * 64;
 
 int launch_narrow2(ccd_ctx *ctx, bool vf, const double *qs, const double *qe, const int32_t *keys,
                    const double *eta, double eta_s, int64_t n, uint8_t *hit, double *t, uint8_t *sub, void *list)
 {
     if (n == 0) return CCD_OK;
-    if (n >= SCREEN_MIN && n <= 0x7fffffffll) {   // (the screening form counts stencils in 31 bits)
+    if (n > RESIDENT_LANES_PER_CU * ctx->num_cus && n <= 0x7fffffffll) {   // (the screening form counts stencils in 31 bits)
         if (!list) list = open_list(ctx, n);
         if (!list) return CCD_E_OOM;
         NarrowOut o;

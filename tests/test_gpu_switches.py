@@ -1,6 +1,6 @@
 """Both sides of the sizes at which the detection changes its way: the levels of the pair search (512 records are
-scanned from end to end), the screened narrowphase (4,096 stencils), its coarse refinement (128 open stencils in a
-region)."""
+scanned from end to end), the screened narrowphase (131,072 stencils on 256 compute units), its coarse refinement
+(128 open stencils in a region)."""
 import numpy as np
 import pytest
 
@@ -58,11 +58,11 @@ def contact(core_harness):
                     for keys, is_ee in zip(sets, (False, True))}
 
 
-@pytest.mark.parametrize("n", [4095, 4096, 4097])
+@pytest.mark.parametrize("n", [4096, 131071, 131072, 131073])
 def test_narrowphase_at_the_screen(contact, n):
     s, eta, sets = contact
     rng = np.random.default_rng(n)
-    pick = {is_ee: rng.choice(len(x[0]), size=n, replace=False) for is_ee, x in sets.items()}
+    pick = {is_ee: rng.choice(len(x[0]), size=n) for is_ee, x in sets.items()}
     r = api.narrowphase(s["qstart"], s["qend"], sets[False][0][pick[False]], sets[True][0][pick[True]], eta)
     for is_ee, pre in ((False, "vf"), (True, "ee")):
         _check(r, pre, *(x[pick[is_ee]] for x in sets[is_ee][1:]))
