@@ -711,7 +711,7 @@ def set_edge_edge_split(on: bool, ctx: Context | None = None):
 # ------------------------------------------------------------------------------------------------
 class Server:
     """Device-resident sessions behind a continuous-batching request loop (ccd_server_* in
-    include/ccd_amd.h).  Sessions refit their tree per request; requests of different sessions
+    include/ccd_amd.h).  Sessions keep their Morton order from request to request; requests of different sessions
     overlap on the device."""
 
     def __init__(self, hbm_budget_bytes=8 << 30, max_inflight=8, device=0):

@@ -9,9 +9,9 @@
 // Times for 0.27M vertex-face and 0.47M edge-edge stencils over 4 entries per vertex, and for 15,000 and 26,000
 // over 48, vertex-face + edge-edge:
 //   stitched windows, the cascade in the lane: 0.59 + 1.59 ms, 1.00 + 1.96 ms (a wavefront a stencil); here
-//     0.35 + 0.60 ms, 0.23 + 0.39 ms;
+//     0.34 + 0.59 ms, 0.21 + 0.34 ms;
 //   separating plane, the cascade in the lane: 1.38 + 1.96 ms, 2.71 + 3.23 ms (a wavefront a stencil); here
-//     0.73 + 0.91 ms, 0.90 + 1.01 ms.
+//     0.81 + 0.98 ms, 0.89 + 1.04 ms.
 // A pool that is too small costs time only: the last kernel runs the stencils without room from the start, a
 // wavefront each.
 #include "narrow_common.h"

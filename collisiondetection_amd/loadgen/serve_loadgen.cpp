@@ -7,7 +7,7 @@
 // SESSIONS is a binary file: int64 count, then per session int64 F, int64 V, double eta, int32 faces[3F],
 // double positions[3V] (start = end = these).  Each request picks a session uniformly at random and
 // supplies new end positions = the session's previous end + N(0, sigma^2) per coordinate, a fresh draw
-// per request, so its tree is refit in place.  Requests are generated ahead of their arrival times by T
+// per request, so its Morton order is kept.  Requests are generated ahead of their arrival times by T
 // worker threads (each owns the sessions s with s % T == its index, so a session's requests form one
 // chain) and submitted by the main thread at their scheduled times.  Latency is measured from the
 // scheduled arrival to the result on the host.  The offer stops early when more than RATE * B requests
